@@ -114,11 +114,24 @@ int lvar_dense_attn_rcp_fwd(lvar_tensor_t q, lvar_tensor_t k, lvar_tensor_t v, l
                             float scale, void* stream);
 
 /*
+ * Row statistics alone: lse2[b,h,i] = log2(sum_n exp2(q_i.k_n*scale*log2e)), fp32 contiguous [B,H,Lq], the form the
+ * colsum entry point consumes (what lvar_dense_attn_fwd writes to LSE2, without the product with v).  scratch, if not
+ * NULL and at least lvar_row_lse_scratch_bytes() long, lets the launch cut the keys into ranges where the query rows
+ * alone do not fill the chip; its contents are written and read by this call only.
+ */
+int64_t lvar_row_lse_scratch_bytes(int B, int H, int Lq, int Lk);
+int lvar_row_lse_fwd(lvar_tensor_t q, lvar_tensor_t k, float* lse2, void* scratch, int64_t scratch_bytes,
+                     int B, int H, int kv_heads, int Lq, int Lk, int head_dim, float scale, void* stream);
+
+/* lse2 = M + log2(L) of `rows` contiguous fp32 statistics, as a dense pass returns them. */
+int lvar_lse2_from_stats(const float* M, const float* L, float* lse2, int64_t rows, void* stream);
+
+/*
  * Colsum given the row statistics: cs[b,h,g,n] = sum_{i in group g} exp2(q_i.k_n*scale*log2e - lse2_i),
  * lse2 = M + log2(L) (fp32 contiguous [B,H,Lq], as written by lvar_dense_attn_fwd), groups of
  * q_group_size consecutive query rows (a multiple of 32), rows >= Lq add zero.
  * cs is fp32 contiguous [B,H,G,Lk], G = ceil(Lq/q_group_size); every element is written exactly once
- * (no atomics, no pre-zeroing, deterministic).  block_sums, if not NULL, receives the sums of cs over
+ * (no atomics, no pre-zeroing, deterministic); cs may be NULL when block_sums is given.  block_sums, if not NULL, receives the sums of cs over
  * blocks of 64 consecutive keys, fp32 contiguous [B,H,G,ceil(Lk/64)] (ragged last block).
  * Replaces pass 2 of _full_attn_fwd (kernels/sparse_attn/triton/attn_dense_colsum.py:216-231)
  * and torch.ops.chipmunk.dense_colsum_attn (kernels/chipmunk/csrc/chipmunk.cu:58,

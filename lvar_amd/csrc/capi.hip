@@ -103,6 +103,8 @@ static int dense_common(lvar_tensor_t q, lvar_tensor_t k, lvar_tensor_t v, lvar_
   if (!kv_span_ok(k, Lk, head_dim) || (!lse_only && !kv_span_ok(v, Lk, head_dim))) return LVAR_EINVAL;
   if (!lse_only && (!view_ok(v) || !view_ok(o) || o.stride_row <= 0)) return LVAR_EINVAL;
   if (lse_only && !((M && L) || LSE2 || RCP)) return LVAR_EINVAL;
+  if (lse_only && !M && !L && !RCP)   // the row statistic alone has a kernel of its own
+    return lvar_row_lse_fwd(q, k, LSE2, nullptr, 0, B, H, kv_heads, Lq, Lk, head_dim, scale, stream);
   AttnParams p{};
   fill_qkv(p, q, k, lse_only ? k : v);
   p.o = (bf16_t*)o.ptr; p.o_sb = o.stride_b; p.o_sh = o.stride_h; p.o_sr = o.stride_row;
@@ -131,9 +133,35 @@ int lvar_dense_attn_rcp_fwd(lvar_tensor_t q, lvar_tensor_t k, lvar_tensor_t v, l
   return dense_common(q, k, v, o, nullptr, nullptr, nullptr, rcp, B, H, kv_heads, Lq, Lk, head_dim, scale, nullptr, stream);
 }
 
+int64_t lvar_row_lse_scratch_bytes(int B, int H, int Lq, int Lk) {
+  if (B <= 0 || H <= 0 || Lq <= 0 || Lk <= 0) return LVAR_EINVAL;
+  const int n = row_lse_splits(B, H, Lq, Lk);
+  return n > 1 ? 8ll * n * B * H * Lq : 0;
+}
+
+int lvar_row_lse_fwd(lvar_tensor_t q, lvar_tensor_t k, float* lse2, void* scratch, int64_t scratch_bytes,
+                     int B, int H, int kv_heads, int Lq, int Lk, int head_dim, float scale, void* stream) {
+  if (!shape_ok(B, H, Lq, Lk, scale) || !view_ok(q) || !view_ok(k) || !lse2) return LVAR_EINVAL;
+  if (kv_heads <= 0 || H % kv_heads != 0 || !kv_span_ok(k, Lk, head_dim)) return LVAR_EINVAL;
+  if (scratch && (reinterpret_cast<uintptr_t>(scratch) & 3u)) return LVAR_EINVAL;
+  RowLseParams p{};
+  p.q = (const bf16_t*)q.ptr; p.q_sb = q.stride_b; p.q_sh = q.stride_h; p.q_sr = q.stride_row;
+  p.k = (const bf16_t*)k.ptr; p.k_sb = k.stride_b; p.k_sh = k.stride_h; p.k_sr = k.stride_row;
+  p.lse2 = lse2;
+  p.B = B; p.H = H; p.Lq = Lq; p.Lk = Lk; p.kv_group = H / kv_heads;
+  p.c = scale * kLog2e;
+  p.part = (scratch && scratch_bytes >= lvar_row_lse_scratch_bytes(B, H, Lq, Lk)) ? (float*)scratch : nullptr;
+  return launch_row_lse(p, head_dim, (hipStream_t)stream);
+}
+
+int lvar_lse2_from_stats(const float* M, const float* L, float* lse2, int64_t rows, void* stream) {
+  if (!M || !L || !lse2 || rows <= 0) return LVAR_EINVAL;
+  return launch_lse2_from_stats(M, L, lse2, rows, (hipStream_t)stream);
+}
+
 int lvar_colsum_fwd(lvar_tensor_t q, lvar_tensor_t k, const float* lse2, float* cs, float* block_sums,
                     int B, int H, int kv_heads, int Lq, int Lk, int head_dim, int q_group_size, float scale, void* stream) {
-  if (!shape_ok(B, H, Lq, Lk, scale) || !view_ok(q) || !view_ok(k) || !lse2 || !cs) return LVAR_EINVAL;
+  if (!shape_ok(B, H, Lq, Lk, scale) || !view_ok(q) || !view_ok(k) || !lse2 || (!cs && !block_sums)) return LVAR_EINVAL;
   if (kv_heads <= 0 || H % kv_heads != 0) return LVAR_EINVAL;
   if (q_group_size <= 0 || q_group_size % 32 != 0) return LVAR_EINVAL;
   if (!kv_span_ok(q, Lq, head_dim, 0)) return LVAR_EINVAL;

@@ -125,7 +125,7 @@ __global__ __launch_bounds__(256, (D <= 128 ? 2 : 1)) void colsum_kernel(const C
     }
   };
 
-  float* csp = p.cs + ((int64_t)b * p.H + h) * p.G * (int64_t)p.Lk;
+  float* csp = p.cs ? p.cs + ((int64_t)b * p.H + h) * p.G * (int64_t)p.Lk : nullptr;
   float* bsp = p.bs ? p.bs + ((int64_t)b * p.H + h) * p.G * (int64_t)p.nkb : nullptr;
   // store the finished column sums of group g and reset the accumulators
   auto flush = [&](int g, float (&acc)[2]) {
@@ -135,7 +135,7 @@ __global__ __launch_bounds__(256, (D <= 128 ? 2 : 1)) void colsum_kernel(const C
       const float tot = xhalf_sum(acc[nt]);
       const int key = n0 + nt * 32 + r;
       const bool ok = key < p.Lk;
-      if (hh == 0 && ok) csp[(int64_t)g * p.Lk + key] = tot;
+      if (csp && hh == 0 && ok) csp[(int64_t)g * p.Lk + key] = tot;
       blk += ok ? tot : 0.f;
       acc[nt] = 0.f;
     }

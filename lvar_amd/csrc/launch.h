@@ -53,7 +53,7 @@ struct AttnParams {
 struct ColsumParams {
   const bf16_t *q, *k;
   const float* lse2;  // base-2 log-sum-exp per query row, M + log2(L)
-  float* cs;
+  float* cs;          // [B,H,G,Lk], or null when only the block sums are wanted
   float* bs;          // optional per-64-key block sums [B,H,G,ceil(Lk/64)]
   int64_t q_sb, q_sh, q_sr;
   int64_t k_sb, k_sh, k_sr;
@@ -63,6 +63,20 @@ struct ColsumParams {
   float c;
   int nkt, nkb, total_wg;
   int q_splits, split_rows;   // ranges of query groups per key tile, rows per range (set at launch)
+};
+
+constexpr int ROW_LSE_MAX_SPLITS = 8;   // key ranges of the row-statistics kernel
+
+struct RowLseParams {
+  const bf16_t *q, *k;
+  float* lse2;        // [B,H,Lq]
+  float* part;        // optional scratch: 2 * splits * B*H*Lq floats (null = one key range)
+  int64_t q_sb, q_sh, q_sr;
+  int64_t k_sb, k_sh, k_sr;
+  int B, H, Lq, Lk;
+  int kv_group;       // query heads per key head
+  float c;
+  int nrt, splits, split_keys, total_wg;   // set at launch
 };
 
 struct MaskListParams {
@@ -127,6 +141,9 @@ int launch_remap_concat_lists(const RemapListParams& p, hipStream_t s);
 int launch_mask_to_lists(const MaskCompactParams& p, hipStream_t s);
 int launch_block_topk_lists(const MaskListParams& p, hipStream_t s);
 int launch_attn(const AttnParams& p, int head_dim, int mode, bool accum, bool lse_only, int nwaves, hipStream_t s);
+int launch_row_lse(const RowLseParams& p, int head_dim, hipStream_t s);
+int launch_lse2_from_stats(const float* M, const float* L, float* lse2, int64_t rows, hipStream_t s);
+int row_lse_splits(int B, int H, int Lq, int Lk);   // key ranges that the row-statistics launch takes when it is given scratch
 int launch_colsum(const ColsumParams& p, int head_dim, hipStream_t s);
 int sk_slot_floats(int head_dim, int mode, int nwaves);
 int sk_plan(int total_wg, int nwaves, int slot_floats, int64_t per_tile, int sub, int64_t ws_bytes, int& min_share, int& min_piece);

@@ -311,8 +311,10 @@ def video_window_topk_block_lists(q: torch.Tensor, k: torch.Tensor, scale=None, 
         raise ValueError("block / query_stride must be a multiple of 32 (the colsum group size)")
     nK = (Lk + block - 1) // block
     base = video_window_base_mask(frames, height, width, block, device=q.device)
-    cs = ops.colsum(q[:, :, ::query_stride].contiguous(), k, scale, q_group_size=block // query_stride)
-    score = key_block_sums(cs, block).contiguous()
-    del cs
+    rows = q[:, :, ::query_stride]
+    if block % 64 == 0 and q.shape[-1] >= 64:      # block sums straight from the colsum kernel
+        score = ops._colsum_block_scores(rows, k, scale, block // query_stride, block)
+    else:
+        score = key_block_sums(ops.colsum(rows, k, scale, q_group_size=block // query_stride), block).contiguous()
     num, idx = ops.block_topk_lists(score, int(round(density * nK)), base)
     return num, idx, score

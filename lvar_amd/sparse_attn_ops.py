@@ -209,17 +209,37 @@ def dense_attn(q, k, v, scale=None):
 
 def _lse_only(q, k, scale):
     """Statistics sweep without the PV product: base-2 log-sum-exp ``M + log2(L)``, fp32 [B,H,Lq]."""
-    return _dense_launch(q, k, None, scale, want_o=False, want_ml=False, want_lse2=True)[3]
+    B, H, Lq, d = q.shape
+    Lk = k.shape[2]
+    lse2 = torch.empty((B, H, Lq), dtype=torch.float32, device=q.device)
+    lib = _lib.load()
+    with _on_device(q):
+        nbytes = int(lib.lvar_row_lse_scratch_bytes(B, H, Lq, Lk))
+        scratch = torch.empty(nbytes, dtype=torch.uint8, device=q.device) if nbytes > 0 else None
+        st = lib.lvar_row_lse_fwd(_view(q), _view(k), lse2.data_ptr(), _ptr(scratch), nbytes,
+                                  B, H, k.shape[1], Lq, Lk, d, _scale(q, scale), _stream(q))
+    _lib.check(st, "lvar_row_lse_fwd")
+    return lse2
 
 
-def _colsum_given_lse(q, k, lse2, scale, q_group_size, want_block_sums=False):
+def _lse2_of(lse, shape):
+    """Base-2 log-sum-exp ``M + log2(L)`` of the statistics ``(M, L)`` of a dense pass, fp32 of ``shape``."""
+    M, L = (t.to(torch.float32).contiguous() for t in lse)
+    out = torch.empty(shape, dtype=torch.float32, device=M.device)
+    with _on_device(M):
+        st = _lib.load().lvar_lse2_from_stats(M.data_ptr(), L.data_ptr(), out.data_ptr(), out.numel(), _stream(M))
+    _lib.check(st, "lvar_lse2_from_stats")
+    return out
+
+
+def _colsum_given_lse(q, k, lse2, scale, q_group_size, want_block_sums=False, want_columns=True):
     B, H, Lq, d = q.shape
     Lk = k.shape[2]
     G = (Lq + q_group_size - 1) // q_group_size
-    cs = torch.empty((B, H, G, Lk), dtype=torch.float32, device=q.device)
+    cs = torch.empty((B, H, G, Lk), dtype=torch.float32, device=q.device) if want_columns else None
     bs = torch.empty((B, H, G, (Lk + 63) // 64), dtype=torch.float32, device=q.device) if want_block_sums else None
     with _on_device(q):
-        st = _lib.load().lvar_colsum_fwd(_view(q), _view(k), lse2.data_ptr(), cs.data_ptr(), _ptr(bs),
+        st = _lib.load().lvar_colsum_fwd(_view(q), _view(k), lse2.data_ptr(), _ptr(cs), _ptr(bs),
                                         B, H, k.shape[1], Lq, Lk, d, q_group_size, _scale(q, scale), _stream(q))
     _lib.check(st, "lvar_colsum_fwd")
     return (cs, bs) if want_block_sums else cs
@@ -244,8 +264,21 @@ def colsum(q, k, scale=None, q_group_size: Optional[int] = None, lse: Optional[T
     else:
         M, L = lse
         _require(M.numel() == q.shape[0] * q.shape[1] * q.shape[2] == L.numel(), "lse must be ([B,H,Lq,1], [B,H,Lq,1])")
-        lse2 = (M.to(torch.float32) + torch.log2(L.to(torch.float32))).reshape(q.shape[:3]).contiguous()
+        _require(M.device == q.device and L.device == q.device, "lse must be on q's device")
+        lse2 = _lse2_of(lse, tuple(q.shape[:3]))
     return _colsum_given_lse(q, k, lse2, scale, q_group_size, return_block_sums)
+
+
+def _colsum_block_scores(q, k, scale, q_group_size: int, block_k: int):
+    """Column sums summed over blocks of ``block_k`` keys (a multiple of 64), ``[B,H,G,ceil(Lk/block_k)]``, without the
+    column sums themselves going to memory (self-contained two-pass form)."""
+    q, k = _prep(q, "q"), _prep(k, "k")
+    _check_qkv(q, k, k, gqa=True)
+    _, bs = _colsum_given_lse(q, k, _lse_only(q, k, scale), scale, q_group_size, want_block_sums=True, want_columns=False)
+    m = block_k // 64
+    if m == 1:
+        return bs
+    return torch.nn.functional.pad(bs, (0, -bs.shape[-1] % m)).unflatten(-1, (-1, m)).sum(-1)
 
 
 def dense_colsum_attn(q, k, v, scale=None):
