@@ -131,7 +131,8 @@ int lvar_lse2_from_stats(const float* M, const float* L, float* lse2, int64_t ro
  * lse2 = M + log2(L) (fp32 contiguous [B,H,Lq], as written by lvar_dense_attn_fwd), groups of
  * q_group_size consecutive query rows (a multiple of 32), rows >= Lq add zero.
  * cs is fp32 contiguous [B,H,G,Lk], G = ceil(Lq/q_group_size); every element is written exactly once
- * (no atomics, no pre-zeroing, deterministic); cs may be NULL when block_sums is given.  block_sums, if not NULL, receives the sums of cs over
+ * (no atomics, no pre-zeroing, deterministic); cs may be NULL when block_sums is given (the block sums are
+ * then added as ((x0 + x1) + x2) + x3 over fours of keys and a binary tree over the fours).  block_sums, if not NULL, receives the sums of cs over
  * blocks of 64 consecutive keys, fp32 contiguous [B,H,G,ceil(Lk/64)] (ragged last block).
  * Replaces pass 2 of _full_attn_fwd (kernels/sparse_attn/triton/attn_dense_colsum.py:216-231)
  * and torch.ops.chipmunk.dense_colsum_attn (kernels/chipmunk/csrc/chipmunk.cu:58,
@@ -289,6 +290,15 @@ int lvar_block_topk_lists(const float* block_scores, const uint8_t* base_mask,
 int lvar_topk_token_lists(const float* scores, int64_t score_row_stride,
                           int32_t* indices, int64_t idx_row_stride, int32_t* counts,
                           int rows, int Lk, int k, int zero_to, void* stream);
+
+/*
+ * Selection merged with a given list: out[row, 0:k+n_listed] (int64, contiguous) are the columns of the k largest
+ * values of the row, as lvar_topk_token_lists selects them, and the n_listed columns listed[row, :] (int64 contiguous
+ * [rows, n_listed], any order), together in ascending order; a column that occurs several times is written as often.
+ * Listed columns are clamped to [0, Lk).  Rows of at most 16384 columns, at most 65535 listed columns.
+ */
+int lvar_topk_union_lists(const float* scores, int64_t score_row_stride, const int64_t* listed, int n_listed, int64_t* out,
+                          int rows, int Lk, int k, void* stream);
 
 /*
  * Sparse-step key list in one launch: for every (batch*head) slice bh < BH and query group g < Gk of

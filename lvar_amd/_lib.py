@@ -17,7 +17,7 @@ EXPORTED_SYMBOLS = (
     "lvar_block_sparse_attn_fwd",
     "lvar_attn_workspace_bytes", "lvar_attn_balanced_workgroups", "lvar_dense_attn_ws_fwd", "lvar_csp_attn_ws_fwd", "lvar_csp_attn_upsample_ws_fwd",
     "lvar_block_sparse_attn_ws_fwd", "lvar_block_sparse_attn_static_fwd",
-    "lvar_block_topk_lists", "lvar_topk_token_lists", "lvar_remap_concat_lists", "lvar_mask_to_lists",
+    "lvar_block_topk_lists", "lvar_topk_token_lists", "lvar_topk_union_lists", "lvar_remap_concat_lists", "lvar_mask_to_lists",
     "lvar_window_key_scores",
 )
 
@@ -93,6 +93,8 @@ def load() -> C.CDLL:
     lib.lvar_block_topk_lists.argtypes = [P, P, P, P, I, I, I, I, I, P]
     lib.lvar_topk_token_lists.restype = I
     lib.lvar_topk_token_lists.argtypes = [P, I64, P, I64, P, I, I, I, I, P]
+    lib.lvar_topk_union_lists.restype = I
+    lib.lvar_topk_union_lists.argtypes = [P, I64, P, I, P, I, I, I, P]
     lib.lvar_remap_concat_lists.restype = I
     lib.lvar_remap_concat_lists.argtypes = [P, I64, I, P, I64, I, P, I64, P, I, I, I, I, I, I, P]
     lib.lvar_mask_to_lists.restype = I
@@ -114,7 +116,7 @@ _binding = False      # False: not tried yet; None: not available
 def torch_binding():
     """The compiled torch binding (``_lvar_torch.so`` next to this file), bound to the loaded C-ABI library, or
     None when it is not built, does not load, or ``LVAR_AMD_NO_TORCH_BINDING`` is set.  It only shortens the
-    host side of ``dense_attn``; every call it declines goes through the ctypes path."""
+    host side of the operators; every call it declines goes through the ctypes path."""
     global _binding
     if _binding is not False:
         return _binding
@@ -129,12 +131,12 @@ def torch_binding():
         mod = importlib.util.module_from_spec(spec)
         spec.loader.exec_module(mod)
         lib = load()
-        mod.bind(C.cast(lib.lvar_dense_attn_fwd, C.c_void_p).value, C.cast(lib.lvar_dense_attn_rcp_fwd, C.c_void_p).value)
+        mod.bind([C.cast(getattr(lib, name), C.c_void_p).value for name in mod.entry_names()])
         _binding = mod
     except Exception as e:     # a stale or incompatible module must not take the ctypes path down with it
         import warnings
         warnings.warn(f"lvar_amd: the compiled torch binding {path} did not load ({type(e).__name__}: {e}); "
-                      "dense_attn runs through the slower ctypes path.  Rebuild it with `python -m lvar_amd.build`.",
+                      "the operators run through the slower ctypes path.  Rebuild it with `python -m lvar_amd.build`.",
                       RuntimeWarning, stacklevel=2)
         _binding = None
     return _binding

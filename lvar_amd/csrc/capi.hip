@@ -384,6 +384,17 @@ int lvar_topk_token_lists(const float* scores, int64_t score_row_stride, int32_t
   return launch_topk_token_lists(p, (hipStream_t)stream);
 }
 
+int lvar_topk_union_lists(const float* scores, int64_t score_row_stride, const int64_t* listed, int n_listed, int64_t* out,
+                          int rows, int Lk, int k, void* stream) {
+  if (!scores || !listed || !out || rows < 0 || Lk <= 0 || k <= 0 || k > Lk || score_row_stride < Lk || n_listed <= 0) return LVAR_EINVAL;
+  if (Lk > TOPK_UNION_MAX_N || n_listed > 65535) return LVAR_EUNSUPPORTED;
+  TopkListParams p{};
+  p.scores = scores; p.score_stride = score_row_stride;
+  p.more = listed; p.W = n_listed; p.out64 = out; p.out_stride = (int64_t)k + n_listed;
+  p.rows = rows; p.n = Lk; p.k = k;
+  return launch_topk_token_lists(p, (hipStream_t)stream);
+}
+
 int lvar_remap_concat_lists(const int32_t* src_indices, int64_t src_row_stride, int src_len,
                             const int64_t* local_indices, int64_t local_row_stride, int local_count,
                             int32_t* out_indices, int64_t out_row_stride, int32_t* out_counts,

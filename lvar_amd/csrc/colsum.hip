@@ -129,18 +129,22 @@ __global__ __launch_bounds__(256, (D <= 128 ? 2 : 1)) void colsum_kernel(const C
   float* bsp = p.bs ? p.bs + ((int64_t)b * p.H + h) * p.G * (int64_t)p.nkb : nullptr;
   // store the finished column sums of group g and reset the accumulators
   auto flush = [&](int g, float (&acc)[2]) {
-    float blk = 0.f;
+    float blk = 0.f, val[2];
 #pragma unroll
     for (int nt = 0; nt < 2; nt++) {
       const float tot = xhalf_sum(acc[nt]);
       const int key = n0 + nt * 32 + r;
       const bool ok = key < p.Lk;
       if (csp && hh == 0 && ok) csp[(int64_t)g * p.Lk + key] = tot;
-      blk += ok ? tot : 0.f;
+      val[nt] = ok ? tot : 0.f;
+      blk += val[nt];
       acc[nt] = 0.f;
     }
     if (bsp) {
-      blk = group_sum<32>(blk);
+      // Without the columns in memory the block sum is the caller's only view of them; it is then added up the way a
+      // reduction over the stored columns adds (four neighbours in sequence, then a tree over the fours), so that
+      // whoever ranks blocks gets the same ranking from either form.
+      blk = csp ? group_sum<32>(blk) : quad_tree_sum(val[0]) + quad_tree_sum(val[1]);
       if (lane == 0 && n0 < p.Lk) bsp[(int64_t)g * p.nkb + kblk] = blk;
     }
   };

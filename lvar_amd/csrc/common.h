@@ -62,6 +62,22 @@ __device__ __forceinline__ float group_sum(float x) {
   return x;
 }
 
+// Sum over aligned groups of 32 lanes in the order ((x0 + x1) + x2) + x3 inside fours of neighbours, then a binary tree
+// over the eight fours; every lane of a group receives the total.
+__device__ __forceinline__ float quad_tree_sum(float x) {
+  auto mv = [](float v, auto ctrl) {
+    return __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, v), decltype(ctrl)::value, 0xf, 0xf, true));
+  };
+  float t = mv(x, std::integral_constant<int, 0x00>{});   // quad_perm: lane 0 of the four to all of it, then 1, 2, 3
+  t += mv(x, std::integral_constant<int, 0x55>{});
+  t += mv(x, std::integral_constant<int, 0xAA>{});
+  t += mv(x, std::integral_constant<int, 0xFF>{});
+  t += mv(t, std::integral_constant<int, 0x141>{});       // row_half_mirror: the other four of eight lanes
+  t += mv(t, std::integral_constant<int, 0x140>{});       // row_mirror: the other eight of sixteen
+  t += __shfl_xor(t, 16, 64);
+  return t;
+}
+
 __device__ __forceinline__ uint32_t pack_bf16(float a, float b) {
   f32x2 f = {a, b};
   bf16x2 h = __builtin_convertvector(f, bf16x2);

@@ -94,7 +94,11 @@ struct TopkListParams {
   int64_t score_stride, out_stride;
   int rows, n, k;
   int zero_to;          // columns [k, zero_to) of every index row are set to 0 (0 = left untouched)
+  const int64_t* more;  // [rows, W] columns to merge with the selection, or null
+  int64_t* out64;       // [rows, k + W] with row stride out_stride: the merge (with `more` only)
+  int W;
 };
+constexpr int TOPK_UNION_MAX_N = 16384;   // longest row of the merging form
 
 struct RemapListParams {
   const int32_t* src;    // [BH, Gs, src_stride]

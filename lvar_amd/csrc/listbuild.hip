@@ -46,11 +46,16 @@ __device__ __forceinline__ uint32_t wave_umin(uint32_t v) {
 //   columns in ascending order (ballot compaction into an LDS ring, full-width stores).
 // ---------------------------------------------------------------------------------------------
 constexpr int TOPK_BINS = 2048;
+constexpr int TOPK_FEW_ROWS_PER_CU = 2;
 constexpr int TOPK_CAND = 256;   // keys of the first pass's bin that are resolved by direct comparison
 
-template <int KPT, int NT>
-__global__ __launch_bounds__(NT, (KPT >= 1 && KPT <= 24) ? 6 : 1) void topk_token_lists_kernel(const TopkListParams p) {
+// UNION: the output row is the ascending merge of the selection with the row's own list of W columns (in any order,
+// columns that are listed or selected several times come out as often), as int64.  How often each column is listed sits
+// in LDS as 16-bit counts, so a column's place in the merge is one more term of the scan that places the selection.
+template <int KPT, int NT, bool UNION>
+__global__ __launch_bounds__(NT, (KPT >= 1 && KPT <= 24) ? (NT == 512 ? 6 : 4) : 1) void topk_token_lists_kernel(const TopkListParams p) {
   constexpr int NW = NT / 64;
+  extern __shared__ uint32_t listed[];   // UNION: two 16-bit counts per word
   __shared__ int hist[TOPK_BINS];
   __shared__ __attribute__((aligned(16))) uint32_t cand[TOPK_CAND];
   __shared__ int wsum[NW];
@@ -67,6 +72,8 @@ __global__ __launch_bounds__(NT, (KPT >= 1 && KPT <= 24) ? 6 : 1) void topk_toke
   // columns [k, zero_to) of the list row: defined (zero) instead of whatever the buffer held
   for (int t = want + tid; t < p.zero_to; t += NT) out[t] = 0;
   if (want == 0) return;
+  if constexpr (UNION)
+    for (int t = tid; t < (n + 1) / 2; t += NT) listed[t] = 0u;
 
   // chunk c of wave w covers columns (w * cpw + c) * 64 .. +63
   const int cpw = KPT ? KPT : ((n + NT - 1) / NT);
@@ -121,6 +128,13 @@ __global__ __launch_bounds__(NT, (KPT >= 1 && KPT <= 24) ? 6 : 1) void topk_toke
   __syncthreads();
 #pragma unroll
   for (int w = 0; w < NW; w++) { kmax = max(kmax, (uint32_t)wgt[w]); kmin = min(kmin, (uint32_t)weq[w]); }
+  if constexpr (UNION) {   // (read behind at least one more barrier)
+    const int64_t* more = p.more + (int64_t)row * p.W;
+    for (int t = tid; t < p.W; t += NT) {
+      const int j = (int)max((int64_t)0, min((int64_t)n - 1, more[t]));
+      atomicAdd(&listed[j >> 1], 1u << (16 * (j & 1)));
+    }
+  }
   const int top = 32 - __builtin_clz((kmax ^ kmin) | 1u) + (((kmax ^ kmin) == 0u) ? -1 : 0);   // 0 when all keys are equal
   uint32_t pmask = (top >= 32) ? 0u : ~((1u << top) - 1u);
   uint32_t prefix = kmax & pmask;
@@ -206,11 +220,14 @@ __global__ __launch_bounds__(NT, (KPT >= 1 && KPT <= 24) ? 6 : 1) void topk_toke
   const uint32_t T = prefix;  // key of the k-th largest element
   const int need = want;      // selected keys equal to T (the first `need` of them by column)
 
-  int gt = 0, eq = 0;
+  int gt = 0, eq = 0, times = 0;
+  const uint16_t* listed16 = (const uint16_t*)listed;
   visit([&](int j, uint32_t key) {
     gt += __builtin_popcountll(__builtin_amdgcn_ballot_w64(key > T));
     eq += __builtin_popcountll(__builtin_amdgcn_ballot_w64(key == T));
+    if constexpr (UNION) times += j < n ? (int)listed16[j] : 0;
   });
+  if constexpr (UNION) gt += __builtin_amdgcn_readlane(wave_scan(times, 0, [](int a, int b) { return a + b; }), 63);
   if (lane == 0) { wgt[wave] = gt; weq[wave] = eq; }
   __syncthreads();
   int pos = 0, eq_before = 0;
@@ -219,6 +236,28 @@ __global__ __launch_bounds__(NT, (KPT >= 1 && KPT <= 24) ? 6 : 1) void topk_toke
     eq_before += weq[w];
   }
   int eq_left = max(0, need - eq_before);
+  if constexpr (UNION) {
+    int64_t* out64 = p.out64 + (int64_t)row * p.out_stride;
+    visit([&](int j, uint32_t key) {
+      unsigned long long bk = __builtin_amdgcn_ballot_w64(key > T);
+      const unsigned long long beq = __builtin_amdgcn_ballot_w64(key == T);
+      if (beq != 0ull && eq_left > 0) {
+        bk |= __builtin_amdgcn_ballot_w64(key == T && lanes_below(beq, lane) < eq_left);
+        eq_left = max(0, eq_left - __builtin_popcountll(beq));
+      }
+      const int mult = j < n ? (int)listed16[j] : 0;
+      const int mine = (int)((bk >> lane) & 1ull) + mult;
+      if (__builtin_amdgcn_ballot_w64(mult > 0) == 0ull) {
+        if (mine) out64[pos + lanes_below(bk, lane)] = j;
+        pos += __builtin_popcountll(bk);
+      } else {
+        const int incl = wave_scan(mine, 0, [](int a, int b) { return a + b; });
+        for (int e = 0; e < mine; e++) out64[pos + incl - mine + e] = j;
+        pos += __builtin_amdgcn_readlane(incl, 63);
+      }
+    });
+    return;
+  }
   // The selected columns of a wave are collected in a 128-entry ring in LDS (the histogram is no longer needed: the
   // barrier above lies between its last read and these writes) and leave in full 64-entry, 256-byte stores instead
   // of one partial store per chunk.  LDS operations of one wave complete in order, so the ring needs no barrier.
@@ -243,24 +282,34 @@ __global__ __launch_bounds__(NT, (KPT >= 1 && KPT <= 24) ? 6 : 1) void topk_toke
   if (lane < fill) out[pos + lane] = ring[(head + lane) & 127];
 }
 
-// Keys per thread: every value up to 24 (a row of n keys takes ceil(n / 512) of them: no pass walks more than one
+// Keys per thread: every value up to 24 (a row of n keys takes ceil(n / NT) of them: no pass walks more than one
 // chunk of padding per wave), then 28 and 32; longer rows are re-read from L2 in every pass.
-template <int KPT>
+template <int KPT, int NT, bool UNION>
 static bool topk_try(const TopkListParams& p, hipStream_t stream) {
-  if (p.n > 512 * KPT) return false;
-  hipLaunchKernelGGL((topk_token_lists_kernel<KPT, 512>), dim3(p.rows), dim3(512), 0, stream, p);
+  if (p.n > NT * KPT) return false;
+  hipLaunchKernelGGL((topk_token_lists_kernel<KPT, NT, UNION>), dim3(p.rows), dim3(NT), UNION ? (p.n + 1) / 2 * 4 : 0, stream, p);
   return true;
 }
-template <int... KPT>
+template <int NT, bool UNION, int... KPT>
 static bool topk_dispatch(const TopkListParams& p, hipStream_t stream, std::integer_sequence<int, KPT...>) {
-  return (topk_try<KPT + 1>(p, stream) || ...);
+  return (topk_try<KPT + 1, NT, UNION>(p, stream) || ...);
 }
 
 int launch_topk_token_lists(const TopkListParams& p, hipStream_t stream) {
   if (p.rows == 0) return LVAR_OK;
+  if (p.more) {
+    if (p.n > TOPK_UNION_MAX_N) return LVAR_EUNSUPPORTED;
+    topk_dispatch<1024, true>(p, stream, std::make_integer_sequence<int, TOPK_UNION_MAX_N / 1024>{});
+    return hipGetLastError() == hipSuccess ? LVAR_OK : LVAR_ELAUNCH;
+  }
+  // A row is a chain of short phases that end in a barrier.  With at most one row per compute unit and its neighbour
+  // half as many keys per thread shorten every phase; with more rows the 512-thread workgroups of several rows fill
+  // each other's gaps better.  (Rows of 512 keys and less have one key per thread either way.)
+  const bool few = p.rows <= TOPK_FEW_ROWS_PER_CU * device_cus() && p.n > 512 && p.n <= 16384;
+  if (few) topk_dispatch<1024, false>(p, stream, std::make_integer_sequence<int, 16>{});
   // 512 threads per row keep a row of up to 16384 keys in registers (KPT keys per thread)
-  if (!topk_dispatch(p, stream, std::make_integer_sequence<int, 24>{}) && !topk_try<28>(p, stream) && !topk_try<32>(p, stream))
-    hipLaunchKernelGGL((topk_token_lists_kernel<0, 512>), dim3(p.rows), dim3(512), 0, stream, p);
+  else if (!topk_dispatch<512, false>(p, stream, std::make_integer_sequence<int, 24>{}) && !topk_try<28, 512, false>(p, stream) && !topk_try<32, 512, false>(p, stream))
+    hipLaunchKernelGGL((topk_token_lists_kernel<0, 512, false>), dim3(p.rows), dim3(512), 0, stream, p);
   return hipGetLastError() == hipSuccess ? LVAR_OK : LVAR_ELAUNCH;
 }
 

@@ -2,14 +2,14 @@
 // log-sum-exp that the column-sum kernel subtracts.
 //
 // Query-stationary twin of the colsum kernel: a wave keeps 64 query rows (the B operand, Q^T) in registers for its
-// whole sweep over the keys; the workgroup (4 waves = 256 rows) streams 64-key K stages through a 4-deep LDS ring
-// filled by global->LDS DMA three stages ahead.  In the 32x32 accumulator a lane owns ONE query row and 16 keys, so
+// whole sweep over the keys; the workgroup (4 waves = 256 rows) streams 64-key K stages through a 2-deep LDS ring
+// filled by global->LDS DMA one stage (about 3 us) ahead.  In the 32x32 accumulator a lane owns ONE query row and 16 keys, so
 // the sum over keys is an in-register add.
 //
 // Bound by the vector port (per logit: scale-and-subtract, exp2, add = 19 cycles of one SIMD against 16.6 of its
 // matrix pipe), so nothing else may run per logit.  In particular there is no row maximum: the reference that keeps
-// exp2 in range is the maximum of the first 16 logits a lane sees, and once per 32 x 64 tile the running sum is looked
-// at and, when it has outgrown SUM_LIMIT, its exponent moves into the reference (a power of two: exact).  A logit that
+// exp2 in range is the maximum of the first 64 logits of a row, and once per 64-key stage the running sum is looked
+// at and, when it has outgrown LSE_SUM_LIMIT, its exponent moves into the reference (a power of two).  A logit that
 // lies more than 2^127 above the running sum overflows the sum; the wave then repeats its rows with a tracked maximum.
 // 64 rows per wave instead of the 32 of the attention kernel halve the LDS reads and the L2->LDS fills per flop.
 #include <type_traits>
@@ -19,9 +19,11 @@
 namespace lvar {
 
 constexpr float LSE_SUM_LIMIT = 65536.f;
+constexpr int ROW_LSE_STAGES = 2;   // depth of the LDS ring
+constexpr int ROW_LSE_WGS = 3;      // workgroups per compute unit (head_dim 64 and 128): 168 registers per wave, 32 KiB of LDS
 
 template <int D>
-__global__ __launch_bounds__(256, (D <= 128 ? 2 : 1)) void row_lse_kernel(const RowLseParams p) {
+__global__ __launch_bounds__(256, (D <= 128 ? ROW_LSE_WGS : 1)) void row_lse_kernel(const RowLseParams p) {
 #if defined(__HIP_DEVICE_COMPILE__)
   constexpr int KS = D / 16;
   constexpr int ROWB = D * 2, CPR = ROWB / 16;
@@ -29,7 +31,7 @@ __global__ __launch_bounds__(256, (D <= 128 ? 2 : 1)) void row_lse_kernel(const 
   constexpr int SWD = ROWB >= 256 ? 1 : 256 / ROWB;   // chunk swizzle of row t: (t / SWD) & SWM, 16 rows per period
   constexpr int SWM = ROWB >= 256 ? 15 : CPR - 1;
   constexpr int KTILE = 64 * ROWB;         // one 64-key stage
-  constexpr int NSTAGE = 4;
+  constexpr int NSTAGE = ROW_LSE_STAGES, PF = NSTAGE - 1;   // PF stages in flight ahead of the one being used
   extern __shared__ __attribute__((aligned(1024))) char smem[];  // NSTAGE * KTILE bytes
 
   // consecutive workgroup ids are dealt round-robin to the 8 XCDs: each XCD walks a contiguous range
@@ -91,17 +93,20 @@ __global__ __launch_bounds__(256, (D <= 128 ? 2 : 1)) void row_lse_kernel(const 
   constexpr auto vm = [](int n) constexpr { return 0x0f70 | (n & 15) | (((n >> 4) & 3) << 14); };
   // wait until at most `younger` later stages of this wave's fills are still in flight
   auto wait_fills = [&](int younger) {
-    if (younger >= 2) __builtin_amdgcn_s_waitcnt(vm(2 * SLOTS));
-    else if (younger == 1) __builtin_amdgcn_s_waitcnt(vm(SLOTS));
+    if (PF >= 3 && younger >= 2) __builtin_amdgcn_s_waitcnt(vm(2 * SLOTS));
+    else if (younger >= 1) __builtin_amdgcn_s_waitcnt(vm(SLOTS));
     else __builtin_amdgcn_s_waitcnt(vm(0));
   };
 
   const int S = (Lk_l + 63) >> 6;          // stages of this range
   const int U = (Lk_l + 31) >> 5;          // 32-key tiles
   const int kbase_l = r * ROWB + ((hh ^ ((r / SWD) & SWM)) << 4);
-  float m[2], l[2] = {0.f, 0.f};           // reference and sum of this lane's half of the keys, per query row
+  // Reference and sum of this lane's half of the keys, per query row.  The sum runs in the order of the attention
+  // kernel's row sum (even and odd elements of a 64-key stage apart; the two halves of the last stage apart), with the
+  // same first reference: statistics of one key range have the bits that the attention kernel gives.
+  float m[2], l[2] = {0.f, 0.f}, la[2], lb[2];
 
-  // after a tile: when a sum has outgrown the limit its exponent moves into the reference
+  // after a stage: when a sum has outgrown the limit its exponent moves into the reference
   auto renorm = [&]() {
     if (__builtin_amdgcn_ballot_w64(fmaxf(l[0], l[1]) > LSE_SUM_LIMIT) != 0) {
 #pragma unroll
@@ -129,110 +134,133 @@ __global__ __launch_bounds__(256, (D <= 128 ? 2 : 1)) void row_lse_kernel(const 
     float a = s[0], bmx = s[1];
 #pragma unroll
     for (int i = 2; i < 16; i += 2) { a = fmaxf(a, s[i]); bmx = fmaxf(bmx, s[i + 1]); }
-    return fmaxf(a, bmx) * c;
-  };
-  auto first_reference = [&](const f32x16& s0, const f32x16& s1) {
-    // A whole number, so that moving exponents into it later does not round.  (A lane whose 16 keys all lie beyond the
-    // range takes the reference 0 and keeps the sum 0.)
-    const float a = tile_max(s0), bmx = tile_max(s1);
-    m[0] = a > -INFINITY ? __builtin_rintf(a) : 0.f;
-    m[1] = bmx > -INFINITY ? __builtin_rintf(bmx) : 0.f;
+    return fmaxf(a, bmx);
   };
 
-  // prologue: up to three stages in flight
-  issue_stage(0);
-  if (S > 1) issue_stage(1);
-  if (S > 2) issue_stage(2);
-  wait_fills(min(2, S - 1));
-  __syncthreads();
-
-  // S(u) = K_tile(u) Q^T -> (n0a, n1a) on the matrix cores, the sum over tile u-1 from (c0, c1) on the vector ALU as a
-  // three-stage pipeline over the MFMA steps (scale | exp2 | add), interleaved by hand
-  auto step = [&](int u, f32x16& n0a, f32x16& n1a, const f32x16& c0, const f32x16& c1, bool have_prev) {
+  // S(u) = K_tile(u) Q^T -> (n0a, n1a) on the matrix cores, nothing beside it
+  auto qk_tile = [&](int u, f32x16& n0a, f32x16& n1a) {
     const char* kb = smem + ((u >> 1) & (NSTAGE - 1)) * KTILE + (u & 1) * 32 * ROWB;
-    constexpr int AHEAD = 3;
+#pragma unroll
+    for (int ks = 0; ks < KS; ks++) {
+      const bf16x8 f = *(const bf16x8*)(kb + (kbase_l ^ (ks << 5)));
+      n0a = mfma32(f, qf[0][ks], ks == 0 ? zero : n0a);
+      n1a = mfma32(f, qf[1][ks], ks == 0 ? zero : n1a);
+    }
+  };
+  // exponentials of a tile of the last stage, or of one without a successor: one sum
+  auto tile_sum = [&](const f32x16& s0, const f32x16& s1, float (&to)[2]) {
+    to[0] = to[1] = 0.f;
+#pragma unroll
+    for (int i = 0; i < 16; i++) {
+      to[0] += fast_exp2(fmaf(s0[i], c, -m[0]));
+      to[1] += fast_exp2(fmaf(s1[i], c, -m[1]));
+    }
+  };
+
+  // S(u) on the matrix cores, the exponentials of tile u-1 from (c0, c1) on the vector ALU as a three-stage pipeline
+  // over the MFMA steps (scale | exp2 | add), interleaved by hand.  One per 64-key stage opens the two sums (tile u-1
+  // is the first of its stage), the other closes them; `whole`: the first tile of the last stage, one sum.
+  auto step = [&](int u, f32x16& n0a, f32x16& n1a, const f32x16& c0, const f32x16& c1, auto opens, auto whole) {
+    constexpr bool OPENS = decltype(opens)::value, WHOLE = decltype(whole)::value;
+    const char* kb = smem + ((u >> 1) & (NSTAGE - 1)) * KTILE + (u & 1) * 32 * ROWB;
+    constexpr int AHEAD = 2;
     bf16x8 frag[KS];
 #pragma unroll
     for (int j = 0; j < AHEAD && j < KS; j++) frag[j] = *(const bf16x8*)(kb + (kbase_l ^ (j << 5)));
-    if (have_prev) {
-      constexpr int EPS = 16 / KS;
-      const float negm0 = -m[0], negm1 = -m[1];
-      float pa = 0.f, pb = 0.f;
-      float xs0[16], xs1[16];
-      auto st_scale = [&](int g) {
+    constexpr int EPS = 16 / KS;
+    const float negm0 = -m[0], negm1 = -m[1];
+    if (OPENS) la[0] = la[1] = lb[0] = lb[1] = 0.f;
+    float xs0[16], xs1[16];
+    auto st_scale = [&](int g) {
 #pragma unroll
-        for (int e = 0; e < EPS; e++) {
-          const int i = g * EPS + e;
-          xs0[i] = fmaf(c0[i], c, negm0);
-          xs1[i] = fmaf(c1[i], c, negm1);
-        }
-      };
-      auto st_exp = [&](int g) {
+      for (int e = 0; e < EPS; e++) {
+        const int i = g * EPS + e;
+        xs0[i] = fmaf(c0[i], c, negm0);
+        xs1[i] = fmaf(c1[i], c, negm1);
+      }
+    };
+    auto st_exp = [&](int g) {
 #pragma unroll
-        for (int e = 0; e < EPS; e++) {
-          const int i = g * EPS + e;
-          xs0[i] = fast_exp2(xs0[i]);
-          xs1[i] = fast_exp2(xs1[i]);
-        }
-      };
-      auto st_add = [&](int g) {
+      for (int e = 0; e < EPS; e++) {
+        const int i = g * EPS + e;
+        xs0[i] = fast_exp2(xs0[i]);
+        xs1[i] = fast_exp2(xs1[i]);
+      }
+    };
+    auto st_add = [&](int g) {
 #pragma unroll
-        for (int e = 0; e < EPS; e++) {
-          const int i = g * EPS + e;
-          pa += xs0[i];
-          pb += xs1[i];
-        }
-      };
-      st_scale(0);
+      for (int e = 0; e < EPS; e++) {
+        const int i = g * EPS + e;
+        if (WHOLE || (i & 1) == 0) { la[0] += xs0[i]; la[1] += xs1[i]; }
+        else { lb[0] += xs0[i]; lb[1] += xs1[i]; }
+      }
+    };
+    st_scale(0);
+    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+    for (int ks = 0; ks < KS; ks++) {
+      if (ks + AHEAD < KS) frag[ks + AHEAD] = *(const bf16x8*)(kb + (kbase_l ^ ((ks + AHEAD) << 5)));
+      n0a = mfma32(frag[ks], qf[0][ks], ks == 0 ? zero : n0a);
+      n1a = mfma32(frag[ks], qf[1][ks], ks == 0 ? zero : n1a);
+      if (ks >= 1) st_add(ks - 1);
+      st_exp(ks);
+      if (ks + 1 < KS) st_scale(ks + 1);
       __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-      for (int ks = 0; ks < KS; ks++) {
-        if (ks + AHEAD < KS) frag[ks + AHEAD] = *(const bf16x8*)(kb + (kbase_l ^ ((ks + AHEAD) << 5)));
-        n0a = mfma32(frag[ks], qf[0][ks], ks == 0 ? zero : n0a);
-        n1a = mfma32(frag[ks], qf[1][ks], ks == 0 ? zero : n1a);
-        if (ks >= 1) st_add(ks - 1);
-        st_exp(ks);
-        if (ks + 1 < KS) st_scale(ks + 1);
-        __builtin_amdgcn_sched_barrier(0);
-      }
-      st_add(KS - 1);
-      l[0] += pa;
-      l[1] += pb;
+    }
+    st_add(KS - 1);
+    if (!OPENS) {
+      l[0] += la[0] + lb[0];
+      l[1] += la[1] + lb[1];
       renorm();
-    } else {
-#pragma unroll
-      for (int ks = 0; ks < KS; ks++) {
-        if (ks + AHEAD < KS) frag[ks + AHEAD] = *(const bf16x8*)(kb + (kbase_l ^ ((ks + AHEAD) << 5)));
-        n0a = mfma32(frag[ks], qf[0][ks], ks == 0 ? zero : n0a);
-        n1a = mfma32(frag[ks], qf[1][ks], ks == 0 ? zero : n1a);
-      }
-      if (U == 1) mask_tile(0, n0a, n1a);
-      first_reference(n0a, n1a);
     }
   };
+  using yes = std::true_type;
+  using no = std::false_type;
 
-  // Tiles 0 .. U-2 are summed inside the step of their successor, the last (possibly ragged) one below.
+  // prologue: the ring filled; the first stage gives the reference
+#pragma unroll
+  for (int s = 0; s < NSTAGE; s++)
+    if (s < S) issue_stage(s);
+  wait_fills(min(PF, S - 1));
+  __syncthreads();
   f32x16 sa0, sa1, sb0, sb1;
-  for (int s = 0; s < S; s++) {
-    if (s + 3 < S) issue_stage(s + 3);
-    const int u0 = 2 * s;
-    step(u0, sa0, sa1, sb0, sb1, u0 > 0);
-    if (u0 + 1 < U) step(u0 + 1, sb0, sb1, sa0, sa1, true);
-    wait_fills(min(s + 3, S - 1) - (s + 1));
-    __syncthreads();
-  }
-  auto last_tile = [&](f32x16& s0, f32x16& s1) {
-    mask_tile(U - 1, s0, s1);
-    float pa = 0.f, pb = 0.f;
+  qk_tile(0, sa0, sa1);
+  qk_tile(1, sb0, sb1);
+  if (S == 1) { mask_tile(0, sa0, sa1); mask_tile(1, sb0, sb1); }
+  m[0] = xhalf_max(fmaxf(tile_max(sa0), tile_max(sb0))) * c;
+  m[1] = xhalf_max(fmaxf(tile_max(sa1), tile_max(sb1))) * c;
+  if (S > 1) {
+    la[0] = la[1] = lb[0] = lb[1] = 0.f;
 #pragma unroll
     for (int i = 0; i < 16; i++) {
-      pa += fast_exp2(fmaf(s0[i], c, -m[0]));
-      pb += fast_exp2(fmaf(s1[i], c, -m[1]));
+      const float x0 = fast_exp2(fmaf(sa0[i], c, -m[0])), x1 = fast_exp2(fmaf(sa1[i], c, -m[1]));
+      if (i & 1) { lb[0] += x0; lb[1] += x1; } else { la[0] += x0; la[1] += x1; }
     }
-    l[0] += pa;
-    l[1] += pb;
-  };
-  if (U & 1) last_tile(sa0, sa1); else last_tile(sb0, sb1);
+    wait_fills(min(PF, S - 1) - 1);
+    __syncthreads();
+    for (int s = 1; s + 1 < S; s++) {
+      if (s + PF < S) issue_stage(s + PF);
+      step(2 * s, sa0, sa1, sb0, sb1, no{}, no{});
+      step(2 * s + 1, sb0, sb1, sa0, sa1, yes{}, no{});
+      wait_fills(min(s + PF, S - 1) - (s + 1));
+      __syncthreads();
+    }
+    step(2 * S - 2, sa0, sa1, sb0, sb1, no{}, no{});
+    if (U & 1) {
+      mask_tile(U - 1, sa0, sa1);
+      tile_sum(sa0, sa1, la);
+      lb[0] = lb[1] = 0.f;
+    } else {
+      step(2 * S - 1, sb0, sb1, sa0, sa1, yes{}, yes{});
+      mask_tile(U - 1, sb0, sb1);
+      tile_sum(sb0, sb1, lb);
+    }
+  } else {
+    tile_sum(sa0, sa1, la);
+    tile_sum(sb0, sb1, lb);
+  }
+  l[0] += la[0] + lb[0];
+  l[1] += la[1] + lb[1];
 
   if (__builtin_amdgcn_ballot_w64(!(fmaxf(l[0], l[1]) < INFINITY)) != 0) {
     // a sum has overflowed: this wave's rows again, straight from memory, with the maximum tracked tile by tile
@@ -252,7 +280,7 @@ __global__ __launch_bounds__(256, (D <= 128 ? 2 : 1)) void row_lse_kernel(const 
 #pragma unroll
       for (int nt = 0; nt < 2; nt++) {
         const f32x16& s = nt ? sa1 : sa0;
-        const float m_new = fmaxf(m[nt], tile_max(s));
+        const float m_new = fmaxf(m[nt], tile_max(s) * c);
         float t = 0.f;
 #pragma unroll
         for (int i = 0; i < 16; i++) t += fast_exp2(fmaf(s[i], c, -m_new));
@@ -312,11 +340,11 @@ int launch_lse2_from_stats(const float* M, const float* L, float* lse2, int64_t 
   return hipGetLastError() == hipSuccess ? LVAR_OK : LVAR_ELAUNCH;
 }
 
-// Key ranges per row tile: workgroups are handed to the resident slots (two per compute unit) as slots fall free, so a
+// Key ranges per row tile: workgroups are handed to the resident slots as slots fall free, so a
 // launch takes its total work over the slots plus a part of the longest workgroup while the chip drains (the model of
 // the colsum launch, in 64-key stages of about 2 us), and the merge of several ranges costs a launch of its own.
 int row_lse_splits(int B, int H, int Lq, int Lk) {
-  const int base_wg = B * H * ((Lq + 255) / 256), slots = 2 * device_cus(), stages = (Lk + 63) / 64;
+  const int base_wg = B * H * ((Lq + 255) / 256), slots = ROW_LSE_WGS * device_cus(), stages = (Lk + 63) / 64;
   if (slots <= 0 || base_wg >= 4 * slots) return 1;
   int best_n = 1;
   double best = -1.0;
@@ -343,7 +371,7 @@ static int launch_rl(const RowLseParams& p0, hipStream_t stream) {
   p.split_keys = per * 64;
   p.total_wg = p.B * p.H * p.nrt * p.splits;
   const int grid = ((p.total_wg + 7) / 8) * 8;
-  constexpr int SMEM = 4 * 64 * D * 2;
+  constexpr int SMEM = ROW_LSE_STAGES * 64 * D * 2;
   static std::atomic<uint64_t> lds_ready{0};
   if (!ensure_lds_limit((const void*)row_lse_kernel<D>, SMEM, lds_ready)) return LVAR_ELAUNCH;
   hipLaunchKernelGGL((row_lse_kernel<D>), dim3(grid), dim3(256), SMEM, stream, p);

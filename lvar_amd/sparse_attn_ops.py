@@ -172,6 +172,17 @@ def _workspace(t: torch.Tensor, stream: int):
     return hit[0]
 
 
+def _native():
+    """The compiled host path of the operators (``csrc/torch_binding.cpp``), or None: not built, or the calls have to
+    carry a workspace.  Its functions return None for inputs that the general path has to look at."""
+    return None if _balanced else _lib.torch_binding()
+
+
+def _plain_scale(scale):
+    """A scale the compiled path takes as it is (numbers of other types are converted)."""
+    return scale if scale is None or type(scale) is float else float(scale)
+
+
 def _dense_launch(q, k, v, scale, want_o=True, want_ml=True, want_lse2=False):
     B, H, Lq, d = q.shape
     Lk = k.shape[2]
@@ -192,10 +203,9 @@ def _dense_launch(q, k, v, scale, want_o=True, want_ml=True, want_lse2=False):
 def dense_attn(q, k, v, scale=None):
     """Dense flash attention, ``(o, (M, L))`` (reference ``dense_attn``, sparse_attn_ops.py:21-59,
     Triton-provider return convention: ``lse`` is the tuple ``(M, L)``, each ``[B,H,Lq,1]``)."""
-    fast = None if _balanced else _lib.torch_binding()   # (the compiled path takes no workspace)
+    fast = _native()
     if fast is not None:
-        # None unless the inputs are the plain contiguous bf16 case
-        r = fast.fast_dense_attn(q, k, v, None if scale is None else float(scale)) if isinstance(q, torch.Tensor) else None
+        r = fast.fast_dense_attn(q, k, v, _plain_scale(scale))
         if r is not None:
             return r[0], (r[1], r[2])
     q, k, v, d_small = _pad_head_dim(q, k, v)
@@ -207,14 +217,15 @@ def dense_attn(q, k, v, scale=None):
     return (o if d_small is None else o[..., :d_small].contiguous()), (M, L)
 
 
-def _lse_only(q, k, scale):
-    """Statistics sweep without the PV product: base-2 log-sum-exp ``M + log2(L)``, fp32 [B,H,Lq]."""
+def _lse_only(q, k, scale, cut_keys: bool = True):
+    """``cut_keys``: the launch may cut the keys into ranges where the rows do not fill the chip (another summation order).
+    Statistics sweep without the PV product: base-2 log-sum-exp ``M + log2(L)``, fp32 [B,H,Lq]."""
     B, H, Lq, d = q.shape
     Lk = k.shape[2]
     lse2 = torch.empty((B, H, Lq), dtype=torch.float32, device=q.device)
     lib = _lib.load()
     with _on_device(q):
-        nbytes = int(lib.lvar_row_lse_scratch_bytes(B, H, Lq, Lk))
+        nbytes = int(lib.lvar_row_lse_scratch_bytes(B, H, Lq, Lk)) if cut_keys else 0
         scratch = torch.empty(nbytes, dtype=torch.uint8, device=q.device) if nbytes > 0 else None
         st = lib.lvar_row_lse_fwd(_view(q), _view(k), lse2.data_ptr(), _ptr(scratch), nbytes,
                                   B, H, k.shape[1], Lq, Lk, d, _scale(q, scale), _stream(q))
@@ -251,6 +262,13 @@ def colsum(q, k, scale=None, q_group_size: Optional[int] = None, lse: Optional[T
     (default: the kernel config's ``bm`` = 192), fp32 ``[B,H,G,Lk]``.  Self-contained two-pass form
     (statistics sweep, then column sweep) unless ``lse=(M, L)`` from a previous dense pass is given.
     With ``return_block_sums`` also returns the sums over blocks of 64 keys, ``[B,H,G,ceil(Lk/64)]``."""
+    fast = _native()
+    if fast is not None:
+        M, L = (None, None) if lse is None else lse
+        r = fast.fast_colsum(q, k, _plain_scale(scale), get_kernel_config_attn()["bm"] if q_group_size is None else q_group_size,
+                             M, L, bool(return_block_sums), True)
+        if r is not None:
+            return r if return_block_sums else r[0]
     q, k, _, d_small = _pad_head_dim(q, k)
     if d_small is not None:
         scale = _scale_for(d_small, scale)
@@ -271,10 +289,16 @@ def colsum(q, k, scale=None, q_group_size: Optional[int] = None, lse: Optional[T
 
 def _colsum_block_scores(q, k, scale, q_group_size: int, block_k: int):
     """Column sums summed over blocks of ``block_k`` keys (a multiple of 64), ``[B,H,G,ceil(Lk/block_k)]``, without the
-    column sums themselves going to memory (self-contained two-pass form)."""
-    q, k = _prep(q, "q"), _prep(k, "k")
-    _check_qkv(q, k, k, gqa=True)
-    _, bs = _colsum_given_lse(q, k, _lse_only(q, k, scale), scale, q_group_size, want_block_sums=True, want_columns=False)
+    column sums themselves going to memory (self-contained two-pass form).  Every sum has the bits of
+    ``key_block_sums(colsum(...), block_k)`` over whole blocks of 128 keys, with the keys uncut: a ranking of close scores
+    does not depend on which form computed them."""
+    fast = _native()
+    r = None if fast is None else fast.fast_colsum(q, k, _plain_scale(scale), q_group_size, None, None, True, False)
+    if r is None:
+        q, k = _prep(q, "q"), _prep(k, "k")
+        _check_qkv(q, k, k, gqa=True)
+        r = _colsum_given_lse(q, k, _lse_only(q, k, scale, cut_keys=False), scale, q_group_size, want_block_sums=True, want_columns=False)
+    bs = r[1]
     m = block_k // 64
     if m == 1:
         return bs
@@ -285,6 +309,11 @@ def dense_colsum_attn(q, k, v, scale=None):
     """Kernel-level op ``(o, blocksums, (M, L))`` (reference Triton ``dense_colsum_attn``,
     kernels/sparse_attn/triton/attn_dense_colsum.py:237-296): dense attention, then the column
     sweep that reuses its row statistics."""
+    fast = _native()
+    if fast is not None:
+        r = fast.fast_dense_colsum_attn(q, k, v, _plain_scale(scale), get_kernel_config_attn()["bm"])
+        if r is not None:
+            return r[0], r[1], (r[2], r[3])
     q, k, v, d_small = _pad_head_dim(q, k, v)
     if d_small is not None:
         scale = _scale_for(d_small, scale)
@@ -374,6 +403,11 @@ def csp_attn(q, k, v, scale, indices, indices_counts, o, o_scale):
     """``o + o_scale * softmax(q k[idx]^T scale) v[idx]`` with per-192-row-group key-token lists
     (reference ``csp_attn``, sparse_attn_ops.py:273-292).  Returns a new tensor; ``o`` is not
     modified (the reference's Triton behaviour).  The sum is formed in fp32 and rounded once."""
+    fast = _native()
+    if fast is not None:
+        r = fast.fast_csp_attn(q, k, v, _plain_scale(scale), indices, indices_counts, o, o_scale, get_kernel_config_attn()["bm"], 0, 0)
+        if r is not None:
+            return r
     _require(indices.dim() == 4 and indices.shape[-1] == k.shape[-2] and indices.shape[:2] == q.shape[:2],
              lambda: f"Indices shape mismatch - indices: {tuple(indices.shape)}, q: {tuple(q.shape)}, k: {tuple(k.shape)}")
     _require(tuple(o.shape) == tuple(q.shape), lambda: f"Output shape mismatch - o: {tuple(o.shape)}, q: {tuple(q.shape)}")
@@ -393,6 +427,11 @@ def csp_attn_upsampled(q, k, v, scale, indices, indices_counts, o_cache, o_scale
     _require(o_cache.dim() == 4, "o_cache must be [B,H,h*h,d]")
     src, dst = math.isqrt(o_cache.shape[-2]), math.isqrt(q.shape[-2])
     _require(src * src == o_cache.shape[-2] and dst * dst == q.shape[-2], "o_cache and q must hold square token grids")
+    fast = _native()
+    if fast is not None:
+        r = fast.fast_csp_attn(q, k, v, _plain_scale(scale), indices, indices_counts, o_cache, o_scale, get_kernel_config_attn()["bm"], src, dst)
+        if r is not None:
+            return r
     out, _, _ = _csp_launch(q, k, v, indices, indices_counts, o_cache, o_scale, scale, False, upsample_from=(src, dst))
     return out
 
@@ -409,6 +448,11 @@ def block_sparse_attn(q, k, v, kv_num_blocks, kv_indices, block_q: int = 128, bl
     ``BlockMask`` layout consumed by ``SparseFlexAttn`` (models/sparvar/basic_sparvar.py:55-72,187-194):
     ``kv_num_blocks`` int32 ``[B|1,H|1,nQ]``, ``kv_indices`` int32 ``[B|1,H|1,nQ,nKmax]``.
     Returns ``(o, (M, L))``."""
+    fast = _native()
+    if fast is not None:
+        r = fast.fast_block_sparse_attn(q, k, v, kv_num_blocks, kv_indices, block_q, block_k, _plain_scale(scale), True)
+        if r is not None:
+            return r[0], (r[1], r[2])
     q, k, v, d_small = _pad_head_dim(q, k, v)
     if d_small is not None:
         o, ml = block_sparse_attn(q, k, v, kv_num_blocks, kv_indices, block_q, block_k, _scale_for(d_small, scale))
@@ -446,11 +490,26 @@ def block_sparse_attn(q, k, v, kv_num_blocks, kv_indices, block_q: int = 128, bl
     return o, (M, L)
 
 
+def block_sparse_attn_out(q, k, v, kv_num_blocks, kv_indices, block_q: int = 128, block_k: int = 64, scale=None):
+    """:func:`block_sparse_attn` for callers that take the output alone: the row statistics are not written."""
+    fast = _native()
+    if fast is not None:
+        r = fast.fast_block_sparse_attn(q, k, v, kv_num_blocks, kv_indices, block_q, block_k, _plain_scale(scale), False)
+        if r is not None:
+            return r[0]
+    return block_sparse_attn(q, k, v, kv_num_blocks, kv_indices, block_q, block_k, scale)[0]
+
+
 def block_topk_lists(block_scores, target: int, base_mask=None):
     """Block lists from block scores on the GPU: per ``[B,H,nQ]`` row keep the blocks of ``base_mask``
     (bool/uint8 ``[nQ,nK]``, optional) plus the best-scoring others up to ``target`` blocks; returns
     ``(kv_num_blocks int32 [B,H,nQ], kv_indices int32 [B,H,nQ,nK])`` in ascending block order with a
     zero tail, ready for :func:`block_sparse_attn`.  Ties go to the smaller block index."""
+    fast = _native()
+    if fast is not None:
+        r = fast.fast_block_topk_lists(block_scores, target, base_mask)
+        if r is not None:
+            return r
     _require(block_scores.dim() == 4, "block_scores must be [B,H,nQ,nK]")
     if not block_scores.is_cuda:
         raise RuntimeError("block_scores must live on a HIP device; lvar_amd has no CPU path")
@@ -479,6 +538,11 @@ def topk_token_lists(scores, k: int, out_len: Optional[int] = None, order: str =
     lists them in ascending column order, which is also the best order for the gather kernel;
     ``order="value"`` re-orders them by descending score like ``torch.topk``
     (models/sparvar/sparse_attn.py:1016).  Ties at the k-th value go to the smaller column."""
+    fast = _native() if order == "index" and scores.dim() > 0 else None
+    if fast is not None:
+        r = fast.fast_topk_token_lists(scores, k, scores.shape[-1] if out_len is None else out_len, bool(zero_tail))
+        if r is not None:
+            return r
     _require(scores.dim() >= 1, "scores must have a key axis")
     if not scores.is_cuda:
         raise RuntimeError("scores must live on a HIP device; lvar_amd has no CPU path")
@@ -515,6 +579,12 @@ def remap_concat_lists(src_indices, src_count: int, cur_q_len: int, cur_k_len: i
     models/sparvar/sparse_attn.py:1113-1117; nothing reads them), which saves writing the full-width rows.  Equals
     ``append_local_run(map_inds_counts_across_scales(...))`` of :mod:`lvar_amd.mask_build`
     (models/sparvar/sparse_attn.py:366-421, 1096-1121)."""
+    fast = _native()
+    if fast is not None:
+        r = fast.fast_remap_concat_lists(src_indices, src_count, (int(cur_q_len) + bm - 1) // bm, cur_k_len, local_indices, indices_pad_to,
+                                         cur_k_len if out_len is None else out_len, bool(zero_tail))
+        if r is not None:
+            return r
     _require(src_indices.dim() == 4, "src_indices must be [B,H,Gs,Ks]")
     if not src_indices.is_cuda:
         raise RuntimeError("src_indices must live on a HIP device; lvar_amd has no CPU path")
@@ -549,6 +619,11 @@ def mask_to_lists(mask, multiple_of: int = 1):
     Counterpart of the reference's ``mask_to_indices`` (kernels/chipmunk/csrc/indexed_io/mask_to_indices.cu:21-97):
     the same set, but in ascending order (the reference's order is thread-strided) and with the padded count
     capped at ``n`` (the reference's rounded count can exceed the row)."""
+    fast = _native()
+    if fast is not None:
+        r = fast.fast_mask_to_lists(mask, multiple_of)
+        if r is not None:
+            return r
     if not mask.is_cuda:
         raise RuntimeError("mask must live on a HIP device; lvar_amd has no CPU path")
     # a bool tensor is one byte per entry with the values 0 / 1: viewed, not converted
@@ -640,6 +715,11 @@ def window_key_scores(q, k, window_keys, kernel_size: int = 5, pooling: str = "a
     along the key axis (``avgpool`` with zero padding or ``maxpool``, odd ``kernel_size``, stride 1) and masked
     again.  ``q`` ``[B,H,Lq,d]`` are the queries of the newest ``Lq`` keys of ``k`` ``[B,H,Lk,d]``;
     ``window_keys`` int64 ``[B,H,W]`` are key positions.  Returns fp32 ``[B,H,Lk]``.  One pass over K."""
+    fast = _native() if pooling in ("avgpool", "maxpool") else None
+    if fast is not None:
+        r = fast.fast_window_keys(q, k, window_keys, kernel_size, pooling == "maxpool", _plain_scale(scale), 0)
+        if r is not None:
+            return r
     q, k = _prep(q, "q"), _prep(k, "k")
     _check_qkv(q, k, k)
     B, H, Lq, d = q.shape
@@ -661,12 +741,19 @@ def window_key_scores(q, k, window_keys, kernel_size: int = 5, pooling: str = "a
 def scalekv_keep_indices(q, k, window_keys, max_capacity: int, kernel_size: int = 5, pooling: str = "avgpool"):
     """Key positions a ScaleKV-style cache keeps (models/scalekv/scale_kv.py:229-282): the window keys plus
     the ``max_capacity - W`` best-scoring other keys, ascending; int64 ``[B,H,min(max_capacity, Lk)]``.
-    Scores and the top-k selection run in the HIP library (ties go to the smaller key position)."""
+    Scores and the top-k selection run in the HIP library (ties go to the smaller key position).  Window keys are
+    positions in ``[0, Lk)``."""
     B, H, W = window_keys.shape
     Lk = k.shape[2]
     keep = min(max(0, int(max_capacity) - W), Lk - W)
     if keep <= 0:
         return torch.sort(window_keys.to(torch.int64), dim=-1).values
+    # one pass over K and one selection that writes the merged positions
+    fast = _native() if pooling in ("avgpool", "maxpool") else None
+    if fast is not None:
+        r = fast.fast_window_keys(q, k, window_keys, kernel_size, pooling == "maxpool", None, keep)
+        if r is not None:
+            return r
     scores = window_key_scores(q, k, window_keys, kernel_size, pooling)
     rest, _ = topk_token_lists(scores, keep, out_len=keep)
     combined = torch.cat([rest.to(torch.int64), window_keys.to(device=rest.device, dtype=torch.int64)], dim=-1)

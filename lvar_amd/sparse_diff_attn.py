@@ -4,6 +4,7 @@ full-step / sparse-step arithmetic, with the per-layer storage reduced to plain 
 reference's CPU offload pipeline is disabled in its shipped configuration and is not rebuilt)."""
 from __future__ import annotations
 
+import math
 from typing import Dict, Optional, Sequence, Tuple
 
 import torch
@@ -58,7 +59,18 @@ class SparseDiffAttn(torch.nn.Module):
         if not GLOBAL_CONFIG["attn"]["is_enabled"]:
             return ops.dense_attn(q, k, v, scale)[0]
         top_keys = GLOBAL_CONFIG["attn"]["top_keys"]
+        fast = ops._native()
         if do_full_step:                                           # sparse_attn.py:991-1051
+            if fast is not None:
+                # the launches below behind one host call
+                count = mb.indices_count(top_keys, k.shape[-2], self.multiple_of)
+                r = fast.fast_full_step(q, k, v, ops._plain_scale(scale), get_kernel_config_attn()["bm"], count, self.use_o_cache)
+                if r is not None:
+                    o, self.indices, self.counts, cache = r
+                    self.count_host = count
+                    if self.use_o_cache:
+                        self.out_cache = cache
+                    return o
             o, bs = self.dense_colsum_attn(q, k, v, scale)
             inds, counts = mb.topk_index_list(bs, top_keys, self.multiple_of, self.indices_pad_to, order="index", zero_tail=False)
             self.indices, self.counts = inds, counts
@@ -76,16 +88,23 @@ class SparseDiffAttn(torch.nn.Module):
         if local_inds.device != inds.device:
             local_inds = local_inds.to(inds.device)
             self.local_inds[scale_ind] = (local_inds, local_count)
+        last = scale_ind == len(self.scales) - 1
+        if fast is not None and self.use_o_cache:
+            # list remap and attention behind one host call
+            cache = self.out_cache if self.out_cache.shape[0] == q.shape[0] else self.out_cache[:q.shape[0]]
+            r = fast.fast_sparse_step(q, k, v, ops._plain_scale(scale), inds, s_count, local_inds, self.bm, self.indices_pad_to, cache,
+                                      math.isqrt(cache.shape[-2]), math.isqrt(q.shape[-2])) if self.bm == get_kernel_config_attn()["bm"] else None
+            if r is not None:
+                assert (s_count + local_count) % self.multiple_of == 0, f"after add local sparse index, mismatch multiple_of={self.multiple_of}"
+                self._keep_lists(r[1], r[2], s_count, local_count, last)
+                return r[0]
         # group remap + clamp + local-run append + counts in one launch (sparse_attn.py:1056-1121)
         # (columns behind the list stay as allocated, as the reference's torch.empty padding, sparse_attn.py:1113-1117)
         inds, counts = ops.remap_concat_lists(inds, s_count, q.shape[-2], k.shape[-2], local_inds,
                                               bm=self.bm, indices_pad_to=self.indices_pad_to, zero_tail=False)
         assert int(inds.shape[-1]) >= s_count + local_count and (s_count + local_count) % self.multiple_of == 0, \
             f"after add local sparse index, mismatch multiple_of={self.multiple_of}"
-        if scale_ind != len(self.scales) - 1:
-            self.indices, self.counts = inds, counts               # cached for the next scale
-            pad = self.indices_pad_to
-            self.count_host = max(pad, (s_count + pad - 1) // pad * pad) + local_count
+        self._keep_lists(inds, counts, s_count, local_count, last)
         if self.use_o_cache:
             o = self.out_cache
             if o.shape[0] != q.shape[0]:
@@ -94,3 +113,9 @@ class SparseDiffAttn(torch.nn.Module):
             return ops.csp_attn_upsampled(q, k, v, scale, inds, counts, o, 1)
         return ops.csp_attn(q, k, v, scale, inds, counts, torch.zeros_like(q), 1)
 
+    def _keep_lists(self, inds, counts, s_count: int, local_count: int, last: bool) -> None:
+        """Caches the lists of this scale for the next one."""
+        if not last:
+            self.indices, self.counts = inds, counts
+            pad = self.indices_pad_to
+            self.count_host = max(pad, (s_count + pad - 1) // pad * pad) + local_count

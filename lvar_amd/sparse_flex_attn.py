@@ -45,6 +45,6 @@ class SparseFlexAttn(torch.nn.Module):
         if self.kv_num_blocks.device != q.device:
             self.kv_num_blocks = self.kv_num_blocks.to(q.device)
             self.kv_indices = self.kv_indices.to(q.device)
-        out, _ = ops.block_sparse_attn(q.to(v.dtype), k.to(v.dtype), v, self.kv_num_blocks, self.kv_indices,
-                                       self.block_size, self.block_size, scale)
-        return out
+        if q.dtype is not v.dtype or k.dtype is not v.dtype:
+            q, k = q.to(v.dtype), k.to(v.dtype)
+        return ops.block_sparse_attn_out(q, k, v, self.kv_num_blocks, self.kv_indices, self.block_size, self.block_size, scale)
