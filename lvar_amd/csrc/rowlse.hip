@@ -40,9 +40,10 @@ __global__ __launch_bounds__(256, (D <= 128 ? ROW_LSE_WGS : 1)) void row_lse_ker
   if (w >= p.total_wg) return;
   // workgroup = (batch*head, key range, tile of 256 query rows)
   const int per_bh = p.nrt * p.splits;
-  const int bh = w / per_bh, rem = w - bh * per_bh;
-  const int sp = rem / p.nrt, rt = rem - sp * p.nrt;
-  const int b = bh / p.H, h = bh - b * p.H;
+  // (the quotients are formed on the vector ALU: moved to scalar registers, so are the addresses that hang on them)
+  const int bh = __builtin_amdgcn_readfirstlane(w / per_bh), rem = w - bh * per_bh;
+  const int sp = __builtin_amdgcn_readfirstlane(rem / p.nrt), rt = rem - sp * p.nrt;
+  const int b = __builtin_amdgcn_readfirstlane(bh / p.H), h = bh - b * p.H;
   const int koff = __builtin_amdgcn_readfirstlane(sp * p.split_keys);       // first key of this range (a multiple of 64)
   const int Lk_l = min(p.Lk, koff + p.split_keys) - koff;                   // keys of this range
   const int tid = threadIdx.x, lane = tid & 63;
@@ -53,7 +54,7 @@ __global__ __launch_bounds__(256, (D <= 128 ? ROW_LSE_WGS : 1)) void row_lse_ker
 
   // stationary Q^T fragments: lane holds query row n0 + nt*32 + r, d = ks*16 + 8*hh .. +7
   const bf16_t* qbase = p.q + b * p.q_sb + h * p.q_sh;
-  const bf16_t* kbase = p.k + b * p.k_sb + (h / p.kv_group) * p.k_sh;   // grouped-query attention: shared key heads
+  const bf16_t* kbase = p.k + b * p.k_sb + __builtin_amdgcn_readfirstlane(h / p.kv_group) * p.k_sh;   // grouped-query attention: shared key heads
   bf16x8 qf[2][KS];
 #pragma unroll
   for (int nt = 0; nt < 2; nt++) {
