@@ -152,6 +152,16 @@ at::Tensor empty(at::IntArrayRef sizes, at::ScalarType ty, int dev) {
 at::Tensor empty_o(const Qkv& a) { return empty({a.B, a.H, a.Lq, a.d}, at::kBFloat16, a.dev); }
 at::Tensor empty_stat(const Qkv& a) { return empty({a.B, a.H, a.Lq, 1}, at::kFloat, a.dev); }
 
+// M and L in one allocation: L is a view of the storage behind M
+void empty_stats(const Qkv& a, at::Tensor& M, at::Tensor& L) {
+  const int64_t rows = int64_t(a.B) * a.H * a.Lq;
+  M = empty({2, a.B, a.H, a.Lq, 1}, at::kFloat, a.dev);
+  L = at::detail::make_tensor<c10::TensorImpl>(c10::Storage(M.storage()), M.key_set(), M.dtype());
+  L.unsafeGetTensorImpl()->set_sizes_contiguous({a.B, a.H, a.Lq, 1});
+  L.unsafeGetTensorImpl()->set_storage_offset(rows);
+  M.unsafeGetTensorImpl()->set_sizes_contiguous({a.B, a.H, a.Lq, 1});
+}
+
 PyObject* none() { Py_RETURN_NONE; }
 
 template <class... T>
@@ -172,7 +182,8 @@ LVAR_FAST(fast_dense_attn) {
   Qkv x;
   float scale;
   LVAR_NEED(n == 4 && qkv_ok(x, a[0], a[1], a[2], true) && as_scale(a[3], x.d, scale));
-  at::Tensor o = empty_o(x), M = empty_stat(x), L = empty_stat(x);
+  at::Tensor o = empty_o(x), M, L;
+  empty_stats(x, M, L);
   LVAR_NEED(api.lvar_dense_attn_fwd(view(*x.q), view(*x.k), view(*x.v), view(o), M.data_ptr<float>(), L.data_ptr<float>(), nullptr,
                                     x.B, x.H, x.Hkv, x.Lq, x.Lk, x.d, scale, x.stream) == LVAR_OK);
   return tuple(std::move(o), std::move(M), std::move(L));
@@ -188,7 +199,8 @@ LVAR_FAST(fast_dense_colsum_attn) {
   float scale;
   int64_t bm;
   LVAR_NEED(n == 5 && qkv_ok(x, a[0], a[1], a[2], true) && as_scale(a[3], x.d, scale) && as_long(a[4], bm) && bm > 0 && bm % 32 == 0);
-  at::Tensor o = empty_o(x), M = empty_stat(x), L = empty_stat(x), lse2 = empty_stat(x);
+  at::Tensor o = empty_o(x), lse2 = empty_stat(x), M, L;
+  empty_stats(x, M, L);
   at::Tensor cs = empty({x.B, x.H, groups_of(x.Lq, bm), x.Lk}, at::kFloat, x.dev);
   LVAR_NEED(api.lvar_dense_attn_fwd(view(*x.q), view(*x.k), view(*x.v), view(o), M.data_ptr<float>(), L.data_ptr<float>(), lse2.data_ptr<float>(),
                                     x.B, x.H, x.Hkv, x.Lq, x.Lk, x.d, scale, x.stream) == LVAR_OK);
@@ -354,7 +366,7 @@ LVAR_FAST(fast_block_sparse_attn) {
             is[3] > 0 && is[3] <= INT32_MAX);
   const bool per_b = ns[0] == x.B && x.B > 1, per_h = ns[1] == x.H && x.H > 1;
   at::Tensor o = empty_o(x), M, L;
-  if (stats) { M = empty_stat(x); L = empty_stat(x); }
+  if (stats) empty_stats(x, M, L);
   LVAR_NEED(api.lvar_block_sparse_attn_fwd(view(*x.q), view(*x.k), view(*x.v), view(o), stats ? M.data_ptr<float>() : nullptr, stats ? L.data_ptr<float>() : nullptr,
                                            num->data_ptr<int32_t>(), per_b ? num->stride(0) : 0, per_h ? num->stride(1) : 0, idx->data_ptr<int32_t>(),
                                            per_b ? idx->stride(0) : 0, per_h ? idx->stride(1) : 0, is[3], static_cast<int>(is[3]), static_cast<int>(bq),

@@ -1,0 +1,63 @@
+"""Dense and block-list attention with the keys of a query tile split over two teams of waves: the sizes at which the
+launch takes 64- or 128-row workgroups of two teams, at the edges of tiles and with odd, short and empty lists."""
+import pytest
+import torch
+
+import oracle
+from conftest import make_qkv
+
+pytestmark = pytest.mark.gpu
+
+
+def _close(o, ref):
+    assert torch.allclose(o.float().cpu(), ref, atol=2e-2, rtol=1e-2)
+
+
+# (B*H) * ceil(Lq/64) <= 256 takes 64-row workgroups from 4 tiles on, (B*H) * ceil(Lq/128) <= 256 128-row ones from 8
+@pytest.mark.parametrize("B,H,Hkv,Lq,Lk,d", [
+    (1, 2, 2, 1, 193, 128), (1, 2, 2, 64, 256, 128), (2, 2, 1, 65, 257, 64), (1, 3, 3, 129, 319, 128), (1, 2, 2, 200, 449, 64),
+    (1, 140, 140, 128, 512, 128), (1, 140, 140, 100, 577, 128), (1, 130, 65, 127, 513, 64), (2, 64, 64, 200, 640, 64),
+])
+def test_dense_two_teams(B, H, Hkv, Lq, Lk, d):
+    from lvar_amd import sparse_attn_ops as ops
+    q, k, v = make_qkv(B, H, Lq, Lk, d, seed=Lq + Lk)
+    k, v = k[:, :Hkv].contiguous(), v[:, :Hkv].contiguous()
+    o, (M, L) = ops.dense_attn(q.cuda(), k.cuda(), v.cuda())
+    hs = slice(0, min(H, 6))
+    kx, vx = k.repeat_interleave(H // Hkv, 1)[:, hs], v.repeat_interleave(H // Hkv, 1)[:, hs]
+    o_ref, M_ref, L_ref = oracle.dense_attn(q[:, hs], kx, vx)
+    _close(o[:, hs], o_ref)
+    lse = (M + torch.log2(L))[:, hs].cpu()
+    assert torch.allclose(lse, M_ref + torch.log2(L_ref), atol=1e-3, rtol=0)
+    if H > 6:   # every head of the launch, against the statement in float32 on the device
+        s = torch.matmul(q.cuda().float(), k.cuda().float().repeat_interleave(H // Hkv, 1).transpose(-1, -2).contiguous()) * d ** -0.5
+        ref = torch.matmul(s.softmax(-1), v.cuda().float().repeat_interleave(H // Hkv, 1))
+        assert torch.allclose(o.float(), ref, atol=2e-2, rtol=1e-2)
+
+
+def test_dense_two_teams_growing_logits():
+    """Row maxima that grow along the keys: the teams end with different references."""
+    from lvar_amd import sparse_attn_ops as ops
+    q, k, v = make_qkv(1, 2, 100, 700, 128, seed=9)
+    k = (k.float() * torch.linspace(0.1, 6.0, 700).view(1, 1, -1, 1)).to(torch.bfloat16)
+    o, _ = ops.dense_attn(q.cuda(), k.cuda(), v.cuda())
+    _close(o, oracle.dense_attn(q, k, v)[0])
+
+
+@pytest.mark.parametrize("H,Lq,Lk,d,bq,bk", [(2, 300, 1000, 128, 128, 64), (3, 130, 900, 64, 128, 128), (2, 200, 1100, 128, 64, 64),
+                                             (140, 128, 1024, 128, 128, 64), (135, 120, 1300, 64, 128, 256)])
+def test_block_lists_two_teams(H, Lq, Lk, d, bq, bk):
+    from lvar_amd import sparse_attn_ops as ops
+    q, k, v = make_qkv(1, H, Lq, Lk, d, seed=Lq)
+    nQ, nK = -(-Lq // bq), -(-Lk // bk)
+    g = torch.Generator().manual_seed(Lk)
+    mask = torch.rand(1, H, nQ, nK, generator=g) < 0.4
+    mask[0, 0, 0] = False                      # an empty list
+    mask[0, 1, 0] = False
+    mask[0, 1, 0, nK - 1] = True               # one block, the ragged last one
+    num, idx = ops.mask_to_lists(mask.cuda())
+    o, (M, L) = ops.block_sparse_attn(q.cuda(), k.cuda(), v.cuda(), num, idx, bq, bk)
+    hs = slice(0, min(H, 6))
+    o_ref = oracle.block_sparse_attn(q[:, hs], k[:, hs], v[:, hs], num.cpu()[:, hs], idx.cpu()[:, hs], bq, bk)[0]
+    _close(o[:, hs], o_ref)
+    assert bool((o[0, 0, :min(bq, Lq)] == 0).all())
