@@ -67,6 +67,13 @@ struct Swz {
   __device__ static __forceinline__ int fv(int row) { return (D >= 128) ? ((row & 3) << 2) : (((row >> 1) & 1) << 2); }
 };
 
+// LDS of a workgroup: K and V buffers of every team; the epilogue's transpose buffer of eight computing waves is larger
+template <int D, int NWAVES, int MODE, int KSPLIT>
+constexpr int attn_lds_bytes() {
+  const int bufs = KSPLIT * 4 * 64 * D * 2, epi = NWAVES * 32 * (D * 2 + 16);
+  return (MODE == MODE_BLOCK && KSPLIT == 1 && epi > bufs) ? epi : bufs;
+}
+
 // Context of a balanced launch (see sk_partition.h); unused by the plain launch.
 #if defined(__HIP_DEVICE_COMPILE__)
 struct SkCtx {
@@ -100,7 +107,7 @@ __device__ __forceinline__ void attn_item(const AttnParams& p, char* smem, const
   constexpr bool CONST_OFF = MODE == MODE_BLOCK && ((FW * RPI) % 16 == 0 || 16 % (FW * RPI) == 0) && NI % FW == 0;
   constexpr int CONST_PER = (FW * RPI) >= 16 ? 1 : 16 / (FW * RPI);
   constexpr int OSTR = D * 2 + 16;  // epilogue transpose buffer row stride (bytes)
-  static_assert(NCOMP * 32 * OSTR <= 4 * TILE, "epilogue buffer must fit in the K/V buffers");
+  static_assert(NCOMP * 32 * OSTR <= attn_lds_bytes<D, NWAVES, MODE, KSPLIT>(), "the epilogue buffer must fit");
   static_assert(KSPLIT == 1 || (KSPLIT == 2 && MODE == MODE_BLOCK && !SK && !ACCUM && NPROD == 0), "two teams: block lists and dense attention");
   // LDS map: K buffers at 0 and TILE, V buffers at 2*TILE and 3*TILE (the second team's follow)
 
@@ -1017,10 +1024,11 @@ __global__ __launch_bounds__(256) void plan_kernel(const AttnParams p, int* plan
 // which walk two tiles in 1.6 of the time of one (576 x 1497: 27.6 -> 24.9 us, 1024 x 2521: 47.6 -> 45.2 us).  Beyond
 // that the second resident workgroup does the same without a merge.  The merge costs about a microsecond, so lists of a
 // few tiles are walked by one team (the length of a block list is known to the device only; the width of the table
-// stands in for it).  A launch that hands the row statistic to a ranking (LSE2: column sums, top-k lists) keeps one team:
-// two add the rows up in another order, and close scores would change places with the launch shape.
+// stands in for it).  A launch whose row statistic feeds a ranking (LSE2 without M and L: the decision-scale step, whose
+// column sums become top-k lists) keeps one team: two add the rows up in another order, and close scores would change
+// places with the launch shape.
 static int two_team_rows(const AttnParams& p, int nwaves) {
-  if (p.LSE2) return 0;
+  if (p.LSE2 && !p.M) return 0;
   const int64_t all = (p.Lk + 63) / 64, tiles = p.list ? std::min((int64_t)p.list_len << p.sub_shift, all) : all;
   const int64_t bh = (int64_t)p.B * p.H, cus = device_cus();
   if (tiles >= 4 && bh * ((p.Lq + 63) / 64) <= cus) return 64;
@@ -1028,22 +1036,41 @@ static int two_team_rows(const AttnParams& p, int nwaves) {
   return 0;
 }
 
+// Dense attention with 256 query rows per workgroup (eight waves on one pair of K/V buffers, one workgroup per compute
+// unit): half the L2->LDS fills per flop, 4 % faster than two 128-row workgroups side by side (B2 H16 d128: 4096 x 10521
+// 635 -> 608 us, 1600 x 4121 117 -> 113 us) unless the coarser tiles leave more of the last round idle.  In units of a
+// lone 128-row tile: a pair of 128-row workgroups takes 1.6 of it, a 256-row one 1.6 * 0.95; at head_dim 64 three small
+// workgroups share a compute unit and only launches of a single round gain.
+static bool wide_tiles(const AttnParams& p, int head_dim) {
+  if (p.list) return false;
+  const int64_t bh = (int64_t)p.B * p.H, cus = device_cus();
+  if (cus <= 0) return false;
+  const int64_t n128 = bh * ((p.Lq + 127) / 128), n256 = bh * ((p.Lq + 255) / 256);
+  if (n128 <= cus) return false;
+  if (head_dim == 64) return n256 <= cus;
+  const int64_t full = n128 / (2 * cus), rest = n128 % (2 * cus);
+  const double narrow = 1.6 * full + (rest == 0 ? 0.0 : rest <= cus ? 1.0 : 1.6);
+  const double wide = 1.6 * 0.95 * ((n256 + cus - 1) / cus);
+  return wide < narrow;
+}
+
 template <int D, int NWAVES, int MODE, bool ACCUM, bool LSE_ONLY, int KSPLIT = 1>
 static int launch_one(const AttnParams& p0, hipStream_t stream) {
   AttnParams p = p0;
   if (p.kv_group < 1) p.kv_group = 1;
   constexpr int WGROWS = ((MODE == MODE_GATHER && NWAVES == 8) ? 6 : NWAVES / KSPLIT) * 32;   // two of eight token-list waves only fetch
-  constexpr int SMEM = KSPLIT * 4 * 64 * D * 2;
+  constexpr int SMEM = attn_lds_bytes<D, NWAVES, MODE, KSPLIT>();
   if (MODE == MODE_BLOCK && p.list == nullptr) p.group_rows = WGROWS;  // dense: any row grouping
   if (p.group_rows % WGROWS != 0) return LVAR_EINVAL;
   p.nqt = (p.Lq + WGROWS - 1) / WGROWS;
   p.total_wg = p.B * p.H * p.nqt;
+  constexpr bool WIDE = MODE == MODE_BLOCK && NWAVES == 8 && KSPLIT == 1;   // 256 query rows
   if constexpr (!LSE_ONLY && KSPLIT == 1) {
     const bool dense = (MODE == MODE_BLOCK && p.list == nullptr);
     const int64_t per_tile = (MODE == MODE_BLOCK) ? (p.list ? p.list_len : (p.Lk + 63) / 64) : (p.list_len + 63) / 64;
     const int sub = (MODE == MODE_BLOCK && p.list) ? p.sub_shift : 0;
     // (64-row query blocks always take the plain launch)
-    p.sk_wgs = (p.sk_ws && NWAVES != 2 && D <= 128) ? sk_plan(p.total_wg, NWAVES, sk_slot_floats(D, MODE, NWAVES), per_tile, sub, p.sk_ws_bytes,
+    p.sk_wgs = (p.sk_ws && NWAVES != 2 && !WIDE && D <= 128) ? sk_plan(p.total_wg, NWAVES, sk_slot_floats(D, MODE, NWAVES), per_tile, sub, p.sk_ws_bytes,
                                  p.sk_min_share, p.sk_min_piece) : 0;
     p.sk_uniform_n = 0;
     if (p.sk_wgs > 0 && dense) {
@@ -1051,7 +1078,7 @@ static int launch_one(const AttnParams& p0, hipStream_t stream) {
       p.sk_uniform_n = sk_dense_pieces(p.total_wg, (int)per_tile, p.sk_wgs, p.sk_min_share, p.sk_min_piece);
       if (p.sk_uniform_n == 0) p.sk_wgs = 0;   // whole tiles: the plain launch
     }
-    if constexpr (NWAVES != 2 && D <= 128) if (p.sk_wgs > 0) {
+    if constexpr (NWAVES != 2 && !WIDE && D <= 128) if (p.sk_wgs > 0) {
       p.sk_counters = (int*)p.sk_ws;
       p.sk_slots = (float*)((char*)p.sk_ws + SK_COUNTER_BYTES + sk_plan_bytes(p.sk_wgs));
       int grid_sk;
@@ -1079,7 +1106,8 @@ static int launch_one(const AttnParams& p0, hipStream_t stream) {
       return hipGetLastError() == hipSuccess ? LVAR_OK : LVAR_ELAUNCH;
     }
   }
-  if constexpr (MODE == MODE_BLOCK && !LSE_ONLY && KSPLIT == 1 && D <= 128) {
+  if constexpr (MODE == MODE_BLOCK && !LSE_ONLY && KSPLIT == 1 && !WIDE && D <= 128) {
+    if (NWAVES == 4 && wide_tiles(p0, D)) return launch_one<D, 8, MODE_BLOCK, false, false, 1>(p0, stream);
     const int rows = two_team_rows(p0, NWAVES);
     AttnParams p2 = p0;
     p2.sk_ws = nullptr;

@@ -1,5 +1,5 @@
-"""Dense and block-list attention with the keys of a query tile split over two teams of waves: the sizes at which the
-launch takes 64- or 128-row workgroups of two teams, at the edges of tiles and with odd, short and empty lists."""
+"""Workgroup shapes of dense and block-list attention: the sizes at which the launch takes 64- or 128-row workgroups of two
+teams of waves, or 256-row workgroups, at the edges of tiles and with odd, short and empty lists."""
 import pytest
 import torch
 
@@ -33,6 +33,18 @@ def test_dense_two_teams(B, H, Hkv, Lq, Lk, d):
         s = torch.matmul(q.cuda().float(), k.cuda().float().repeat_interleave(H // Hkv, 1).transpose(-1, -2).contiguous()) * d ** -0.5
         ref = torch.matmul(s.softmax(-1), v.cuda().float().repeat_interleave(H // Hkv, 1))
         assert torch.allclose(o.float(), ref, atol=2e-2, rtol=1e-2)
+
+
+@pytest.mark.parametrize("B,H,Lq,Lk,d", [(2, 64, 257, 65, 128), (1, 200, 250, 300, 64), (2, 70, 385, 130, 128), (1, 256, 512, 64, 128), (1, 250, 512, 1, 128)])
+def test_dense_256_row_workgroups(B, H, Lq, Lk, d):
+    """More than one 128-row tile per compute unit and at most one 256-row tile (or whole rounds of them)."""
+    from lvar_amd import sparse_attn_ops as ops
+    g = torch.Generator(device="cuda").manual_seed(Lq)
+    q, k, v = (torch.randn(B, H, L, d, generator=g, device="cuda").to(torch.bfloat16) for L in (Lq, Lk, Lk))
+    o, (M, L) = ops.dense_attn(q, k, v)
+    s = torch.matmul(q.float(), k.float().transpose(-1, -2).contiguous()) * d ** -0.5
+    assert torch.allclose(o.float(), torch.matmul(s.softmax(-1), v.float()), atol=2e-2, rtol=1e-2)
+    assert torch.allclose(M + torch.log2(L), torch.logsumexp(s, -1, keepdim=True) * 1.4426950408889634, atol=1e-3, rtol=0)
 
 
 def test_dense_two_teams_growing_logits():
