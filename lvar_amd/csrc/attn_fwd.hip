@@ -1036,13 +1036,13 @@ static int two_team_rows(const AttnParams& p, int nwaves) {
   return 0;
 }
 
-// Dense attention with 256 query rows per workgroup (eight waves on one pair of K/V buffers, one workgroup per compute
+// 256 query rows per workgroup (eight waves on one pair of K/V buffers, one workgroup per compute
 // unit): half the L2->LDS fills per flop, 4 % faster than two 128-row workgroups side by side (B2 H16 d128: 4096 x 10521
 // 635 -> 608 us, 1600 x 4121 117 -> 113 us) unless the coarser tiles leave more of the last round idle.  In units of a
 // lone 128-row tile: a pair of 128-row workgroups takes 1.6 of it, a 256-row one 1.6 * 0.95; at head_dim 64 three small
 // workgroups share a compute unit and only launches of a single round gain.
 static bool wide_tiles(const AttnParams& p, int head_dim) {
-  if (p.list) return false;
+  if (p.list && p.group_rows % 256 != 0) return false;   // (lists of 256-row query blocks run the same way)
   const int64_t bh = (int64_t)p.B * p.H, cus = device_cus();
   if (cus <= 0) return false;
   const int64_t n128 = bh * ((p.Lq + 127) / 128), n256 = bh * ((p.Lq + 255) / 256);

@@ -73,3 +73,22 @@ def test_block_lists_two_teams(H, Lq, Lk, d, bq, bk):
     o_ref = oracle.block_sparse_attn(q[:, hs], k[:, hs], v[:, hs], num.cpu()[:, hs], idx.cpu()[:, hs], bq, bk)[0]
     _close(o[:, hs], o_ref)
     assert bool((o[0, 0, :min(bq, Lq)] == 0).all())
+
+
+@pytest.mark.parametrize("B,H,Lq,Lk,d,bq,bk", [(1, 3, 300, 500, 128, 128, 64), (2, 20, 1000, 900, 64, 128, 128), (1, 7, 700, 1100, 128, 64, 64),
+                                               (2, 70, 640, 300, 128, 256, 256), (1, 9, 700, 800, 128, 256, 64), (2, 40, 520, 600, 128, 384, 128)])
+def test_block_lists_of_several_workgroups(B, H, Lq, Lk, d, bq, bk):
+    """Query blocks of several workgroups and of 256-row workgroups, a ragged last block among them."""
+    from lvar_amd import sparse_attn_ops as ops
+    g = torch.Generator(device="cuda").manual_seed(Lq + bk)
+    q, k, v = (torch.randn(B, H, L, d, generator=g, device="cuda").to(torch.bfloat16) for L in (Lq, Lk, Lk))
+    nQ, nK = -(-Lq // bq), -(-Lk // bk)
+    num, idx = ops.mask_to_lists(torch.rand(1, 1, nQ, nK, generator=g, device="cuda") < 0.5)
+    ref, _ = ops.block_sparse_attn(q, k, v, num, idx, bq, bk)
+    assert torch.equal(ops.block_sparse_attn_out(q, k, v, num, idx, bq, bk), ref)
+    m = torch.zeros(nQ, nK, dtype=torch.bool, device="cuda")
+    for i in range(nQ):
+        m[i, idx[0, 0, i, :int(num[0, 0, i])].long()] = True
+    m = m.repeat_interleave(bq, 0)[:Lq].repeat_interleave(bk, 1)[:, :Lk]
+    s = (torch.matmul(q.float(), k.float().transpose(-1, -2).contiguous()) * d ** -0.5).masked_fill(~m, float("-inf"))
+    assert torch.allclose(ref.float(), torch.matmul(s.softmax(-1).nan_to_num(0.0), v.float()), atol=2e-2, rtol=1e-2)
