@@ -146,6 +146,22 @@ int lvar_colsum_fwd(lvar_tensor_t q, lvar_tensor_t k, const float* lse2, float* 
                     float scale, void* stream);
 
 /*
+ * Scores of key blocks without the column sums: scores[b,h,g,j] = sum_{i in group g} sum_{n in block j}
+ * exp2(q_i.k_n*scale*log2e - lse2_i), fp32 contiguous [B,H,G,ceil(Lk/block_k)], in one sweep over the logits (the
+ * statistics come from the same sweep).  block_k is a multiple of 64, q_group_size 32 or a multiple of 64 up to 1024
+ * (others: LVAR_EUNSUPPORTED).  Sums run over the keys of a block first and then over the rows, so a score differs from
+ * the sum of lvar_colsum_fwd's columns in the last bits.  For callers that rank the blocks, `target` > 0 gives the
+ * number of blocks they will keep per row (as lvar_block_topk_lists counts them, base_mask [G, ceil(Lk/block_k)] or
+ * NULL): scores within 2^-18 (relative) of the cut are then replaced by the sum of lvar_colsum_fwd's block sums, and
+ * the selection does not depend on which of the two computed the scores (up to 2048 blocks per row).
+ * scratch: at least lvar_block_scores_scratch_bytes(), 16-byte aligned; written and read by this call only.
+ */
+int64_t lvar_block_scores_scratch_bytes(int B, int H, int Lq, int Lk, int q_group_size, int block_k);
+int lvar_block_scores_fwd(lvar_tensor_t q, lvar_tensor_t k, float* scores, const uint8_t* base_mask, int target,
+                          void* scratch, int64_t scratch_bytes, int B, int H, int kv_heads, int Lq, int Lk, int head_dim,
+                          int q_group_size, int block_k, float scale, void* stream);
+
+/*
  * Column-sparse (token-list) attention:
  *   o[b,h,i,:] = o_accum[b,h,i,:] + o_scale * softmax(q_i k[idx]^T scale) v[idx],
  *   idx = indices[b,h,g,0:counts[b,h,g]],  g = i / group_rows,

@@ -176,6 +176,45 @@ int lvar_colsum_fwd(lvar_tensor_t q, lvar_tensor_t k, const float* lse2, float* 
   return launch_colsum(p, head_dim, (hipStream_t)stream);
 }
 
+// Scratch of a block-score call, in 4-byte words: lse2 | first references | number of scores to compute again, and which | block sums.
+struct ScoreLayout { int64_t refs, work, sums, total; };
+static ScoreLayout score_layout(int B, int H, int Lq, int Lk, int q_group_size, int block_k) {
+  ScoreLayout l{};
+  const int64_t bh = (int64_t)B * H, nK = (Lk + block_k - 1) / block_k;
+  l.refs = bh * Lq;
+  l.work = 2 * l.refs;
+  l.sums = (l.work + 1 + bh * ((Lq + q_group_size - 1) / q_group_size) * nK + 63) / 64 * 64;
+  l.total = l.sums + bh * ((Lq + 255) / 256) * 256 * nK;
+  return l;
+}
+
+int64_t lvar_block_scores_scratch_bytes(int B, int H, int Lq, int Lk, int q_group_size, int block_k) {
+  if (B <= 0 || H <= 0 || Lq <= 0 || Lk <= 0 || q_group_size <= 0 || block_k <= 0 || block_k % 64 != 0) return LVAR_EINVAL;
+  return 4 * score_layout(B, H, Lq, Lk, q_group_size, block_k).total;
+}
+
+int lvar_block_scores_fwd(lvar_tensor_t q, lvar_tensor_t k, float* scores, const uint8_t* base_mask, int target, void* scratch, int64_t scratch_bytes,
+                          int B, int H, int kv_heads, int Lq, int Lk, int head_dim, int q_group_size, int block_k, float scale, void* stream) {
+  if (!shape_ok(B, H, Lq, Lk, scale) || !view_ok(q) || !view_ok(k) || !scores || target < 0) return LVAR_EINVAL;
+  if (kv_heads <= 0 || H % kv_heads != 0 || !kv_span_ok(k, Lk, head_dim)) return LVAR_EINVAL;
+  if (block_k <= 0 || block_k % 64 != 0 || q_group_size <= 0 || q_group_size % 32 != 0) return LVAR_EINVAL;
+  if ((q_group_size != 32 && q_group_size % 64 != 0) || q_group_size > 1024) return LVAR_EUNSUPPORTED;
+  const ScoreLayout l = score_layout(B, H, Lq, Lk, q_group_size, block_k);
+  if (l.sums > INT32_MAX) return LVAR_EUNSUPPORTED;   // (scores are counted in 32 bits)
+  if (!scratch || (reinterpret_cast<uintptr_t>(scratch) & 15u) || scratch_bytes < 4 * l.total) return LVAR_EINVAL;
+  float* const f = (float*)scratch;
+  BlockScoreParams p{};
+  p.r.q = (const bf16_t*)q.ptr; p.r.q_sb = q.stride_b; p.r.q_sh = q.stride_h; p.r.q_sr = q.stride_row;
+  p.r.k = (const bf16_t*)k.ptr; p.r.k_sb = k.stride_b; p.r.k_sh = k.stride_h; p.r.k_sr = k.stride_row;
+  p.r.lse2 = f; p.r.first_ref = f + l.refs; p.r.work = (int*)f + l.work; p.r.tsum = f + l.sums;
+  p.r.B = B; p.r.H = H; p.r.Lq = Lq; p.r.Lk = Lk; p.r.kv_group = H / kv_heads;
+  p.r.c = scale * kLog2e;
+  p.r.block_stages = block_k / 64;
+  p.scores = scores; p.base = base_mask; p.target = target;
+  p.group_rows = q_group_size; p.G = (Lq + q_group_size - 1) / q_group_size; p.nK = p.r.key_blocks = (Lk + block_k - 1) / block_k;
+  return launch_block_scores(p, head_dim, (hipStream_t)stream);
+}
+
 static int csp_common(lvar_tensor_t q, lvar_tensor_t k, lvar_tensor_t v, lvar_tensor_t o_accum, int up_src, int up_dst,
                       lvar_tensor_t o, float* M, float* L, const int32_t* indices, const int32_t* counts, int G,
                       int64_t idx_row_stride, int group_rows, int B, int H, int Lq, int Lk, int head_dim,

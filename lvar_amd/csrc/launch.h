@@ -76,8 +76,23 @@ struct RowLseParams {
   int B, H, Lq, Lk;
   int kv_group;       // query heads per key head
   float c;
+  // block scores (null tsum: row statistics alone; no part: one key range)
+  float* tsum;        // sums per (workgroup, wave, key block, row of the wave)
+  float* first_ref;   // [B*H*Lq] the reference that the sums of a row count from
+  int block_stages;   // 64-key stages per key block
+  int key_blocks;
+  int* work;          // work[0] is cleared by the sweep
   int nrt, splits, split_keys, total_wg;   // set at launch
 };
+
+// Scores of key blocks from the sums that the row-statistics kernel keeps (see blockscore.hip)
+struct BlockScoreParams {
+  RowLseParams r;     // q, k, lse2, tsum, first_ref, work and the partition of the sweep
+  float* scores;      // [B*H, G, nK]
+  const uint8_t* base;  // [G, nK] always-on blocks, or null
+  int G, nK, group_rows, target;
+};
+int launch_block_scores(const BlockScoreParams& p, int head_dim, hipStream_t s);
 
 struct MaskListParams {
   const float* scores;     // [rows, nK]

@@ -12,6 +12,12 @@
 // at and, when it has outgrown LSE_SUM_LIMIT, its exponent moves into the reference (a power of two).  A logit that
 // lies more than 2^127 above the running sum overflows the sum; the wave then repeats its rows with a tracked maximum.
 // 64 rows per wave instead of the 32 of the attention kernel halve the LDS reads and the L2->LDS fills per flop.
+//
+// SCORES: the sweep also yields the softmax mass of every key block, summed over groups of query rows.  While a row's
+// log-sum-exp is not known yet, the sum of its exponentials over a block of keys can be kept against the row's first
+// reference (one float per row and block: 1/128 of the logits at 128-key blocks), and block_score_finish_kernel applies
+// exp2(reference - lse2) and adds the rows up.  The second sweep over all logits (the column sums) is not needed then:
+// B1 H24 d128, 8192 rows x 32768 keys, 128-key blocks: this sweep 1472 us, finish 58, refinement 14, in place of 1415 for the statistics and 1690 for the column sums.
 #include <type_traits>
 #include "common.h"
 #include "launch.h"
@@ -20,9 +26,10 @@ namespace lvar {
 
 constexpr float LSE_SUM_LIMIT = 65536.f;
 constexpr int ROW_LSE_STAGES = 2;   // depth of the LDS ring
+constexpr float SCORE_REF_LIMIT = 96.f;   // SCORES: largest distance (log2) of a row's reference from its first one
 constexpr int ROW_LSE_WGS = 3;      // workgroups per compute unit (head_dim 64 and 128): 168 registers per wave, 32 KiB of LDS
 
-template <int D>
+template <int D, bool SCORES>
 __global__ __launch_bounds__(256, (D <= 128 ? ROW_LSE_WGS : 1)) void row_lse_kernel(const RowLseParams p) {
 #if defined(__HIP_DEVICE_COMPILE__)
   constexpr int KS = D / 16;
@@ -37,6 +44,7 @@ __global__ __launch_bounds__(256, (D <= 128 ? ROW_LSE_WGS : 1)) void row_lse_ker
   // consecutive workgroup ids are dealt round-robin to the 8 XCDs: each XCD walks a contiguous range
   const int per_xcd = gridDim.x >> 3;
   const int w = (blockIdx.x & 7) * per_xcd + (blockIdx.x >> 3);
+  if (SCORES && blockIdx.x == 0 && threadIdx.x == 0) p.work[0] = 0;
   if (w >= p.total_wg) return;
   // workgroup = (batch*head, key range, tile of 256 query rows)
   const int per_bh = p.nrt * p.splits;
@@ -106,7 +114,33 @@ __global__ __launch_bounds__(256, (D <= 128 ? ROW_LSE_WGS : 1)) void row_lse_ker
   // kernel's row sum (even and odd elements of a 64-key stage apart; the two halves of the last stage apart), with the
   // same first reference: statistics of one key range have the bits that the attention kernel gives.
   float m[2], l[2] = {0.f, 0.f}, la[2], lb[2];
-
+  // SCORES: stages left in the open key block, and its sum against the first reference; lane = row of the wave (both
+  // halves of the keys added up), one register.  (Two sums, one per half, spill; sums in LDS cost the loop 40 %: an
+  // LDS atomic takes about 100 cycles.)  The first references sit in LDS and are read once a reference has moved.
+  int left = p.block_stages, blk = 0;
+  float bsum = 0.f;
+  bool moved = false;
+  float* const tp = SCORES ? p.tsum + ((int64_t)w * 4 + wave) * p.key_blocks * 64 : nullptr;
+  auto lane_id = []() {   // formed where it is needed: every register counts in the loop
+    int ln;
+    asm volatile("v_mbcnt_lo_u32_b32 %0, -1, 0\n\tv_mbcnt_hi_u32_b32 %0, -1, %0" : "=v"(ln));
+    return ln;
+  };
+  auto first = [&](int nt) -> LVAR_LDS float& { return ((LVAR_LDS float*)(smem + NSTAGE * KTILE))[wave * 128 + nt * 64 + lane_id()]; };
+  auto add_block = [&](float t0, float t1) {
+    if (moved) {
+      t0 *= fast_exp2(m[0] - first(0));
+      t1 *= fast_exp2(m[1] - first(1));
+    }
+    const auto sw = __builtin_amdgcn_permlane32_swap(__builtin_bit_cast(int, t0), __builtin_bit_cast(int, t1), false, false);
+    bsum += __builtin_bit_cast(float, (int)sw[0]) + __builtin_bit_cast(float, (int)sw[1]);
+  };
+  auto emit = [&]() {
+    tp[blk * 64 + lane_id()] = bsum;
+    bsum = 0.f;
+    blk++;
+    left = p.block_stages;
+  };
   // after a stage: when a sum has outgrown the limit its exponent moves into the reference
   auto renorm = [&]() {
     if (__builtin_amdgcn_ballot_w64(fmaxf(l[0], l[1]) > LSE_SUM_LIMIT) != 0) {
@@ -115,9 +149,12 @@ __global__ __launch_bounds__(256, (D <= 128 ? ROW_LSE_WGS : 1)) void row_lse_ker
         // exponent of the sum (an infinite one stays infinite whatever is taken off)
         const int e = (int)((__builtin_bit_cast(uint32_t, l[nt]) >> 23) & 255u) - 127;
         const int d = (l[nt] > LSE_SUM_LIMIT && e < 128) ? e : 0;
-        l[nt] = __builtin_amdgcn_ldexpf(l[nt], -d);
-        m[nt] += (float)d;
+        // (the reference rounds when the exponent is added to it: what it has not moved stays with the sums)
+        const float mn = m[nt] + (float)d, rest = fast_exp2((float)d - (mn - m[nt]));
+        l[nt] = __builtin_amdgcn_ldexpf(l[nt], -d) * rest;
+        m[nt] = mn;
       }
+      moved = true;
     }
   };
   const f32x16 zero = {0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0};   // constant addend of the first MFMA
@@ -210,8 +247,10 @@ __global__ __launch_bounds__(256, (D <= 128 ? ROW_LSE_WGS : 1)) void row_lse_ker
     }
     st_add(KS - 1);
     if (!OPENS) {
-      l[0] += la[0] + lb[0];
-      l[1] += la[1] + lb[1];
+      const float t0 = la[0] + lb[0], t1 = la[1] + lb[1];
+      l[0] += t0;
+      l[1] += t1;
+      if (SCORES) add_block(t0, t1);
       renorm();
     }
   };
@@ -230,6 +269,10 @@ __global__ __launch_bounds__(256, (D <= 128 ? ROW_LSE_WGS : 1)) void row_lse_ker
   if (S == 1) { mask_tile(0, sa0, sa1); mask_tile(1, sb0, sb1); }
   m[0] = xhalf_max(fmaxf(tile_max(sa0), tile_max(sb0))) * c;
   m[1] = xhalf_max(fmaxf(tile_max(sa1), tile_max(sb1))) * c;
+  if (SCORES) {
+    first(0) = m[0];
+    first(1) = m[1];
+  }
   if (S > 1) {
     la[0] = la[1] = lb[0] = lb[1] = 0.f;
 #pragma unroll
@@ -240,13 +283,19 @@ __global__ __launch_bounds__(256, (D <= 128 ? ROW_LSE_WGS : 1)) void row_lse_ker
     wait_fills(min(PF, S - 1) - 1);
     __syncthreads();
     for (int s = 1; s + 1 < S; s++) {
+      // (before the fills, so that one wait covers both, and with nothing conditional behind a step: the compiler
+      // moves a step's exponentials past it, out of the shadow of its matrix instructions)
+      if (SCORES && left == 0) emit();
       if (s + PF < S) issue_stage(s + PF);
       step(2 * s, sa0, sa1, sb0, sb1, no{}, no{});
+      if (SCORES) left--;
       step(2 * s + 1, sb0, sb1, sa0, sa1, yes{}, no{});
       wait_fills(min(s + PF, S - 1) - (s + 1));
       __syncthreads();
     }
+    if (SCORES && left == 0) emit();
     step(2 * S - 2, sa0, sa1, sb0, sb1, no{}, no{});
+    if (SCORES && --left == 0) emit();
     if (U & 1) {
       mask_tile(U - 1, sa0, sa1);
       tile_sum(sa0, sa1, la);
@@ -262,12 +311,16 @@ __global__ __launch_bounds__(256, (D <= 128 ? ROW_LSE_WGS : 1)) void row_lse_ker
   }
   l[0] += la[0] + lb[0];
   l[1] += la[1] + lb[1];
+  if (SCORES) {
+    add_block(la[0] + lb[0], la[1] + lb[1]);
+    emit();
+  }
 
-  if (__builtin_amdgcn_ballot_w64(!(fmaxf(l[0], l[1]) < INFINITY)) != 0) {
+  bool again = !(fmaxf(l[0], l[1]) < INFINITY);
+  if (SCORES) again = again || fmaxf(m[0] - first(0), m[1] - first(1)) > SCORE_REF_LIMIT;
+  if (__builtin_amdgcn_ballot_w64(again) != 0) {
     // a sum has overflowed: this wave's rows again, straight from memory, with the maximum tracked tile by tile
-    l[0] = l[1] = 0.f;
-    m[0] = m[1] = -1.0e30f;
-    for (int u = 0; u < U; u++) {
+    auto tile_mem = [&](int u) {
       const bf16_t* kp = kbase + (int64_t)min(koff + u * 32 + r, p.Lk - 1) * p.k_sr + hh * 8;
       sa0 = zero;
       sa1 = zero;
@@ -278,6 +331,11 @@ __global__ __launch_bounds__(256, (D <= 128 ? ROW_LSE_WGS : 1)) void row_lse_ker
         sa1 = mfma32(kfr, qf[1][ks], sa1);
       }
       mask_tile(u, sa0, sa1);
+    };
+    l[0] = l[1] = 0.f;
+    m[0] = m[1] = -1.0e30f;
+    for (int u = 0; u < U; u++) {
+      tile_mem(u);
 #pragma unroll
       for (int nt = 0; nt < 2; nt++) {
         const f32x16& s = nt ? sa1 : sa0;
@@ -287,6 +345,28 @@ __global__ __launch_bounds__(256, (D <= 128 ? ROW_LSE_WGS : 1)) void row_lse_ker
         for (int i = 0; i < 16; i++) t += fast_exp2(fmaf(s[i], c, -m_new));
         l[nt] = fmaf(l[nt], fast_exp2(m[nt] - m_new), t);
         m[nt] = m_new;
+      }
+    }
+    if (SCORES) {
+      // and the block sums against that maximum (`blk` is past the end: the stores of the first sweep are overwritten)
+#pragma unroll
+      for (int nt = 0; nt < 2; nt++) {
+        const float mm = xhalf_max(m[nt]);
+        l[nt] *= fast_exp2(m[nt] - mm);
+        m[nt] = first(nt) = mm;
+      }
+      blk = 0;
+      moved = false;
+      for (int u = 0; u < U; u++) {
+        tile_mem(u);
+        float t0 = 0.f, t1 = 0.f;
+#pragma unroll
+        for (int i = 0; i < 16; i++) {
+          t0 += fast_exp2(fmaf(sa0[i], c, -m[0]));
+          t1 += fast_exp2(fmaf(sa1[i], c, -m[1]));
+        }
+        add_block(t0, t1);
+        if (u + 1 == U || (u + 1) % (2 * p.block_stages) == 0) emit();
       }
     }
   }
@@ -300,6 +380,7 @@ __global__ __launch_bounds__(256, (D <= 128 ? ROW_LSE_WGS : 1)) void row_lse_ker
     const float ll = xhalf_sum(l[nt] * fast_exp2(fminf(m[nt] - mm, 0.f)));
     const int row = n0 + nt * 32 + r;
     if (hh == 0 && row < p.Lq) {
+      if (SCORES) p.first_ref[row0 + row] = first(nt);
       if (p.splits == 1) {
         p.lse2[row0 + row] = mm + __builtin_amdgcn_logf(ll);
       } else {
@@ -360,7 +441,7 @@ int row_lse_splits(int B, int H, int Lq, int Lk) {
   return best_n;
 }
 
-template <int D>
+template <int D, bool SCORES>
 static int launch_rl(const RowLseParams& p0, hipStream_t stream) {
   RowLseParams p = p0;
   if (p.kv_group < 1) p.kv_group = 1;
@@ -372,10 +453,10 @@ static int launch_rl(const RowLseParams& p0, hipStream_t stream) {
   p.split_keys = per * 64;
   p.total_wg = p.B * p.H * p.nrt * p.splits;
   const int grid = ((p.total_wg + 7) / 8) * 8;
-  constexpr int SMEM = ROW_LSE_STAGES * 64 * D * 2;
+  constexpr int SMEM = ROW_LSE_STAGES * 64 * D * 2 + (SCORES ? 4 * 128 * 4 : 0);
   static std::atomic<uint64_t> lds_ready{0};
-  if (!ensure_lds_limit((const void*)row_lse_kernel<D>, SMEM, lds_ready)) return LVAR_ELAUNCH;
-  hipLaunchKernelGGL((row_lse_kernel<D>), dim3(grid), dim3(256), SMEM, stream, p);
+  if (!ensure_lds_limit((const void*)row_lse_kernel<D, SCORES>, SMEM, lds_ready)) return LVAR_ELAUNCH;
+  hipLaunchKernelGGL((row_lse_kernel<D, SCORES>), dim3(grid), dim3(256), SMEM, stream, p);
   if (hipGetLastError() != hipSuccess) return LVAR_ELAUNCH;
   if (p.splits > 1) {
     const int64_t rows = (int64_t)p.B * p.H * p.Lq;
@@ -386,9 +467,15 @@ static int launch_rl(const RowLseParams& p0, hipStream_t stream) {
 }
 
 int launch_row_lse(const RowLseParams& p, int head_dim, hipStream_t s) {
-  if (head_dim == 128) return launch_rl<128>(p, s);
-  if (head_dim == 64) return launch_rl<64>(p, s);
-  if (head_dim == 256) return launch_rl<256>(p, s);
+  if (p.tsum) {
+    if (head_dim == 128) return launch_rl<128, true>(p, s);
+    if (head_dim == 64) return launch_rl<64, true>(p, s);
+    if (head_dim == 256) return launch_rl<256, true>(p, s);
+    return LVAR_EUNSUPPORTED;
+  }
+  if (head_dim == 128) return launch_rl<128, false>(p, s);
+  if (head_dim == 64) return launch_rl<64, false>(p, s);
+  if (head_dim == 256) return launch_rl<256, false>(p, s);
   return LVAR_EUNSUPPORTED;
 }
 

@@ -312,9 +312,10 @@ def video_window_topk_block_lists(q: torch.Tensor, k: torch.Tensor, scale=None, 
     nK = (Lk + block - 1) // block
     base = video_window_base_mask(frames, height, width, block, device=q.device)
     rows = q[:, :, ::query_stride]
-    if block % 64 == 0 and q.shape[-1] >= 64:      # block sums straight from the colsum kernel
-        score = ops._colsum_block_scores(rows, k, scale, block // query_stride, block)
+    target = int(round(density * nK))
+    if block % 64 == 0 and q.shape[-1] >= 64:      # block sums without the column sums themselves
+        score = ops._block_scores_for_topk(rows, k, scale, block // query_stride, block, base, target)
     else:
         score = key_block_sums(ops.colsum(rows, k, scale, q_group_size=block // query_stride), block).contiguous()
-    num, idx = ops.block_topk_lists(score, int(round(density * nK)), base)
+    num, idx = ops.block_topk_lists(score, target, base)
     return num, idx, score

@@ -305,6 +305,29 @@ def _colsum_block_scores(q, k, scale, q_group_size: int, block_k: int):
     return torch.nn.functional.pad(bs, (0, -bs.shape[-1] % m)).unflatten(-1, (-1, m)).sum(-1)
 
 
+def _block_scores_for_topk(q, k, scale, q_group_size: int, block_k: int, base_mask, target: int):
+    """Block scores that :func:`block_topk_lists` will rank with ``base_mask`` and ``target``, from one sweep over the
+    logits: the blocks it selects are those that the sums of :func:`_colsum_block_scores` select, the scores themselves
+    agree to the rounding of 32-bit sums.  Group sizes without a one-sweep kernel, and rows of more blocks than it can
+    compare, take the two-pass form."""
+    B, H, Lq, d = q.shape
+    Lk = k.shape[2]
+    nK = (Lk + block_k - 1) // block_k
+    if not (q_group_size == 32 or (q_group_size % 64 == 0 and q_group_size <= 1024)) or nK > 2048 or target <= 0:
+        return _colsum_block_scores(q, k, scale, q_group_size, block_k)
+    q, k = _prep(q, "q"), _prep(k, "k")
+    _check_qkv(q, k, k, gqa=True)
+    scores = torch.empty((B, H, (Lq + q_group_size - 1) // q_group_size, nK), dtype=torch.float32, device=q.device)
+    lib = _lib.load()
+    with _on_device(q):
+        nbytes = int(lib.lvar_block_scores_scratch_bytes(B, H, Lq, Lk, q_group_size, block_k))
+        scratch = torch.empty(nbytes, dtype=torch.uint8, device=q.device)
+        st = lib.lvar_block_scores_fwd(_view(q), _view(k), scores.data_ptr(), _ptr(base_mask), target, scratch.data_ptr(), nbytes,
+                                       B, H, k.shape[1], Lq, Lk, d, q_group_size, block_k, _scale(q, scale), _stream(q))
+    _lib.check(st, "lvar_block_scores_fwd")
+    return scores
+
+
 def dense_colsum_attn(q, k, v, scale=None):
     """Kernel-level op ``(o, blocksums, (M, L))`` (reference Triton ``dense_colsum_attn``,
     kernels/sparse_attn/triton/attn_dense_colsum.py:237-296): dense attention, then the column

@@ -65,3 +65,69 @@ def test_block_scores_without_the_column_sums():
     cs = ops.colsum(rows, k, None, q_group_size=32)
     ref = torch.nn.functional.pad(cs, (0, 68)).unflatten(-1, (6, 128)).sum(-1)
     assert got.shape == ref.shape and torch.allclose(got, ref, rtol=1e-5, atol=0)   # 128 terms in another order: 128 * 2^-24
+
+
+# ---- scores of key blocks from the statistics sweep ----
+
+def _scores_ref(q, k, scale, group, block_k):
+    k = k.repeat_interleave(q.shape[1] // k.shape[1], dim=1)
+    p = (torch.matmul(q.double().cpu(), k.double().cpu().transpose(-1, -2)) * scale).softmax(-1)
+    Lq, Lk = p.shape[-2:]
+    p = torch.nn.functional.pad(p, (0, -Lk % block_k, 0, -Lq % group))
+    return p.unflatten(-1, (-1, block_k)).sum(-1).unflatten(-2, (-1, group)).sum(-2)
+
+
+def _check_scores(q, k, scale, group, block_k, target, base=None):
+    from lvar_amd import sparse_attn_ops as ops
+    got = ops._block_scores_for_topk(q, k, scale, group, block_k, base, target)
+    ref = _scores_ref(q, k, scale, group, block_k)
+    assert got.shape == ref.shape
+    # exponents carry 2^-24 of the largest logit and statistic (log2 units, < 2^11 here): 2^-13 ln2 relative, far less
+    # for plain inputs; what lies 2^-100 below the largest score is not looked at
+    big = float(ref.abs().max())
+    assert torch.allclose(got.double().cpu(), ref, rtol=2e-4, atol=big * 1e-6), float((got.double().cpu() - ref).abs().max())
+    two_pass = ops._colsum_block_scores(q, k, scale, group, block_k)
+    lists, lists2 = ops.block_topk_lists(got, target, base), ops.block_topk_lists(two_pass, target, base)
+    assert torch.equal(lists[0], lists2[0]) and torch.equal(lists[1], lists2[1])
+
+
+@pytest.mark.parametrize("B,H,Hkv,Lq,Lk,d,group,block_k", [
+    (1, 1, 1, 1, 1, 128, 32, 128), (1, 2, 2, 33, 64, 64, 32, 64), (2, 2, 1, 95, 129, 128, 32, 128), (1, 3, 3, 256, 257, 128, 64, 128),
+    (1, 2, 2, 300, 1000, 256, 128, 128), (1, 2, 2, 513, 2049, 64, 32, 128), (2, 2, 2, 700, 1500, 128, 128, 64), (1, 4, 2, 1024, 4096, 128, 32, 128),
+    (1, 3, 3, 200, 640, 128, 96, 128), (1, 24, 24, 2048, 1024, 64, 32, 128), (1, 40, 40, 2048, 704, 128, 64, 64),
+])
+def test_block_scores_sizes(B, H, Hkv, Lq, Lk, d, group, block_k):
+    """Edges of stages, key blocks, key ranges, wave tiles and groups (96: the two-pass form)."""
+    g = torch.Generator().manual_seed(Lq + 3 * Lk)
+    q = (torch.randn(B, H, Lq, d, generator=g) * 0.5).to(torch.bfloat16).cuda()
+    k = (torch.randn(B, Hkv, Lk, d, generator=g) * 0.5).to(torch.bfloat16).cuda()
+    nQ, nK = -(-Lq // group), -(-Lk // block_k)
+    base = (torch.rand(nQ, nK, generator=g) < 0.2).cuda()
+    _check_scores(q, k, d ** -0.5, group, block_k, max(1, nK // 3), base)
+    _check_scores(q, k, d ** -0.5, group, block_k, max(1, nK // 2))
+
+
+@pytest.mark.parametrize("kind", ["ramp_up", "ramp_down", "late_spike", "first_tile_low"])
+def test_block_scores_references_far_from_the_first_tile(kind):
+    g = torch.Generator().manual_seed(4)
+    Lq, Lk, d = 200, 700, 128
+    q = torch.zeros(1, 2, Lq, d)
+    q[..., 0] = 1.0
+    q[..., 1:] = torch.randn(1, 2, Lq, d - 1, generator=g) * 0.05
+    k = torch.randn(1, 2, Lk, d, generator=g) * 0.05
+    n = torch.arange(Lk, dtype=torch.float32)
+    k[..., 0] = {"ramp_up": n * 2.0, "ramp_down": -n * 2.0, "late_spike": torch.where(n == 500, 900.0, 0.0),
+                 "first_tile_low": torch.where(n < 40, -800.0, 3.0)}[kind]
+    q[:, :, ::3, 0] = 0.25
+    _check_scores(q.to(torch.bfloat16).cuda(), k.to(torch.bfloat16).cuda(), 1.0, 32, 128, 2)
+
+
+def test_block_scores_ties_at_the_cut():
+    """Equal key blocks in other orders: the two-pass ranking decides (one key range: the statistics have equal bits)."""
+    g = torch.Generator().manual_seed(6)
+    q = (torch.randn(1, 8, 1024, 128, generator=g) * 0.5).to(torch.bfloat16).cuda()
+    one = torch.randn(1, 8, 1, 128, 128, generator=g) * 0.5
+    k = one.repeat(1, 1, 3, 1, 1).to(torch.bfloat16)
+    for j in range(1, 3):
+        k[:, :, j] = k[:, :, j, torch.randperm(128, generator=g)]
+    _check_scores(q, k.flatten(2, 3).contiguous().cuda(), 128 ** -0.5, 32, 128, 2)
