@@ -1122,6 +1122,17 @@ static int launch_one(const AttnParams& p0, hipStream_t stream) {
   return hipGetLastError() == hipSuccess ? LVAR_OK : LVAR_ELAUNCH;
 }
 
+// Token lists at head_dim 64: 192-row groups as two 3-wave workgroups (several share a compute unit, each fetches for
+// itself) instead of one of 8 waves, with the same bits, where the 8-wave workgroups leave their last round at most half
+// full.  832 / 2560 keys per list, 8-wave against 3-wave: 96 groups 18.9 / 43.2 against 16.3 / 37.7 us, 384 groups 36.2 /
+// 84.3 against 32.7 / 79.2 us; full rounds the other way (256 groups 20.7 / 44.9 against 23.2 / 52.1 us, 704 groups 53.3 /
+// 127 against 56.2 / 140 us).  From the fourth round on the choice is within a few percent and stays.  (At head_dim 128 the
+// 3-wave form wins only on nearly empty launches: 16 groups 25.1 against 23.2 us, 96 groups 27.1 against 27.9 us.)
+static bool three_wave_groups(const AttnParams& p) {
+  const int64_t n = (int64_t)p.B * p.H * ((p.Lq + 191) / 192), cus = device_cus();
+  return cus > 0 && p.group_rows % 192 == 0 && n < 3 * cus && n % cus != 0 && 2 * (n % cus) <= cus;
+}
+
 template <int D>
 static int launch_d(const AttnParams& p, int mode, bool accum, bool lse_only, int nwaves, hipStream_t s) {
   if (mode == MODE_BLOCK) {
@@ -1131,6 +1142,7 @@ static int launch_d(const AttnParams& p, int mode, bool accum, bool lse_only, in
   } else if (mode == MODE_GATHER) {
     // (head_dim 256: a wave needs more than 256 registers, so one wave per SIMD: 192-row groups run as two 3-wave workgroups)
     if constexpr (D > 128) { if (nwaves == 8) nwaves = 3; }
+    else if (D == 64 && nwaves == 8 && !p.sk_ws && three_wave_groups(p)) return launch_one<D, 3, MODE_GATHER, true, false>(p, s);
     else if (nwaves == 8) return launch_one<D, 8, MODE_GATHER, true, false>(p, s);
     if (nwaves == 3) return launch_one<D, 3, MODE_GATHER, true, false>(p, s);
     if (nwaves == 2) return launch_one<D, 2, MODE_GATHER, true, false>(p, s);

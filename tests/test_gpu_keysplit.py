@@ -92,3 +92,18 @@ def test_block_lists_of_several_workgroups(B, H, Lq, Lk, d, bq, bk):
     m = m.repeat_interleave(bq, 0)[:Lq].repeat_interleave(bk, 1)[:, :Lk]
     s = (torch.matmul(q.float(), k.float().transpose(-1, -2).contiguous()) * d ** -0.5).masked_fill(~m, float("-inf"))
     assert torch.allclose(ref.float(), torch.matmul(s.softmax(-1).nan_to_num(0.0), v.float()), atol=2e-2, rtol=1e-2)
+
+
+@pytest.mark.parametrize("H,G", [(40, 2), (128, 1), (130, 1), (80, 2), (150, 2), (200, 2)])
+def test_token_lists_head_dim_64_both_workgroup_shapes(H, G):
+    """192-row groups run as 8-wave or as two 3-wave workgroups, by how full the last round of 8-wave ones is: the same
+    bits as with the lists repeated for groups of 96 rows (which always take the 3-wave form)."""
+    from test_gpu_random_shapes import _csp_abi
+    g = torch.Generator(device="cuda").manual_seed(H + G)
+    Lq, Lk, d = G * 192 - 37, 330, 64
+    q, o0, k, v = (torch.randn(1, H, L, d, generator=g, device="cuda").to(torch.bfloat16) for L in (Lq, Lq, Lk, Lk))
+    idx = torch.randint(0, Lk, (1, H, G, Lk), generator=g, device="cuda", dtype=torch.int32)
+    cnt = torch.randint(0, Lk + 1, (1, H, G), generator=g, device="cuda", dtype=torch.int32)
+    st, out = _csp_abi(q, k, v, idx, cnt, o0, 192, -1)
+    st2, out2 = _csp_abi(q, k, v, idx.repeat_interleave(2, dim=2).contiguous(), cnt.repeat_interleave(2, dim=2).contiguous(), o0, 96, -1)
+    assert st == 0 and st2 == 0 and torch.equal(out, out2)
