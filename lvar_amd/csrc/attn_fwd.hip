@@ -1021,18 +1021,19 @@ __global__ __launch_bounds__(256) void plan_kernel(const AttnParams p, int* plan
 // with one wave per SIMD, split the keys of a query tile over two teams.  With at most one 64-row tile per compute unit:
 // 64 rows per workgroup, twice as many compute units at work and half the walk for each (B2 H16 d128, 400 x 921: 18.7 ->
 // 13.7 us, 256 x 521: 13.0 -> 10.5 us).  With at most one 128-row tile per compute unit: 128 rows, two waves per SIMD,
-// which walk two tiles in 1.6 of the time of one (576 x 1497: 27.6 -> 24.9 us, 1024 x 2521: 47.6 -> 45.2 us).  Beyond
-// that the second resident workgroup does the same without a merge.  The merge costs about a microsecond, so lists of a
+// which walk two tiles in 1.6 of the time of one (576 x 1497: 27.6 -> 24.9 us, 1024 x 2521: 47.6 -> 45.2 us); short
+// walks do not pay for the merge at head_dim 128 (B2 H16, 676 x 696, 11 tiles: 16.1 -> 17.0 us; 17 tiles: 23.6 -> 23.3 us),
+// at head_dim 64 they do from 8 tiles on (11 tiles: 15.6 -> 13.4 us).  Beyond that the second resident workgroup does the same without a merge.  The merge costs about a microsecond, so lists of a
 // few tiles are walked by one team (the length of a block list is known to the device only; the width of the table
 // stands in for it).  A launch whose row statistic feeds a ranking (LSE2 without M and L: the decision-scale step, whose
 // column sums become top-k lists) keeps one team: two add the rows up in another order, and close scores would change
 // places with the launch shape.
-static int two_team_rows(const AttnParams& p, int nwaves) {
+static int two_team_rows(const AttnParams& p, int nwaves, int head_dim) {
   if (p.LSE2 && !p.M) return 0;
   const int64_t all = (p.Lk + 63) / 64, tiles = p.list ? std::min((int64_t)p.list_len << p.sub_shift, all) : all;
   const int64_t bh = (int64_t)p.B * p.H, cus = device_cus();
   if (tiles >= 4 && bh * ((p.Lq + 63) / 64) <= cus) return 64;
-  if (tiles >= 8 && nwaves == 4 && bh * ((p.Lq + 127) / 128) <= cus) return 128;
+  if (tiles >= (head_dim == 64 ? 8 : 16) && nwaves == 4 && bh * ((p.Lq + 127) / 128) <= cus) return 128;
   return 0;
 }
 
@@ -1108,7 +1109,7 @@ static int launch_one(const AttnParams& p0, hipStream_t stream) {
   }
   if constexpr (MODE == MODE_BLOCK && !LSE_ONLY && KSPLIT == 1 && !WIDE && D <= 128) {
     if (NWAVES == 4 && wide_tiles(p0, D)) return launch_one<D, 8, MODE_BLOCK, false, false, 1>(p0, stream);
-    const int rows = two_team_rows(p0, NWAVES);
+    const int rows = two_team_rows(p0, NWAVES, D);
     AttnParams p2 = p0;
     p2.sk_ws = nullptr;
     if (rows == 64) return launch_one<D, 4, MODE_BLOCK, false, false, 2>(p2, stream);

@@ -13,10 +13,11 @@ def _close(o, ref):
     assert torch.allclose(o.float().cpu(), ref, atol=2e-2, rtol=1e-2)
 
 
-# (B*H) * ceil(Lq/64) <= 256 takes 64-row workgroups from 4 tiles on, (B*H) * ceil(Lq/128) <= 256 128-row ones from 8
+# (B*H) * ceil(Lq/64) <= 256 takes 64-row workgroups from 4 tiles on, (B*H) * ceil(Lq/128) <= 256 128-row ones from 8 (head_dim 64) or 16
 @pytest.mark.parametrize("B,H,Hkv,Lq,Lk,d", [
     (1, 2, 2, 1, 193, 128), (1, 2, 2, 64, 256, 128), (2, 2, 1, 65, 257, 64), (1, 3, 3, 129, 319, 128), (1, 2, 2, 200, 449, 64),
     (1, 140, 140, 128, 512, 128), (1, 140, 140, 100, 577, 128), (1, 130, 65, 127, 513, 64), (2, 64, 64, 200, 640, 64),
+    (1, 140, 140, 128, 1024, 128), (1, 140, 140, 100, 1090, 128),
 ])
 def test_dense_two_teams(B, H, Hkv, Lq, Lk, d):
     from lvar_amd import sparse_attn_ops as ops
@@ -57,7 +58,7 @@ def test_dense_two_teams_growing_logits():
 
 
 @pytest.mark.parametrize("H,Lq,Lk,d,bq,bk", [(2, 300, 1000, 128, 128, 64), (3, 130, 900, 64, 128, 128), (2, 200, 1100, 128, 64, 64),
-                                             (140, 128, 1024, 128, 128, 64), (135, 120, 1300, 64, 128, 256)])
+                                             (140, 128, 1024, 128, 128, 64), (135, 120, 1300, 64, 128, 256), (140, 120, 1000, 128, 128, 64)])
 def test_block_lists_two_teams(H, Lq, Lk, d, bq, bk):
     from lvar_amd import sparse_attn_ops as ops
     q, k, v = make_qkv(1, H, Lq, Lk, d, seed=Lq)
