@@ -83,8 +83,9 @@ const char* lvar_status_string(int status);
  * kernels/chipmunk/csrc/attn/dense_attn.cu:248-372) and sattn_triton.dense_attn
  * (kernels/sparse_attn/triton/attn_dense.py:186-231).
  * LSE2, if not NULL, receives the base-2 log-sum-exp M + log2(L) (fp32 [B,H,Lq]), the form the
- * colsum entry point consumes.  o may be NULL (statistics only); M, L and LSE2 may each be NULL.  With LSE2 and without M
- * the rows are summed in one order whatever workgroup shape the launch takes, so that rankings built on it do not move.
+ * colsum entry point consumes.  o may be NULL (statistics only); M, L and LSE2 may each be NULL.  The plain
+ * launch sums a query row in one order whatever workgroup shape it takes: the outputs of a (batch, head) do not depend on
+ * how many others the call holds, and neither do rankings built on them.
  * head_dim in {64, 128, 256} (256: one wave per SIMD with 512 registers and 128 KiB of LDS per workgroup, always
  * the plain launch; built for coverage of the reference's Triton range, kernels/sparse_attn/triton/
  * attn_dense_colsum.py:246, not tuned).  This holds for every attention, colsum and window-score entry point

@@ -22,7 +22,6 @@
 // Softmax runs in the exp2 domain with a lazily updated reference maximum: accumulators are
 // rescaled only when some row maximum grows by more than RESCALE_TAU, which is exact
 // because numerator and denominator share the same reference.
-#include <algorithm>
 #include <type_traits>
 #include "common.h"
 #include "launch.h"
@@ -67,11 +66,11 @@ struct Swz {
   __device__ static __forceinline__ int fv(int row) { return (D >= 128) ? ((row & 3) << 2) : (((row >> 1) & 1) << 2); }
 };
 
-// LDS of a workgroup: K and V buffers of every team; the epilogue's transpose buffer of eight computing waves is larger
-template <int D, int NWAVES, int MODE, int KSPLIT>
+// LDS of a workgroup: K and V buffers; the epilogue's transpose buffer of eight computing waves is larger
+template <int D, int NWAVES, int MODE>
 constexpr int attn_lds_bytes() {
-  const int bufs = KSPLIT * 4 * 64 * D * 2, epi = NWAVES * 32 * (D * 2 + 16);
-  return (MODE == MODE_BLOCK && KSPLIT == 1 && epi > bufs) ? epi : bufs;
+  const int bufs = 4 * 64 * D * 2, epi = NWAVES * 32 * (D * 2 + 16);
+  return (MODE == MODE_BLOCK && epi > bufs) ? epi : bufs;
 }
 
 // Context of a balanced launch (see sk_partition.h); unused by the plain launch.
@@ -84,9 +83,7 @@ struct SkCtx {
 };
 
 // One query tile w (or, in a balanced launch, the units [u0, u1) of its tile list; `whole` = all of them).
-// KSPLIT = 2: the waves form two teams that share the query rows and take every other tile of the list, each with K/V
-// buffers of its own; the second team hands its accumulators over through LDS at the end.
-template <int D, int NWAVES, int MODE, bool ACCUM, bool LSE_ONLY, bool SK, int KSPLIT = 1>
+template <int D, int NWAVES, int MODE, bool ACCUM, bool LSE_ONLY, bool SK>
 __device__ __forceinline__ void attn_item(const AttnParams& p, char* smem, const int w, const int u0, const int u1,
                                           const bool whole, const SkCtx& sk) {
   // Token lists with 8 waves: waves 0..5 compute (one 192-row group), waves 6 and 7 only fetch -- they read
@@ -94,8 +91,8 @@ __device__ __forceinline__ void attn_item(const AttnParams& p, char* smem, const
   // slots of a CU; the two fetch waves take the idle ones and the compute waves lose ~10 % of their
   // instructions.  Everywhere else all waves do both.
   constexpr int NPROD = (MODE == MODE_GATHER && NWAVES == 8) ? 2 : 0;
-  constexpr int NCOMP = (NWAVES - NPROD) / KSPLIT;     // computing waves (of a team), 32 query rows each
-  constexpr int FW = NPROD ? NPROD : NCOMP;  // waves that issue the fills (of a team)
+  constexpr int NCOMP = NWAVES - NPROD;     // computing waves, 32 query rows each
+  constexpr int FW = NPROD ? NPROD : NWAVES;  // waves that issue the fills
   constexpr int WGROWS = NCOMP * 32;
   constexpr int KS = D / 16, MTD = D / 32;
   constexpr int ROWB = Swz<D>::ROWB, CPR = Swz<D>::CPR;
@@ -107,16 +104,13 @@ __device__ __forceinline__ void attn_item(const AttnParams& p, char* smem, const
   constexpr bool CONST_OFF = MODE == MODE_BLOCK && ((FW * RPI) % 16 == 0 || 16 % (FW * RPI) == 0) && NI % FW == 0;
   constexpr int CONST_PER = (FW * RPI) >= 16 ? 1 : 16 / (FW * RPI);
   constexpr int OSTR = D * 2 + 16;  // epilogue transpose buffer row stride (bytes)
-  static_assert(NCOMP * 32 * OSTR <= attn_lds_bytes<D, NWAVES, MODE, KSPLIT>(), "the epilogue buffer must fit");
-  static_assert(KSPLIT == 1 || (KSPLIT == 2 && MODE == MODE_BLOCK && !SK && !ACCUM && NPROD == 0), "two teams: block lists and dense attention");
-  // LDS map: K buffers at 0 and TILE, V buffers at 2*TILE and 3*TILE (the second team's follow)
+  static_assert(NCOMP * 32 * OSTR <= attn_lds_bytes<D, NWAVES, MODE>(), "the epilogue buffer must fit");
+  // LDS map: K buffers at 0 and TILE, V buffers at 2*TILE and 3*TILE
 
   const int bh = w / p.nqt, qt = w - bh * p.nqt;
   const int b = bh / p.H, h = bh - b * p.H;
   const int tid = threadIdx.x, lane = tid & 63;
-  const int wave_id = __builtin_amdgcn_readfirstlane(tid >> 6);
-  const int team = KSPLIT > 1 ? wave_id / NCOMP : 0, wave = wave_id - team * NCOMP;   // wave: index inside the team
-  char* const tbuf = smem + team * (4 * TILE);                                          // this team's K/V buffers
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int hh = lane >> 5, r = lane & 31;
   const int fwave = NPROD ? wave - NCOMP : wave;   // index among the filling waves (negative: this wave does not fill)
   const int q0 = qt * WGROWS;
@@ -135,15 +129,14 @@ __device__ __forceinline__ void attn_item(const AttnParams& p, char* smem, const
   if (identity) {
     count = (p.Lk + 63) >> 6;
     if (SK) { tile0 = u0; count = max(0, min(u1, count) - u0); }
-    T = (count + KSPLIT - 1) / KSPLIT;   // (a tile of the last round that the list does not have is masked as a whole)
+    T = count;
   } else {
     list = p.list + b * p.list_sb + h * p.list_sh + (int64_t)g * p.list_sg;
     const int first = SK ? (MODE == MODE_BLOCK ? u0 : (u0 << 6)) : 0;   // first list entry of this piece
     if (MODE == MODE_BLOCK) {
 #pragma unroll
       for (int i = 0; i < 4; i++)
-        if (KSPLIT == 1) { if (first + i < p.list_len) head[i] = list[first + i]; }
-        else { const int e = (i * KSPLIT + team) >> p.sub_shift; if (e < p.list_len) head[i] = list[e]; }
+        if (first + i < p.list_len) head[i] = list[first + i];
     }
     count = max(0, min(p.cnt[b * p.cnt_sb + h * p.cnt_sh + g], p.list_len));
     avail = p.list_len - first;
@@ -152,7 +145,7 @@ __device__ __forceinline__ void attn_item(const AttnParams& p, char* smem, const
       count = max(0, min(count, last) - first);
       list += first;
     }
-    T = (MODE == MODE_BLOCK) ? ((count << p.sub_shift) + KSPLIT - 1) / KSPLIT : ((count + 63) >> 6);
+    T = (MODE == MODE_BLOCK) ? (count << p.sub_shift) : ((count + 63) >> 6);
   }
   const int sub_shift = identity ? 0 : p.sub_shift;
 
@@ -179,7 +172,7 @@ __device__ __forceinline__ void attn_item(const AttnParams& p, char* smem, const
     const int hkv = h / p.kv_group;   // grouped-query attention: kv_group query heads share a K/V head
     const i32x4 krsrc = make_rsrc(p.k + b * p.k_sb + hkv * p.k_sh, (p.Lk - 1) * k_srb + ROWB);
     const i32x4 vrsrc = make_rsrc(p.v + b * p.v_sb + hkv * p.v_sh, (p.Lk - 1) * v_srb + ROWB);
-    const uint32_t lds0 = (uint32_t)(uintptr_t)(LVAR_LDS char*)tbuf;
+    const uint32_t lds0 = (uint32_t)(uintptr_t)(LVAR_LDS char*)smem;
 
     // per-lane role in a tile load: row (within the RPI rows of one instruction) and chunk slot
     const int lrow = lane / CPR, lcs = lane % CPR;
@@ -192,8 +185,7 @@ __device__ __forceinline__ void attn_item(const AttnParams& p, char* smem, const
     constexpr int NR = (MODE == MODE_GATHER) ? SLOTS : 1;
     auto prefetch_raw = [&](int t, int (&raw)[NR]) {
       if (MODE == MODE_BLOCK) {
-        const int tt = t * KSPLIT + team;
-        raw[0] = identity ? tt + tile0 : list[KSPLIT == 1 ? t >> sub_shift : min(tt >> sub_shift, count - 1)];
+        raw[0] = identity ? t + tile0 : list[t >> sub_shift];
       } else {
         // bounded by the row of the list, not by the count: entries behind the count are never used (they are
         // clamped and masked), and the read then does not have to wait for the count to arrive
@@ -209,10 +201,8 @@ __device__ __forceinline__ void attn_item(const AttnParams& p, char* smem, const
       if (MODE == MODE_BLOCK) {
         // a block index outside the key range (a caller's mistake) is clamped before it is scaled
         const int blk = max(0, min(__builtin_amdgcn_readfirstlane(raw[0]), (p.Lk - 1) >> (6 + sub_shift)));
-        const int tt = t * KSPLIT + team;
-        rows[0] = ((blk << sub_shift) + (tt & ((1 << sub_shift) - 1))) << 6;
+        rows[0] = ((blk << sub_shift) + (t & ((1 << sub_shift) - 1))) << 6;
         nvalid = max(0, min(64, p.Lk - rows[0]));
-        if (KSPLIT > 1 && (tt >> sub_shift) >= count) nvalid = 0;
       } else {
         nvalid = min(64, count - (t << 6));
 #pragma unroll
@@ -421,7 +411,7 @@ __device__ __forceinline__ void attn_item(const AttnParams& p, char* smem, const
       // tiles 0..3: block lists use the entries read next to the count
       auto first_raw = [&](int t, int (&raw)[NR]) {
         if (MODE == MODE_BLOCK && !identity) {
-          const int e = KSPLIT == 1 ? t >> sub_shift : t;   // (two teams: head holds the blocks of this team's tiles)
+          const int e = t >> sub_shift;
           raw[0] = (e == 0) ? head[0] : (e == 1) ? head[1] : (e == 2) ? head[2] : head[3];
         } else {
           prefetch_raw(t, raw);
@@ -452,7 +442,7 @@ __device__ __forceinline__ void attn_item(const AttnParams& p, char* smem, const
     __builtin_amdgcn_s_waitcnt(0x0f70);  // vmcnt(0): this wave's LDS fills have landed
     __syncthreads();
     f32x16 sa0, sa1, sb0, sb1;
-    qk_tile(tbuf, sa0, sa1);
+    qk_tile(smem, sa0, sa1);
     // K(2) is fetched into the buffer of K(0) at the top of the first iteration: every wave must have read
     // K(0) before any wave issues that fill
     __syncthreads();
@@ -501,8 +491,8 @@ __device__ __forceinline__ void attn_item(const AttnParams& p, char* smem, const
       // S(t).  Phase B: PV MFMA j | the two transposing V reads of MFMA j+4 | the last softmax slots
       // of S(t) (first half) or a slice of the row-maximum reduction of S(t+1) (second half).
       constexpr int NQK = 2 * KS, NPV = LSE_ONLY ? 0 : 4 * MTD, AHEAD = READ_AHEAD;
-      const char* kbuf = tbuf + (1 - PAR) * TILE;
-      const char* vbuf = tbuf + (2 + PAR) * TILE;
+      const char* kbuf = smem + (1 - PAR) * TILE;
+      const char* vbuf = smem + (2 + PAR) * TILE;
       auto kread = [&](int j) -> bf16x8 {
         return *(const bf16x8*)(kbuf + (kbase_l ^ ((j >> 1) << 5)) + (j & 1) * 32 * ROWB);
       };
@@ -617,7 +607,7 @@ __device__ __forceinline__ void attn_item(const AttnParams& p, char* smem, const
       constexpr int PAR = decltype(par)::value;
       bf16x8 pb[4];
       exp_tile(c0, c1, pb);
-      if (!LSE_ONLY) pv_tile(pb, tbuf + (2 + PAR) * TILE);
+      if (!LSE_ONLY) pv_tile(pb, smem + (2 + PAR) * TILE);
       __syncthreads();
     };
 
@@ -724,38 +714,6 @@ __device__ __forceinline__ void attn_item(const AttnParams& p, char* smem, const
         m_ref = m_star;
       }
     }
-  }
-
-  if constexpr (KSPLIT == 2) {
-    // ---- the second team parks its accumulators in its own K/V buffers (every wave is past its last read of them) and
-    // its statistics in the first team's V buffer; the first team brings both to a common reference and adds ----
-    char* const park = smem + 4 * TILE + wave * (D * 128);
-    float* const stat = (float*)(smem + 3 * TILE) + wave * 192 + lane;
-    if (team == 1) {
-#pragma unroll
-      for (int m = 0; m < MTD; m++)
-#pragma unroll
-        for (int a = 0; a < 4; a++)
-          *(f32x4*)(park + (m * 4 + a) * 1024 + lane * 16) = f32x4{oacc[m][4 * a], oacc[m][4 * a + 1], oacc[m][4 * a + 2], oacc[m][4 * a + 3]};
-      stat[0] = m_ref;
-      stat[64] = lsum;
-      stat[128] = m_true;
-    }
-    __syncthreads();
-    if (team == 1) return;
-    const float m1 = stat[0], m_star = fmaxf(m_ref, m1);
-    const float a0 = fast_exp2(m_ref - m_star), a1 = fast_exp2(m1 - m_star);
-    lsum = fmaf(stat[64], a1, lsum * a0);
-    m_true = fmaxf(m_true, stat[128]);
-    m_ref = m_star;
-#pragma unroll
-    for (int m = 0; m < MTD; m++)
-#pragma unroll
-      for (int a = 0; a < 4; a++) {
-        const f32x4 x = *(const f32x4*)(park + (m * 4 + a) * 1024 + lane * 16);
-#pragma unroll
-        for (int e = 0; e < 4; e++) oacc[m][4 * a + e] = fmaf(x[e], a1, oacc[m][4 * a + e] * a0);
-      }
   }
 
   // ---- epilogue ----
@@ -872,7 +830,7 @@ __device__ __forceinline__ void attn_item(const AttnParams& p, char* smem, const
 }
 #endif  // __HIP_DEVICE_COMPILE__
 
-template <int D, int NWAVES, int MODE, bool ACCUM, bool LSE_ONLY, int KSPLIT = 1>
+template <int D, int NWAVES, int MODE, bool ACCUM, bool LSE_ONLY>
 __global__ __launch_bounds__(NWAVES * 64, ((NWAVES <= 4 && D <= 128) ? (D == 64 && MODE == MODE_BLOCK && !LSE_ONLY ? 3 : 2) : 1)) void attn_fwd_kernel(const AttnParams p) {
   // The body is compiled for the device only: the host pass just needs the launch stub, and it
   // silently drops the stub when the body uses the LDS-DMA builtins.
@@ -883,7 +841,7 @@ __global__ __launch_bounds__(NWAVES * 64, ((NWAVES <= 4 && D <= 128) ? (D == 64 
   const int per_xcd = gridDim.x >> 3;
   const int w = (blockIdx.x & 7) * per_xcd + (blockIdx.x >> 3);
   if (w >= p.total_wg) return;
-  attn_item<D, NWAVES, MODE, ACCUM, LSE_ONLY, false, KSPLIT>(p, smem, w, 0, 0, true, SkCtx{});
+  attn_item<D, NWAVES, MODE, ACCUM, LSE_ONLY, false>(p, smem, w, 0, 0, true, SkCtx{});
 #endif
 }
 
@@ -1017,26 +975,6 @@ __global__ __launch_bounds__(256) void plan_kernel(const AttnParams p, int* plan
   }
 }
 
-// Query rows per workgroup of two teams of waves (KSPLIT), or 0 for one team.  Launches that leave compute units idle, or
-// with one wave per SIMD, split the keys of a query tile over two teams.  With at most one 64-row tile per compute unit:
-// 64 rows per workgroup, twice as many compute units at work and half the walk for each (B2 H16 d128, 400 x 921: 18.7 ->
-// 13.7 us, 256 x 521: 13.0 -> 10.5 us).  With at most one 128-row tile per compute unit: 128 rows, two waves per SIMD,
-// which walk two tiles in 1.6 of the time of one (576 x 1497: 27.6 -> 24.9 us, 1024 x 2521: 47.6 -> 45.2 us); short
-// walks do not pay for the merge at head_dim 128 (B2 H16, 676 x 696, 11 tiles: 16.1 -> 17.0 us; 17 tiles: 23.6 -> 23.3 us),
-// at head_dim 64 they do from 8 tiles on (11 tiles: 15.6 -> 13.4 us).  Beyond that the second resident workgroup does the same without a merge.  The merge costs about a microsecond, so lists of a
-// few tiles are walked by one team (the length of a block list is known to the device only; the width of the table
-// stands in for it).  A launch whose row statistic feeds a ranking (LSE2 without M and L: the decision-scale step, whose
-// column sums become top-k lists) keeps one team: two add the rows up in another order, and close scores would change
-// places with the launch shape.
-static int two_team_rows(const AttnParams& p, int nwaves, int head_dim) {
-  if (p.LSE2 && !p.M) return 0;
-  const int64_t all = (p.Lk + 63) / 64, tiles = p.list ? std::min((int64_t)p.list_len << p.sub_shift, all) : all;
-  const int64_t bh = (int64_t)p.B * p.H, cus = device_cus();
-  if (tiles >= 4 && bh * ((p.Lq + 63) / 64) <= cus) return 64;
-  if (tiles >= (head_dim == 64 ? 8 : 16) && nwaves == 4 && bh * ((p.Lq + 127) / 128) <= cus) return 128;
-  return 0;
-}
-
 // 256 query rows per workgroup (eight waves on one pair of K/V buffers, one workgroup per compute
 // unit): half the L2->LDS fills per flop, 4 % faster than two 128-row workgroups side by side (B2 H16 d128: 4096 x 10521
 // 635 -> 608 us, 1600 x 4121 117 -> 113 us) unless the coarser tiles leave more of the last round idle.  In units of a
@@ -1055,18 +993,18 @@ static bool wide_tiles(const AttnParams& p, int head_dim) {
   return wide < narrow;
 }
 
-template <int D, int NWAVES, int MODE, bool ACCUM, bool LSE_ONLY, int KSPLIT = 1>
+template <int D, int NWAVES, int MODE, bool ACCUM, bool LSE_ONLY>
 static int launch_one(const AttnParams& p0, hipStream_t stream) {
   AttnParams p = p0;
   if (p.kv_group < 1) p.kv_group = 1;
-  constexpr int WGROWS = ((MODE == MODE_GATHER && NWAVES == 8) ? 6 : NWAVES / KSPLIT) * 32;   // two of eight token-list waves only fetch
-  constexpr int SMEM = attn_lds_bytes<D, NWAVES, MODE, KSPLIT>();
+  constexpr int WGROWS = ((MODE == MODE_GATHER && NWAVES == 8) ? 6 : NWAVES) * 32;   // two of eight token-list waves only fetch
+  constexpr int SMEM = attn_lds_bytes<D, NWAVES, MODE>();
   if (MODE == MODE_BLOCK && p.list == nullptr) p.group_rows = WGROWS;  // dense: any row grouping
   if (p.group_rows % WGROWS != 0) return LVAR_EINVAL;
   p.nqt = (p.Lq + WGROWS - 1) / WGROWS;
   p.total_wg = p.B * p.H * p.nqt;
-  constexpr bool WIDE = MODE == MODE_BLOCK && NWAVES == 8 && KSPLIT == 1;   // 256 query rows
-  if constexpr (!LSE_ONLY && KSPLIT == 1) {
+  constexpr bool WIDE = MODE == MODE_BLOCK && NWAVES == 8;   // 256 query rows
+  if constexpr (!LSE_ONLY) {
     const bool dense = (MODE == MODE_BLOCK && p.list == nullptr);
     const int64_t per_tile = (MODE == MODE_BLOCK) ? (p.list ? p.list_len : (p.Lk + 63) / 64) : (p.list_len + 63) / 64;
     const int sub = (MODE == MODE_BLOCK && p.list) ? p.sub_shift : 0;
@@ -1107,16 +1045,11 @@ static int launch_one(const AttnParams& p0, hipStream_t stream) {
       return hipGetLastError() == hipSuccess ? LVAR_OK : LVAR_ELAUNCH;
     }
   }
-  if constexpr (MODE == MODE_BLOCK && !LSE_ONLY && KSPLIT == 1 && !WIDE && D <= 128) {
-    if (NWAVES == 4 && wide_tiles(p0, D)) return launch_one<D, 8, MODE_BLOCK, false, false, 1>(p0, stream);
-    const int rows = two_team_rows(p0, NWAVES, D);
-    AttnParams p2 = p0;
-    p2.sk_ws = nullptr;
-    if (rows == 64) return launch_one<D, 4, MODE_BLOCK, false, false, 2>(p2, stream);
-    if (rows == 128) return launch_one<D, 8, MODE_BLOCK, false, false, 2>(p2, stream);
+  if constexpr (MODE == MODE_BLOCK && !LSE_ONLY && NWAVES == 4 && D <= 128) {
+    if (wide_tiles(p0, D)) return launch_one<D, 8, MODE_BLOCK, false, false>(p0, stream);
   }
   const int grid = ((p.total_wg + 7) / 8) * 8;
-  auto kern = attn_fwd_kernel<D, NWAVES, MODE, ACCUM, LSE_ONLY, KSPLIT>;
+  auto kern = attn_fwd_kernel<D, NWAVES, MODE, ACCUM, LSE_ONLY>;
   static std::atomic<uint64_t> lds_ready{0};
   if (!ensure_lds_limit((const void*)kern, SMEM, lds_ready)) return LVAR_ELAUNCH;
   hipLaunchKernelGGL(kern, dim3(grid), dim3(NWAVES * 64), SMEM, stream, p);

@@ -57,7 +57,7 @@ def _dense_colsum_attn(q, k, v, p):
     ops._check_qkv(q, k, v, gqa=True)                    # dense_colsum_attn.cu:386-387
     if tuple(p.shape) != (q.shape[0], q.shape[1], q.shape[2], 1):
         raise ops.ShapeError(f"P shape mismatch - p: {tuple(p.shape)}, q: {tuple(q.shape)}")
-    o, _, _, lse2 = ops._dense_launch(q, k, v, 1.0, want_lse2=True)   # (with M and L: the launch dense_attn takes)
+    o, _, _, lse2 = ops._dense_launch(q, k, v, 1.0, want_ml=False, want_lse2=True)
     prev = (-torch.log2(p.to(torch.float32))).reshape(q.shape[:3]).contiguous()
     cs = ops._colsum_given_lse(q, k, prev, 1.0, get_kernel_config_attn()["bm"])
     return [o, cs, torch.exp2(-lse2).unsqueeze(-1)]

@@ -1,5 +1,5 @@
-"""Workgroup shapes of dense and block-list attention: the sizes at which the launch takes 64- or 128-row workgroups of two
-teams of waves, or 256-row workgroups, at the edges of tiles and with odd, short and empty lists."""
+"""Workgroup shapes of dense and block-list attention: launches that leave compute units idle or fill them once with 128-row
+workgroups, and launches of 256-row workgroups, at the edges of tiles and with odd, short and empty lists."""
 import pytest
 import torch
 
@@ -13,13 +13,13 @@ def _close(o, ref):
     assert torch.allclose(o.float().cpu(), ref, atol=2e-2, rtol=1e-2)
 
 
-# (B*H) * ceil(Lq/64) <= 256 takes 64-row workgroups from 4 tiles on, (B*H) * ceil(Lq/128) <= 256 128-row ones from 8 (head_dim 64) or 16
+# at most one 128-row workgroup per compute unit
 @pytest.mark.parametrize("B,H,Hkv,Lq,Lk,d", [
     (1, 2, 2, 1, 193, 128), (1, 2, 2, 64, 256, 128), (2, 2, 1, 65, 257, 64), (1, 3, 3, 129, 319, 128), (1, 2, 2, 200, 449, 64),
     (1, 140, 140, 128, 512, 128), (1, 140, 140, 100, 577, 128), (1, 130, 65, 127, 513, 64), (2, 64, 64, 200, 640, 64),
     (1, 140, 140, 128, 1024, 128), (1, 140, 140, 100, 1090, 128),
 ])
-def test_dense_two_teams(B, H, Hkv, Lq, Lk, d):
+def test_dense_128_row_workgroups(B, H, Hkv, Lq, Lk, d):
     from lvar_amd import sparse_attn_ops as ops
     q, k, v = make_qkv(B, H, Lq, Lk, d, seed=Lq + Lk)
     k, v = k[:, :Hkv].contiguous(), v[:, :Hkv].contiguous()
@@ -48,8 +48,8 @@ def test_dense_256_row_workgroups(B, H, Lq, Lk, d):
     assert torch.allclose(M + torch.log2(L), torch.logsumexp(s, -1, keepdim=True) * 1.4426950408889634, atol=1e-3, rtol=0)
 
 
-def test_dense_two_teams_growing_logits():
-    """Row maxima that grow along the keys: the teams end with different references."""
+def test_dense_growing_logits():
+    """Row maxima that grow along the keys: the reference moves again and again."""
     from lvar_amd import sparse_attn_ops as ops
     q, k, v = make_qkv(1, 2, 100, 700, 128, seed=9)
     k = (k.float() * torch.linspace(0.1, 6.0, 700).view(1, 1, -1, 1)).to(torch.bfloat16)
@@ -59,7 +59,7 @@ def test_dense_two_teams_growing_logits():
 
 @pytest.mark.parametrize("H,Lq,Lk,d,bq,bk", [(2, 300, 1000, 128, 128, 64), (3, 130, 900, 64, 128, 128), (2, 200, 1100, 128, 64, 64),
                                              (140, 128, 1024, 128, 128, 64), (135, 120, 1300, 64, 128, 256), (140, 120, 1000, 128, 128, 64)])
-def test_block_lists_two_teams(H, Lq, Lk, d, bq, bk):
+def test_block_lists_128_row_workgroups(H, Lq, Lk, d, bq, bk):
     from lvar_amd import sparse_attn_ops as ops
     q, k, v = make_qkv(1, H, Lq, Lk, d, seed=Lq)
     nQ, nK = -(-Lq // bq), -(-Lk // bk)
