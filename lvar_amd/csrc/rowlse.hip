@@ -315,6 +315,10 @@ __global__ __launch_bounds__(256, (D <= 128 ? ROW_LSE_WGS : 1)) void row_lse_ker
     add_block(la[0] + lb[0], la[1] + lb[1]);
     emit();
   }
+  // The last stage too: a sum of up to 2^127 against a reference that lies as far below the other half of the row, or
+  // below another key range, would vanish from the weighted sum of the two; and SCORES judges the distance of the
+  // statistic, not of the reference before the last keys, from the first reference.
+  renorm();
 
   bool again = !(fmaxf(l[0], l[1]) < INFINITY);
   if (SCORES) again = again || fmaxf(m[0] - first(0), m[1] - first(1)) > SCORE_REF_LIMIT;

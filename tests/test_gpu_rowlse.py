@@ -55,6 +55,36 @@ def test_row_lse_references_far_from_the_first_tile(kind):
     _check(q.to(torch.bfloat16).cuda(), k.to(torch.bfloat16).cuda(), 1.0)
 
 
+# (position, logit in nats) of the largest keys of a row; the last 64-key stage begins at 640, key ranges end at 256, 384 or 512
+LATE = [[(690, 60.0)], [(690, 69.5)], [(690, 87.5)], [(690, 88.0)], [(690, 88.5)], [(699, 88.5)], [(300, 60.0), (692, 100.0)],
+        [(300, 30.0), (692, 90.0)], [(300, 62.0), (692, 104.0)], [(300, 88.5), (691, 88.5)], [(303, 88.5), (692, 88.5)], [(691, 88.5), (692, 88.5)],
+        [(255, 88.5), (300, 88.5)], [(383, 88.5), (600, 88.5)], [(500, 88.5), (600, 88.5)], [(200, 88.5), (500, 88.5), (690, 88.5)]]
+
+
+def _late_qk(peaks, seed):
+    g = torch.Generator().manual_seed(seed)
+    q = torch.zeros(1, 2, 200, 128)
+    q[..., 0] = 1.0
+    k = torch.randn(1, 2, 700, 128, generator=g) * 0.05
+    k[..., 0] = 0.0
+    for n, x in peaks:
+        k[:, :, n, 0] = x
+    q[:, :, 1::5, 0] = 0.5                     # lanes of one wave that jump by different amounts
+    return q.to(torch.bfloat16).cuda(), k.to(torch.bfloat16).cuda()
+
+
+@pytest.mark.parametrize("cut_keys", [False, True])
+@pytest.mark.parametrize("peaks", LATE)
+def test_row_lse_largest_keys_in_the_last_stage(peaks, cut_keys):
+    """Sums that jump in the last stage of a range, by up to 2^128 against the reference, alone and beside a half of the
+    lanes, or a range, whose reference has moved that far before."""
+    from lvar_amd import sparse_attn_ops as ops
+    q, k = _late_qk(peaks, 11)
+    got = ops._lse_only(q, k, 1.0, cut_keys=cut_keys).double().cpu()
+    ref = _ref(q, k, 1.0)
+    assert (got - ref).abs().max() <= 2.0 ** -15 + 2.0 ** -17 * ref.abs().max()    # the bound of _check
+
+
 def test_block_scores_without_the_column_sums():
     from lvar_amd import sparse_attn_ops as ops
     g = torch.Generator().manual_seed(5)
@@ -120,6 +150,15 @@ def test_block_scores_references_far_from_the_first_tile(kind):
                  "first_tile_low": torch.where(n < 40, -800.0, 3.0)}[kind]
     q[:, :, ::3, 0] = 0.25
     _check_scores(q.to(torch.bfloat16).cuda(), k.to(torch.bfloat16).cuda(), 1.0, 32, 128, 2)
+
+
+@pytest.mark.parametrize("peaks", LATE)
+def test_block_scores_largest_keys_in_the_last_stage(peaks):
+    """A block sum counts from the row's first reference: one that lies further from the statistic than the exponent range
+    must not come out as 0 or NaN."""
+    q, k = _late_qk(peaks, 12)
+    _check_scores(q, k, 1.0, 32, 128, 2)
+    _check_scores(q, k, 1.0, 64, 64, 3)
 
 
 def test_block_scores_ties_at_the_cut():
