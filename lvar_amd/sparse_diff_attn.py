@@ -14,6 +14,10 @@ from . import sparse_attn_ops as ops
 from .sparse_attn_config import GLOBAL_CONFIG, get_kernel_config_attn
 
 
+# what the constructor may set as `dense_colsum_attn`; the compiled full step stands for either
+_COLSUM_OPERATORS = (ops.dense_colsum_attn_s, ops.dense_colsum_attn_q)
+
+
 class SparseDiffAttn(torch.nn.Module):
     """Constructor arguments as the reference's (models/sparvar/sparse_attn.py:866-873; constructed at
     basic_sparvar.py:255-259 as ``SparseDiffAttn(layer_num, layer_counter, use_o_cache=True, spsd_scale=...)``).
@@ -61,8 +65,8 @@ class SparseDiffAttn(torch.nn.Module):
         top_keys = GLOBAL_CONFIG["attn"]["top_keys"]
         fast = ops._native()
         if do_full_step:                                           # sparse_attn.py:991-1051
-            if fast is not None:
-                # the launches below behind one host call
+            if fast is not None and self.dense_colsum_attn in _COLSUM_OPERATORS:
+                # the launches below behind one host call (an operator that the caller has put in is called)
                 count = mb.indices_count(top_keys, k.shape[-2], self.multiple_of)
                 r = fast.fast_full_step(q, k, v, ops._plain_scale(scale), get_kernel_config_attn()["bm"], count, self.use_o_cache)
                 if r is not None:

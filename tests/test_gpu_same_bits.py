@@ -50,3 +50,24 @@ def test_full_step_lists_do_not_depend_on_the_host_path(B, H, n, S, monkeypatch)
         got.append((o, layer.out_cache, layer.indices[..., :layer.count_host], layer.counts))
     for a, b in zip(*got):
         assert torch.equal(a, b)
+
+
+def test_full_step_calls_a_replaced_colsum_operator():
+    """``dense_colsum_attn`` is an attribute of the layer that a caller may replace."""
+    from lvar_amd import mask_build as mb
+    from lvar_amd.sparse_diff_attn import SparseDiffAttn
+    scales = mb.INFINITY_SCALES[:7] + (20,)
+    q, k, v = _rand(1, 2, 400, sum(s * s for s in scales), 128, seed=3)
+    layer = SparseDiffAttn(scales=scales, spsd_scale=len(scales) - 1)
+    plain = layer(q, k, v, None, do_full_step=True, scale_ind=len(scales) - 1)
+    inner, calls = layer.dense_colsum_attn, []
+
+    def reversed_sums(*a):
+        calls.append(len(a))
+        o, cs = inner(*a)
+        return o, (-cs).contiguous()
+    first = layer.indices[..., :layer.count_host].clone()
+    layer.dense_colsum_attn = reversed_sums
+    o = layer(q, k, v, None, do_full_step=True, scale_ind=len(scales) - 1)
+    assert calls == [4] and torch.equal(o, plain)
+    assert not torch.equal(layer.indices[..., :layer.count_host], first)      # the least-attended keys now
