@@ -164,7 +164,7 @@ int lvar_colsum_fwd(lvar_tensor_t q, lvar_tensor_t k, const float* lse2, float* 
   if (!shape_ok(B, H, Lq, Lk, scale) || !view_ok(q) || !view_ok(k) || !lse2 || (!cs && !block_sums)) return LVAR_EINVAL;
   if (kv_heads <= 0 || H % kv_heads != 0) return LVAR_EINVAL;
   if (q_group_size <= 0 || q_group_size % 32 != 0) return LVAR_EINVAL;
-  if (!kv_span_ok(q, Lq, head_dim, 0)) return LVAR_EINVAL;
+  if (!kv_span_ok(q, Lq, head_dim, 64)) return LVAR_EINVAL;   // (a ragged last stage forms offsets of up to 63 rows beyond)
   ColsumParams p{};
   p.q = (const bf16_t*)q.ptr; p.q_sb = q.stride_b; p.q_sh = q.stride_h; p.q_sr = q.stride_row;
   p.k = (const bf16_t*)k.ptr; p.k_sb = k.stride_b; p.k_sh = k.stride_h; p.k_sr = k.stride_row;

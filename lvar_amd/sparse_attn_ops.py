@@ -243,7 +243,13 @@ def _lse2_of(lse, shape):
     return out
 
 
+def _near_rows(q):
+    """``q`` with rows near enough for the 32-bit offsets of the column-sum kernel (up to 63 rows beyond the last one)."""
+    return q if q.stride(2) * 2 * (q.shape[2] + 64) + q.shape[3] * 2 < 2 ** 31 - 1 else q.contiguous()
+
+
 def _colsum_given_lse(q, k, lse2, scale, q_group_size, want_block_sums=False, want_columns=True):
+    q = _near_rows(q)
     B, H, Lq, d = q.shape
     Lk = k.shape[2]
     G = (Lq + q_group_size - 1) // q_group_size

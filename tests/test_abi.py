@@ -67,6 +67,19 @@ def test_argument_validation_without_device(lib):
     assert lib.lvar_block_sparse_attn_fwd(fake, fake, fake, fake, None, None, None, 0, 0, one, 0, 0, 4, 4, 128, 64, 1, 1, 16, 16, 128, 1.0, None) == -1
 
 
+def test_colsum_query_span_limit(lib):
+    """The fills of a ragged last 64-row stage form 32-bit offsets of up to 63 rows beyond the last query row: rows of
+    2 MiB, of which 2^31 bytes hold 1024: 959 rows pass the check (and nothing can be launched here), more do not."""
+    import torch
+    if torch.cuda.is_available():
+        pytest.skip("the call in range would be launched")
+    from lvar_amd._lib import LvarTensor
+    wide, fake = LvarTensor(0x1000, 1 << 40, 1 << 32, 1 << 20), LvarTensor(0x1000, 128 * 16 * 128, 16 * 128, 128)
+    one = ctypes.c_void_p(0x2000)
+    for rows, status in ((959, -3), (960, -1), (1000, -1), (1023, -1), (1024, -1)):
+        assert lib.lvar_colsum_fwd(wide, fake, one, one, None, 1, 1, 1, rows, 16, 128, 192, 1.0, None) == status, rows
+
+
 def test_list_build_and_upsample_argument_validation(lib):
     from lvar_amd._lib import LvarTensor
     null = LvarTensor(None, 0, 0, 0)

@@ -170,3 +170,15 @@ def test_block_scores_ties_at_the_cut():
     for j in range(1, 3):
         k[:, :, j] = k[:, :, j, torch.randperm(128, generator=g)]
     _check_scores(q, k.flatten(2, 3).contiguous().cuda(), 128 ** -0.5, 32, 128, 2)
+
+
+def test_column_sums_of_queries_with_far_rows():
+    """Query rows 4 MiB apart span more than the kernel's 32-bit offsets reach: the operator works on a copy."""
+    from lvar_amd import sparse_attn_ops as ops
+    g = torch.Generator(device="cuda").manual_seed(8)
+    rows, k = ((torch.randn(1, 1, L, 64, generator=g, device="cuda") * 0.5).to(torch.bfloat16) for L in (520, 300))
+    far = torch.empty(520 << 21, dtype=torch.bfloat16, device="cuda").as_strided((1, 1, 520, 64), (1 << 31, 1 << 31, 1 << 21, 1))
+    far.copy_(rows)
+    assert torch.equal(ops.colsum(far, k, None, 192), ops.colsum(rows, k, None, 192))
+    assert torch.equal(ops._colsum_block_scores(far, k, None, 32, 128), ops._colsum_block_scores(rows, k, None, 32, 128))
+    assert torch.equal(ops._block_scores_for_topk(far, k, None, 32, 128, None, 1), ops._block_scores_for_topk(rows, k, None, 32, 128, None, 1))
