@@ -4,12 +4,14 @@
 //                               group; for callers that rank the blocks it lists the scores too close to the cut for
 //                               32-bit sums to tell apart
 //   refine_scores_kernel        computes those again the way the column-sum kernel does
+// A row with many such scores (keys or queries that repeat, zeros) is handed to the column-sum kernel itself.
 #include "common.h"
 #include "launch.h"
 
 namespace lvar {
 
 constexpr int SCORE_MAX_GROUP = 1024;   // query rows per group (their weights sit in LDS)
+constexpr int REFINE_MAX_ITEMS = 8;     // scores of a row that are computed one by one, see list_close_scores
 constexpr int REFINE_MAX_NK = 2048;     // blocks per row that can be ranked (their keys sit in LDS); the limit of the block top-k kernel
 // Two orders of the sums of a score differ by a few units in the last place (5e-7 at most over the declared video sizes);
 // scores this far apart (relative, 64 units) keep their order.
@@ -18,7 +20,11 @@ constexpr float REFINE_EPS = 0x1p-18f;
 __device__ __forceinline__ float key_value(uint32_t k) { return __builtin_bit_cast(float, k ^ ((k >> 31) ? 0x80000000u : 0xffffffffu)); }
 
 // One wave per row: appends the row's scores that lie within REFINE_EPS of the cut of "base blocks plus the best others up
-// to `target`" to the work list, when both sides of the cut do.
+// to `target`" to the work list, when both sides of the cut do.  A score alone costs a wave its operands straight from
+// memory, 40 KiB; the column-sum kernel forms all 256 of a row for the price of twenty.  So a row with more than a few is
+// listed as a row (the complement of its number) and the column sums of its (batch, head) run: with zero queries (every
+// score of every row close) the 24-head 8 x 64 x 64 video lists took 15.3 ms score by score and take 2.6 ms now, against
+// 1.6 ms without ties; the launch costs 3 us where no row asks for it.
 __device__ __forceinline__ void list_close_scores(const BlockScoreParams& p, const uint32_t* key, int row) {
   const int lane = threadIdx.x & 63, nK = p.nK;
   int others = 0;
@@ -44,10 +50,19 @@ __device__ __forceinline__ void list_close_scores(const BlockScoreParams& p, con
   }
   const float hi = key_value(cut), lo = key_value(below), eps = REFINE_EPS * fabsf(hi);
   if (!(hi - lo <= eps)) return;
-  for (int j = lane; j < nK; j += 64) {
-    const uint32_t k = key[j];
-    if (k != 0u && key_value(k) >= lo - eps && key_value(k) <= hi + eps) p.r.work[1 + atomicAdd(p.r.work, 1)] = row * nK + j;
+  auto close = [&](int j) { return j < nK && key[j] != 0u && key_value(key[j]) >= lo - eps && key_value(key[j]) <= hi + eps; };
+  int n = 0;
+  for (int j0 = 0; j0 < nK; j0 += 64) n += __builtin_popcountll(__builtin_amdgcn_ballot_w64(close(j0 + lane)));
+  int* const items = p.r.work + 1 + p.r.B * p.r.H;
+  if (n > REFINE_MAX_ITEMS) {
+    if (lane == 0) {
+      items[atomicAdd(p.r.work, 1)] = ~row;
+      atomicAdd(p.r.work + 1 + row / p.G, 1);
+    }
+    return;
   }
+  for (int j = lane; j < nK; j += 64)
+    if (close(j)) items[atomicAdd(p.r.work, 1)] = row * nK + j;
 }
 
 // Bound by the reads of the kept sums (4 bytes per row and block; B1 H24, 8192 rows x 256 blocks: 58 us, 3.5 TB/s).  One workgroup per
@@ -103,9 +118,9 @@ __global__ __launch_bounds__(256) void block_score_finish_kernel(const BlockScor
 
 constexpr int REFINE_WGS = 256;   // of four waves
 
-// One wave per listed score: the value that the block sums of colsum_kernel have (same products, same order of additions),
-// so that the selection is the same whichever way the scores were computed.  A row in twenty has such scores at 256
-// blocks, so the operands are read straight from memory.
+// One wave per work item.  A score: the value that the block sums of colsum_kernel have (same products, same order of
+// additions), so that the selection is the same whichever way the scores were computed.  A row in twenty has such scores at
+// 256 blocks, so the operands are read straight from memory.  A row: its scores from those block sums.
 template <int D>
 __global__ __launch_bounds__(256) void refine_scores_kernel(const BlockScoreParams p) {
 #if defined(__HIP_DEVICE_COMPILE__)
@@ -114,7 +129,18 @@ __global__ __launch_bounds__(256) void refine_scores_kernel(const BlockScorePara
   const int nK = p.nK, items = p.r.work[0];
   const f32x16 zero = {0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0};
   for (int it = blockIdx.x * 4 + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6); it < items; it += REFINE_WGS * 4) {
-    const int item = __builtin_amdgcn_readfirstlane(p.r.work[1 + it]);
+    const int item = __builtin_amdgcn_readfirstlane(p.r.work[1 + p.r.B * p.r.H + it]);
+    if (item < 0) {
+      const int nkb = (p.r.Lk + 63) >> 6;
+      const float* bs = p.r.tsum + (int64_t)~item * nkb;
+      for (int j = lane; j < nK; j += 64) {
+        const int first = j * p.r.block_stages, end = min(first + p.r.block_stages, nkb);
+        float total = bs[first];
+        for (int i = first + 1; i < end; i++) total += bs[i];
+        p.scores[(int64_t)~item * nK + j] = total;
+      }
+      continue;
+    }
     const int row = item / nK, j = item - row * nK, bh = row / p.G, g = row - bh * p.G, b = bh / p.r.H, h = bh - b * p.r.H;
     const bf16_t* qbase = p.r.q + b * p.r.q_sb + h * p.r.q_sh;
     const bf16_t* kbase = p.r.k + b * p.r.k_sb + (h / p.r.kv_group) * p.r.k_sh;
@@ -180,6 +206,14 @@ int launch_block_scores(const BlockScoreParams& p0, int head_dim, hipStream_t st
     hipLaunchKernelGGL(block_score_finish_kernel<false>, dim3(bh * p.G), dim3(256), rank ? 4 * p.nK : 0, stream, p);
   if (hipGetLastError() != hipSuccess) return LVAR_ELAUNCH;
   if (rank) {
+    ColsumParams c{};
+    c.q = p.r.q; c.q_sb = p.r.q_sb; c.q_sh = p.r.q_sh; c.q_sr = p.r.q_sr;
+    c.k = p.r.k; c.k_sb = p.r.k_sb; c.k_sh = p.r.k_sh; c.k_sr = p.r.k_sr;
+    c.lse2 = p.r.lse2; c.bs = p.r.tsum; c.some = p.r.work + 1;
+    c.B = p.r.B; c.H = p.r.H; c.Lq = p.r.Lq; c.Lk = p.r.Lk; c.kv_group = p.r.kv_group;
+    c.group_rows = p.group_rows; c.G = p.G; c.c = p.r.c;
+    const int st2 = launch_colsum(c, head_dim, stream);
+    if (st2 != LVAR_OK) return st2;
     if (head_dim == 128) hipLaunchKernelGGL(refine_scores_kernel<128>, dim3(REFINE_WGS), dim3(256), 0, stream, p);
     else if (head_dim == 64) hipLaunchKernelGGL(refine_scores_kernel<64>, dim3(REFINE_WGS), dim3(256), 0, stream, p);
     else hipLaunchKernelGGL(refine_scores_kernel<256>, dim3(REFINE_WGS), dim3(256), 0, stream, p);

@@ -1,5 +1,6 @@
 // extern "C" entry points declared in include/lvar_sparse_attn.h: argument validation and
 // parameter packing; all device work is in attn_fwd.hip / colsum.hip.
+#include <algorithm>
 #include <cmath>
 #include "../../include/lvar_sparse_attn.h"
 #include "launch.h"
@@ -176,15 +177,17 @@ int lvar_colsum_fwd(lvar_tensor_t q, lvar_tensor_t k, const float* lse2, float* 
   return launch_colsum(p, head_dim, (hipStream_t)stream);
 }
 
-// Scratch of a block-score call, in 4-byte words: lse2 | first references | number of scores to compute again, and which | block sums.
+// Scratch of a block-score call, in 4-byte words: lse2 | first references | number of work items, rows among them per
+// (batch, head), the items | sums of the sweep, and after it the block sums of the column sums.
 struct ScoreLayout { int64_t refs, work, sums, total; };
 static ScoreLayout score_layout(int B, int H, int Lq, int Lk, int q_group_size, int block_k) {
   ScoreLayout l{};
   const int64_t bh = (int64_t)B * H, nK = (Lk + block_k - 1) / block_k;
   l.refs = bh * Lq;
   l.work = 2 * l.refs;
-  l.sums = (l.work + 1 + bh * ((Lq + q_group_size - 1) / q_group_size) * nK + 63) / 64 * 64;
-  l.total = l.sums + bh * ((Lq + 255) / 256) * 256 * nK;
+  const int64_t G = (Lq + q_group_size - 1) / q_group_size;
+  l.sums = (l.work + 1 + bh + bh * G * nK + 63) / 64 * 64;
+  l.total = l.sums + std::max(bh * ((Lq + 255) / 256) * 256 * nK, bh * G * ((Lk + 63) / 64));
   return l;
 }
 
@@ -196,7 +199,7 @@ int64_t lvar_block_scores_scratch_bytes(int B, int H, int Lq, int Lk, int q_grou
 int lvar_block_scores_fwd(lvar_tensor_t q, lvar_tensor_t k, float* scores, const uint8_t* base_mask, int target, void* scratch, int64_t scratch_bytes,
                           int B, int H, int kv_heads, int Lq, int Lk, int head_dim, int q_group_size, int block_k, float scale, void* stream) {
   if (!shape_ok(B, H, Lq, Lk, scale) || !view_ok(q) || !view_ok(k) || !scores || target < 0) return LVAR_EINVAL;
-  if (kv_heads <= 0 || H % kv_heads != 0 || !kv_span_ok(k, Lk, head_dim)) return LVAR_EINVAL;
+  if (kv_heads <= 0 || H % kv_heads != 0 || !kv_span_ok(k, Lk, head_dim) || !kv_span_ok(q, Lq, head_dim, 64)) return LVAR_EINVAL;
   if (block_k <= 0 || block_k % 64 != 0 || q_group_size <= 0 || q_group_size % 32 != 0) return LVAR_EINVAL;
   if ((q_group_size != 32 && q_group_size % 64 != 0) || q_group_size > 1024) return LVAR_EUNSUPPORTED;
   const ScoreLayout l = score_layout(B, H, Lq, Lk, q_group_size, block_k);

@@ -20,7 +20,7 @@ namespace lvar {
 
 constexpr int CS_WGS = 3;   // workgroups per compute unit (head_dim 64 and 128): 168 registers per wave, 33 KiB of LDS
 
-template <int D>
+template <int D, bool SOME>
 __global__ __launch_bounds__(256, (D <= 128 ? CS_WGS : 1)) void colsum_kernel(const ColsumParams p) {
 #if defined(__HIP_DEVICE_COMPILE__)
   constexpr int KS = D / 16;
@@ -42,6 +42,7 @@ __global__ __launch_bounds__(256, (D <= 128 ? CS_WGS : 1)) void colsum_kernel(co
   // (the quotients are formed on the vector ALU: moved to scalar registers, so are the addresses that hang on them)
   const int bh = __builtin_amdgcn_readfirstlane(w / per_bh), rem = w - bh * per_bh;
   const int kt = __builtin_amdgcn_readfirstlane(rem / p.q_splits), sp = rem - kt * p.q_splits;
+  if (SOME && p.some[bh] == 0) return;
   const int b = __builtin_amdgcn_readfirstlane(bh / p.H), h = bh - b * p.H;
   const int qoff = __builtin_amdgcn_readfirstlane(sp * p.split_rows);   // first query row of this range (a multiple of 64 and of group_rows)
   const int Lq_l = min(p.Lq, qoff + p.split_rows) - qoff;   // rows of this range
@@ -289,7 +290,7 @@ __global__ __launch_bounds__(256, (D <= 128 ? CS_WGS : 1)) void colsum_kernel(co
 #endif  // __HIP_DEVICE_COMPILE__
 }
 
-template <int D>
+template <int D, bool SOME>
 static int launch_cs(const ColsumParams& p0, hipStream_t stream) {
   ColsumParams p = p0;
   if (p.kv_group < 1) p.kv_group = 1;
@@ -320,15 +321,15 @@ static int launch_cs(const ColsumParams& p0, hipStream_t stream) {
   const int grid = ((p.total_wg + 7) / 8) * 8;
   constexpr int SMEM = 2 * 64 * D * 2 + 4 * 256;
   static std::atomic<uint64_t> lds_ready{0};
-  if (!ensure_lds_limit((const void*)colsum_kernel<D>, SMEM, lds_ready)) return LVAR_ELAUNCH;
-  hipLaunchKernelGGL((colsum_kernel<D>), dim3(grid), dim3(256), SMEM, stream, p);
+  if (!ensure_lds_limit((const void*)colsum_kernel<D, SOME>, SMEM, lds_ready)) return LVAR_ELAUNCH;
+  hipLaunchKernelGGL((colsum_kernel<D, SOME>), dim3(grid), dim3(256), SMEM, stream, p);
   return hipGetLastError() == hipSuccess ? LVAR_OK : LVAR_ELAUNCH;
 }
 
 int launch_colsum(const ColsumParams& p, int head_dim, hipStream_t s) {
-  if (head_dim == 128) return launch_cs<128>(p, s);
-  if (head_dim == 64) return launch_cs<64>(p, s);
-  if (head_dim == 256) return launch_cs<256>(p, s);
+  if (head_dim == 128) return p.some ? launch_cs<128, true>(p, s) : launch_cs<128, false>(p, s);
+  if (head_dim == 64) return p.some ? launch_cs<64, true>(p, s) : launch_cs<64, false>(p, s);
+  if (head_dim == 256) return p.some ? launch_cs<256, true>(p, s) : launch_cs<256, false>(p, s);
   return LVAR_EUNSUPPORTED;
 }
 

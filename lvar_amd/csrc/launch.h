@@ -55,6 +55,7 @@ struct ColsumParams {
   const float* lse2;  // base-2 log-sum-exp per query row, M + log2(L)
   float* cs;          // [B,H,G,Lk], or null when only the block sums are wanted
   float* bs;          // optional per-64-key block sums [B,H,G,ceil(Lk/64)]
+  const int* some;    // optional [B*H]: the sums of a (batch, head) are only formed where this is not 0
   int64_t q_sb, q_sh, q_sr;
   int64_t k_sb, k_sh, k_sr;
   int B, H, Lq, Lk, G;
@@ -81,11 +82,12 @@ struct RowLseParams {
   float* first_ref;   // [B*H*Lq] the reference that the sums of a row count from
   int block_stages;   // 64-key stages per key block
   int key_blocks;
-  int* work;          // work[0] is cleared by the sweep
+  int* work;          // work[0 .. B*H] are cleared by the sweep: number of work items, then per (batch, head) the rows among them
   int nrt, splits, split_keys, total_wg;   // set at launch
 };
 
-// Scores of key blocks from the sums that the row-statistics kernel keeps (see blockscore.hip)
+// Scores of key blocks from the sums that the row-statistics kernel keeps (see blockscore.hip); r.tsum also holds the
+// column sums' block sums, [B*H, G, ceil(Lk/64)] floats, once the scores are written
 struct BlockScoreParams {
   RowLseParams r;     // q, k, lse2, tsum, first_ref, work and the partition of the sweep
   float* scores;      // [B*H, G, nK]

@@ -44,7 +44,8 @@ __global__ __launch_bounds__(256, (D <= 128 ? ROW_LSE_WGS : 1)) void row_lse_ker
   // consecutive workgroup ids are dealt round-robin to the 8 XCDs: each XCD walks a contiguous range
   const int per_xcd = gridDim.x >> 3;
   const int w = (blockIdx.x & 7) * per_xcd + (blockIdx.x >> 3);
-  if (SCORES && blockIdx.x == 0 && threadIdx.x == 0) p.work[0] = 0;
+  if (SCORES && blockIdx.x == 0)
+    for (int i = threadIdx.x; i <= p.B * p.H; i += 256) p.work[i] = 0;
   if (w >= p.total_wg) return;
   // workgroup = (batch*head, key range, tile of 256 query rows)
   const int per_bh = p.nrt * p.splits;

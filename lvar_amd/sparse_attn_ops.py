@@ -320,10 +320,10 @@ def _block_scores_for_topk(q, k, scale, q_group_size: int, block_k: int, base_ma
     Lk = k.shape[2]
     nK = (Lk + block_k - 1) // block_k
     one_sweep = (q_group_size == 32 or (q_group_size % 64 == 0 and q_group_size <= 1024)) and nK <= 2048 and target > 0
-    words = B * H * ((Lq + q_group_size - 1) // q_group_size * nK + 2 * Lq)      # (counted in 32 bits)
+    words = B * H * ((Lq + q_group_size - 1) // q_group_size * nK + 2 * Lq + 1)  # (counted in 32 bits)
     if not one_sweep or words >= 2 ** 31 - 128:
         return _colsum_block_scores(q, k, scale, q_group_size, block_k)
-    q, k = _prep(q, "q"), _prep(k, "k")
+    q, k = _near_rows(_prep(q, "q")), _prep(k, "k")
     _check_qkv(q, k, k, gqa=True)
     scores = torch.empty((B, H, (Lq + q_group_size - 1) // q_group_size, nK), dtype=torch.float32, device=q.device)
     lib = _lib.load()

@@ -182,3 +182,57 @@ def test_column_sums_of_queries_with_far_rows():
     assert torch.equal(ops.colsum(far, k, None, 192), ops.colsum(rows, k, None, 192))
     assert torch.equal(ops._colsum_block_scores(far, k, None, 32, 128), ops._colsum_block_scores(rows, k, None, 32, 128))
     assert torch.equal(ops._block_scores_for_topk(far, k, None, 32, 128, None, 1), ops._block_scores_for_topk(rows, k, None, 32, 128, None, 1))
+
+
+@pytest.mark.parametrize("kind", ["zero_queries", "zero_keys", "some_heads", "some_rows", "few_ties", "far_below"])
+@pytest.mark.parametrize("group,block_k,d", [(32, 128, 128), (64, 64, 64), (32, 192, 128), (128, 128, 256)])
+def test_block_scores_rows_with_many_ties(kind, group, block_k, d):
+    """Up to eight scores about the cut are computed one by one; rows with more of them take their scores from the column
+    sums of their (batch, head)."""
+    g = torch.Generator().manual_seed(21)
+    q, k = torch.randn(2, 3, 420, d, generator=g) * 0.5, torch.randn(2, 3, 2000, d, generator=g) * 0.5
+    if kind == "zero_queries":
+        q[:] = 0
+    elif kind == "zero_keys":
+        k[:] = 0
+    elif kind == "some_heads":
+        q[0, 1] = 0
+        q[1, 2, :, 5:] = 0
+    elif kind == "some_rows":
+        q[:, :, 64:160] = 0
+        q[1, 0, 400:] = 0
+    elif kind == "few_ties":
+        nb = 5                                            # five equal blocks among others
+        k[:, :, block_k:(nb + 1) * block_k] = k[:, :, :block_k].repeat(1, 1, nb, 1)
+    else:                                                 # all mass in one block: the others' scores are 0 or next to it
+        k[..., 0] = -900.0
+        k[:, :, 3] = 0
+        q[..., 0] = 1.0
+    q, k = q.to(torch.bfloat16).cuda(), k.to(torch.bfloat16).cuda()
+    nQ, nK = -(-420 // group), -(-2000 // block_k)
+    base = (torch.rand(nQ, nK, generator=g) < 0.1).cuda()
+    for target in (1, nK // 3, nK - 1):
+        _check_scores(q, k, d ** -0.5, group, block_k, target)
+        _check_scores(q, k, d ** -0.5, group, block_k, target, base)
+
+
+def test_block_scores_of_equal_blocks_cost_no_more_than_two_passes():
+    """Every score of every row about the cut: the scores must not be computed one by one (six times the two-pass form)."""
+    from lvar_amd import sparse_attn_ops as ops
+    g = torch.Generator(device="cuda").manual_seed(22)
+    k = (torch.randn(1, 8, 16384, 128, generator=g, device="cuda") * 0.5).to(torch.bfloat16)
+    q = torch.zeros(1, 8, 4096, 128, device="cuda", dtype=torch.bfloat16)
+
+    def time_of(f):
+        f()
+        times = []
+        for _ in range(5):
+            a, b = torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True)
+            a.record()
+            f()
+            b.record()
+            torch.cuda.synchronize()
+            times.append(a.elapsed_time(b))
+        return sorted(times)[2]
+    one, two = time_of(lambda: ops._block_scores_for_topk(q, k, None, 32, 128, None, 12)), time_of(lambda: ops._colsum_block_scores(q, k, None, 32, 128))
+    assert one < 2 * two, (one, two)
