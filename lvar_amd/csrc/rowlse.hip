@@ -321,9 +321,11 @@ __global__ __launch_bounds__(256, (D <= 128 ? ROW_LSE_WGS : 1)) void row_lse_ker
   // statistic, not of the reference before the last keys, from the first reference.
   renorm();
 
-  bool again = !(fmaxf(l[0], l[1]) < INFINITY);
-  if (SCORES) again = again || fmaxf(m[0] - first(0), m[1] - first(1)) > SCORE_REF_LIMIT;
-  if (__builtin_amdgcn_ballot_w64(again) != 0) {
+  const bool overflow = __builtin_amdgcn_ballot_w64(!(fmaxf(l[0], l[1]) < INFINITY)) != 0;
+  bool again = overflow;
+  if (SCORES) again = again || __builtin_amdgcn_ballot_w64(fmaxf(m[0] - first(0), m[1] - first(1)) > SCORE_REF_LIMIT) != 0;
+  const float m_sweep[2] = {m[0], m[1]}, l_sweep[2] = {l[0], l[1]};
+  if (again) {
     // a sum has overflowed: this wave's rows again, straight from memory, with the maximum tracked tile by tile
     auto tile_mem = [&](int u) {
       const bf16_t* kp = kbase + (int64_t)min(koff + u * 32 + r, p.Lk - 1) * p.k_sr + hh * 8;
@@ -372,6 +374,14 @@ __global__ __launch_bounds__(256, (D <= 128 ? ROW_LSE_WGS : 1)) void row_lse_ker
         }
         add_block(t0, t1);
         if (u + 1 == U || (u + 1) % (2 * p.block_stages) == 0) emit();
+      }
+      // the statistic of a sweep that was only repeated for its block sums stands: it has the bits of the one without SCORES
+      if (!overflow) {
+#pragma unroll
+        for (int nt = 0; nt < 2; nt++) {
+          m[nt] = m_sweep[nt];
+          l[nt] = l_sweep[nt];
+        }
       }
     }
   }

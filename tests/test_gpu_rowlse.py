@@ -236,3 +236,22 @@ def test_block_scores_of_equal_blocks_cost_no_more_than_two_passes():
         return sorted(times)[2]
     one, two = time_of(lambda: ops._block_scores_for_topk(q, k, None, 32, 128, None, 12)), time_of(lambda: ops._colsum_block_scores(q, k, None, 32, 128))
     assert one < 2 * two, (one, two)
+
+
+@pytest.mark.parametrize("amp", [1.0, 16.0, 64.0, 256.0])
+@pytest.mark.parametrize("group,low", [(32, 0.0), (64, 0.0), (32, 40.0)])
+def test_block_scores_ties_at_the_cut_of_large_logits(amp, group, low):
+    """The rounding of the exponents grows with their size, and so does the distance within which the two-pass sums decide.
+    Six orders of one block; ``low``: behind a first stage of logits that far below, so that references and statistics part."""
+    g = torch.Generator().manual_seed(7)
+    q = torch.randn(1, 8, 1024, 128, generator=g) * 0.5 * amp
+    one = torch.randn(1, 8, 1, 128, 128, generator=g) * 0.5
+    k = one.repeat(1, 1, 7, 1, 1)
+    for j in range(1, 7):
+        k[:, :, j] = k[:, :, j, torch.randperm(128, generator=g)]
+    if low:
+        q[..., 0] = 1.0
+        k[..., 0] = 0.0
+        k[:, :, 0, :, 0] = -low * 128 ** 0.5
+    k = k.flatten(2, 3) if low else k[:, :, 1:].flatten(2, 3)
+    _check_scores(q.to(torch.bfloat16).cuda(), k.to(torch.bfloat16).contiguous().cuda(), 128 ** -0.5, group, 128, 3)
