@@ -153,8 +153,9 @@ int lvar_colsum_fwd(lvar_tensor_t q, lvar_tensor_t k, const float* lse2, float* 
  * (others: LVAR_EUNSUPPORTED).  Sums run over the keys of a block first and then over the rows, so a score differs from
  * the sum of lvar_colsum_fwd's columns in the last bits.  For callers that rank the blocks, `target` > 0 gives the
  * number of blocks they will keep per row (as lvar_block_topk_lists counts them, base_mask [G, ceil(Lk/block_k)] or
- * NULL): scores within 2^-18 (relative) of the cut are then replaced by the sum of lvar_colsum_fwd's block sums, and
- * the selection does not depend on which of the two computed the scores (up to 2048 blocks per row).
+ * NULL): scores whose distance from the cut the rounding of the sums and of the exponents might bridge (relative 2^-20,
+ * and 2^-23 of the exponents' size) are then replaced by the sum of lvar_colsum_fwd's block sums, so that the selection is
+ * the one that those sums give (up to 2048 blocks per row).
  * scratch: at least lvar_block_scores_scratch_bytes(), 16-byte aligned; written and read by this call only.
  */
 int64_t lvar_block_scores_scratch_bytes(int B, int H, int Lq, int Lk, int q_group_size, int block_k);

@@ -13,19 +13,25 @@ namespace lvar {
 constexpr int SCORE_MAX_GROUP = 1024;   // query rows per group (their weights sit in LDS)
 constexpr int REFINE_MAX_ITEMS = 8;     // scores of a row that are computed one by one, see list_close_scores
 constexpr int REFINE_MAX_NK = 2048;     // blocks per row that can be ranked (their keys sit in LDS); the limit of the block top-k kernel
-// Two orders of the sums of a score differ by a few units in the last place (5e-7 at most over the declared video sizes);
-// scores this far apart (relative, 64 units) keep their order.
-constexpr float REFINE_EPS = 0x1p-18f;
+// Distance (relative) from which two scores keep their order whichever of the two forms computed them: twice what the forms
+// differ by.  The sums and the exponentials: a few units of 2^-24 (4 for N(0, 1) * 0.5 inputs), 16 allowed for the pair.
+// The exponents, rounded to 2^-24 of their size: one form rounds (logit - reference) and (reference - statistic), the
+// other (logit - statistic).  With D the largest distance of a first reference from the statistic among the rows, N terms
+// per score and the score V, the terms' mean distance from their statistics is at most log2(N) - log2(V) (concavity), so
+// that the pair differs in the order of 2^-23 (D + log2(N) + |log2(V)|): about 60 units for N(0, 1) * 0.5 inputs, 240 for
+// logits of 90 (measured there: 80 for one score, 160 for a pair).
+constexpr float REFINE_EPS = 0x1p-20f, REFINE_EPS_EXP = 0x1p-23f;
+constexpr float REFINE_FLOOR = 0x1p-120f;   // scores below this are close to one another (terms flush to zero in one form and not in the other)
 
 __device__ __forceinline__ float key_value(uint32_t k) { return __builtin_bit_cast(float, k ^ ((k >> 31) ? 0x80000000u : 0xffffffffu)); }
 
-// One wave per row: appends the row's scores that lie within REFINE_EPS of the cut of "base blocks plus the best others up
+// One wave per row: appends the row's scores that lie within that distance of the cut of "base blocks plus the best others up
 // to `target`" to the work list, when both sides of the cut do.  A score alone costs a wave its operands straight from
 // memory, 40 KiB; the column-sum kernel forms all 256 of a row for the price of twenty.  So a row with more than a few is
 // listed as a row (the complement of its number) and the column sums of its (batch, head) run: with zero queries (every
 // score of every row close) the 24-head 8 x 64 x 64 video lists took 15.3 ms score by score and take 2.6 ms now, against
 // 1.6 ms without ties; the launch costs 3 us where no row asks for it.
-__device__ __forceinline__ void list_close_scores(const BlockScoreParams& p, const uint32_t* key, int row) {
+__device__ __forceinline__ void list_close_scores(const BlockScoreParams& p, const uint32_t* key, const float* wt, int n_wt, int row) {
   const int lane = threadIdx.x & 63, nK = p.nK;
   int others = 0;
   for (int j0 = 0; j0 < nK; j0 += 64) others += __builtin_popcountll(__builtin_amdgcn_ballot_w64(j0 + lane < nK && key[j0 + lane] != 0u));
@@ -48,7 +54,12 @@ __device__ __forceinline__ void list_close_scores(const BlockScoreParams& p, con
       if (key[j] < cut) below = max(below, key[j]);
     for (int d = 32; d > 0; d >>= 1) below = max(below, (uint32_t)__shfl_xor((int)below, d, 64));
   }
-  const float hi = key_value(cut), lo = key_value(below), eps = REFINE_EPS * fabsf(hi);
+  float w = 1.f;   // smallest weight exp2(reference - statistic) of the rows
+  for (int t = lane; t < n_wt; t += 64) w = wt[t] > 0.f ? fminf(w, wt[t]) : w;
+  for (int d = 32; d > 0; d >>= 1) w = fminf(w, __shfl_xor(w, d, 64));
+  const float hi = key_value(cut), lo = key_value(below);
+  const float size = __builtin_amdgcn_logf((float)p.group_rows * (float)(p.r.block_stages * 64)) - __builtin_amdgcn_logf(w) + fabsf(__builtin_amdgcn_logf(fmaxf(hi, REFINE_FLOOR)));
+  const float eps = fmaf(fmaf(REFINE_EPS_EXP, size, REFINE_EPS), hi, REFINE_FLOOR);
   if (!(hi - lo <= eps)) return;
   auto close = [&](int j) { return j < nK && key[j] != 0u && key_value(key[j]) >= lo - eps && key_value(key[j]) <= hi + eps; };
   int n = 0;
@@ -113,7 +124,7 @@ __global__ __launch_bounds__(256) void block_score_finish_kernel(const BlockScor
   if (!rank) return;
   __syncthreads();
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-  if (wave < (HALF ? 2 : 1) && g0 + wave < p.G) list_close_scores(p, keys + wave * nK, bh * p.G + g0 + wave);
+  if (wave < (HALF ? 2 : 1) && g0 + wave < p.G) list_close_scores(p, keys + wave * nK, wt + wave * 32, HALF ? 32 : have * 64, bh * p.G + g0 + wave);
 }
 
 constexpr int REFINE_WGS = 256;   // of four waves

@@ -113,7 +113,8 @@ __global__ __launch_bounds__(256, (D <= 128 ? ROW_LSE_WGS : 1)) void row_lse_ker
   const int kbase_l = r * ROWB + ((hh ^ ((r / SWD) & SWM)) << 4);
   // Reference and sum of this lane's half of the keys, per query row.  The sum runs in the order of the attention
   // kernel's row sum (even and odd elements of a 64-key stage apart; the two halves of the last stage apart), with the
-  // same first reference: statistics of one key range have the bits that the attention kernel gives.
+  // same first reference: while neither kernel moves its reference (the attention kernel does for a logit 2^8 above it,
+  // this one for a sum above LSE_SUM_LIMIT), statistics of one key range have the bits that the attention kernel gives.
   float m[2], l[2] = {0.f, 0.f}, la[2], lb[2];
   // SCORES: stages left in the open key block, and its sum against the first reference; lane = row of the wave (both
   // halves of the keys added up), one register.  (Two sums, one per half, spill; sums in LDS cost the loop 40 %: an

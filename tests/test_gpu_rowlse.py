@@ -255,3 +255,29 @@ def test_block_scores_ties_at_the_cut_of_large_logits(amp, group, low):
         k[:, :, 0, :, 0] = -low * 128 ** 0.5
     k = k.flatten(2, 3) if low else k[:, :, 1:].flatten(2, 3)
     _check_scores(q.to(torch.bfloat16).cuda(), k.to(torch.bfloat16).contiguous().cuda(), 128 ** -0.5, group, 128, 3)
+
+
+@pytest.mark.parametrize("amp,low", [(1, 0), (1, 60), (4, 45), (16, 0), (16, 30), (16, 60), (64, 0), (64, 20), (64, 30)])
+def test_block_scores_differ_from_two_passes_by_less_than_half_the_distance_looked_at(amp, low):
+    """Scores from one sweep, none computed again, against the column sums: half of the distance from the cut within which
+    both forms are compared, 2^-20 + 2^-23 (D + log2(terms) + |log2(score)|), D = statistic less the first stage's maximum.
+    (The other half is the other score's.  Measured: 4 units of 2^-24 for plain inputs, 80 at the largest logits here.)"""
+    from lvar_amd import _lib, sparse_attn_ops as ops
+    g = torch.Generator(device="cuda").manual_seed(amp * 100 + low)
+    q = torch.randn(1, 4, 1024, 128, generator=g, device="cuda") * 0.5 * amp
+    k = torch.randn(1, 4, 2048, 128, generator=g, device="cuda") * 0.5
+    q[..., 0] = 1.0
+    k[..., 0] = 0.0
+    k[:, :, :64, 0] = -low * 128 ** 0.5
+    q, k, scale = q.to(torch.bfloat16), k.to(torch.bfloat16), 128 ** -0.5
+    lib = _lib.load()
+    one = torch.empty(1, 4, 32, 16, device="cuda")
+    nbytes = lib.lvar_block_scores_scratch_bytes(1, 4, 1024, 2048, 32, 128)
+    scratch = torch.empty(nbytes, dtype=torch.uint8, device="cuda")
+    assert lib.lvar_block_scores_fwd(ops._view(q), ops._view(k), one.data_ptr(), None, 0, scratch.data_ptr(), nbytes, 1, 4, 4, 1024, 2048, 128,
+                                     32, 128, scale, ops._stream(q)) == 0
+    two = ops._colsum_block_scores(q, k, scale, 32, 128).double()
+    s = torch.matmul(q.double(), k.double().transpose(-1, -2).contiguous()) * (scale * LOG2E)
+    far = (torch.logsumexp(s * math.log(2.0), -1) / math.log(2.0) - s[..., :64].amax(-1)).unflatten(-1, (32, 32)).amax(-1, keepdim=True)
+    limit = 2.0 ** -20 + 2.0 ** -23 * (far + math.log2(32 * 128) + two.clamp_min(2.0 ** -120).log2().abs())
+    assert bool(((one.double() - two).abs() <= 0.5 * limit * two + 2.0 ** -120).all())
