@@ -104,7 +104,10 @@ static int dense_common(lvar_tensor_t q, lvar_tensor_t k, lvar_tensor_t v, lvar_
   if (!kv_span_ok(k, Lk, head_dim) || (!lse_only && !kv_span_ok(v, Lk, head_dim))) return LVAR_EINVAL;
   if (!lse_only && (!view_ok(v) || !view_ok(o) || o.stride_row <= 0)) return LVAR_EINVAL;
   if (lse_only && !((M && L) || LSE2 || RCP)) return LVAR_EINVAL;
-  if (lse_only && !M && !L && !RCP)   // the row statistic alone has a kernel of its own
+  // The row statistic alone has a kernel of its own, which gives 256 rows to a workgroup; with uncut keys it is the faster
+  // one once the attention kernel's 128-row workgroups are more than the compute units (its time against the attention
+  // kernel's, B2 H16 d128: 1024 x 2521 40.5 / 36.1 us, 1056 x 2521 39.7 / 48.9; B1 H2 128 x 4121: d128 56.0 / 48.3, d256 94.6 / 71.8).
+  if (lse_only && !M && !L && !RCP && (int64_t)B * H * ((Lq + 127) / 128) > device_cus())
     return lvar_row_lse_fwd(q, k, LSE2, nullptr, 0, B, H, kv_heads, Lq, Lk, head_dim, scale, stream);
   AttnParams p{};
   fill_qkv(p, q, k, lse_only ? k : v);

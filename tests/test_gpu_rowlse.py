@@ -281,3 +281,46 @@ def test_block_scores_differ_from_two_passes_by_less_than_half_the_distance_look
     far = (torch.logsumexp(s * math.log(2.0), -1) / math.log(2.0) - s[..., :64].amax(-1)).unflatten(-1, (32, 32)).amax(-1, keepdim=True)
     limit = 2.0 ** -20 + 2.0 ** -23 * (far + math.log2(32 * 128) + two.clamp_min(2.0 ** -120).log2().abs())
     assert bool(((one.double() - two).abs() <= 0.5 * limit * two + 2.0 ** -120).all())
+
+
+def _dense_stats(q, k, want_ml):
+    """lvar_dense_attn_fwd without an output: LSE2 alone, or M and L."""
+    from lvar_amd import _lib, sparse_attn_ops as ops
+    B, H, Lq, d = q.shape
+    out = torch.empty(2, B, H, Lq, device="cuda")
+    none = _lib.LvarTensor(None, 0, 0, 0)
+    a, b, c = (out[0].data_ptr(), out[1].data_ptr(), None) if want_ml else (None, None, out[0].data_ptr())
+    assert _lib.load().lvar_dense_attn_fwd(ops._view(q), ops._view(k), none, none, a, b, c, B, H, k.shape[1], Lq, k.shape[2], d, d ** -0.5, ops._stream(q)) == 0
+    return out[0] + torch.log2(out[1]) if want_ml else out[0]
+
+
+# at most one 128-row workgroup of the attention kernel per compute unit, and more
+@pytest.mark.parametrize("B,H,Hkv,Lq,Lk,d", [(1, 2, 1, 128, 4121, 128), (2, 16, 16, 1024, 700, 64), (2, 16, 16, 1025, 700, 64), (1, 260, 130, 77, 300, 128),
+                                             (1, 2, 2, 300, 127, 256), (3, 100, 100, 100, 65, 256)])
+def test_statistic_alone_from_either_kernel(B, H, Hkv, Lq, Lk, d):
+    g = torch.Generator(device="cuda").manual_seed(Lq)
+    q = torch.randn(B, H, Lq, d, generator=g, device="cuda").to(torch.bfloat16)
+    k = torch.randn(B, Hkv, Lk, d, generator=g, device="cuda").to(torch.bfloat16)
+    got = _dense_stats(q, k, False)
+    assert (got.double().cpu() - _ref(q, k, d ** -0.5)).abs().max() <= 2.0 ** -13      # 2^-17 of the largest statistic (< 2^4), see _check
+    assert torch.allclose(got, _dense_stats(q, k, True), rtol=0, atol=2.0 ** -18)       # the sum's logarithm and one addition, rounded
+
+
+def test_statistic_alone_of_few_rows_costs_no_more_than_with_the_maximum():
+    """256 rows per workgroup and uncut keys take a third longer where the rows leave compute units idle."""
+    g = torch.Generator(device="cuda").manual_seed(2)
+    q, k = (torch.randn(1, 2, L, 256, generator=g, device="cuda").to(torch.bfloat16) for L in (128, 8192))
+
+    def time_of(want_ml):
+        times = []
+        for _ in range(6):
+            a, b = torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True)
+            a.record()
+            for _ in range(20):
+                _dense_stats(q, k, want_ml)
+            b.record()
+            torch.cuda.synchronize()
+            times.append(a.elapsed_time(b))
+        return sorted(times[1:])[2]
+    with_max = time_of(True)
+    assert time_of(False) < 1.15 * with_max
