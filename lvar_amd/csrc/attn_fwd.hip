@@ -830,8 +830,9 @@ __device__ __forceinline__ void attn_item(const AttnParams& p, char* smem, const
 }
 #endif  // __HIP_DEVICE_COMPILE__
 
-template <int D, int NWAVES, int MODE, bool ACCUM, bool LSE_ONLY>
-__global__ __launch_bounds__(NWAVES * 64, ((NWAVES <= 4 && D <= 128) ? (D == 64 && MODE == MODE_BLOCK && !LSE_ONLY ? 3 : 2) : 1)) void attn_fwd_kernel(const AttnParams p) {
+// THIRD: registers of a wave limited so that three workgroups share a compute unit, see third_workgroup
+template <int D, int NWAVES, int MODE, bool ACCUM, bool LSE_ONLY, bool THIRD = false>
+__global__ __launch_bounds__(NWAVES * 64, ((NWAVES <= 4 && D <= 128) ? (THIRD ? 3 : 2) : 1)) void attn_fwd_kernel(const AttnParams p) {
   // The body is compiled for the device only: the host pass just needs the launch stub, and it
   // silently drops the stub when the body uses the LDS-DMA builtins.
 #if defined(__HIP_DEVICE_COMPILE__)
@@ -993,6 +994,13 @@ static bool wide_tiles(const AttnParams& p, int head_dim) {
   return wide < narrow;
 }
 
+// Three 128-row workgroups per compute unit at head_dim 64: 168 registers per wave instead of 180, two of them spilled.  Where
+// two per compute unit hold the launch the third slot stays empty and the spills cost 1 to 4 % (two against three: B8 H16
+// 256 x 680 12.4 / 12.9 us, B2 H16 2048 x 4121 in lists of 30 % 29.3 / 29.9 us); larger launches are up to 9 % faster (B2 H17
+// 2048 x 4121 115 / 105 us, B2 H16 2304 x 6425 177 / 164 us).  The 2-wave workgroups of 64-row query blocks are not (B2 H16
+// 4096 x 10521 in lists of 30 %: 149 / 162 us).
+static bool third_workgroup(int total_wg) { return total_wg > 2 * device_cus(); }
+
 template <int D, int NWAVES, int MODE, bool ACCUM, bool LSE_ONLY>
 static int launch_one(const AttnParams& p0, hipStream_t stream) {
   AttnParams p = p0;
@@ -1049,6 +1057,13 @@ static int launch_one(const AttnParams& p0, hipStream_t stream) {
     if (wide_tiles(p0, D)) return launch_one<D, 8, MODE_BLOCK, false, false>(p0, stream);
   }
   const int grid = ((p.total_wg + 7) / 8) * 8;
+  if constexpr (D == 64 && NWAVES == 4 && MODE == MODE_BLOCK && !LSE_ONLY) {
+    if (third_workgroup(p.total_wg)) {
+      static_assert(SMEM <= 48 * 1024, "three workgroups share the LDS of a compute unit; no larger limit has to be asked for");
+      hipLaunchKernelGGL((attn_fwd_kernel<D, NWAVES, MODE, ACCUM, LSE_ONLY, true>), dim3(grid), dim3(NWAVES * 64), SMEM, stream, p);
+      return hipGetLastError() == hipSuccess ? LVAR_OK : LVAR_ELAUNCH;
+    }
+  }
   auto kern = attn_fwd_kernel<D, NWAVES, MODE, ACCUM, LSE_ONLY>;
   static std::atomic<uint64_t> lds_ready{0};
   if (!ensure_lds_limit((const void*)kern, SMEM, lds_ready)) return LVAR_ELAUNCH;

@@ -28,6 +28,24 @@ def test_attention_of_a_head_does_not_depend_on_the_others(B, H, Lq, Lk, d):
         assert torch.equal(o1[0], ob[b, h]) and torch.equal(M1[0], Mb[b, h]) and torch.equal(L1[0], Lb[b, h])
 
 
+# head_dim 64: as many 128-row workgroups as two per compute unit hold, and one row more per head; lists of 128 and of 64 rows
+@pytest.mark.parametrize("extra,bq", [(0, 128), (1, 128), (0, 64), (1, 64)])
+def test_head_dim_64_on_both_sides_of_two_workgroups_per_compute_unit(extra, bq):
+    from lvar_amd import sparse_attn_ops as ops
+    H, Lk = torch.cuda.get_device_properties(0).multi_processor_count // 4, 300
+    q, k, v = _rand(1, H, 1024 + extra, Lk, 64, seed=extra)               # 8 or 9 tiles of 128 rows per head
+    g = torch.Generator(device="cuda").manual_seed(bq)
+    num, idx = ops.mask_to_lists(torch.rand(1, H, -(-(1024 + extra) // bq), -(-Lk // 64), generator=g, device="cuda") < 0.6)
+    o, (M, L) = ops.block_sparse_attn(q, k, v, num, idx, bq, 64)
+    od, (Md, Ld) = ops.dense_attn(q, k, v)
+    h = slice(H - 2, H)
+    part = [t[:, h].contiguous() for t in (q, k, v)]
+    o1, (M1, L1) = ops.block_sparse_attn(*part, num[:, h].contiguous(), idx[:, h].contiguous(), bq, 64)
+    assert torch.equal(o1, o[:, h]) and torch.equal(M1, M[:, h]) and torch.equal(L1, L[:, h])
+    o1, (M1, L1) = ops.dense_attn(*part)
+    assert torch.equal(o1, od[:, h]) and torch.equal(M1, Md[:, h]) and torch.equal(L1, Ld[:, h])
+
+
 @pytest.mark.parametrize("B,H,n,S", [(1, 4, 7, 20), (2, 16, 5, 12), (1, 8, 8, 24), (2, 16, 10, 40)])
 def test_full_step_lists_do_not_depend_on_the_host_path(B, H, n, S, monkeypatch):
     """Column sums of three repeats of the same keys in other orders: scores that are equal up to the order of their sums."""
