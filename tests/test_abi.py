@@ -103,6 +103,46 @@ def test_list_build_and_upsample_argument_validation(lib):
     assert lib.lvar_csp_attn_upsample_fwd(fake, fake, fake, null, 2, 4, fake, None, None, *args) == -1
 
 
+def test_statistics_score_and_merge_argument_validation(lib):
+    from lvar_amd._lib import LvarTensor
+    null = LvarTensor(None, 0, 0, 0)
+    fake = LvarTensor(0x1000, 128 * 16 * 128, 16 * 128, 128)
+    odd = LvarTensor(0x1008, 128 * 16 * 128, 16 * 128, 128)
+    far = LvarTensor(0x1000, 1 << 40, 1 << 36, 1 << 27)                  # 16 rows span 2^32 bytes
+    one, odd4 = ctypes.c_void_p(0x2000), ctypes.c_void_p(0x2002)
+    # row statistics: q, k, lse2, scratch, bytes, B, H, kv_heads, Lq, Lk, head_dim
+    for q, k, out, scratch, dims, status in (
+            (null, fake, one, None, (1, 1, 1, 16, 16, 128), -1), (fake, odd, one, None, (1, 1, 1, 16, 16, 128), -1),
+            (fake, fake, None, None, (1, 1, 1, 16, 16, 128), -1), (fake, fake, one, odd4, (1, 1, 1, 16, 16, 128), -1),
+            (fake, fake, one, None, (1, 6, 4, 16, 16, 128), -1), (fake, fake, one, None, (1, 6, 0, 16, 16, 128), -1),
+            (fake, fake, one, None, (1, 1, 1, 0, 16, 128), -1), (fake, fake, one, None, (1, 1, 1, 16, -1, 128), -1),
+            (fake, far, one, None, (1, 1, 1, 16, 16, 128), -1), (fake, fake, one, None, (1, 1, 1, 16, 16, 96), -2)):
+        assert lib.lvar_row_lse_fwd(q, k, out, scratch, 64, *dims, 1.0, None) == status, dims
+    assert lib.lvar_row_lse_fwd(fake, fake, one, None, 0, 1, 1, 1, 16, 16, 128, -1.0, None) == -1
+    assert lib.lvar_row_lse_scratch_bytes(0, 1, 16, 16) == -1 and lib.lvar_row_lse_scratch_bytes(1, 1, 16, 0) == -1
+    for m, l, out, rows in ((None, one, one, 4), (one, None, one, 4), (one, one, None, 4), (one, one, one, 0)):
+        assert lib.lvar_lse2_from_stats(m, l, out, rows, None) == -1
+    # block scores
+    need = lib.lvar_block_scores_scratch_bytes(1, 1, 16, 16, 32, 128)
+    assert need > 0
+    assert all(lib.lvar_block_scores_scratch_bytes(1, 1, 16, 16, g, b) == -1 for g, b in ((0, 128), (32, 0), (32, 96)))
+
+    def scores(q=fake, k=fake, out=one, target=1, scratch=one, nbytes=need, H=1, kv=1, d=128, group=32, block=128, scale=1.0):
+        return lib.lvar_block_scores_fwd(q, k, out, None, target, scratch, nbytes, 1, H, kv, 16, 16, d, group, block, scale, None)
+    big = dict(nbytes=1 << 40)
+    for bad in (dict(q=null), dict(k=odd), dict(out=None), dict(target=-1), dict(scratch=None), dict(scratch=ctypes.c_void_p(0x2008)),
+                dict(nbytes=need - 1), dict(H=6, kv=4, **big), dict(k=far), dict(q=far), dict(group=0), dict(group=33), dict(block=96), dict(scale=0.0)):
+        assert scores(**bad) == -1, bad
+    for bad in (dict(group=96, **big), dict(group=1088, **big), dict(d=96)):   # group sizes and head sizes without a one-sweep kernel
+        assert scores(**bad) == -2, bad
+    # merged selection: scores, row stride, listed, how many, out, rows, Lk, k
+    for args, status in (((None, 100, one, 4, one, 2, 100, 10), -1), ((one, 100, None, 4, one, 2, 100, 10), -1), ((one, 100, one, 4, None, 2, 100, 10), -1),
+                         ((one, 100, one, 0, one, 2, 100, 10), -1), ((one, 99, one, 4, one, 2, 100, 10), -1), ((one, 100, one, 4, one, 2, 100, 101), -1),
+                         ((one, 100, one, 4, one, 2, 100, 0), -1), ((one, 100, one, 4, one, -1, 100, 10), -1), ((one, 16385, one, 4, one, 2, 16385, 10), -2),
+                         ((one, 100, one, 65536, one, 2, 100, 10), -2), ((one, 100, one, 4, one, 0, 100, 10), 0)):
+        assert lib.lvar_topk_union_lists(*args, None) == status, args
+
+
 def test_header_is_plain_c(tmp_path):
     """The public header must be usable from C (the reference's other bindings are C/C++)."""
     import shutil
