@@ -1,0 +1,184 @@
+"""Every instance of the selection kernels, and every operator through both of its host paths."""
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+
+
+def _scores(kind, rows, n, seed):
+    g = torch.Generator(device="cuda").manual_seed(seed)
+    x = torch.rand(rows, n, generator=g, device="cuda")
+    if kind == "ties":
+        x = (x * 7).floor() - 3.0
+    elif kind == "equal":
+        x = torch.full_like(x, 0.25)
+    elif kind == "one_binade":
+        x = 1.0 + x
+    return x
+
+
+def _selected(x, k):
+    """Columns of the k largest values of every row, equal ones by column, ascending."""
+    return torch.sort(x, dim=-1, descending=True, stable=True).indices[:, :k].sort(dim=-1).values
+
+
+# keys per thread: up to 24 of 512 threads, 28, 32, and rows that are read again in every pass; 1024 threads, up to 16
+# keys, where there are at most two rows per compute unit
+@pytest.mark.parametrize("kind", ["distinct", "ties"])
+@pytest.mark.parametrize("few_rows,step", [*((False, s) for s in (*range(1, 25), 28, 32, 33)), *((True, s) for s in range(1, 17))])
+def test_topk_lists_at_every_number_of_keys_per_thread(few_rows, step, kind):
+    from lvar_amd import sparse_attn_ops as ops
+    threads = 1024 if few_rows else 512
+    rows = 3 if few_rows else 2 * torch.cuda.get_device_properties(0).multi_processor_count + 1
+    for n in (threads * (step - 1) + 1, threads * step):
+        x = _scores(kind, rows, n, seed=n)
+        for k in sorted({1, max(1, n // 5), n}):
+            idx, cnt = ops.topk_token_lists(x, k)
+            assert torch.equal(idx[:, :k].long(), _selected(x, k)), (n, k)
+            assert bool((idx[:, k:] == 0).all()) and bool((cnt == k).all())
+
+
+# 1024 threads with up to 16 keys each
+@pytest.mark.parametrize("kind", ["distinct", "ties", "equal", "one_binade"])
+@pytest.mark.parametrize("n", [1, 2, 3, 63, 64, 65, 1023, *[m for s in range(1, 16) for m in (1024 * s, 1024 * s + 1)], 16383, 16384])
+def test_merged_selection_at_every_number_of_keys_per_thread(n, kind):
+    """Every selected column once and every listed one as often as it is listed, in ascending order."""
+    from lvar_amd import _lib
+    lib, rows = _lib.load(), 3
+    x = _scores(kind, rows, n, seed=n + 1)
+    g = torch.Generator(device="cuda").manual_seed(n)
+    for k, W in ((1, 1), (max(1, n // 3), 9), (max(1, n - 1), 256), (n, 300)):
+        more = torch.randint(0, n, (rows, W), generator=g, device="cuda")
+        more[1] = int(more[1, 0])                              # one column W times
+        if W > 8:
+            more[0, 3], more[0, 5], more[2, 1] = -7, n + 5, n - 1   # (columns outside the row count as the nearest one)
+        out = torch.full((rows, k + W), -1, dtype=torch.int64, device="cuda")
+        st = lib.lvar_topk_union_lists(x.data_ptr(), n, more.data_ptr(), W, out.data_ptr(), rows, n, k, torch.cuda.current_stream().cuda_stream)
+        assert st == 0
+        assert torch.equal(out, torch.cat([_selected(x, k), more.clamp(0, n - 1)], -1).sort(dim=-1).values), (k, W)
+
+
+def test_merged_selection_of_the_longest_list():
+    from lvar_amd import _lib
+    x = _scores("distinct", 2, 5, seed=1)
+    more = torch.full((2, 65535), 3, dtype=torch.int64, device="cuda")
+    more[1] = torch.arange(65535, device="cuda") % 5
+    out = torch.full((2, 65537), -1, dtype=torch.int64, device="cuda")
+    assert _lib.load().lvar_topk_union_lists(x.data_ptr(), 5, more.data_ptr(), 65535, out.data_ptr(), 2, 5, 2, torch.cuda.current_stream().cuda_stream) == 0
+    assert torch.equal(out, torch.cat([_selected(x, 2), more], -1).sort(dim=-1).values)
+
+
+class _Taken:
+    """The compiled host path, with a record of the functions that did not decline."""
+
+    def __init__(self, mod):
+        self.mod, self.names = mod, []
+
+    def __getattr__(self, name):
+        fn = getattr(self.mod, name)
+
+        def call(*a):
+            r = fn(*a)
+            if r is not None:
+                self.names.append(name)
+            return r
+        return call
+
+
+def _inputs(B, H, Hkv, Lq, Lk, d, strided, seed):
+    g = torch.Generator(device="cuda").manual_seed(seed)
+
+    def one(h, L):
+        if strided:   # [B, L, H, d] in memory, as a fused projection leaves it
+            return (torch.randn(B, L, h, d, generator=g, device="cuda") * 0.5).to(torch.bfloat16).transpose(1, 2)
+        return (torch.randn(B, h, L, d, generator=g, device="cuda") * 0.5).to(torch.bfloat16)
+    return one(H, Lq), one(Hkv, Lk), one(Hkv, Lk)
+
+
+def _calls(B, H, Hkv, Lq, Lk, d, strided, scale):
+    """(name of the compiled function, call) for every operator that takes these inputs."""
+    from lvar_amd import sparse_attn_ops as ops
+    q, k, v = _inputs(B, H, Hkv, Lq, Lk, d, strided, seed=Lq)
+    g = torch.Generator(device="cuda").manual_seed(Lk)
+    G, nQ, nK = -(-Lq // 192), -(-Lq // 128), -(-Lk // 64)
+    yield "fast_dense_attn", lambda: ops.dense_attn(q, k, v, scale)
+    yield "fast_dense_colsum_attn", lambda: ops.dense_colsum_attn(q, k, v, scale)
+    yield "fast_colsum", lambda: ops.colsum(q, k, scale)
+    yield "fast_colsum", lambda: ops.colsum(q, k, scale, q_group_size=64, return_block_sums=True)
+    lse = ops.dense_attn(q, k, v, scale)[1]
+    yield "fast_colsum", lambda: ops.colsum(q, k, scale, lse=lse)
+    yield "fast_colsum", lambda: ops._colsum_block_scores(q, k, scale, 128, 128)
+    x = torch.rand(B, H, G, Lk, generator=g, device="cuda")
+    keep = Lk // 3
+    idx, cnt = ops.topk_token_lists(x, keep)
+    yield "fast_topk_token_lists", lambda: ops.topk_token_lists(x, keep, out_len=keep + 5)
+    local = torch.randint(0, Lk, (G + 2, 7), generator=g, device="cuda")
+    yield "fast_remap_concat_lists", lambda: ops.remap_concat_lists(idx, keep, 192 * (G + 2) - 100, Lk, local)
+    yield "fast_remap_concat_lists", lambda: ops.remap_concat_lists(idx, keep, 192 * (G + 2) - 100, Lk, out_len=Lk + 3)
+    mask = torch.rand(B, H, nQ, nK, generator=g, device="cuda") < 0.5
+    yield "fast_mask_to_lists", lambda: ops.mask_to_lists(mask, 2)
+    s = torch.rand(B, H, nQ, nK, generator=g, device="cuda")
+    yield "fast_block_topk_lists", lambda: ops.block_topk_lists(s, max(1, nK // 2))
+    yield "fast_block_topk_lists", lambda: ops.block_topk_lists(s, max(1, nK // 2), mask[0, 0])
+    if H != Hkv:
+        return
+    acc = _inputs(B, H, H, Lq, Lk, d, strided, seed=7)[0]
+    yield "fast_csp_attn", lambda: ops.csp_attn(q, k, v, scale, idx, cnt, acc, -1)
+    if Lq in (100, 400):   # square grids
+        coarse = _inputs(B, H, H, 25, Lk, d, strided, seed=8)[0]
+        yield "fast_csp_attn", lambda: ops.csp_attn_upsampled(q, k, v, scale, idx, cnt, coarse)
+    num, blocks = ops.mask_to_lists(mask)
+    yield "fast_block_sparse_attn", lambda: ops.block_sparse_attn(q, k, v, num, blocks, 128, 64, scale)
+    yield "fast_block_sparse_attn", lambda: ops.block_sparse_attn_out(q, k, v, num[:1, :1].contiguous(), blocks[:1, :1].contiguous(), 128, 64, scale)
+    if Lq <= Lk:
+        win = torch.randint(Lk - Lq, Lk, (B, H, 5), generator=g, device="cuda")
+        yield "fast_window_keys", lambda: ops.window_key_scores(q, k, win, 5, "maxpool", scale)
+        yield "fast_window_keys", lambda: ops.scalekv_keep_indices(q, k, win, min(Lk, 40), 5, "avgpool")
+
+
+def _flat(x):
+    return [t for y in x for t in _flat(y)] if isinstance(x, (tuple, list)) else [x]
+
+
+@pytest.mark.parametrize("B,H,Hkv,Lq,Lk,d,strided,scale", [
+    (1, 2, 2, 1, 40, 128, False, None), (2, 3, 3, 100, 333, 64, True, 0.2), (1, 4, 4, 400, 921, 128, False, None),
+    (2, 2, 2, 191, 200, 128, True, None), (1, 4, 2, 385, 450, 128, True, 1), (1, 2, 1, 193, 130, 256, False, None)])
+def test_operators_do_not_depend_on_the_host_path(B, H, Hkv, Lq, Lk, d, strided, scale, monkeypatch):
+    from lvar_amd import _lib, sparse_attn_ops as ops
+    if _lib.torch_binding() is None:
+        pytest.skip("torch binding not built")
+    for name, call in _calls(B, H, Hkv, Lq, Lk, d, strided, scale):
+        taken = _Taken(_lib.torch_binding())
+        with monkeypatch.context() as m:
+            m.setattr(ops, "_native", lambda: taken)
+            a = _flat(call())
+        with monkeypatch.context() as m:
+            m.setattr(ops, "_native", lambda: None)
+            b = _flat(call())
+        assert name in taken.names, name
+        assert len(a) == len(b)
+        for x, y in zip(a, b):
+            assert (x is None and y is None) or (x.shape == y.shape and x.dtype == y.dtype and torch.equal(x, y)), name
+
+
+@pytest.mark.parametrize("B,d,strided", [(1, 128, False), (2, 64, True)])
+def test_sparse_steps_do_not_depend_on_the_host_path(B, d, strided, monkeypatch):
+    from lvar_amd import _lib, mask_build as mb, sparse_attn_ops as ops
+    from lvar_amd.sparse_diff_attn import SparseDiffAttn
+    if _lib.torch_binding() is None:
+        pytest.skip("torch binding not built")
+    scales = mb.INFINITY_SCALES[:8] + (20, 24, 28)
+    results = []
+    for native in (True, False):
+        taken = _Taken(_lib.torch_binding())
+        monkeypatch.setattr(ops, "_native", (lambda: taken) if native else (lambda: None))
+        layer = SparseDiffAttn(scales=scales, spsd_scale=8)
+        got = []
+        for ind in (8, 9, 10):
+            q, k, v = _inputs(B, 2, 2, scales[ind] ** 2, sum(s * s for s in scales[:ind + 1]), d, strided, seed=ind)
+            got.append(layer(q, k, v, None, do_full_step=ind == 8, scale_ind=ind))
+        results.append(got)
+        if native:
+            assert taken.names.count("fast_full_step") == 1 and taken.names.count("fast_sparse_step") == 2
+    for a, b in zip(*results):
+        assert torch.equal(a, b)
