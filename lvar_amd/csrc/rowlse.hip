@@ -101,10 +101,10 @@ __global__ __launch_bounds__(256, (D <= 128 ? ROW_LSE_WGS : 1)) void row_lse_ker
     }
   };
   constexpr auto vm = [](int n) constexpr { return 0x0f70 | (n & 15) | (((n >> 4) & 3) << 14); };
-  // wait until at most `younger` later stages of this wave's fills are still in flight
+  // wait until at most `younger` later stages (0 or 1: the ring has two) of this wave's fills are still in flight
+  static_assert(PF == 1, "wait_fills knows one stage ahead");
   auto wait_fills = [&](int younger) {
-    if (PF >= 3 && younger >= 2) __builtin_amdgcn_s_waitcnt(vm(2 * SLOTS));
-    else if (younger >= 1) __builtin_amdgcn_s_waitcnt(vm(SLOTS));
+    if (younger >= 1) __builtin_amdgcn_s_waitcnt(vm(SLOTS));
     else __builtin_amdgcn_s_waitcnt(vm(0));
   };
 
@@ -440,7 +440,7 @@ int launch_lse2_from_stats(const float* M, const float* L, float* lse2, int64_t 
 
 // Key ranges per row tile: workgroups are handed to the resident slots as slots fall free, so a
 // launch takes its total work over the slots plus a part of the longest workgroup while the chip drains (the model of
-// the colsum launch, in 64-key stages of about 2 us), and the merge of several ranges costs a launch of its own.
+// the colsum launch, in 64-key stages of about 3 us), and the merge of several ranges costs a launch of its own.
 int row_lse_splits(int B, int H, int Lq, int Lk) {
   const int base_wg = B * H * ((Lq + 255) / 256), slots = ROW_LSE_WGS * device_cus(), stages = (Lk + 63) / 64;
   if (slots <= 0 || base_wg >= 4 * slots) return 1;
