@@ -46,7 +46,7 @@ __device__ __forceinline__ uint32_t wave_umin(uint32_t v) {
 //   columns in ascending order (ballot compaction into an LDS ring, full-width stores).
 // ---------------------------------------------------------------------------------------------
 constexpr int TOPK_BINS = 2048;
-constexpr int TOPK_FEW_ROWS_PER_CU = 2;
+constexpr int TOPK_SHARED_MAX_N = 12288;   // longest row of 1024 threads where two rows share a compute unit
 constexpr int TOPK_CAND = 256;   // keys of the first pass's bin that are resolved by direct comparison
 
 // UNION: the output row is the ascending merge of the selection with the row's own list of W columns (in any order,
@@ -302,10 +302,15 @@ int launch_topk_token_lists(const TopkListParams& p, hipStream_t stream) {
     topk_dispatch<1024, true>(p, stream, std::make_integer_sequence<int, TOPK_UNION_MAX_N / 1024>{});
     return hipGetLastError() == hipSuccess ? LVAR_OK : LVAR_ELAUNCH;
   }
-  // A row is a chain of short phases that end in a barrier.  With at most one row per compute unit and its neighbour
-  // half as many keys per thread shorten every phase; with more rows the 512-thread workgroups of several rows fill
-  // each other's gaps better.  (Rows of 512 keys and less have one key per thread either way.)
-  const bool few = p.rows <= TOPK_FEW_ROWS_PER_CU * device_cus() && p.n > 512 && p.n <= 16384;
+  // A row is a chain of short phases that end in a barrier.  With at most one row per compute unit half as many keys per
+  // thread shorten every phase (1024 against 512 threads, 256 rows: of 6000 keys 8.3 / 11.6 us, of 10521 10.9 / 12.3, of
+  // 16384 14.8 / 17.2).  With a second row per compute unit they still win or tie up to 12 keys per thread (512 rows of
+  // 10521: 15.7 / 17.0, 257 rows: 14.5 / 14.6), but not beyond: two workgroups then no longer run side by side (512 rows of
+  // 12288: 17.9 / 19.8, of 12289: 22.5 / 21.9, of 14336: 25.2 / 22.7; the instances with 13 keys and more are the first
+  // with more than 80 scalar registers).  With more rows the 512-thread workgroups of several rows fill each other's
+  // gaps better.  (Rows of 512 keys and less have one key per thread either way.)
+  const int cus = device_cus();
+  const bool few = p.n > 512 && (p.rows <= cus ? p.n <= 16384 : p.rows <= 2 * cus && p.n <= TOPK_SHARED_MAX_N);
   if (few) topk_dispatch<1024, false>(p, stream, std::make_integer_sequence<int, 16>{});
   // 512 threads per row keep a row of up to 16384 keys in registers (KPT keys per thread)
   else if (!topk_dispatch<512, false>(p, stream, std::make_integer_sequence<int, 24>{}) && !topk_try<28, 512, false>(p, stream) && !topk_try<32, 512, false>(p, stream))

@@ -38,6 +38,37 @@ def test_topk_lists_at_every_number_of_keys_per_thread(few_rows, step, kind):
             assert bool((idx[:, k:] == 0).all()) and bool((cnt == k).all())
 
 
+# two rows per compute unit: 1024 threads up to 12288 keys, 512 beyond
+@pytest.mark.parametrize("n", [12288, 12289])
+@pytest.mark.parametrize("more", [0, 1])
+@pytest.mark.parametrize("per_cu", [1, 2])
+def test_topk_lists_on_both_sides_of_the_thread_rule(per_cu, more, n):
+    from lvar_amd import sparse_attn_ops as ops
+    rows = per_cu * torch.cuda.get_device_properties(0).multi_processor_count + more
+    x = _scores("ties", rows, n, seed=rows)
+    idx, _ = ops.topk_token_lists(x, n // 3)
+    assert torch.equal(idx[:, :n // 3].long(), _selected(x, n // 3))
+
+
+@pytest.mark.parametrize("per_cu,more", [(1, 1), (2, 0)])
+def test_topk_lists_of_two_rows_per_compute_unit_do_not_step_behind_the_rule(per_cu, more):
+    """Rows of 14336 keys, a sixth more than 12288: 1.42 and 1.43 times as long with 1024 threads, 1.18 and 1.23 with 512."""
+    from lvar_amd import sparse_attn_ops as ops
+    rows = per_cu * torch.cuda.get_device_properties(0).multi_processor_count + more
+    g = torch.Generator(device="cuda").manual_seed(1)
+    calls, best = [torch.randn(rows, n, generator=g, device="cuda") for n in (12288, 14336)], [float("inf")] * 2
+    for _ in range(8):
+        for i, s in enumerate(calls):
+            start, end = (torch.cuda.Event(enable_timing=True) for _ in range(2))
+            start.record()
+            for _ in range(50):
+                ops.topk_token_lists(s, s.shape[-1] // 5)
+            end.record()
+            end.synchronize()
+            best[i] = min(best[i], start.elapsed_time(end))
+    assert best[1] < 1.32 * best[0]
+
+
 # 1024 threads with up to 16 keys each
 @pytest.mark.parametrize("kind", ["distinct", "ties", "equal", "one_binade"])
 @pytest.mark.parametrize("n", [1, 2, 3, 63, 64, 65, 1023, *[m for s in range(1, 16) for m in (1024 * s, 1024 * s + 1)], 16383, 16384])
