@@ -314,7 +314,10 @@ def video_window_topk_block_lists(q: torch.Tensor, k: torch.Tensor, scale=None, 
     rows = q[:, :, ::query_stride]
     target = int(round(density * nK))
     if block % 64 == 0 and q.shape[-1] >= 64:      # block sums without the column sums themselves
-        score = ops._block_scores_for_topk(rows, k, scale, block // query_stride, block, base, target)
+        if q.is_cuda and ops._few_rows_for_one_sweep(rows, k):
+            score = ops._block_scores_of_few_rows(rows, k, scale, block // query_stride, block)
+        else:
+            score = ops._block_scores_for_topk(rows, k, scale, block // query_stride, block, base, target)
     else:
         score = key_block_sums(ops.colsum(rows, k, scale, q_group_size=block // query_stride), block).contiguous()
     num, idx = ops.block_topk_lists(score, target, base)

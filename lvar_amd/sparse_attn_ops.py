@@ -304,11 +304,35 @@ def _colsum_block_scores(q, k, scale, q_group_size: int, block_k: int):
         q, k = _prep(q, "q"), _prep(k, "k")
         _check_qkv(q, k, k, gqa=True)
         r = _colsum_given_lse(q, k, _lse_only(q, k, scale, cut_keys=False), scale, q_group_size, want_block_sums=True, want_columns=False)
-    bs = r[1]
+    return _sum_blocks(r[1], block_k)
+
+
+def _sum_blocks(bs, block_k: int):
+    """Sums of 64-key blocks added up to blocks of ``block_k`` keys."""
     m = block_k // 64
     if m == 1:
         return bs
     return torch.nn.functional.pad(bs, (0, -bs.shape[-1] % m)).unflatten(-1, (-1, m)).sum(-1)
+
+
+def _few_rows_for_one_sweep(q, k) -> bool:
+    """Whether :func:`_block_scores_of_few_rows` beats the sweep of :func:`_block_scores_for_topk`.  The sweep gives 256 rows
+    to a workgroup and does not cut the keys; the statistics sweep of the attention kernel gives 128, and the column sums
+    cut the rows.  Head_dim 128, 32-row groups, 128-key blocks: 4 workgroups of the sweep and 64 stages of 64 keys 70.8 us
+    against 59.2; 16 and 128 stages 125.8 / 111.0; 32 and 512 stages 480 / 452; 48: 254 / 252; 64: 485 / 521.  At
+    head_dim 256 64 workgroups 820 / 807, 80: 426 / 445.  With few keys the launches count: 24 workgroups, 16 stages
+    25.0 / 27.0, 4 workgroups, 32 stages 38.9 / 35.1."""
+    workgroups = q.shape[0] * q.shape[1] * ((q.shape[2] + 255) // 256)
+    eighth = torch.cuda.get_device_properties(q.device).multi_processor_count // 8
+    return workgroups <= (2 * eighth if q.shape[3] == 256 else eighth) and k.shape[2] > 31 * 64
+
+
+def _block_scores_of_few_rows(q, k, scale, q_group_size: int, block_k: int):
+    """The scores of :func:`_colsum_block_scores`, with the row statistic from the attention kernel's statistics sweep."""
+    q, k = _prep(q, "q"), _prep(k, "k")
+    _check_qkv(q, k, k, gqa=True)
+    lse2 = _dense_launch(q, k, k, scale, want_o=False, want_ml=False, want_lse2=True)[3]
+    return _sum_blocks(_colsum_given_lse(q, k, lse2, scale, q_group_size, want_block_sums=True, want_columns=False)[1], block_k)
 
 
 def _block_scores_for_topk(q, k, scale, q_group_size: int, block_k: int, base_mask, target: int):
