@@ -67,9 +67,9 @@ struct Swz {
 };
 
 // LDS of a workgroup: K and V buffers; the epilogue's transpose buffer of eight computing waves is larger
-template <int D, int NWAVES, int MODE>
+template <int D, int NCOMP, int MODE>
 constexpr int attn_lds_bytes() {
-  const int bufs = 4 * 64 * D * 2, epi = NWAVES * 32 * (D * 2 + 16);
+  const int bufs = 4 * 64 * D * 2, epi = NCOMP * 32 * (D * 2 + 16);
   return (MODE == MODE_BLOCK && epi > bufs) ? epi : bufs;
 }
 
@@ -83,14 +83,12 @@ struct SkCtx {
 };
 
 // One query tile w (or, in a balanced launch, the units [u0, u1) of its tile list; `whole` = all of them).
-template <int D, int NWAVES, int MODE, bool ACCUM, bool LSE_ONLY, bool SK>
-__device__ __forceinline__ void attn_item(const AttnParams& p, char* smem, const int w, const int u0, const int u1,
-                                          const bool whole, const SkCtx& sk) {
-  // Token lists with 8 waves: waves 0..5 compute (one 192-row group), waves 6 and 7 only fetch -- they read
-  // the list, form the gather addresses and issue every K/V fill.  One 6-wave group fills 6 of the 8 wave
-  // slots of a CU; the two fetch waves take the idle ones and the compute waves lose ~10 % of their
-  // instructions.  Everywhere else all waves do both.
-  constexpr int NPROD = (MODE == MODE_GATHER && NWAVES == 8) ? 2 : 0;
+template <int D, int NWAVES, int MODE, bool ACCUM, bool LSE_ONLY, bool SK, int NPROD>
+__device__ __forceinline__ void attn_item(const AttnParams& p, char* smem, const int w, const int bh, const int qt,
+                                          const int u0, const int u1, const bool whole, const SkCtx& sk) {
+  // NPROD: the last waves only fetch -- they read the list, form the addresses and issue every K/V fill -- and the
+  // others compute.  Token lists with 8 waves: six compute (one 192-row group fills 6 of the 8 wave slots of a CU) and
+  // two fetch, so the computing waves lose ~10 % of their instructions.  Everywhere else all waves do both.
   constexpr int NCOMP = NWAVES - NPROD;     // computing waves, 32 query rows each
   constexpr int FW = NPROD ? NPROD : NWAVES;  // waves that issue the fills
   constexpr int WGROWS = NCOMP * 32;
@@ -104,10 +102,9 @@ __device__ __forceinline__ void attn_item(const AttnParams& p, char* smem, const
   constexpr bool CONST_OFF = MODE == MODE_BLOCK && ((FW * RPI) % 16 == 0 || 16 % (FW * RPI) == 0) && NI % FW == 0;
   constexpr int CONST_PER = (FW * RPI) >= 16 ? 1 : 16 / (FW * RPI);
   constexpr int OSTR = D * 2 + 16;  // epilogue transpose buffer row stride (bytes)
-  static_assert(NCOMP * 32 * OSTR <= attn_lds_bytes<D, NWAVES, MODE>(), "the epilogue buffer must fit");
+  static_assert(NCOMP * 32 * OSTR <= attn_lds_bytes<D, NCOMP, MODE>(), "the epilogue buffer must fit");
   // LDS map: K buffers at 0 and TILE, V buffers at 2*TILE and 3*TILE
 
-  const int bh = w / p.nqt, qt = w - bh * p.nqt;
   const int b = bh / p.H, h = bh - b * p.H;
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -264,33 +261,53 @@ __device__ __forceinline__ void attn_item(const AttnParams& p, char* smem, const
     // valid keys of tile t of a token list (only the last tile can be ragged)
     auto nvalid_gather = [&](int t) { return max(0, min(64, count - (t << 6))); };
 
-    if (NPROD && wave >= NCOMP) {
+    // tiles 0..3: block lists use the entries read next to the count
+    auto first_raw = [&](int t, int (&raw)[NR]) {
+      if (MODE == MODE_BLOCK && !identity) {
+        const int e = t >> sub_shift;
+        raw[0] = (e == 0) ? head[0] : (e == 1) ? head[1] : (e == 2) ? head[2] : head[3];
+      } else {
+        prefetch_raw(t, raw);
+      }
+    };
+
+    // A computing wave of a ragged last query tile that owns no row does not compute: it keeps its part of the fills and
+    // meets the barriers, so the waves with rows have the matrix cores and the LDS reads to themselves, and a launch at
+    // the power limit keeps its clock (dense B2 H16 d128, 1600 x 4121 in 256-row tiles, an eighth of them padding: 111.7 ->
+    // 106.5 us).  Not where the second role costs registers that have to be spilled, nor at head_dim 256 (+1 %).
+    const bool no_rows = !SK && (NPROD > 0 || (MODE == MODE_BLOCK && D == 128)) && q0 + wave * 32 >= p.Lq;
+    if ((NPROD > 0 && wave >= NCOMP) || no_rows) {
       // ---- fetch waves: the fill schedule of the loop below and nothing else; one barrier per tile ----
+      const bool fills = !NPROD || wave >= NCOMP;
       int rows_v[NR], rows_k[NR], rows_n[NR], raw[NR], rows0[NR];
       int nv_unused;
 #pragma unroll
       for (int s = 0; s < NR; s++) { rows_v[s] = 0; rows_k[s] = 0; rows_n[s] = 0; raw[s] = 0; }
       // the list entries of the first four tiles are requested together (one memory round trip, not one per tile)
       int raw0[NR], raw1[NR], raw2[NR];
-      prefetch_raw(0, raw0);
-      prefetch_raw(1, raw1);
-      prefetch_raw(2, raw2);
-      prefetch_raw(3, raw);
-      finish_rows(0, raw0, rows0, nv_unused);
-      finish_rows(1, raw1, rows_v, nv_unused);
-      finish_rows(2, raw2, rows_k, nv_unused);
-      issue(krsrc, k_srb, false, rows0, lds0);
-      issue(vrsrc, v_srb, true, rows0, lds0 + 2 * TILE);
-      if (T > 1) issue(krsrc, k_srb, false, rows_v, lds0 + TILE);
+      if (fills) {
+        first_raw(0, raw0);
+        first_raw(1, raw1);
+        first_raw(2, raw2);
+        first_raw(3, raw);
+        finish_rows(0, raw0, rows0, nv_unused);
+        finish_rows(1, raw1, rows_v, nv_unused);
+        finish_rows(2, raw2, rows_k, nv_unused);
+        issue(krsrc, k_srb, false, rows0, lds0);
+        if (!LSE_ONLY) issue(vrsrc, v_srb, true, rows0, lds0 + 2 * TILE);
+        if (T > 1) issue(krsrc, k_srb, false, rows_v, lds0 + TILE);
+      }
       __builtin_amdgcn_s_waitcnt(0x0f70);
       __syncthreads();
       __syncthreads();   // the computing waves have read K(0): its buffer may be refilled
       for (int t = 0; t + 1 < T; t++) {
-        const int par = t & 1;
-        issue(vrsrc, v_srb, true, rows_v, lds0 + (3 - par) * TILE);
-        if (t + 2 < T) issue(krsrc, k_srb, false, rows_k, lds0 + par * TILE);
-        if (t + 3 < T) finish_rows(t + 3, raw, rows_n, nv_unused);
-        if (t + 4 < T) prefetch_raw(t + 4, raw);
+        if (fills) {
+          const int par = t & 1;
+          if (!LSE_ONLY) issue(vrsrc, v_srb, true, rows_v, lds0 + (3 - par) * TILE);
+          if (t + 2 < T) issue(krsrc, k_srb, false, rows_k, lds0 + par * TILE);
+          if (t + 3 < T) finish_rows(t + 3, raw, rows_n, nv_unused);
+          if (t + 4 < T) prefetch_raw(t + 4, raw);
+        }
         __builtin_amdgcn_s_waitcnt(0x0f70);
         __syncthreads();
 #pragma unroll
@@ -404,19 +421,10 @@ __device__ __forceinline__ void attn_item(const AttnParams& p, char* smem, const
 #pragma unroll
     for (int s = 0; s < NR; s++) { rows_v[s] = 0; rows_k[s] = 0; rows_n[s] = 0; raw[s] = 0; }
     int nv0, nv1 = 64, nv2 = 64, nv3 = 64;
-    if (NPROD) {
+    if constexpr (NPROD && MODE == MODE_GATHER) {
       nv0 = nvalid_gather(0); nv1 = nvalid_gather(1); nv2 = nvalid_gather(2);
     } else {
       int rows0[NR];
-      // tiles 0..3: block lists use the entries read next to the count
-      auto first_raw = [&](int t, int (&raw)[NR]) {
-        if (MODE == MODE_BLOCK && !identity) {
-          const int e = t >> sub_shift;
-          raw[0] = (e == 0) ? head[0] : (e == 1) ? head[1] : (e == 2) ? head[2] : head[3];
-        } else {
-          prefetch_raw(t, raw);
-        }
-      };
       if constexpr (MODE == MODE_GATHER) {
         // the list entries of the first four tiles are requested together (one memory round trip, not one per tile)
         int raw0[NR], raw1[NR], raw2[NR];
@@ -435,9 +443,11 @@ __device__ __forceinline__ void attn_item(const AttnParams& p, char* smem, const
         if (T > 2) { first_raw(2, raw); finish_rows(2, raw, rows_k, nv2); }
         if (T > 3) first_raw(3, raw);
       }
-      issue(krsrc, k_srb, false, rows0, lds0);
-      if (!LSE_ONLY) issue(vrsrc, v_srb, true, rows0, lds0 + 2 * TILE);
-      if (T > 1) issue(krsrc, k_srb, false, rows_v, lds0 + TILE);
+      if constexpr (!NPROD) {
+        issue(krsrc, k_srb, false, rows0, lds0);
+        if (!LSE_ONLY) issue(vrsrc, v_srb, true, rows0, lds0 + 2 * TILE);
+        if (T > 1) issue(krsrc, k_srb, false, rows_v, lds0 + TILE);
+      }
     }
     __builtin_amdgcn_s_waitcnt(0x0f70);  // vmcnt(0): this wave's LDS fills have landed
     __syncthreads();
@@ -476,10 +486,10 @@ __device__ __forceinline__ void attn_item(const AttnParams& p, char* smem, const
           }
         }
       };
-      if (NPROD) {
+      if constexpr (NPROD && MODE == MODE_GATHER) {
         nv3 = nvalid_gather(t + 3);
       } else {
-        if constexpr (FSTRIDE == 0) {
+        if constexpr (!NPROD && FSTRIDE == 0) {
           if (!LSE_ONLY) issue(vrsrc, v_srb, true, rows_v, lds0 + (3 - PAR) * TILE);
           if (fill_k) issue(krsrc, k_srb, false, rows_k, lds0 + PAR * TILE);
         }
@@ -593,7 +603,7 @@ __device__ __forceinline__ void attn_item(const AttnParams& p, char* smem, const
       __syncthreads();
       rescale_check(mx);
       nv0 = nv1; nv1 = nv2; nv2 = nv3;
-      if (!NPROD) {
+      if constexpr (!(NPROD && MODE == MODE_GATHER)) {
 #pragma unroll
         for (int s = 0; s < NR; s++) { rows_v[s] = rows_k[s]; rows_k[s] = rows_n[s]; }
       }
@@ -831,7 +841,7 @@ __device__ __forceinline__ void attn_item(const AttnParams& p, char* smem, const
 #endif  // __HIP_DEVICE_COMPILE__
 
 // THIRD: registers of a wave limited so that three workgroups share a compute unit, see third_workgroup
-template <int D, int NWAVES, int MODE, bool ACCUM, bool LSE_ONLY, bool THIRD = false>
+template <int D, int NWAVES, int MODE, bool ACCUM, bool LSE_ONLY, int NPROD, bool THIRD = false>
 __global__ __launch_bounds__(NWAVES * 64, ((NWAVES <= 4 && D <= 128) ? (THIRD ? 3 : 2) : 1)) void attn_fwd_kernel(const AttnParams p) {
   // The body is compiled for the device only: the host pass just needs the launch stub, and it
   // silently drops the stub when the body uses the LDS-DMA builtins.
@@ -839,10 +849,20 @@ __global__ __launch_bounds__(NWAVES * 64, ((NWAVES <= 4 && D <= 128) ? (THIRD ? 
   extern __shared__ __attribute__((aligned(1024))) char smem[];
   // Consecutive workgroup ids are dealt round-robin to the 8 XCDs; remap so that each XCD
   // walks a contiguous range of (batch, head, q-tile) and K/V of one head stay in its L2.
-  const int per_xcd = gridDim.x >> 3;
-  const int w = (blockIdx.x & 7) * per_xcd + (blockIdx.x >> 3);
-  if (w >= p.total_wg) return;
-  attn_item<D, NWAVES, MODE, ACCUM, LSE_ONLY, false>(p, smem, w, 0, 0, true, SkCtx{});
+  const int xcd = blockIdx.x & 7, i = blockIdx.x >> 3;
+  int bh, qt;
+  if (i < p.whole_per_xcd) {
+    const int w = xcd * p.whole_per_xcd + i;
+    if (w >= p.whole_wg) return;
+    bh = w / p.whole_nqt;
+    qt = w - bh * p.whole_nqt;
+  } else {
+    // ragged last tiles of the (batch, head) slices, behind the whole ones (see launch_one)
+    bh = xcd * p.ragged_per_xcd + (i - p.whole_per_xcd);
+    if (i - p.whole_per_xcd >= p.ragged_per_xcd || bh >= p.B * p.H) return;
+    qt = p.whole_nqt;
+  }
+  attn_item<D, NWAVES, MODE, ACCUM, LSE_ONLY, false, NPROD>(p, smem, 0, bh, qt, 0, 0, true, SkCtx{});
 #endif
 }
 
@@ -884,7 +904,8 @@ __global__ __launch_bounds__(NWAVES * 64, (NWAVES <= 4 ? 2 : 1)) void attn_fwd_b
     // a damaged table must not send a store outside the workspace
     if (sk.pieces < 1 || sk.pieces > SK_MAX_PIECES || sk.kp < 0 || sk.kp >= sk.pieces || (sk.pieces > 1 && (sk.slot0 < 0 || sk.slot0 + sk.pieces > 2 * p.sk_wgs))) return;
   }
-  attn_item<D, NWAVES, MODE, ACCUM, false, true>(p, smem, w, u0, u1, sk.pieces == 1, sk);
+  const int bh = w / p.nqt;
+  attn_item<D, NWAVES, MODE, ACCUM, false, true, (MODE == MODE_GATHER && NWAVES == 8) ? 2 : 0>(p, smem, w, bh, w - bh * p.nqt, u0, u1, sk.pieces == 1, sk);
 #endif
 }
 
@@ -1001,18 +1022,18 @@ static bool wide_tiles(const AttnParams& p, int head_dim) {
 // 4096 x 10521 in lists of 30 %: 149 / 162 us).
 static bool third_workgroup(int total_wg) { return total_wg > 2 * device_cus(); }
 
-template <int D, int NWAVES, int MODE, bool ACCUM, bool LSE_ONLY>
+template <int D, int NWAVES, int MODE, bool ACCUM, bool LSE_ONLY, int NPROD = (MODE == MODE_GATHER && NWAVES == 8) ? 2 : 0>
 static int launch_one(const AttnParams& p0, hipStream_t stream) {
   AttnParams p = p0;
   if (p.kv_group < 1) p.kv_group = 1;
-  constexpr int WGROWS = ((MODE == MODE_GATHER && NWAVES == 8) ? 6 : NWAVES) * 32;   // two of eight token-list waves only fetch
-  constexpr int SMEM = attn_lds_bytes<D, NWAVES, MODE>();
+  constexpr int WGROWS = (NWAVES - NPROD) * 32;
+  constexpr int SMEM = attn_lds_bytes<D, NWAVES - NPROD, MODE>();
   if (MODE == MODE_BLOCK && p.list == nullptr) p.group_rows = WGROWS;  // dense: any row grouping
   if (p.group_rows % WGROWS != 0) return LVAR_EINVAL;
   p.nqt = (p.Lq + WGROWS - 1) / WGROWS;
   p.total_wg = p.B * p.H * p.nqt;
-  constexpr bool WIDE = MODE == MODE_BLOCK && NWAVES == 8;   // 256 query rows
-  if constexpr (!LSE_ONLY) {
+  constexpr bool WIDE = MODE == MODE_BLOCK && NWAVES == 8;   // 256 query rows, or 128 and fetch waves
+  if constexpr (!LSE_ONLY && !(MODE == MODE_BLOCK && NPROD > 0)) {
     const bool dense = (MODE == MODE_BLOCK && p.list == nullptr);
     const int64_t per_tile = (MODE == MODE_BLOCK) ? (p.list ? p.list_len : (p.Lk + 63) / 64) : (p.list_len + 63) / 64;
     const int sub = (MODE == MODE_BLOCK && p.list) ? p.sub_shift : 0;
@@ -1056,15 +1077,23 @@ static int launch_one(const AttnParams& p0, hipStream_t stream) {
   if constexpr (MODE == MODE_BLOCK && !LSE_ONLY && NWAVES == 4 && D <= 128) {
     if (wide_tiles(p0, D)) return launch_one<D, 8, MODE_BLOCK, false, false>(p0, stream);
   }
-  const int grid = ((p.total_wg + 7) / 8) * 8;
+  // Ragged last tiles start behind all whole ones: their waves without rows do not compute, so they are the shorter
+  // workgroups, and what is dispatched last decides how long the launch drains (token lists of 832 keys, 288 groups of
+  // which 32 have 64 rows, on 256 compute units: 54 -> 47 us with the idle waves).
+  const bool ragged = p.nqt > 1 && p.Lq % WGROWS != 0;
+  p.whole_nqt = ragged ? p.nqt - 1 : p.nqt;
+  p.whole_wg = p.B * p.H * p.whole_nqt;
+  p.whole_per_xcd = (p.whole_wg + 7) / 8;
+  p.ragged_per_xcd = ragged ? (p.B * p.H + 7) / 8 : 0;
+  const int grid = 8 * (p.whole_per_xcd + p.ragged_per_xcd);
   if constexpr (D == 64 && NWAVES == 4 && MODE == MODE_BLOCK && !LSE_ONLY) {
     if (third_workgroup(p.total_wg)) {
       static_assert(SMEM <= 48 * 1024, "three workgroups share the LDS of a compute unit; no larger limit has to be asked for");
-      hipLaunchKernelGGL((attn_fwd_kernel<D, NWAVES, MODE, ACCUM, LSE_ONLY, true>), dim3(grid), dim3(NWAVES * 64), SMEM, stream, p);
+      hipLaunchKernelGGL((attn_fwd_kernel<D, NWAVES, MODE, ACCUM, LSE_ONLY, NPROD, true>), dim3(grid), dim3(NWAVES * 64), SMEM, stream, p);
       return hipGetLastError() == hipSuccess ? LVAR_OK : LVAR_ELAUNCH;
     }
   }
-  auto kern = attn_fwd_kernel<D, NWAVES, MODE, ACCUM, LSE_ONLY>;
+  auto kern = attn_fwd_kernel<D, NWAVES, MODE, ACCUM, LSE_ONLY, NPROD>;
   static std::atomic<uint64_t> lds_ready{0};
   if (!ensure_lds_limit((const void*)kern, SMEM, lds_ready)) return LVAR_ELAUNCH;
   hipLaunchKernelGGL(kern, dim3(grid), dim3(NWAVES * 64), SMEM, stream, p);

@@ -36,6 +36,9 @@ struct AttnParams {
   int up_src, up_dst;  // token-list variant: o_accum is an up_src x up_src token grid, bilinearly
                        // resampled to the up_dst x up_dst grid of the queries (0 = o_accum has Lq rows)
   int nqt, total_wg;
+  // plain launch: query tiles of a (batch, head) that run first (all but a ragged last one), how many these are and how
+  // many an XCD takes, ragged last tiles per XCD
+  int whole_nqt, whole_wg, whole_per_xcd, ragged_per_xcd;
   // balanced launch: workspace handed in by the caller (null = plain launch).  The launch code fills in sk_wgs
   // (0 = plain launch after all), sk_counters (per-query-tile arrival counters, all zero between launches) and
   // sk_slots (2 * sk_wgs slots of partial results).
