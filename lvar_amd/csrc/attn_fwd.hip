@@ -88,7 +88,8 @@ __device__ __forceinline__ void attn_item(const AttnParams& p, char* smem, const
                                           const int u0, const int u1, const bool whole, const SkCtx& sk) {
   // NPROD: the last waves only fetch -- they read the list, form the addresses and issue every K/V fill -- and the
   // others compute.  Token lists with 8 waves: six compute (one 192-row group fills 6 of the 8 wave slots of a CU) and
-  // two fetch, so the computing waves lose ~10 % of their instructions.  Everywhere else all waves do both.
+  // two fetch, so the computing waves lose ~10 % of their instructions.  Launches of at most one 128-row workgroup per
+  // CU: four and four (see fetch_waves).  Everywhere else all waves do both.
   constexpr int NCOMP = NWAVES - NPROD;     // computing waves, 32 query rows each
   constexpr int FW = NPROD ? NPROD : NWAVES;  // waves that issue the fills
   constexpr int WGROWS = NCOMP * 32;
@@ -1022,6 +1023,14 @@ static bool wide_tiles(const AttnParams& p, int head_dim) {
 // 4096 x 10521 in lists of 30 %: 149 / 162 us).
 static bool third_workgroup(int total_wg) { return total_wg > 2 * device_cus(); }
 
+// Fetch-only waves beside four computing ones.  A launch of at most one 128-row workgroup per compute unit leaves half of
+// the wave slots empty, and its lone waves pay for every instruction in full: 16 of the 100-odd that a wave issues per
+// tile beside its MFMAs are fills.  Without / with four fetch waves, B2 H16 d128: 144 x 265 9.8 / 9.0 us, 576 x 1497 27.3 /
+// 24.4, 1024 x 2521 (256 workgroups) 46.5 / 44.3; B1 H4 4096 x 10521 153 / 134; d64 B8 H16 256 x 680 12.2 / 11.4; lists
+// alike (B1 H16 784 x 1924 at 25 % 20.6 / 18.4).  With a second workgroup on a compute unit there are no empty slots, and at
+// head_dim 256 a wave fills its SIMD.  Same bits.
+static bool fetch_waves(int total_wg) { return total_wg <= device_cus(); }
+
 template <int D, int NWAVES, int MODE, bool ACCUM, bool LSE_ONLY, int NPROD = (MODE == MODE_GATHER && NWAVES == 8) ? 2 : 0>
 static int launch_one(const AttnParams& p0, hipStream_t stream) {
   AttnParams p = p0;
@@ -1076,6 +1085,7 @@ static int launch_one(const AttnParams& p0, hipStream_t stream) {
   }
   if constexpr (MODE == MODE_BLOCK && !LSE_ONLY && NWAVES == 4 && D <= 128) {
     if (wide_tiles(p0, D)) return launch_one<D, 8, MODE_BLOCK, false, false>(p0, stream);
+    if (fetch_waves(p.total_wg)) return launch_one<D, 8, MODE_BLOCK, false, false, 4>(p0, stream);
   }
   // Ragged last tiles start behind all whole ones: their waves without rows do not compute, so they are the shorter
   // workgroups, and what is dispatched last decides how long the launch drains (token lists of 832 keys, 288 groups of

@@ -1,4 +1,6 @@
-"""Query tiles whose last rows are missing (waves without rows do not compute, ragged tiles run last), against the oracle."""
+"""Query tiles whose last rows are missing (waves without rows do not compute, ragged tiles run last) and launches whose
+workgroups have fetch-only waves: every count of key tiles around the depth of the fill pipeline, against the oracle and
+against the same heads in a launch that is large enough to take the other form."""
 import pytest
 import torch
 
@@ -14,6 +16,31 @@ def _rand(B, H, Lq, Lk, d, seed):
 
 def _close(o, ref):
     return torch.allclose(o.float().cpu(), ref, atol=2e-2, rtol=1e-2)     # the attention tolerance of bf16 outputs
+
+
+@pytest.mark.parametrize("d", [64, 128])
+@pytest.mark.parametrize("Lq,Lk", [(1, 1), (32, 64), (33, 65), (128, 128), (129, 192), (160, 193), (250, 257), (300, 330)])
+def test_few_query_tiles(Lq, Lk, d):
+    from lvar_amd import sparse_attn_ops as ops
+    H = 270                                                     # more query tiles than compute units: no fetch-only waves
+    (q, k, v), g = _rand(1, H, Lq, Lk, d, seed=Lq + d)
+    qg, kg, vg = q.cuda(), k.cuda(), v.cuda()
+    h = slice(H - 3, H)
+    part = [t[:, h].contiguous() for t in (qg, kg, vg)]
+    o, (M, L) = ops.dense_attn(*part)
+    ob, (Mb, Lb) = ops.dense_attn(qg, kg, vg)
+    assert torch.equal(o, ob[:, h]) and torch.equal(M, Mb[:, h]) and torch.equal(L, Lb[:, h])
+    o_ref, M_ref, L_ref = oracle.dense_attn(q[:, h], k[:, h], v[:, h])
+    assert _close(o, o_ref)
+    assert torch.allclose((M + L.log2()).cpu(), M_ref + L_ref.log2(), atol=1e-3)
+    for bk in (64, 128):
+        mask = torch.rand(1, H, -(-Lq // 128), -(-Lk // bk), generator=g) < 0.6      # some lists are empty
+        num, idx = oracle.block_mask_to_lists(mask)
+        o, (M, L) = ops.block_sparse_attn(*part, num[:, h].contiguous().cuda(), idx[:, h].contiguous().cuda(), 128, bk)
+        ob, (Mb, Lb) = ops.block_sparse_attn(qg, kg, vg, num.cuda(), idx.cuda(), 128, bk)
+        assert torch.equal(o, ob[:, h]) and torch.equal(M, Mb[:, h]) and torch.equal(L, Lb[:, h])
+        o_ref, _, _ = oracle.block_sparse_attn(q[:, h], k[:, h], v[:, h], num[:, h], idx[:, h], 128, bk)
+        assert _close(o, o_ref)
 
 
 # rows of the last query group / tile: one, a wave less one row, a wave, all but a wave; heads that do not divide by eight
