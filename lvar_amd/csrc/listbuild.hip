@@ -48,6 +48,7 @@ __device__ __forceinline__ uint32_t wave_umin(uint32_t v) {
 constexpr int TOPK_BINS = 2048;
 constexpr int TOPK_SHARED_MAX_N = 12288;   // longest row of 1024 threads where two rows share a compute unit
 constexpr int TOPK_CAND = 256;   // keys of the first pass's bin that are resolved by direct comparison
+constexpr uint32_t KEY_NEG_INF = 0x007fffffu, KEY_POS_INF = 0xff800000u;   // real_key of -inf and +inf
 
 // UNION: the output row is the ascending merge of the selection with the row's own list of W columns (in any order,
 // columns that are listed or selected several times come out as often), as int64.  How often each column is listed sits
@@ -73,7 +74,12 @@ __global__ __launch_bounds__(NT, (KPT >= 1 && KPT <= 24) ? (NT == 512 ? 6 : 4) :
   for (int t = want + tid; t < p.zero_to; t += NT) out[t] = 0;
   if (want == 0) return;
   if constexpr (UNION)
+    for (int t = tid; t < TOPK_BINS; t += NT) hist[t] = 0;
+  int64_t more_first = 0;   // this thread's first entry of the row's own list, requested ahead of the scores
+  if constexpr (UNION) {
+    if (tid < p.W) more_first = p.more[(int64_t)row * p.W + tid];
     for (int t = tid; t < (n + 1) / 2; t += NT) listed[t] = 0u;
+  }
 
   // chunk c of wave w covers columns (w * cpw + c) * 64 .. +63
   const int cpw = KPT ? KPT : ((n + NT - 1) / NT);
@@ -92,7 +98,7 @@ __global__ __launch_bounds__(NT, (KPT >= 1 && KPT <= 24) ? (NT == 512 ? 6 : 4) :
       const bool real = col0 + c * 64 < n;
       keys[c] = real ? real_key(__builtin_bit_cast(float, raw[c])) : 0u;
       kmax = max(kmax, keys[c]);
-      kmin = min(kmin, real ? keys[c] : 0xffffffffu);
+      kmin = min(kmin, real && (!UNION || keys[c] > KEY_NEG_INF) ? keys[c] : 0xffffffffu);
     }
   } else {
     for (int c = 0; c < cpw; c++) {
@@ -131,27 +137,32 @@ __global__ __launch_bounds__(NT, (KPT >= 1 && KPT <= 24) ? (NT == 512 ? 6 : 4) :
   if constexpr (UNION) {   // (read behind at least one more barrier)
     const int64_t* more = p.more + (int64_t)row * p.W;
     for (int t = tid; t < p.W; t += NT) {
-      const int j = (int)max((int64_t)0, min((int64_t)n - 1, more[t]));
+      const int j = (int)max((int64_t)0, min((int64_t)n - 1, t < NT ? more_first : more[t]));
       atomicAdd(&listed[j >> 1], 1u << (16 * (j & 1)));
     }
   }
-  const int top = 32 - __builtin_clz((kmax ^ kmin) | 1u) + (((kmax ^ kmin) == 0u) ? -1 : 0);   // 0 when all keys are equal
+  // (UNION: the smallest key leaves out the -inf of the columns that do not compete, so nothing is known from it)
+  const int top = UNION ? 32 : 32 - __builtin_clz((kmax ^ kmin) | 1u) + (((kmax ^ kmin) == 0u) ? -1 : 0);   // 0 when all keys are equal
   uint32_t pmask = (top >= 32) ? 0u : ~((1u << top) - 1u);
   uint32_t prefix = kmax & pmask;
-  if (top == 0) __syncthreads();   // no pass below to separate these reads of wgt / weq from their reuse
-  bool first = true;
-  for (int hi = top; hi > 0;) {
-    const int shift = max(0, hi - 11);
-    const int bits = hi - shift;
-    hi = shift;
-    const int nbins = 1 << bits;
-    for (int t = tid; t < nbins; t += NT) hist[t] = 0;
-    __syncthreads();
-    visit([&](int j, uint32_t key) {
-      if ((key & pmask) == prefix) atomicAdd(&hist[(key >> shift) & (nbins - 1)], 1);
-    });
-    __syncthreads();
-    // thread t owns the bpt bins nbins-1 - t*bpt .. (descending); find the bin holding the want-th key from the top
+  // UNION, first pass: the scores are sums of signed products, so the top bits of their keys (sign, exponent, two bits of
+  // mantissa) fill a few dozen bins and the bin of the threshold holds several hundred keys of 10521: two more passes.
+  // Bins of equal width between the smallest finite score and the largest hold about ten each (32 rows: 16.7 -> 12.4 us
+  // with the row's own list requested first and no scan where a column is listed once).  The map is monotonic in the key
+  // (subtraction, product and truncation are), so a bin is a run of keys like any other; where one score lies far from
+  // all others the passes by digits follow, over the keys of that bin.
+  bool linear = false;
+  int lbin = 0;
+  float x0 = 0.f, xs = 0.f;
+  auto bin_of = [&](uint32_t key) -> int {
+    const uint32_t k = max(key, KEY_NEG_INF);
+    const float x = __builtin_bit_cast(float, k ^ ((k >> 31) ? 0x80000000u : 0xffffffffu));
+    return (int)__builtin_amdgcn_fmed3f((x - x0) * xs, 0.f, (float)(TOPK_BINS - 1));
+  };
+  auto in_play = [&](uint32_t key) -> bool { return (key & pmask) == prefix && (!UNION || !linear || bin_of(key) == lbin); };
+  // The bin that holds the want-th key from the top, and how many of its keys are wanted: thread t owns the bpt bins
+  // nbins-1 - t*bpt .. (descending).
+  auto find_bin = [&](int nbins) {
     const int bpt = (nbins + NT - 1) / NT;   // 1 when there are as many threads as bins (then every thread owns one)
     const int btop = nbins - 1 - tid * bpt;
     int mine = 0;
@@ -172,49 +183,86 @@ __global__ __launch_bounds__(NT, (KPT >= 1 && KPT <= 24) ? (NT == 512 ? 6 : 4) :
       sel[1] = want - acc;
     }
     __syncthreads();
-    prefix |= (uint32_t)sel[0] << shift;
-    pmask |= (uint32_t)(nbins - 1) << shift;
     want = sel[1];
     // (the next write of `sel` lies behind three more barriers: no barrier needed after these reads)
-    if (first && hi > 0) {
-      // After the first pass the chosen bin usually holds a few dozen keys.  They are copied to LDS, and if they
-      // fit, every one of them counts the candidates above it: the one with fewer than `want` above and at least
-      // `want` at or above is the threshold, and the other passes are not needed.
-      first = false;
-      visit([&](int j, uint32_t key) {
-        const bool m = (key & pmask) == prefix;
-        const unsigned long long bm = __builtin_amdgcn_ballot_w64(m);
-        if (bm != 0ull) {
-          int base = 0;
-          if (lane == 0) base = atomicAdd(&ncand, __builtin_popcountll(bm));
-          base = __builtin_amdgcn_readfirstlane(base);
-          const int at = base + lanes_below(bm, lane);
-          if (m && at < TOPK_CAND) cand[at] = key;
-        }
-      });
-      __syncthreads();
-      const int nc = ncand;
-      if (nc <= TOPK_CAND) {
-        if (tid < nc) {
-          const uint32_t kt = cand[tid];
-          int above = 0, at_or_above = 0;
-          // four candidates per LDS read (all lanes read the same address): the loop is bound by the latency of its reads
-          for (int u = 0; u < nc; u += 4) {
-            const u32x4 ku = *(const u32x4*)(cand + u);
-#pragma unroll
-            for (int e = 0; e < 4; e++) {
-              const bool in = u + e < nc;
-              above += in && ku[e] > kt;
-              at_or_above += in && ku[e] >= kt;
-            }
-          }
-          if (above < want && want <= at_or_above) { sel[0] = (int)kt; sel[1] = want - above; }   // equal keys write equal values
-        }
-        __syncthreads();
-        prefix = (uint32_t)sel[0];
-        want = sel[1];
-        break;
+  };
+  // After the first pass the chosen bin usually holds a few dozen keys.  They are copied to LDS, and if they
+  // fit, every one of them counts the candidates above it: the one with fewer than `want` above and at least
+  // `want` at or above is the threshold, and the other passes are not needed.
+  auto resolve = [&]() -> bool {
+    visit([&](int j, uint32_t key) {
+      const bool m = in_play(key);
+      const unsigned long long bm = __builtin_amdgcn_ballot_w64(m);
+      if (bm != 0ull) {
+        int base = 0;
+        if (lane == 0) base = atomicAdd(&ncand, __builtin_popcountll(bm));
+        base = __builtin_amdgcn_readfirstlane(base);
+        const int at = base + lanes_below(bm, lane);
+        if (m && at < TOPK_CAND) cand[at] = key;
       }
+    });
+    __syncthreads();
+    const int nc = ncand;
+    if (nc > TOPK_CAND) return false;
+    if (tid < nc) {
+      const uint32_t kt = cand[tid];
+      int above = 0, at_or_above = 0;
+      // four candidates per LDS read (all lanes read the same address): the loop is bound by the latency of its reads
+      for (int u = 0; u < nc; u += 4) {
+        const u32x4 ku = *(const u32x4*)(cand + u);
+#pragma unroll
+        for (int e = 0; e < 4; e++) {
+          const bool in = u + e < nc;
+          above += in && ku[e] > kt;
+          at_or_above += in && ku[e] >= kt;
+        }
+      }
+      if (above < want && want <= at_or_above) { sel[0] = (int)kt; sel[1] = want - above; }   // equal keys write equal values
+    }
+    __syncthreads();
+    prefix = (uint32_t)sel[0];
+    want = sel[1];
+    return true;
+  };
+  bool found = false, first = true;
+  if constexpr (UNION) {
+    if (kmin < kmax && kmax < KEY_POS_INF) {
+      x0 = __builtin_bit_cast(float, kmin ^ ((kmin >> 31) ? 0x80000000u : 0xffffffffu));
+      const float range = __builtin_bit_cast(float, kmax ^ ((kmax >> 31) ? 0x80000000u : 0xffffffffu)) - x0;
+      const uint32_t rb = __builtin_bit_cast(uint32_t, range);
+      if (rb > 0x08000000u && rb < 0x7f800000u) {   // above 2^-111 (its reciprocal is finite) and finite
+        linear = true;
+        xs = (float)(TOPK_BINS - 1) / range;
+      }
+    }
+    if (linear) {
+      visit([&](int j, uint32_t key) { atomicAdd(&hist[bin_of(key)], 1); });
+      __syncthreads();
+      find_bin(TOPK_BINS);
+      lbin = sel[0];
+      found = resolve();
+      if (!found) __syncthreads();    // every wave has read the number of candidates before it is cleared
+      if (!found && tid == 0) ncand = 0;
+    }
+  }
+  for (int hi = found ? 0 : top; hi > 0;) {
+  if (top == 0) __syncthreads();   // no pass below to separate these reads of wgt / weq from their reuse
+    const int shift = max(0, hi - 11);
+    const int bits = hi - shift;
+    hi = shift;
+    const int nbins = 1 << bits;
+    for (int t = tid; t < nbins; t += NT) hist[t] = 0;
+    __syncthreads();
+    visit([&](int j, uint32_t key) {
+      if (in_play(key)) atomicAdd(&hist[(key >> shift) & (nbins - 1)], 1);
+    });
+    __syncthreads();
+    find_bin(nbins);
+    prefix |= (uint32_t)sel[0] << shift;
+    pmask |= (uint32_t)(nbins - 1) << shift;
+    if (first && hi > 0) {
+      first = false;
+      if (resolve()) break;
     }
   }
   const uint32_t T = prefix;  // key of the k-th largest element
@@ -247,7 +295,9 @@ __global__ __launch_bounds__(NT, (KPT >= 1 && KPT <= 24) ? (NT == 512 ? 6 : 4) :
       }
       const int mult = j < n ? (int)listed16[j] : 0;
       const int mine = (int)((bk >> lane) & 1ull) + mult;
-      if (__builtin_amdgcn_ballot_w64(mult > 0) == 0ull) {
+      if (__builtin_amdgcn_ballot_w64(mine > 1) == 0ull) {
+        // (the usual case: listed columns are listed once and not selected)
+        bk = __builtin_amdgcn_ballot_w64(mine > 0);
         if (mine) out64[pos + lanes_below(bk, lane)] = j;
         pos += __builtin_popcountll(bk);
       } else {

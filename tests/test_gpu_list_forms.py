@@ -89,6 +89,46 @@ def test_merged_selection_at_every_number_of_keys_per_thread(n, kind):
         assert torch.equal(out, torch.cat([_selected(x, k), more.clamp(0, n - 1)], -1).sort(dim=-1).values), (k, W)
 
 
+def _wide_scores(kind, rows, n, seed):
+    g = torch.Generator(device="cuda").manual_seed(seed)
+    x = torch.randn(rows, n, generator=g, device="cuda")
+    hole = torch.rand(rows, n, generator=g, device="cuda") < 0.1
+    if kind == "holes":                       # columns that do not compete, as the window's own keys
+        x[hole] = -float("inf")
+    elif kind == "outlier":                   # equal-width bins hold everything else in one of them
+        x[:, n // 2], x[:, n // 3] = 1e30, -1e30
+    elif kind == "tails":
+        x = x.sign() * (x.abs() * 12).exp()
+    elif kind == "infinite":
+        x[hole], x[:, n // 2] = float("inf"), -float("inf")
+    elif kind == "none":
+        x[:] = -float("inf")
+    elif kind == "one":
+        x[:] = -float("inf")
+        x[:, n // 2] = 0.5
+    elif kind == "tiny":
+        x = x * 1e-39
+    elif kind == "zeros":
+        x = torch.where(hole, -0.0, 0.0) + torch.where(x > 1.5, 1.0, 0.0)
+    return x
+
+
+@pytest.mark.parametrize("kind", ["plain", "holes", "outlier", "tails", "infinite", "none", "one", "tiny", "zeros"])
+@pytest.mark.parametrize("n", [60, 1000, 10521, 16384])
+def test_merged_selection_of_any_spread_of_scores(n, kind):
+    """The first pass counts in bins of equal width between the smallest and the largest finite score."""
+    from lvar_amd import _lib
+    rows, W = 3, 17
+    x = _wide_scores(kind, rows, n, seed=n)
+    g = torch.Generator(device="cuda").manual_seed(n + 1)
+    more = torch.randint(0, n, (rows, W), generator=g, device="cuda")
+    for k in (1, 7, n // 6, n // 2, n - n // 20, n):
+        out = torch.full((rows, k + W), -1, dtype=torch.int64, device="cuda")
+        st = _lib.load().lvar_topk_union_lists(x.data_ptr(), n, more.data_ptr(), W, out.data_ptr(), rows, n, k, torch.cuda.current_stream().cuda_stream)
+        assert st == 0
+        assert torch.equal(out, torch.cat([_selected(x, k), more], -1).sort(dim=-1).values), k
+
+
 def test_merged_selection_of_the_longest_list():
     from lvar_amd import _lib
     x = _scores("distinct", 2, 5, seed=1)
