@@ -129,6 +129,28 @@ def test_merged_selection_of_any_spread_of_scores(n, kind):
         assert torch.equal(out, torch.cat([_selected(x, k), more], -1).sort(dim=-1).values), k
 
 
+# 128 keys per workgroup up to two workgroups per compute unit, 512 beyond: the same bits, and the oracle's scores
+@pytest.mark.parametrize("d,Lk,W,ksize", [(64, 1, 1, 1), (128, 127, 3, 33), (256, 129, 40, 3), (128, 513, 300, 5), (64, 640, 17, 33)])
+@pytest.mark.parametrize("pool", ["avgpool", "maxpool"])
+def test_window_scores_on_both_sides_of_the_chunk_rule(d, Lk, W, ksize, pool):
+    import oracle
+    from lvar_amd import sparse_attn_ops as ops
+    H = 2 * torch.cuda.get_device_properties(0).multi_processor_count // -(-Lk // 128) + 1
+    Lq = -(-Lk // 2)
+    g = torch.Generator(device="cuda").manual_seed(Lk + d)
+    q, k = [(torch.randn(1, H, L, d, generator=g, device="cuda") * 0.5).to(torch.bfloat16) for L in (Lq, Lk)]
+    win = torch.randint(Lk - Lq, Lk, (1, H, W), generator=g, device="cuda")
+    many = ops.window_key_scores(q, k, win, ksize, pool)
+    h = slice(H - 2, H)
+    few = ops.window_key_scores(q[:, h].contiguous(), k[:, h].contiguous(), win[:, h].contiguous(), ksize, pool)
+    assert torch.equal(few, many[:, h])
+    ref = oracle.window_key_scores(q[:, h].cpu(), k[:, h].cpu(), win[:, h].cpu(), ksize, pool, dtype=torch.float64)
+    fin = torch.isfinite(ref)
+    assert torch.equal(torch.isfinite(few.cpu()), fin)
+    # fp32 sums of W + d products of values of order one: far below 1e-3 of the largest score
+    assert not fin.any() or (few.cpu()[fin] - ref[fin]).abs().max() <= 1e-3 * max(1.0, float(ref[fin].abs().max()))
+
+
 def test_merged_selection_of_the_longest_list():
     from lvar_amd import _lib
     x = _scores("distinct", 2, 5, seed=1)
