@@ -245,8 +245,8 @@ __global__ __launch_bounds__(NT, (KPT >= 1 && KPT <= 24) ? (NT == 512 ? 6 : 4) :
       if (!found && tid == 0) ncand = 0;
     }
   }
-  for (int hi = found ? 0 : top; hi > 0;) {
   if (top == 0) __syncthreads();   // no pass below to separate these reads of wgt / weq from their reuse
+  for (int hi = found ? 0 : top; hi > 0;) {
     const int shift = max(0, hi - 11);
     const int bits = hi - shift;
     hi = shift;

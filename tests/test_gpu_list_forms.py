@@ -38,6 +38,16 @@ def test_topk_lists_at_every_number_of_keys_per_thread(few_rows, step, kind):
             assert bool((idx[:, k:] == 0).all()) and bool((cnt == k).all())
 
 
+@pytest.mark.parametrize("rows,n", [(288, 4121), (704, 10521), (300, 20000)])
+def test_topk_lists_of_rows_of_equal_scores(rows, n):
+    """No histogram pass, and none of its barriers, runs for such a row."""
+    from lvar_amd import sparse_attn_ops as ops
+    x = _scores("equal", rows, n, seed=n)
+    for k in (1, n // 5, n):
+        idx, _ = ops.topk_token_lists(x, k)
+        assert torch.equal(idx[:, :k].long(), torch.arange(k, device="cuda").expand(rows, k)), k
+
+
 # two rows per compute unit: 1024 threads up to 12288 keys, 512 beyond
 @pytest.mark.parametrize("n", [12288, 12289])
 @pytest.mark.parametrize("more", [0, 1])
