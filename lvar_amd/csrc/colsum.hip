@@ -119,6 +119,25 @@ __global__ __launch_bounds__(256, (D <= 128 ? CS_WGS : 1)) void colsum_kernel(co
     else __builtin_amdgcn_s_waitcnt(vm(0));
   };
 
+  const int S = (Lq_l + 63) >> 6;          // stages of this range
+  const int U = (Lq_l + 31) >> 5;          // 32-row tiles
+  // both stages of the ring and the key fragments are one round trip to memory
+  issue_stage(0);
+  if (S > 1) issue_stage(1);
+  if (n0 >= p.Lk) {
+    // A wave without keys (the last key tile of a slice; three of its four waves at 4121, 6425 and 10521 keys) keeps its part
+    // of the fills and meets the barriers.  With the first two stages requested together, B2 H16 d128: 1600 x 4121 68.2 ->
+    // 67.3 us, 2304 x 6425 126.4 -> 125.0, 4096 x 10521 347.6 -> 345.0.  (Starting these tiles last is 0.3 % slower.)
+    wait_fills(0);
+    __syncthreads();
+    for (int s = 0; s < S; s++) {
+      if (s > 0 && s + 1 < S) issue_stage(s + 1);
+      wait_fills(0);
+      __syncthreads();
+    }
+    return;
+  }
+
   float* csp = p.cs ? p.cs + ((int64_t)b * p.H + h) * p.G * (int64_t)p.Lk : nullptr;
   float* bsp = p.bs ? p.bs + ((int64_t)b * p.H + h) * p.G * (int64_t)p.nkb : nullptr;
   int flush_stores = 0;   // stores of the flushes since the last fill
@@ -149,8 +168,6 @@ __global__ __launch_bounds__(256, (D <= 128 ? CS_WGS : 1)) void colsum_kernel(co
     }
   };
 
-  const int S = (Lq_l + 63) >> 6;          // stages of this range
-  const int U = (Lq_l + 31) >> 5;          // 32-row tiles
   const int kbase_l = r * ROWB + ((hh ^ ((r / SWD) & SWM)) << 4);
   float acc[2] = {0.f, 0.f};
   // the group being summed and the row of this range that it ends with (ranges begin with a group)
@@ -184,7 +201,6 @@ __global__ __launch_bounds__(256, (D <= 128 ? CS_WGS : 1)) void colsum_kernel(co
     if (qend == group_end || qend >= Lq_l) flush(group, acc);
   };
 
-  issue_stage(0);
   wait_fills(0);
   __syncthreads();
 
@@ -273,7 +289,6 @@ __global__ __launch_bounds__(256, (D <= 128 ? CS_WGS : 1)) void colsum_kernel(co
   // Tiles 0 .. U-2 go through the pipelined step (their successor exists); every tile whose rows are
   // all valid is consumed inside the next step, the last tile (possibly ragged) by exp_acc below.
   f32x16 sa0, sa1, sb0, sb1;
-  if (S > 1) issue_stage(1);
   qk_tile(0, sa0, sa1);
   for (int s = 0; s < S; s++) {
     flush_stores = 0;

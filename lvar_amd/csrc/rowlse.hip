@@ -61,18 +61,7 @@ __global__ __launch_bounds__(256, (D <= 128 ? ROW_LSE_WGS : 1)) void row_lse_ker
   const int n0 = rt * 256 + wave * 64;     // first query row of this wave
   const float c = p.c;
 
-  // stationary Q^T fragments: lane holds query row n0 + nt*32 + r, d = ks*16 + 8*hh .. +7
-  const bf16_t* qbase = p.q + b * p.q_sb + h * p.q_sh;
   const bf16_t* kbase = p.k + b * p.k_sb + __builtin_amdgcn_readfirstlane(h / p.kv_group) * p.k_sh;   // grouped-query attention: shared key heads
-  bf16x8 qf[2][KS];
-#pragma unroll
-  for (int nt = 0; nt < 2; nt++) {
-    const int qrow = min(n0 + nt * 32 + r, p.Lq - 1);
-    const bf16_t* qp = qbase + (int64_t)qrow * p.q_sr + hh * 8;
-#pragma unroll
-    for (int ks = 0; ks < KS; ks++) qf[nt][ks] = *(const bf16x8*)(qp + ks * 16);
-  }
-
   // buffer descriptor that ends with the last key row: the rows of a ragged last stage beyond it read as zeros
   const int k_srb = (int)p.k_sr * 2;
   const uint64_t ka = (uint64_t)kbase;
@@ -109,6 +98,35 @@ __global__ __launch_bounds__(256, (D <= 128 ? ROW_LSE_WGS : 1)) void row_lse_ker
   };
 
   const int S = (Lk_l + 63) >> 6;          // stages of this range
+  // the ring filled; with the query fragments one round trip to memory
+#pragma unroll
+  for (int s = 0; s < NSTAGE; s++)
+    if (s < S) issue_stage(s);
+  if (n0 >= p.Lq) {
+    // A wave without rows (the last row tile of a slice) keeps its part of the fills and meets
+    // the barriers (1600 rows: 25 of 28 waves have rows; with the column sums behind it 124.7 -> 123.1 us).
+    wait_fills(0);
+    __syncthreads();
+    if (S > 1) __syncthreads();
+    for (int s = 1; s + 1 < S; s++) {
+      if (s + PF < S) issue_stage(s + PF);
+      wait_fills(0);
+      __syncthreads();
+    }
+    return;
+  }
+
+  // stationary Q^T fragments: lane holds query row n0 + nt*32 + r, d = ks*16 + 8*hh .. +7
+  const bf16_t* qbase = p.q + b * p.q_sb + h * p.q_sh;
+  bf16x8 qf[2][KS];
+#pragma unroll
+  for (int nt = 0; nt < 2; nt++) {
+    const int qrow = min(n0 + nt * 32 + r, p.Lq - 1);
+    const bf16_t* qp = qbase + (int64_t)qrow * p.q_sr + hh * 8;
+#pragma unroll
+    for (int ks = 0; ks < KS; ks++) qf[nt][ks] = *(const bf16x8*)(qp + ks * 16);
+  }
+
   const int U = (Lk_l + 31) >> 5;          // 32-key tiles
   const int kbase_l = r * ROWB + ((hh ^ ((r / SWD) & SWM)) << 4);
   // Reference and sum of this lane's half of the keys, per query row.  The sum runs in the order of the attention
@@ -259,11 +277,8 @@ __global__ __launch_bounds__(256, (D <= 128 ? ROW_LSE_WGS : 1)) void row_lse_ker
   using yes = std::true_type;
   using no = std::false_type;
 
-  // prologue: the ring filled; the first stage gives the reference
-#pragma unroll
-  for (int s = 0; s < NSTAGE; s++)
-    if (s < S) issue_stage(s);
-  wait_fills(min(PF, S - 1));
+  // prologue: the first stage gives the reference
+  wait_fills(0);
   __syncthreads();
   f32x16 sa0, sa1, sb0, sb1;
   qk_tile(0, sa0, sa1);
@@ -282,8 +297,7 @@ __global__ __launch_bounds__(256, (D <= 128 ? ROW_LSE_WGS : 1)) void row_lse_ker
       const float x0 = fast_exp2(fmaf(sa0[i], c, -m[0])), x1 = fast_exp2(fmaf(sa1[i], c, -m[1]));
       if (i & 1) { lb[0] += x0; lb[1] += x1; } else { la[0] += x0; la[1] += x1; }
     }
-    wait_fills(min(PF, S - 1) - 1);
-    __syncthreads();
+    __syncthreads();   // every wave has read stage 0: its place may be filled
     for (int s = 1; s + 1 < S; s++) {
       // (before the fills, so that one wait covers both, and with nothing conditional behind a step: the compiler
       // moves a step's exponentials past it, out of the shadow of its matrix instructions)
