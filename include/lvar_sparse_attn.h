@@ -215,6 +215,18 @@ int lvar_csp_attn_upsample_fwd(lvar_tensor_t q, lvar_tensor_t k, lvar_tensor_t v
                                int B, int H, int Lq, int Lk, int head_dim,
                                float o_scale, float scale, void* stream);
 
+/*
+ * lvar_csp_attn_upsample_fwd over the lists that lvar_remap_concat_lists would write (row gS(g) of src_indices, int32
+ * [B, H, Gs, src_row_stride] with src_len >= count valid columns, clamped to the keys, then row g of local_indices),
+ * without writing them: for a step whose lists no later step reads.  The same bits as the two calls.  The groups are
+ * ceil(Lq / group_rows).  group_rows a multiple of 192 and head_dim 64 or 128, otherwise LVAR_EUNSUPPORTED.
+ * Replaces models/sparvar/sparse_attn.py:1096-1144 at the last scale.
+ */
+int lvar_csp_attn_remap_fwd(lvar_tensor_t q, lvar_tensor_t k, lvar_tensor_t v, lvar_tensor_t o_cache, int src_side, int dst_side,
+                            lvar_tensor_t o, const int32_t* src_indices, int64_t src_row_stride, int src_len, int Gs, int count,
+                            const int64_t* local_indices, int64_t local_row_stride, int local_count, int group_rows, int B, int H,
+                            int Lq, int Lk, int head_dim, float o_scale, float scale, void* stream);
+
 /* lvar_csp_attn_upsample_fwd with a partial-result workspace (see lvar_workspace_t). */
 int lvar_csp_attn_upsample_ws_fwd(lvar_tensor_t q, lvar_tensor_t k, lvar_tensor_t v,
                                   lvar_tensor_t o_cache, int src_side, int dst_side,

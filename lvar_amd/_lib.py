@@ -14,6 +14,7 @@ EXPORTED_SYMBOLS = (
     "lvar_version", "lvar_target_arch", "lvar_status_string",
     "lvar_dense_attn_fwd", "lvar_dense_attn_rcp_fwd", "lvar_row_lse_scratch_bytes", "lvar_row_lse_fwd", "lvar_lse2_from_stats",
     "lvar_colsum_fwd", "lvar_block_scores_scratch_bytes", "lvar_block_scores_fwd", "lvar_csp_attn_fwd", "lvar_csp_attn_upsample_fwd",
+    "lvar_csp_attn_remap_fwd",
     "lvar_block_sparse_attn_fwd",
     "lvar_attn_workspace_bytes", "lvar_attn_balanced_workgroups", "lvar_dense_attn_ws_fwd", "lvar_csp_attn_ws_fwd", "lvar_csp_attn_upsample_ws_fwd",
     "lvar_block_sparse_attn_ws_fwd", "lvar_block_sparse_attn_static_fwd",
@@ -76,6 +77,8 @@ def load() -> C.CDLL:
     lib.lvar_csp_attn_fwd.argtypes = [T, T, T, T, T, P, P, P, P, I, I64, I, I, I, I, I, I, F, F, P]
     lib.lvar_csp_attn_upsample_fwd.restype = I
     lib.lvar_csp_attn_upsample_fwd.argtypes = [T, T, T, T, I, I, T, P, P, P, P, I, I64, I, I, I, I, I, I, F, F, P]
+    lib.lvar_csp_attn_remap_fwd.restype = I
+    lib.lvar_csp_attn_remap_fwd.argtypes = [T, T, T, T, I, I, T, P, I64, I, I, I, P, I64, I, I, I, I, I, I, I, F, F, P]
     lib.lvar_block_sparse_attn_fwd.restype = I
     lib.lvar_block_sparse_attn_fwd.argtypes = [T, T, T, T, P, P, P, I64, I64, P, I64, I64, I64, I, I, I, I, I, I, I, I, F, P]
     W = LvarWorkspace

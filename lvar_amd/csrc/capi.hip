@@ -221,16 +221,19 @@ int lvar_block_scores_fwd(lvar_tensor_t q, lvar_tensor_t k, float* scores, const
   return launch_block_scores(p, head_dim, (hipStream_t)stream);
 }
 
+// rows that the lists of a token-list call are formed from, see lvar_csp_attn_remap_fwd
+struct RemapRows { int Gs, count; const int64_t* local; int64_t local_stride; int local_count; };
+
 static int csp_common(lvar_tensor_t q, lvar_tensor_t k, lvar_tensor_t v, lvar_tensor_t o_accum, int up_src, int up_dst,
                       lvar_tensor_t o, float* M, float* L, const int32_t* indices, const int32_t* counts, int G,
                       int64_t idx_row_stride, int group_rows, int B, int H, int Lq, int Lk, int head_dim,
-                      float o_scale, float scale, const lvar_workspace_t* ws, void* stream) {
+                      float o_scale, float scale, const lvar_workspace_t* ws, void* stream, const RemapRows* remap = nullptr) {
   if (!shape_ok(B, H, Lq, Lk, scale) || !view_ok(q) || !view_ok(k) || !view_ok(v) || !view_ok(o)) return LVAR_EINVAL;
   if (o.stride_row <= 0 || (o_accum.ptr && (!view_ok(o_accum) || o_accum.stride_row <= 0))) return LVAR_EINVAL;
   if (!kv_span_ok(k, Lk, head_dim, 0) || !kv_span_ok(v, Lk, head_dim, 0)) return LVAR_EINVAL;
   // gathered rows are addressed with a 24-bit multiply: token index and row stride in bytes below 2^24
   if (Lk > (1 << 24) || k.stride_row * 2 >= (1 << 24) || v.stride_row * 2 >= (1 << 24)) return LVAR_EUNSUPPORTED;
-  if (!indices || !counts || G <= 0 || idx_row_stride <= 0) return LVAR_EINVAL;
+  if (!indices || (!counts && !remap) || G <= 0 || idx_row_stride <= 0) return LVAR_EINVAL;
   if (group_rows <= 0 || (int64_t)G * group_rows < Lq) return LVAR_EINVAL;
   AttnParams p{};
   fill_qkv(p, q, k, v);
@@ -247,6 +250,12 @@ static int csp_common(lvar_tensor_t q, lvar_tensor_t k, lvar_tensor_t v, lvar_te
   p.up_src = up_src; p.up_dst = up_dst;
   const int nw = gather_waves(group_rows);
   if (nw == 0) return LVAR_EUNSUPPORTED;
+  if (remap) {
+    if (nw != 8 || head_dim > 128) return LVAR_EUNSUPPORTED;   // (the shapes whose list readers know two rows)
+    p.list_sh = (int64_t)remap->Gs * idx_row_stride; p.list_sb = (int64_t)H * p.list_sh;
+    p.remap_gs = remap->Gs; p.remap_gk = G; p.remap_cnt = remap->count;
+    p.remap_local = remap->local; p.remap_local_sg = remap->local_stride; p.remap_len = remap->local_count;
+  }
   if (!attach_workspace(p, ws)) return LVAR_EINVAL;
   return launch_attn(p, head_dim, MODE_GATHER, true, false, nw, (hipStream_t)stream);
 }
@@ -290,6 +299,19 @@ int lvar_csp_attn_upsample_ws_fwd(lvar_tensor_t q, lvar_tensor_t k, lvar_tensor_
   if (!upsample_ok(o_cache, src_side, dst_side, Lq)) return LVAR_EINVAL;
   return csp_common(q, k, v, o_cache, src_side, dst_side, o, M, L, indices, counts, G, idx_row_stride, group_rows,
                     B, H, Lq, Lk, head_dim, o_scale, scale, &workspace, stream);
+}
+
+int lvar_csp_attn_remap_fwd(lvar_tensor_t q, lvar_tensor_t k, lvar_tensor_t v, lvar_tensor_t o_cache, int src_side, int dst_side,
+                            lvar_tensor_t o, const int32_t* src_indices, int64_t src_row_stride, int src_len, int Gs, int count,
+                            const int64_t* local_indices, int64_t local_row_stride, int local_count, int group_rows, int B, int H,
+                            int Lq, int Lk, int head_dim, float o_scale, float scale, void* stream) {
+  if (!upsample_ok(o_cache, src_side, dst_side, Lq) || group_rows <= 0) return LVAR_EINVAL;
+  if (Gs <= 0 || count < 0 || src_len < count || src_row_stride < src_len || local_count < 0 || count > INT32_MAX - 64 - local_count ||
+      (local_count > 0 && (!local_indices || local_row_stride < local_count)))
+    return LVAR_EINVAL;
+  const RemapRows rows{Gs, count, local_indices, local_row_stride, local_count};
+  return csp_common(q, k, v, o_cache, src_side, dst_side, o, nullptr, nullptr, src_indices, nullptr, (Lq + group_rows - 1) / group_rows,
+                    src_row_stride, group_rows, B, H, Lq, Lk, head_dim, o_scale, scale, nullptr, stream, &rows);
 }
 
 // argument checks of the block-list entry points (everything but the workspace)

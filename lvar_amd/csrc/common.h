@@ -106,6 +106,13 @@ __device__ __forceinline__ uint32_t real_key(float x) {
   return k > 1u ? k : 1u;
 }
 
+// Query group of a scale with Gs groups that group g of Gk stands on: the nearest group centre, half to even, in three
+// separately rounded fp32 operations (no fused multiply-add), as an eager tensor expression forms it.
+__device__ __forceinline__ int remap_group(int g, int Gk, int Gs) {
+  const float pos = __fsub_rn(__fmul_rn(__fdiv_rn((float)g + 0.5f, (float)Gk), (float)Gs), 0.5f);
+  return max(0, min(Gs - 1, (int)__builtin_rintf(pos)));
+}
+
 // Transposing LDS read: the 16 lanes of a group each point at 4 consecutive bf16 of a row;
 // lane i of the group receives element (i%4) of the rows addressed by lanes (i/4), (i/4)+4,
 // (i/4)+8, (i/4)+12.  With lane s addressing row (s/4), columns 4*(s%4)..+3 of a 4x16 block,

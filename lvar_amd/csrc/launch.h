@@ -35,6 +35,11 @@ struct AttnParams {
   int sub_shift;   // log2(64-key tiles per key block)
   int up_src, up_dst;  // token-list variant: o_accum is an up_src x up_src token grid, bilinearly
                        // resampled to the up_dst x up_dst grid of the queries (0 = o_accum has Lq rows)
+  // token lists formed from the ones of another scale (remap_gs > 0; plain launch only): the first remap_cnt entries of
+  // group g are row remap_group(g) of the remap_gs rows of `list`, the other remap_len row g of remap_local
+  const int64_t* remap_local;
+  int64_t remap_local_sg;
+  int remap_gs, remap_gk, remap_cnt, remap_len;
   int nqt, total_wg;
   // plain launch: query tiles of a (batch, head) that run first (all but a ragged last one), how many these are and how
   // many an XCD takes, ragged last tiles per XCD

@@ -378,9 +378,7 @@ int launch_topk_token_lists(const TopkListParams& p, hipStream_t stream) {
 __global__ __launch_bounds__(256) void remap_concat_lists_kernel(const RemapListParams p) {
   const int row = blockIdx.x;  // bh * Gk + g
   const int g = row % p.Gk, bh = row / p.Gk;
-  // three separately rounded fp32 operations (no fused multiply-add), as an eager tensor expression does
-  const float pos = __fsub_rn(__fmul_rn(__fdiv_rn((float)g + 0.5f, (float)p.Gk), (float)p.Gs), 0.5f);
-  const int gs = max(0, min(p.Gs - 1, (int)__builtin_rintf(pos)));
+  const int gs = remap_group(g, p.Gk, p.Gs);
   const int32_t* src = p.src + ((int64_t)bh * p.Gs + gs) * p.src_stride;
   int32_t* out = p.out + (int64_t)row * p.out_stride;
   // A row is a few thousand entries: bound by the round trips to memory, so eight reads go out before the first store (one

@@ -36,6 +36,7 @@ namespace {
 #define LVAR_ENTRIES(X)                                                                                                   \
   X(lvar_dense_attn_fwd) X(lvar_dense_attn_rcp_fwd) X(lvar_row_lse_scratch_bytes) X(lvar_row_lse_fwd)                     \
   X(lvar_lse2_from_stats) X(lvar_colsum_fwd) X(lvar_csp_attn_fwd) X(lvar_csp_attn_upsample_fwd)                           \
+  X(lvar_csp_attn_remap_fwd)                                                                                              \
   X(lvar_block_sparse_attn_fwd) X(lvar_block_topk_lists) X(lvar_topk_token_lists) X(lvar_topk_union_lists)                \
   X(lvar_remap_concat_lists) X(lvar_mask_to_lists) X(lvar_window_key_scores)
 struct Api {
@@ -330,19 +331,30 @@ bool remap(const at::Tensor& src, int64_t count, int64_t Gk, int64_t k_len, cons
 
 // Step of a column-sparse layer after the decision scale (models/sparvar/sparse_attn.py:1053-1144): lists remapped to
 // this scale's query groups + local run, then token-list attention on top of the upsampled output cache.
-// (q, k, v, scale, src indices, src count, local, group rows, pad, cache, up_src, up_dst) -> (o, indices, counts)
+// Lists that no later step reads are not written (head_dim 64 and 128, groups of a multiple of 192 rows).
+// (q, k, v, scale, src indices, src count, local, group rows, pad, cache, up_src, up_dst, keep lists) -> (o, indices | None, counts | None)
 LVAR_FAST(fast_sparse_step) {
   HANDLE_TH_ERRORS
   Qkv x;
   float scale;
   int64_t count, bm, pad, up_src, up_dst;
-  LVAR_NEED(n == 12 && qkv_ok(x, a[0], a[1], a[2], false) && as_scale(a[3], x.d, scale) && as_long(a[5], count) && as_long(a[7], bm) && bm > 0 &&
+  bool keep;
+  LVAR_NEED(n == 13 && as_bool(a[12], keep) && qkv_ok(x, a[0], a[1], a[2], false) && as_scale(a[3], x.d, scale) && as_long(a[5], count) && as_long(a[7], bm) && bm > 0 &&
             as_long(a[8], pad) && pad > 0 && as_long(a[10], up_src) && as_long(a[11], up_dst) && up_src > 0 && up_src < 32768 && up_dst < 32768);
   const at::Tensor *src = tensor(a[4]), *local = tensor(a[6]), *cache = tensor(a[9]);
   const int64_t Gk = groups_of(x.Lq, bm);
   LVAR_NEED(packed(src, x.dev, at::kInt) && src->dim() == 4 && src->size(0) == x.B && src->size(1) == x.H && src->size(2) > 0 && count >= 0);
   LVAR_NEED(packed(local, x.dev, at::kLong) && local->dim() == 2 && local->size(0) == Gk && accum_ok(x, cache, up_src, up_dst));
   at::Tensor idx, cnt, o = empty_o(x);
+  const int64_t c = std::max(pad, (count + pad - 1) / pad * pad), L = local->size(1), Ks = src->size(3);
+  if (!keep && c <= Ks && c + L <= x.Lk) {
+    const int st = api.lvar_csp_attn_remap_fwd(view(*x.q), view(*x.k), view(*x.v), view(*cache), static_cast<int>(up_src), static_cast<int>(up_dst), view(o),
+                                               src->data_ptr<int32_t>(), Ks, static_cast<int>(Ks), static_cast<int>(src->size(2)), static_cast<int>(c),
+                                               L > 0 ? local->data_ptr<int64_t>() : nullptr, L, static_cast<int>(L), static_cast<int>(bm), x.B, x.H, x.Lq,
+                                               x.Lk, x.d, 1.f, scale, x.stream);
+    if (st == LVAR_OK) return tuple(std::move(o), std::move(idx), std::move(cnt));
+    LVAR_NEED(st == LVAR_EUNSUPPORTED);
+  }
   LVAR_NEED(remap(*src, count, Gk, x.Lk, local, pad, x.Lk, false, x.dev, x.stream, idx, cnt));
   LVAR_NEED(csp_launch(x, idx, cnt, bm, cache, static_cast<int>(up_src), static_cast<int>(up_dst), o, 1.f, scale) == LVAR_OK);
   return tuple(std::move(o), std::move(idx), std::move(cnt));

@@ -97,7 +97,7 @@ class SparseDiffAttn(torch.nn.Module):
             # list remap and attention behind one host call
             cache = self.out_cache if self.out_cache.shape[0] == q.shape[0] else self.out_cache[:q.shape[0]]
             r = fast.fast_sparse_step(q, k, v, ops._plain_scale(scale), inds, s_count, local_inds, self.bm, self.indices_pad_to, cache,
-                                      math.isqrt(cache.shape[-2]), math.isqrt(q.shape[-2])) if self.bm == get_kernel_config_attn()["bm"] else None
+                                      math.isqrt(cache.shape[-2]), math.isqrt(q.shape[-2]), not last) if self.bm == get_kernel_config_attn()["bm"] else None
             if r is not None:
                 assert (s_count + local_count) % self.multiple_of == 0, f"after add local sparse index, mismatch multiple_of={self.multiple_of}"
                 self._keep_lists(r[1], r[2], s_count, local_count, last)

@@ -100,6 +100,18 @@ def test_list_build_and_upsample_argument_validation(lib):
     # fused upsample: Lq must be dst_side^2 and the cache must exist
     args = (one, one, 1, 16, 192, 1, 1, 16, 16, 128, 1.0, 1.0, None)
     assert lib.lvar_csp_attn_upsample_fwd(fake, fake, fake, fake, 2, 5, fake, None, None, *args) == -1         # 25 != 16
+    remap = lib.lvar_csp_attn_remap_fwd   # rows of 16 entries, 12 of them taken, then 4 local ones; 16 = 4 x 4 queries
+    rows = (1, 1, 16, 16, 128, 1.0, 1.0, None)
+    assert remap(fake, fake, fake, fake, 2, 5, fake, one, 16, 16, 1, 12, one, 4, 4, 192, *rows) == -1           # 25 != 16
+    assert remap(fake, fake, fake, fake, 2, 4, fake, None, 16, 16, 1, 12, one, 4, 4, 192, *rows) == -1
+    assert remap(fake, fake, fake, fake, 2, 4, fake, one, 16, 16, 0, 12, one, 4, 4, 192, *rows) == -1
+    assert remap(fake, fake, fake, fake, 2, 4, fake, one, 16, 11, 1, 12, one, 4, 4, 192, *rows) == -1           # fewer columns than entries
+    assert remap(fake, fake, fake, fake, 2, 4, fake, one, 15, 16, 1, 12, one, 4, 4, 192, *rows) == -1
+    assert remap(fake, fake, fake, fake, 2, 4, fake, one, 16, 16, 1, 12, None, 4, 4, 192, *rows) == -1
+    assert remap(fake, fake, fake, fake, 2, 4, fake, one, 16, 16, 1, 12, one, 3, 4, 192, *rows) == -1
+    assert remap(fake, fake, fake, fake, 2, 4, fake, one, 16, 16, 1, 12, one, 4, 4, 0, *rows) == -1
+    assert remap(fake, fake, fake, fake, 2, 4, fake, one, 16, 16, 1, 12, one, 4, 4, 96, *rows) == -2            # 3-wave workgroups
+    assert remap(fake, fake, fake, fake, 2, 4, fake, one, 16, 16, 1, 12, one, 4, 4, 192, 1, 1, 16, 16, 256, 1.0, 1.0, None) == -2
     assert lib.lvar_csp_attn_upsample_fwd(fake, fake, fake, null, 2, 4, fake, None, None, *args) == -1
 
 

@@ -285,3 +285,30 @@ def test_sparse_steps_do_not_depend_on_the_host_path(B, d, strided, monkeypatch)
             assert taken.names.count("fast_full_step") == 1 and taken.names.count("fast_sparse_step") == 2
     for a, b in zip(*results):
         assert torch.equal(a, b)
+
+
+# lists formed while they are read: one, two and three workgroups per group (head_dim 64 with few groups takes 3-wave ones),
+# either row empty or ending inside a tile, more and fewer groups than the lists come from
+@pytest.mark.parametrize("d", [64, 128])
+@pytest.mark.parametrize("side,Gs,bm", [(5, 1, 192), (14, 3, 192), (20, 9, 192), (28, 2, 384)])
+@pytest.mark.parametrize("count,L", [(0, 1), (0, 70), (1, 0), (64, 0), (63, 1), (65, 63), (200, 130)])
+def test_attention_over_remapped_rows_is_the_attention_over_the_written_lists(d, side, Gs, bm, count, L):
+    from lvar_amd import _lib, sparse_attn_ops as ops
+    lib, B, H, Lq, Lk, src_side = _lib.load(), 2, 3, side * side, 700, 3
+    q, k, v = _inputs(B, H, H, Lq, Lk, d, side == 14, seed=side)
+    cache = _inputs(B, H, H, src_side * src_side, Lk, d, False, seed=1)[0]
+    G, Ks = -(-Lq // bm), count + 3
+    g = torch.Generator(device="cuda").manual_seed(count)
+    src = torch.randint(-2, Lk + 2, (B, H, Gs, Ks), generator=g, device="cuda", dtype=torch.int32)   # (clamped to the keys)
+    local = torch.randint(0, Lk, (G, L), generator=g, device="cuda")
+    lists = torch.empty((B, H, G, count + L), dtype=torch.int32, device="cuda")
+    counts = torch.empty((B, H, G), dtype=torch.int32, device="cuda")
+    o, want = (torch.full((B, H, Lq, d), 7.0, dtype=torch.bfloat16, device="cuda") for _ in range(2))
+    s = torch.cuda.current_stream().cuda_stream
+    loc = local.data_ptr() if L else None
+    assert lib.lvar_remap_concat_lists(src.data_ptr(), Ks, Ks, loc, L, L, lists.data_ptr(), count + L, counts.data_ptr(), B * H, Gs, G, count, Lk, 0, s) == 0
+    assert lib.lvar_csp_attn_upsample_fwd(ops._view(q), ops._view(k), ops._view(v), ops._view(cache), src_side, side, ops._view(want), None, None,
+                                          lists.data_ptr(), counts.data_ptr(), G, count + L, bm, B, H, Lq, Lk, d, 1.0, 0.125, s) == 0
+    assert lib.lvar_csp_attn_remap_fwd(ops._view(q), ops._view(k), ops._view(v), ops._view(cache), src_side, side, ops._view(o),
+                                       src.data_ptr(), Ks, Ks, Gs, count, loc, L, L, bm, B, H, Lq, Lk, d, 1.0, 0.125, s) == 0
+    assert torch.equal(o, want)
