@@ -123,7 +123,7 @@ __device__ __forceinline__ void attn_item(const AttnParams& p, char* smem, const
   int avail = 0;   // entries of the list row from `list` on (token lists)
   // Token lists formed from another scale's (see AttnParams): the waves that read the list take the entries straight from the
   // two rows they come from, so that no launch writes the lists and the count is not waited for.  Step at the last scale with
-  // 20 % of the keys and a local run, B2 H16 d128: 30 x 30 34.1 -> 29.9 us, 48 x 48 86.0 -> 81.6, 64 x 64 170.7 -> 164.6.
+  // 20 % of the keys and a local run, B2 H16 d128: 30 x 30 32.8 -> 29.7 us, 48 x 48 84.5 -> 81.4, 64 x 64 169.3 -> 164.5.
   constexpr bool REMAP = MODE == MODE_GATHER && !SK && (NPROD > 0 || D == 64);
   int n_src = 0x7fffffff;             // entries from `list`, the others from `local`:
   const int32_t* local = nullptr;     // low words of 64-bit entries
