@@ -218,9 +218,10 @@ __global__ __launch_bounds__(256, (D <= 128 ? ROW_LSE_WGS : 1)) void row_lse_ker
   // S(u) on the matrix cores, the exponentials of tile u-1 from (c0, c1) on the vector ALU as a three-stage pipeline
   // over the MFMA steps (scale | exp2 | add), interleaved by hand.  One per 64-key stage opens the two sums (tile u-1
   // is the first of its stage), the other closes them; `whole`: the first tile of the last stage, one sum.
-  auto step = [&](int u, f32x16& n0a, f32x16& n1a, const f32x16& c0, const f32x16& c1, auto opens, auto whole) {
+  // (`buf`: the stage's place in the ring, a constant in the loop of SCORES)
+  auto step = [&](auto buf, int u, f32x16& n0a, f32x16& n1a, const f32x16& c0, const f32x16& c1, auto opens, auto whole) {
     constexpr bool OPENS = decltype(opens)::value, WHOLE = decltype(whole)::value;
-    const char* kb = smem + ((u >> 1) & (NSTAGE - 1)) * KTILE + (u & 1) * 32 * ROWB;
+    const char* kb = smem + buf * KTILE + (u & 1) * 32 * ROWB;
     constexpr int AHEAD = 2;
     bf16x8 frag[KS];
 #pragma unroll
@@ -266,6 +267,8 @@ __global__ __launch_bounds__(256, (D <= 128 ? ROW_LSE_WGS : 1)) void row_lse_ker
       __builtin_amdgcn_sched_barrier(0);
     }
     st_add(KS - 1);
+    // (the sums are wanted here: left to itself the compiler moves exponentials into the next step, behind its MFMAs)
+    if (SCORES && OPENS) asm volatile("" : "+v"(la[0]), "+v"(la[1]), "+v"(lb[0]), "+v"(lb[1]));
     if (!OPENS) {
       const float t0 = la[0] + lb[0], t1 = la[1] + lb[1];
       l[0] += t0;
@@ -298,26 +301,42 @@ __global__ __launch_bounds__(256, (D <= 128 ? ROW_LSE_WGS : 1)) void row_lse_ker
       if (i & 1) { lb[0] += x0; lb[1] += x1; } else { la[0] += x0; la[1] += x1; }
     }
     __syncthreads();   // every wave has read stage 0: its place may be filled
-    for (int s = 1; s + 1 < S; s++) {
+    auto stage = [&](auto buf, int s) {
       // (before the fills, so that one wait covers both, and with nothing conditional behind a step: the compiler
       // moves a step's exponentials past it, out of the shadow of its matrix instructions)
       if (SCORES && left == 0) emit();
       if (s + PF < S) issue_stage(s + PF);
-      step(2 * s, sa0, sa1, sb0, sb1, no{}, no{});
+      step(buf, 2 * s, sa0, sa1, sb0, sb1, no{}, no{});
       if (SCORES) left--;
-      step(2 * s + 1, sb0, sb1, sa0, sa1, yes{}, no{});
+      step(buf, 2 * s + 1, sb0, sb1, sa0, sa1, yes{}, no{});
       wait_fills(min(s + PF, S - 1) - (s + 1));
       __syncthreads();
+    };
+    if constexpr (SCORES) {
+      // two stages per turn: the place in the ring is part of the reads, which saves eight vector additions per stage
+      // (B1 H24 d128, 8 x 64 x 64 tokens, lists in all: 1526 -> 1515 us; H8, 4 x 48 x 48: 183.9 -> 180.6; H16 d64, 4 x 64 x 64: 254 -> 249).  Without SCORES
+      // the registers that this takes spill around the loop, and short sweeps lose as much (1600 x 4121: +1 us).
+      using P0 = std::integral_constant<int, 0>;
+      using P1 = std::integral_constant<int, 1>;
+      int s = 1;
+      for (; s + 2 < S; s += 2) {
+        stage(P1{}, s);
+        stage(P0{}, s + 1);
+      }
+      if (s + 1 < S) stage(P1{}, s);
+    } else {
+      for (int s = 1; s + 1 < S; s++) stage(s & (NSTAGE - 1), s);
     }
+    const int buf = (S - 1) & (NSTAGE - 1);
     if (SCORES && left == 0) emit();
-    step(2 * S - 2, sa0, sa1, sb0, sb1, no{}, no{});
+    step(buf, 2 * S - 2, sa0, sa1, sb0, sb1, no{}, no{});
     if (SCORES && --left == 0) emit();
     if (U & 1) {
       mask_tile(U - 1, sa0, sa1);
       tile_sum(sa0, sa1, la);
       lb[0] = lb[1] = 0.f;
     } else {
-      step(2 * S - 1, sb0, sb1, sa0, sa1, yes{}, yes{});
+      step(buf, 2 * S - 1, sb0, sb1, sa0, sa1, yes{}, yes{});
       mask_tile(U - 1, sb0, sb1);
       tile_sum(sb0, sb1, lb);
     }
