@@ -83,7 +83,7 @@ struct SkCtx {
 };
 
 // One query tile w (or, in a balanced launch, the units [u0, u1) of its tile list; `whole` = all of them).
-template <int D, int NWAVES, int MODE, bool ACCUM, bool LSE_ONLY, bool SK, int NPROD>
+template <int D, int NWAVES, int MODE, bool ACCUM, bool LSE_ONLY, bool SK, int NPROD, bool IDLE>
 __device__ __forceinline__ void attn_item(const AttnParams& p, char* smem, const int w, const int bh, const int qt,
                                           const int u0, const int u1, const bool whole, const SkCtx& sk) {
   // NPROD: the last waves only fetch -- they read the list, form the addresses and issue every K/V fill -- and the
@@ -290,8 +290,8 @@ __device__ __forceinline__ void attn_item(const AttnParams& p, char* smem, const
     // A computing wave of a ragged last query tile that owns no row does not compute: it keeps its part of the fills and
     // meets the barriers, so the waves with rows have the matrix cores and the LDS reads to themselves, and a launch at
     // the power limit keeps its clock (dense B2 H16 d128, 1600 x 4121 in 256-row tiles, an eighth of them padding: 111.7 ->
-    // 106.5 us).  Not where the second role costs registers that have to be spilled, nor at head_dim 256 (+1 %).
-    const bool no_rows = !SK && (NPROD > 0 || (MODE == MODE_BLOCK && D == 128)) && q0 + wave * 32 >= p.Lq;
+    // 106.5 us).  Where no wave has that role otherwise (IDLE, see idle_waves) it is an instance of its own.
+    const bool no_rows = !SK && (NPROD > 0 || IDLE) && q0 + wave * 32 >= p.Lq;
     if ((NPROD > 0 && wave >= NCOMP) || no_rows) {
       // ---- fetch waves: the fill schedule of the loop below and nothing else; one barrier per tile ----
       const bool fills = !NPROD || wave >= NCOMP;
@@ -857,7 +857,7 @@ __device__ __forceinline__ void attn_item(const AttnParams& p, char* smem, const
 #endif  // __HIP_DEVICE_COMPILE__
 
 // THIRD: registers of a wave limited so that three workgroups share a compute unit, see third_workgroup
-template <int D, int NWAVES, int MODE, bool ACCUM, bool LSE_ONLY, int NPROD, bool THIRD = false>
+template <int D, int NWAVES, int MODE, bool ACCUM, bool LSE_ONLY, int NPROD, bool IDLE, bool THIRD = false>
 __global__ __launch_bounds__(NWAVES * 64, ((NWAVES <= 4 && D <= 128) ? (THIRD ? 3 : 2) : 1)) void attn_fwd_kernel(const AttnParams p) {
   // The body is compiled for the device only: the host pass just needs the launch stub, and it
   // silently drops the stub when the body uses the LDS-DMA builtins.
@@ -878,7 +878,7 @@ __global__ __launch_bounds__(NWAVES * 64, ((NWAVES <= 4 && D <= 128) ? (THIRD ? 
     if (i - p.whole_per_xcd >= p.ragged_per_xcd || bh >= p.B * p.H) return;
     qt = p.whole_nqt;
   }
-  attn_item<D, NWAVES, MODE, ACCUM, LSE_ONLY, false, NPROD>(p, smem, 0, bh, qt, 0, 0, true, SkCtx{});
+  attn_item<D, NWAVES, MODE, ACCUM, LSE_ONLY, false, NPROD, IDLE>(p, smem, 0, bh, qt, 0, 0, true, SkCtx{});
 #endif
 }
 
@@ -921,7 +921,7 @@ __global__ __launch_bounds__(NWAVES * 64, (NWAVES <= 4 ? 2 : 1)) void attn_fwd_b
     if (sk.pieces < 1 || sk.pieces > SK_MAX_PIECES || sk.kp < 0 || sk.kp >= sk.pieces || (sk.pieces > 1 && (sk.slot0 < 0 || sk.slot0 + sk.pieces > 2 * p.sk_wgs))) return;
   }
   const int bh = w / p.nqt;
-  attn_item<D, NWAVES, MODE, ACCUM, false, true, (MODE == MODE_GATHER && NWAVES == 8) ? 2 : 0>(p, smem, w, bh, w - bh * p.nqt, u0, u1, sk.pieces == 1, sk);
+  attn_item<D, NWAVES, MODE, ACCUM, false, true, (MODE == MODE_GATHER && NWAVES == 8) ? 2 : 0, false>(p, smem, w, bh, w - bh * p.nqt, u0, u1, sk.pieces == 1, sk);
 #endif
 }
 
@@ -1046,6 +1046,12 @@ static bool third_workgroup(int total_wg) { return total_wg > 2 * device_cus(); 
 // head_dim 256 a wave fills its SIMD.  Same bits.
 static bool fetch_waves(int total_wg) { return total_wg <= device_cus(); }
 
+// A last query tile with waves that own no row, where no wave only fetches.  The role is an instance of its own: in one kernel
+// with the others its second loop costs launches without such waves up to 3 % (B2 H16 d128, 2304 rows in lists of 18 tiles on
+// average, with / without: 63.2 / 61.3 us).  Not at head_dim 64, where the role's registers have to be spilled, nor at 256 (+1 %
+// with it).
+static bool idle_waves(int Lq, int rows) { return Lq % rows != 0 && Lq % rows <= rows - 32; }
+
 template <int D, int NWAVES, int MODE, bool ACCUM, bool LSE_ONLY, int NPROD = (MODE == MODE_GATHER && NWAVES == 8) ? 2 : 0>
 static int launch_one(const AttnParams& p0, hipStream_t stream) {
   AttnParams p = p0;
@@ -1114,11 +1120,20 @@ static int launch_one(const AttnParams& p0, hipStream_t stream) {
   if constexpr (D == 64 && NWAVES == 4 && MODE == MODE_BLOCK && !LSE_ONLY) {
     if (third_workgroup(p.total_wg)) {
       static_assert(SMEM <= 48 * 1024, "three workgroups share the LDS of a compute unit; no larger limit has to be asked for");
-      hipLaunchKernelGGL((attn_fwd_kernel<D, NWAVES, MODE, ACCUM, LSE_ONLY, NPROD, true>), dim3(grid), dim3(NWAVES * 64), SMEM, stream, p);
+      hipLaunchKernelGGL((attn_fwd_kernel<D, NWAVES, MODE, ACCUM, LSE_ONLY, NPROD, false, true>), dim3(grid), dim3(NWAVES * 64), SMEM, stream, p);
       return hipGetLastError() == hipSuccess ? LVAR_OK : LVAR_ELAUNCH;
     }
   }
-  auto kern = attn_fwd_kernel<D, NWAVES, MODE, ACCUM, LSE_ONLY, NPROD>;
+  if constexpr (MODE == MODE_BLOCK && D == 128 && NPROD == 0) {
+    if (idle_waves(p.Lq, WGROWS)) {
+      auto kern = attn_fwd_kernel<D, NWAVES, MODE, ACCUM, LSE_ONLY, NPROD, true>;
+      static std::atomic<uint64_t> lds_ready{0};
+      if (!ensure_lds_limit((const void*)kern, SMEM, lds_ready)) return LVAR_ELAUNCH;
+      hipLaunchKernelGGL(kern, dim3(grid), dim3(NWAVES * 64), SMEM, stream, p);
+      return hipGetLastError() == hipSuccess ? LVAR_OK : LVAR_ELAUNCH;
+    }
+  }
+  auto kern = attn_fwd_kernel<D, NWAVES, MODE, ACCUM, LSE_ONLY, NPROD, false>;
   static std::atomic<uint64_t> lds_ready{0};
   if (!ensure_lds_limit((const void*)kern, SMEM, lds_ready)) return LVAR_ELAUNCH;
   hipLaunchKernelGGL(kern, dim3(grid), dim3(NWAVES * 64), SMEM, stream, p);
