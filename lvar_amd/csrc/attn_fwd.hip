@@ -863,21 +863,8 @@ __global__ __launch_bounds__(NWAVES * 64, ((NWAVES <= 4 && D <= 128) ? (THIRD ? 
   // silently drops the stub when the body uses the LDS-DMA builtins.
 #if defined(__HIP_DEVICE_COMPILE__)
   extern __shared__ __attribute__((aligned(1024))) char smem[];
-  // Consecutive workgroup ids are dealt round-robin to the 8 XCDs; remap so that each XCD
-  // walks a contiguous range of (batch, head, q-tile) and K/V of one head stay in its L2.
-  const int xcd = blockIdx.x & 7, i = blockIdx.x >> 3;
   int bh, qt;
-  if (i < p.whole_per_xcd) {
-    const int w = xcd * p.whole_per_xcd + i;
-    if (w >= p.whole_wg) return;
-    bh = w / p.whole_nqt;
-    qt = w - bh * p.whole_nqt;
-  } else {
-    // ragged last tiles of the (batch, head) slices, behind the whole ones (see launch_one)
-    bh = xcd * p.ragged_per_xcd + (i - p.whole_per_xcd);
-    if (i - p.whole_per_xcd >= p.ragged_per_xcd || bh >= p.B * p.H) return;
-    qt = p.whole_nqt;
-  }
+  if (!tile_of(p.order, blockIdx.x, bh, qt)) return;
   attn_item<D, NWAVES, MODE, ACCUM, LSE_ONLY, false, NPROD, IDLE>(p, smem, 0, bh, qt, 0, 0, true, SkCtx{});
 #endif
 }
@@ -1112,11 +1099,8 @@ static int launch_one(const AttnParams& p0, hipStream_t stream) {
   // workgroups, and what is dispatched last decides how long the launch drains (token lists of 832 keys, 288 groups of
   // which 32 have 64 rows, on 256 compute units: 54 -> 47 us with the idle waves).
   const bool ragged = p.nqt > 1 && p.Lq % WGROWS != 0;
-  p.whole_nqt = ragged ? p.nqt - 1 : p.nqt;
-  p.whole_wg = p.B * p.H * p.whole_nqt;
-  p.whole_per_xcd = (p.whole_wg + 7) / 8;
-  p.ragged_per_xcd = ragged ? (p.B * p.H + 7) / 8 : 0;
-  const int grid = 8 * (p.whole_per_xcd + p.ragged_per_xcd);
+  p.order = tile_order(p.B * p.H, p.nqt, ragged);
+  const int grid = TILE_XCDS * p.order.per_xcd;
   if constexpr (D == 64 && NWAVES == 4 && MODE == MODE_BLOCK && !LSE_ONLY) {
     if (third_workgroup(p.total_wg)) {
       static_assert(SMEM <= 48 * 1024, "three workgroups share the LDS of a compute unit; no larger limit has to be asked for");

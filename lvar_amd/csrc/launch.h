@@ -4,6 +4,7 @@
 #include <stdint.h>
 #include <atomic>
 #include "common.h"
+#include "tile_order.h"
 #include "../../include/lvar_sparse_attn.h"
 
 namespace lvar {
@@ -41,9 +42,7 @@ struct AttnParams {
   int64_t remap_local_sg;
   int remap_gs, remap_gk, remap_cnt, remap_len;
   int nqt, total_wg;
-  // plain launch: query tiles of a (batch, head) that run first (all but a ragged last one), how many these are and how
-  // many an XCD takes, ragged last tiles per XCD
-  int whole_nqt, whole_wg, whole_per_xcd, ragged_per_xcd;
+  TileOrder order;   // plain launch: which query tile a workgroup takes
   // balanced launch: workspace handed in by the caller (null = plain launch).  The launch code fills in sk_wgs
   // (0 = plain launch after all), sk_counters (per-query-tile arrival counters, all zero between launches) and
   // sk_slots (2 * sk_wgs slots of partial results).

@@ -1,0 +1,51 @@
+// Host-side check of the order of query tiles (lvar_amd/csrc/tile_order.h), with the arithmetic the device code uses:
+//   * every query tile of every slice is taken by exactly one workgroup of the launch, and nothing else is,
+//   * no XCD gets more tiles than an even split gives the fullest one,
+//   * on every XCD the ragged last tiles come behind the whole ones, and the whole ones are a contiguous range.
+// Prints "ok <cases>" or the first violation.
+#include <cstdio>
+#include <vector>
+#include "../../lvar_amd/csrc/tile_order.h"
+
+using namespace lvar;
+
+static const char* check(int slices, int nqt, bool ragged) {
+  const TileOrder t = tile_order(slices, nqt, ragged);
+  const int tiles = slices * nqt;
+  std::vector<int> taken(tiles, 0);
+  for (int x = 0; x < TILE_XCDS; x++) {
+    int here = 0, last = -1;
+    bool behind = false;
+    for (int i = 0; i < t.per_xcd; i++) {
+      int s = -1, q = -1;
+      if (!tile_of(t, i * TILE_XCDS + x, s, q)) continue;
+      if (s < 0 || s >= slices || q < 0 || q >= nqt) return "tile out of range";
+      taken[s * nqt + q]++;
+      here++;
+      if (ragged && q == nqt - 1) { behind = true; continue; }
+      if (behind) return "whole tile behind a ragged one";
+      const int w = s * t.nqt + q;
+      if (last >= 0 && w != last + 1) return "whole tiles of an XCD not contiguous";
+      last = w;
+    }
+    if (here > (tiles + TILE_XCDS - 1) / TILE_XCDS) return "XCD with more tiles than an even split";
+  }
+  for (int n : taken)
+    if (n != 1) return "tile not taken exactly once";
+  return nullptr;
+}
+
+int main() {
+  long cases = 0;
+  for (int slices = 1; slices <= 72; slices++)
+    for (int nqt = 1; nqt <= 260; nqt += nqt < 40 ? 1 : 7)
+      for (int ragged = 0; ragged <= (nqt > 1 ? 1 : 0); ragged++, cases++)
+        if (const char* why = check(slices, nqt, ragged != 0)) { printf("%s: %d slices of %d tiles, ragged %d\n", why, slices, nqt, ragged); return 1; }
+  // one 128-row workgroup per compute unit of 256: four heads of 8065 .. 8191 rows and the like
+  const int full[][2] = {{1, 256}, {2, 128}, {3, 85}, {4, 64}, {5, 51}, {9, 28}, {16, 16}, {32, 8}, {64, 4}, {128, 2}};
+  for (auto& f : full)
+    for (int ragged = 0; ragged <= 1; ragged++, cases++)
+      if (const char* why = check(f[0], f[1], ragged != 0)) { printf("%s: %d slices of %d tiles, ragged %d\n", why, f[0], f[1], ragged); return 1; }
+  printf("ok %ld\n", cases);
+  return 0;
+}
