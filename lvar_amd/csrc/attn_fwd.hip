@@ -1095,10 +1095,9 @@ static int launch_one(const AttnParams& p0, hipStream_t stream) {
     if (wide_tiles(p0, D)) return launch_one<D, 8, MODE_BLOCK, false, false>(p0, stream);
     if (fetch_waves(p.total_wg)) return launch_one<D, 8, MODE_BLOCK, false, false, 4>(p0, stream);
   }
-  // Ragged last tiles start behind all whole ones: their waves without rows do not compute, so they are the shorter
-  // workgroups, and what is dispatched last decides how long the launch drains (token lists of 832 keys, 288 groups of
-  // which 32 have 64 rows, on 256 compute units: 54 -> 47 us with the idle waves).
-  const bool ragged = p.nqt > 1 && p.Lq % WGROWS != 0;
+  const int rest = p.Lq % WGROWS;
+  const bool ragged = MODE == MODE_GATHER ? NPROD > 0 && ragged_runs_last(p.B * p.H, p.nqt, rest, WGROWS, device_cus())
+                                          : p.list != nullptr && ragged_lists_last(p.B * p.H, p.nqt, rest, device_cus());
   p.order = tile_order(p.B * p.H, p.nqt, ragged);
   const int grid = TILE_XCDS * p.order.per_xcd;
   if constexpr (D == 64 && NWAVES == 4 && MODE == MODE_BLOCK && !LSE_ONLY) {

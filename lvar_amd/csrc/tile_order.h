@@ -55,4 +55,22 @@ LVAR_HD bool tile_of(const TileOrder& t, unsigned id, int& slice, int& qt) {
   return i < t.per_xcd && slice < t.ragged;
 }
 
+// Whether the ragged last tiles of token lists with fetch-only waves (one workgroup per compute unit) run behind the whole
+// ones.  The waves without rows do not compute, so with at least half of them idle such a tile is the shorter workgroup, and
+// it pays where the launch can end on a round of nothing else, with every whole tile in the full rounds before it.  832 of
+// 4121 keys, d128, 192-row groups with 30 rows in the last one, behind against in order: 67 heads of 4 tiles on 256 compute
+// units -20 %, 140 heads -8 %, 275 -3 %; where whole tiles are left for the last round +2 .. +4 % (100 heads of 4, 166 of 3).
+LVAR_HD bool ragged_runs_last(int slices, int nqt, int rest, int rows, int cus) {
+  if (cus <= 0 || nqt < 2 || rest == 0 || 2 * rest > rows) return false;
+  const int total = slices * nqt, left = total % cus;
+  return total > cus && left > 0 && left < slices;
+}
+
+// The same for block lists.  The last tile of a grid has the shorter lists of a sink + window mask (23 drawn layers of grids of side 31 .. 62:
+// -1.1 % on average, -5 .. +1.7 %), and lists of any length come out even (-0.1 %), while its second visit to the K/V of a
+// head costs the more the fewer tiles share it: in order / behind, 25 % of 4121 keys, d128, 1500 tiles in heads of 2 170 / 190
+// us, of 4 152 / 161, of 8 139 / 140.  Dense attention gains nothing from it at any size (2 tiles 71 / 80 us; d256, 3 tiles
+// 436 / 487).
+LVAR_HD bool ragged_lists_last(int slices, int nqt, int rest, int cus) { return rest != 0 && nqt >= 12 && slices * nqt > cus; }
+
 }  // namespace lvar

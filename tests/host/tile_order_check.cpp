@@ -1,7 +1,8 @@
 // Host-side check of the order of query tiles (lvar_amd/csrc/tile_order.h), with the arithmetic the device code uses:
 //   * every query tile of every slice is taken by exactly one workgroup of the launch, and nothing else is,
 //   * no XCD gets more tiles than an even split gives the fullest one,
-//   * on every XCD the ragged last tiles come behind the whole ones, and the whole ones are a contiguous range.
+//   * on every XCD the ragged last tiles come behind the whole ones, and the whole ones are a contiguous range,
+//   * the rules that take ragged tiles out of the order, on both sides of each of their bounds.
 // Prints "ok <cases>" or the first violation.
 #include <cstdio>
 #include <vector>
@@ -46,6 +47,24 @@ int main() {
   for (auto& f : full)
     for (int ragged = 0; ragged <= 1; ragged++, cases++)
       if (const char* why = check(f[0], f[1], ragged != 0)) { printf("%s: %d slices of %d tiles, ragged %d\n", why, f[0], f[1], ragged); return 1; }
+  // ragged tiles leave the order where they alone make the last round, with the waves of half of their rows idle
+  struct { int slices, nqt, rest; bool last; } rule[] = {
+      {67, 4, 30, true}, {140, 4, 96, true}, {250, 2, 96, true}, {275, 4, 30, true},
+      {67, 4, 160, false}, {67, 4, 97, false},          // nearly as long as the others
+      {100, 4, 30, false}, {166, 3, 30, false},         // whole tiles are left for the last round
+      {32, 9, 64, false},                               // the last round holds every ragged tile
+      {64, 4, 64, false}, {32, 4, 64, false}, {300, 1, 64, false}, {288, 2, 0, false}};
+  for (auto& r : rule) {
+    cases++;
+    if (ragged_runs_last(r.slices, r.nqt, r.rest, 192, 256) != r.last) { printf("order of %d slices of %d tiles, rest %d\n", r.slices, r.nqt, r.rest); return 1; }
+  }
+  // block lists: heads of many tiles, more of them than compute units
+  struct { int slices, nqt, rest; bool last; } lists[] = {{24, 12, 36, true}, {48, 16, 16, true}, {750, 2, 27, false}, {375, 4, 91, false}, {60, 11, 89, false},
+                                                          {48, 16, 0, false}, {8, 32, 1, false}, {9, 32, 1, true}};
+  for (auto& r : lists) {
+    cases++;
+    if (ragged_lists_last(r.slices, r.nqt, r.rest, 256) != r.last) { printf("order of %d block-list slices of %d tiles, rest %d\n", r.slices, r.nqt, r.rest); return 1; }
+  }
   printf("ok %ld\n", cases);
   return 0;
 }
