@@ -290,7 +290,7 @@ __device__ __forceinline__ void attn_item(const AttnParams& p, char* smem, const
     // A computing wave of a ragged last query tile that owns no row does not compute: it keeps its part of the fills and
     // meets the barriers, so the waves with rows have the matrix cores and the LDS reads to themselves, and a launch at
     // the power limit keeps its clock (dense B2 H16 d128, 1600 x 4121 in 256-row tiles, an eighth of them padding: 111.7 ->
-    // 106.5 us).  Where no wave has that role otherwise (IDLE, see idle_waves) it is an instance of its own.
+    // 106.5 us).  Where no wave has that role otherwise (IDLE, see idle_waves_pay) it is an instance of its own.
     const bool no_rows = !SK && (NPROD > 0 || IDLE) && q0 + wave * 32 >= p.Lq;
     if ((NPROD > 0 && wave >= NCOMP) || no_rows) {
       // ---- fetch waves: the fill schedule of the loop below and nothing else; one barrier per tile ----
@@ -1033,12 +1033,6 @@ static bool third_workgroup(int total_wg) { return total_wg > 2 * device_cus(); 
 // head_dim 256 a wave fills its SIMD.  Same bits.
 static bool fetch_waves(int total_wg) { return total_wg <= device_cus(); }
 
-// A last query tile with waves that own no row, where no wave only fetches.  The role is an instance of its own: in one kernel
-// with the others its second loop costs launches without such waves up to 3 % (B2 H16 d128, 2304 rows in lists of 18 tiles on
-// average, with / without: 63.2 / 61.3 us).  Not at head_dim 64, where the role's registers have to be spilled, nor at 256 (+1 %
-// with it).
-static bool idle_waves(int Lq, int rows) { return Lq % rows != 0 && Lq % rows <= rows - 32; }
-
 template <int D, int NWAVES, int MODE, bool ACCUM, bool LSE_ONLY, int NPROD = (MODE == MODE_GATHER && NWAVES == 8) ? 2 : 0>
 static int launch_one(const AttnParams& p0, hipStream_t stream) {
   AttnParams p = p0;
@@ -1107,8 +1101,9 @@ static int launch_one(const AttnParams& p0, hipStream_t stream) {
       return hipGetLastError() == hipSuccess ? LVAR_OK : LVAR_ELAUNCH;
     }
   }
-  if constexpr (MODE == MODE_BLOCK && D == 128 && NPROD == 0) {
-    if (idle_waves(p.Lq, WGROWS)) {
+  // (an instance of its own; not at head_dim 64, where the role's registers have to be spilled, nor at 256: +1 % with it)
+  if constexpr (MODE == MODE_BLOCK && D == 128 && NPROD == 0 && NWAVES >= 4) {
+    if (idle_waves_pay(NWAVES, p.nqt, rest)) {
       auto kern = attn_fwd_kernel<D, NWAVES, MODE, ACCUM, LSE_ONLY, NPROD, true>;
       static std::atomic<uint64_t> lds_ready{0};
       if (!ensure_lds_limit((const void*)kern, SMEM, lds_ready)) return LVAR_ELAUNCH;

@@ -66,11 +66,23 @@ LVAR_HD bool ragged_runs_last(int slices, int nqt, int rest, int rows, int cus) 
   return total > cus && left > 0 && left < slices;
 }
 
-// The same for block lists.  The last tile of a grid has the shorter lists of a sink + window mask (23 drawn layers of grids of side 31 .. 62:
-// -1.1 % on average, -5 .. +1.7 %), and lists of any length come out even (-0.1 %), while its second visit to the K/V of a
-// head costs the more the fewer tiles share it: in order / behind, 25 % of 4121 keys, d128, 1500 tiles in heads of 2 170 / 190
-// us, of 4 152 / 161, of 8 139 / 140.  Dense attention gains nothing from it at any size (2 tiles 71 / 80 us; d256, 3 tiles
-// 436 / 487).
+// The same for block lists.  The last tile of a grid has the shorter lists of a sink + window mask (50 drawn layers of at
+// least 12 tiles per head: -0.7 % on average, -5.6 .. +3.7 %), and lists of a score or of random length come out even, while
+// its second visit to the K/V of a head costs the more the fewer tiles share it: in order / behind, 25 % of 4121 keys, d128,
+// 1500 tiles in heads of 2 170 / 190 us, of 4 152 / 161, of 8 139 / 140.  Dense attention gains nothing from it at any size
+// (2 tiles 71 / 80 us; d256, 3 tiles 436 / 487).
 LVAR_HD bool ragged_lists_last(int slices, int nqt, int rest, int cus) { return rest != 0 && nqt >= 12 && slices * nqt > cus; }
+
+// Whether an instance is taken whose waves without rows do not compute, in dense and block-list launches of workgroups
+// where no wave only fetches: a second loop in the kernel costs every workgroup up to a percent, and a last tile has only so
+// many idle waves; what they save is matrix instructions, and so power, in launches that run long enough for the clock to
+// follow.  d128, with it against without, kept up for 150 ms each: dense 128-row workgroups with 3 of 8 waves of a head idle
+// -3 .. -12 %, 2 of 32 -0.4 .. -3 %, 2 of 64 -0.2 .. -0.6 %; lists of 25 % with 3 of 16 -1 .. -5 %, 3 of 48 -0.4 .. -3 %, 3 of
+// 80 +0.1 .. -2.5 %, 2 of 80 +0.6 .. -0.5 %, 1 of 80 +1.6 .. -0.1 %; 256-row ones with 6 of 56 111.7 / 106.5 us, 4 of 144 -0.4 %,
+// 2 of 144 nothing.  64-row workgroups lose up to 1 % at any share.
+LVAR_HD bool idle_waves_pay(int waves, int nqt, int rest) {
+  const int idle = rest == 0 ? 0 : waves - (rest + 31) / 32;
+  return waves >= 4 && idle > 0 && 32 * idle >= waves * nqt;
+}
 
 }  // namespace lvar

@@ -2,7 +2,8 @@
 //   * every query tile of every slice is taken by exactly one workgroup of the launch, and nothing else is,
 //   * no XCD gets more tiles than an even split gives the fullest one,
 //   * on every XCD the ragged last tiles come behind the whole ones, and the whole ones are a contiguous range,
-//   * the rules that take ragged tiles out of the order, on both sides of each of their bounds.
+//   * the rules that take ragged tiles out of the order, on both sides of each of their bounds,
+//   * the rule that takes the instance with idle waves, likewise.
 // Prints "ok <cases>" or the first violation.
 #include <cstdio>
 #include <vector>
@@ -64,6 +65,14 @@ int main() {
   for (auto& r : lists) {
     cases++;
     if (ragged_lists_last(r.slices, r.nqt, r.rest, 256) != r.last) { printf("order of %d block-list slices of %d tiles, rest %d\n", r.slices, r.nqt, r.rest); return 1; }
+  }
+  // idle waves: a 32nd of all, in workgroups of at least 128 rows
+  struct { int waves, nqt, rest; bool pay; } idle[] = {
+      {8, 7, 64, true}, {8, 2, 4, true}, {8, 4, 200, true}, {8, 18, 128, false}, {8, 18, 96, true}, {8, 7, 0, false}, {8, 2, 225, false},
+      {4, 8, 60, true}, {4, 8, 96, true}, {4, 9, 96, false}, {4, 18, 64, false}, {4, 20, 4, true}, {4, 32, 4, false}, {4, 2, 97, false}, {2, 2, 20, false}};
+  for (auto& r : idle) {
+    cases++;
+    if (idle_waves_pay(r.waves, r.nqt, r.rest) != r.pay) { printf("idle waves of %d in %d tiles per head, rest %d\n", r.waves, r.nqt, r.rest); return 1; }
   }
   printf("ok %ld\n", cases);
   return 0;
