@@ -5,6 +5,7 @@
 #include <utility>
 #include "common.h"
 #include "launch.h"
+#include "score_bins.h"
 
 namespace lvar {
 
@@ -32,6 +33,25 @@ __device__ __forceinline__ uint32_t wave_umax(uint32_t v) {
 __device__ __forceinline__ uint32_t wave_umin(uint32_t v) {
   return (uint32_t)__builtin_amdgcn_readlane(wave_scan((int)v, -1, [](int a, int b) { return (int)min((uint32_t)a, (uint32_t)b); }), 63);
 }
+// Smallest value of each aligned group of G lanes (2, 4 or 8), in all of them
+template <int G>
+__device__ __forceinline__ uint32_t group_umin(uint32_t v) {
+  auto mv = [](uint32_t x, auto ctrl) { return (uint32_t)__builtin_amdgcn_update_dpp(0, (int)x, decltype(ctrl)::value, 0xf, 0xf, true); };
+  v = min(v, mv(v, std::integral_constant<int, 0xB1>{}));                        // quad_perm: neighbours
+  if constexpr (G >= 4) v = min(v, mv(v, std::integral_constant<int, 0x4E>{}));  // quad_perm: pairs
+  if constexpr (G >= 8) v = min(v, mv(v, std::integral_constant<int, 0x141>{})); // row_half_mirror: fours
+  return v;
+}
+
+// Reduction over each row of 16 lanes, in all of them
+template <class Op, class T>
+__device__ __forceinline__ void row_all(Op op, T& v) {
+  auto mv = [](T x, auto ctrl) { return __builtin_bit_cast(T, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, x), decltype(ctrl)::value, 0xf, 0xf, true)); };
+  v = op(v, mv(v, std::integral_constant<int, 0xB1>{}));    // quad_perm: neighbours
+  v = op(v, mv(v, std::integral_constant<int, 0x4E>{}));    // quad_perm: pairs
+  v = op(v, mv(v, std::integral_constant<int, 0x141>{}));   // row_half_mirror: fours
+  v = op(v, mv(v, std::integral_constant<int, 0x140>{}));   // row_mirror: eights
+}
 
 // ---------------------------------------------------------------------------------------------
 // Exact top-k per row by radix select.  One 512-thread workgroup per row; wave w owns the w-th
@@ -45,10 +65,9 @@ __device__ __forceinline__ uint32_t wave_umin(uint32_t v) {
 //   a counting pass gives every wave its number of selected keys, the last pass writes the selected
 //   columns in ascending order (ballot compaction into an LDS ring, full-width stores).
 // ---------------------------------------------------------------------------------------------
-constexpr int TOPK_BINS = 2048;
+constexpr int TOPK_BINS = SCORE_BINS;
 constexpr int TOPK_SHARED_MAX_N = 12288;   // longest row of 1024 threads where two rows share a compute unit
 constexpr int TOPK_CAND = 256;   // keys of the first pass's bin that are resolved by direct comparison
-constexpr uint32_t KEY_NEG_INF = 0x007fffffu, KEY_POS_INF = 0xff800000u;   // real_key of -inf and +inf
 
 // UNION: the output row is the ascending merge of the selection with the row's own list of W columns (in any order,
 // columns that are listed or selected several times come out as often), as int64.  How often each column is listed sits
@@ -127,13 +146,36 @@ __global__ __launch_bounds__(NT, (KPT >= 1 && KPT <= 24) ? (NT == 512 ? 6 : 4) :
   // would fall into a handful of bins of the first pass and the LDS atomics of a wave would serialise on them.  The
   // bits that the largest and the smallest key of the row have in common are therefore taken as known, and the
   // digits start at the first bit in which keys differ: `top` low bits are left to resolve, 11 at a time.
+  if constexpr (UNION) {
+    // the bulk of the row, see score_bins.h (threads without a score stay out of it)
+    constexpr int G = score_group(KPT);
+    const bool any = kmin <= kmax;
+    const uint32_t gmax = group_umin<G>(any ? kmax : 0xffffffffu), gmin = ~group_umin<G>(any ? ~kmin : 0xffffffffu);
+    kmax = gmax == 0xffffffffu ? 0u : gmax;
+    kmin = gmin == 0u ? 0xffffffffu : gmin;
+  }
   kmax = wave_umax(kmax);
   kmin = wave_umin(kmin);
   if (lane == 0) { wgt[wave] = (int)kmax; weq[wave] = (int)kmin; }
   if (tid == 0) ncand = 0;
   __syncthreads();
+  float narrow = 0.f, wide = 0.f;   // UNION: of the waves' bulks
+  if constexpr (UNION) {
+    static_assert(NW == 16, "one wave per lane of a row of 16");
+    kmax = (uint32_t)wgt[lane & 15];
+    kmin = (uint32_t)weq[lane & 15];
+    wide = score_width(kmin, kmax);
+    narrow = wide > 0.f ? wide : INFINITY;
+    row_all([](uint32_t a, uint32_t b) { return max(a, b); }, kmax);
+    row_all([](uint32_t a, uint32_t b) { return min(a, b); }, kmin);
+    row_all([](float a, float b) { return fmaxf(a, b); }, wide);
+    row_all([](float a, float b) { return fminf(a, b); }, narrow);
+    kmax = __builtin_amdgcn_readfirstlane(kmax);
+    kmin = __builtin_amdgcn_readfirstlane(kmin);
+  } else {
 #pragma unroll
-  for (int w = 0; w < NW; w++) { kmax = max(kmax, (uint32_t)wgt[w]); kmin = min(kmin, (uint32_t)weq[w]); }
+    for (int w = 0; w < NW; w++) { kmax = max(kmax, (uint32_t)wgt[w]); kmin = min(kmin, (uint32_t)weq[w]); }
+  }
   if constexpr (UNION) {   // (read behind at least one more barrier)
     const int64_t* more = p.more + (int64_t)row * p.W;
     for (int t = tid; t < p.W; t += NT) {
@@ -141,25 +183,36 @@ __global__ __launch_bounds__(NT, (KPT >= 1 && KPT <= 24) ? (NT == 512 ? 6 : 4) :
       atomicAdd(&listed[j >> 1], 1u << (16 * (j & 1)));
     }
   }
-  // (UNION: the smallest key leaves out the -inf of the columns that do not compete, so nothing is known from it)
-  const int top = UNION ? 32 : 32 - __builtin_clz((kmax ^ kmin) | 1u) + (((kmax ^ kmin) == 0u) ? -1 : 0);   // 0 when all keys are equal
-  uint32_t pmask = (top >= 32) ? 0u : ~((1u << top) - 1u);
+  // bits that keys of [lo, hi] need not share
+  auto differing = [](uint32_t lo, uint32_t hi) { return 32 - __builtin_clz((hi ^ lo) | 1u) + (((hi ^ lo) == 0u) ? -1 : 0); };   // 0 when all keys are equal
+  auto above_bits = [](int bits) -> uint32_t { return bits >= 32 ? 0u : ~((1u << bits) - 1u); };
+  // (UNION: its range is not that of all keys, so nothing is known from it)
+  int top = UNION ? 32 : differing(kmin, kmax);
+  uint32_t pmask = above_bits(top);
   uint32_t prefix = kmax & pmask;
-  // UNION, first pass: the scores are sums of signed products, so the top bits of their keys (sign, exponent, two bits of
-  // mantissa) fill a few dozen bins and the bin of the threshold holds several hundred keys of 10521: two more passes.
-  // Bins of equal width between the smallest finite score and the largest hold about ten each (32 rows: 16.7 -> 12.4 us
-  // with the row's own list requested first and no scan where a column is listed once).  The map is monotonic in the key
-  // (subtraction, product and truncation are), so a bin is a run of keys like any other; where one score lies far from
-  // all others the passes by digits follow, over the keys of that bin.
-  bool linear = false;
-  int lbin = 0;
-  float x0 = 0.f, xs = 0.f;
-  auto bin_of = [&](uint32_t key) -> int {
-    const uint32_t k = max(key, KEY_NEG_INF);
-    const float x = __builtin_bit_cast(float, k ^ ((k >> 31) ? 0x80000000u : 0xffffffffu));
-    return (int)__builtin_amdgcn_fmed3f((x - x0) * xs, 0.f, (float)(TOPK_BINS - 1));
+  // UNION, first pass: bins of equal width.  Where that of the threshold is too full after all, the passes by digits follow
+  // over its keys, [klo, khi].
+  int bin[UNION ? KPT : 1], lbin = 0;
+  uint32_t klo = 0u, khi = 0xffffffffu;
+  auto in_play = [&](uint32_t key) -> bool { return (key & pmask) == prefix && (!UNION || (klo <= key && key <= khi)); };
+  // One more key in bin `at`, for the lanes that ask.  UNION, whose digits are a second choice where keys crowd: the lanes that
+  // share the bin of the first one count at once, not one after the other (99 % equal scores 40 -> 21 us).
+  auto tally = [&](int at, bool counts) {
+    if constexpr (UNION) {
+      const unsigned long long asked = __builtin_amdgcn_ballot_w64(counts);
+      if (asked == 0ull) return;
+      const int first = __builtin_ctzll(asked);
+      const int b0 = __builtin_amdgcn_readlane(at, first);
+      const unsigned long long same = __builtin_amdgcn_ballot_w64(counts && at == b0);
+      if (__builtin_popcountll(same) > 8) {
+        if (lane == first) atomicAdd(&hist[b0], __builtin_popcountll(same));
+        counts = counts && at != b0;
+      }
+    }
+    if (counts) atomicAdd(&hist[at], 1);
   };
-  auto in_play = [&](uint32_t key) -> bool { return (key & pmask) == prefix && (!UNION || !linear || bin_of(key) == lbin); };
+  using yes = std::true_type;
+  using no = std::false_type;
   // The bin that holds the want-th key from the top, and how many of its keys are wanted: thread t owns the bpt bins
   // nbins-1 - t*bpt .. (descending).
   auto find_bin = [&](int nbins) {
@@ -189,9 +242,12 @@ __global__ __launch_bounds__(NT, (KPT >= 1 && KPT <= 24) ? (NT == 512 ? 6 : 4) :
   // After the first pass the chosen bin usually holds a few dozen keys.  They are copied to LDS, and if they
   // fit, every one of them counts the candidates above it: the one with fewer than `want` above and at least
   // `want` at or above is the threshold, and the other passes are not needed.
-  auto resolve = [&]() -> bool {
+  auto resolve = [&](auto by_bin) -> bool {
+    int c = 0;
     visit([&](int j, uint32_t key) {
-      const bool m = in_play(key);
+      bool m;
+      if constexpr (decltype(by_bin)::value) m = bin[c++] == lbin;
+      else m = in_play(key);
       const unsigned long long bm = __builtin_amdgcn_ballot_w64(m);
       if (bm != 0ull) {
         int base = 0;
@@ -226,23 +282,34 @@ __global__ __launch_bounds__(NT, (KPT >= 1 && KPT <= 24) ? (NT == 512 ? 6 : 4) :
   };
   bool found = false, first = true;
   if constexpr (UNION) {
-    if (kmin < kmax && kmax < KEY_POS_INF) {
-      x0 = __builtin_bit_cast(float, kmin ^ ((kmin >> 31) ? 0x80000000u : 0xffffffffu));
-      const float range = __builtin_bit_cast(float, kmax ^ ((kmax >> 31) ? 0x80000000u : 0xffffffffu)) - x0;
-      const uint32_t rb = __builtin_bit_cast(uint32_t, range);
-      if (rb > 0x08000000u && rb < 0x7f800000u) {   // above 2^-111 (its reciprocal is finite) and finite
-        linear = true;
-        xs = (float)(TOPK_BINS - 1) / range;
-      }
-    }
-    if (linear) {
-      visit([&](int j, uint32_t key) { atomicAdd(&hist[bin_of(key)], 1); });
+    ScoreBins bins;
+    if (score_bins(kmin, kmax, narrow, wide, bins)) {
+#pragma unroll
+      for (int c = 0; c < KPT; c++) bin[c] = score_bin(bins, keys[c]);
+#pragma unroll
+      for (int c = 0; c < KPT; c++) atomicAdd(&hist[bin[c]], 1);
       __syncthreads();
       find_bin(TOPK_BINS);
       lbin = sel[0];
-      found = resolve();
-      if (!found) __syncthreads();    // every wave has read the number of candidates before it is cleared
-      if (!found && tid == 0) ncand = 0;
+      found = resolve(yes{});
+      if (!found) {
+        uint32_t hi = 0u, lo = 0xffffffffu;
+#pragma unroll
+        for (int c = 0; c < KPT; c++)
+          if (bin[c] == lbin) { hi = max(hi, keys[c]); lo = min(lo, keys[c]); }
+        hi = wave_umax(hi);
+        lo = wave_umin(lo);
+        if (lane == 0) { wgt[wave] = (int)hi; weq[wave] = (int)lo; }
+        __syncthreads();
+#pragma unroll
+        for (int w = 0; w < NW; w++) { hi = max(hi, (uint32_t)wgt[w]); lo = min(lo, (uint32_t)weq[w]); }
+        if (tid == 0) ncand = 0;   // (every wave has read it ahead of that barrier)
+        klo = lo;
+        khi = hi;
+        top = differing(klo, khi);
+        pmask = above_bits(top);
+        prefix = khi & pmask;
+      }
     }
   }
   if (top == 0) __syncthreads();   // no pass below to separate these reads of wgt / weq from their reuse
@@ -254,7 +321,7 @@ __global__ __launch_bounds__(NT, (KPT >= 1 && KPT <= 24) ? (NT == 512 ? 6 : 4) :
     for (int t = tid; t < nbins; t += NT) hist[t] = 0;
     __syncthreads();
     visit([&](int j, uint32_t key) {
-      if (in_play(key)) atomicAdd(&hist[(key >> shift) & (nbins - 1)], 1);
+      tally((key >> shift) & (nbins - 1), in_play(key));
     });
     __syncthreads();
     find_bin(nbins);
@@ -262,7 +329,7 @@ __global__ __launch_bounds__(NT, (KPT >= 1 && KPT <= 24) ? (NT == 512 ? 6 : 4) :
     pmask |= (uint32_t)(nbins - 1) << shift;
     if (first && hi > 0) {
       first = false;
-      if (resolve()) break;
+      if (resolve(no{})) break;
     }
   }
   const uint32_t T = prefix;  // key of the k-th largest element

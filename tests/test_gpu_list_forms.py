@@ -105,10 +105,14 @@ def _wide_scores(kind, rows, n, seed):
     hole = torch.rand(rows, n, generator=g, device="cuda") < 0.1
     if kind == "holes":                       # columns that do not compete, as the window's own keys
         x[hole] = -float("inf")
-    elif kind == "outlier":                   # equal-width bins hold everything else in one of them
+    elif kind == "outlier":                   # far from all others
         x[:, n // 2], x[:, n // 3] = 1e30, -1e30
     elif kind == "tails":
         x = x.sign() * (x.abs() * 12).exp()
+    elif kind == "two widths":                # the bulk of the row is one bin of its range, and digits follow over its keys
+        x[torch.rand(rows, n, generator=g, device="cuda") < 0.6] *= 1e-4
+    elif kind == "mostly equal":
+        x[torch.rand(rows, n, generator=g, device="cuda") < 0.97] = 0.25
     elif kind == "infinite":
         x[hole], x[:, n // 2] = float("inf"), -float("inf")
     elif kind == "none":
@@ -123,10 +127,10 @@ def _wide_scores(kind, rows, n, seed):
     return x
 
 
-@pytest.mark.parametrize("kind", ["plain", "holes", "outlier", "tails", "infinite", "none", "one", "tiny", "zeros"])
+@pytest.mark.parametrize("kind", ["plain", "holes", "outlier", "tails", "two widths", "mostly equal", "infinite", "none", "one", "tiny", "zeros"])
 @pytest.mark.parametrize("n", [60, 1000, 10521, 16384])
 def test_merged_selection_of_any_spread_of_scores(n, kind):
-    """The first pass counts in bins of equal width between the smallest and the largest finite score."""
+    """The first pass counts in bins of equal width over the bulk of the scores."""
     from lvar_amd import _lib
     rows, W = 3, 17
     x = _wide_scores(kind, rows, n, seed=n)
