@@ -89,13 +89,9 @@ __global__ __launch_bounds__(256, (D <= 128 ? ROW_LSE_WGS : 1)) void row_lse_ker
       asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tbuffer_load_dwordx4 %1, %2, %3 offen lds" : : "s"(m0v), "v"(fill_voff[sl % PER]), "s"(krsrc), "s"(soff) : "memory");
     }
   };
-  constexpr auto vm = [](int n) constexpr { return 0x0f70 | (n & 15) | (((n >> 4) & 3) << 14); };
-  // wait until at most `younger` later stages (0 or 1: the ring has two) of this wave's fills are still in flight
-  static_assert(PF == 1, "wait_fills knows one stage ahead");
-  auto wait_fills = [&](int younger) {
-    if (younger >= 1) __builtin_amdgcn_s_waitcnt(vm(SLOTS));
-    else __builtin_amdgcn_s_waitcnt(vm(0));
-  };
+  // (the ring has two stages, so nothing younger than the stage that is waited for is in flight)
+  static_assert(PF == 1, "one stage ahead");
+  auto wait_fills = [&] { __builtin_amdgcn_s_waitcnt(0x0f70); };   // vmcnt(0)
 
   const int S = (Lk_l + 63) >> 6;          // stages of this range
   // the ring filled; with the query fragments one round trip to memory
@@ -105,12 +101,12 @@ __global__ __launch_bounds__(256, (D <= 128 ? ROW_LSE_WGS : 1)) void row_lse_ker
   if (n0 >= p.Lq) {
     // A wave without rows (the last row tile of a slice) keeps its part of the fills and meets
     // the barriers (1600 rows: 25 of 28 waves have rows; with the column sums behind it 124.7 -> 123.1 us).
-    wait_fills(0);
+    wait_fills();
     __syncthreads();
     if (S > 1) __syncthreads();
     for (int s = 1; s + 1 < S; s++) {
       if (s + PF < S) issue_stage(s + PF);
-      wait_fills(0);
+      wait_fills();
       __syncthreads();
     }
     return;
@@ -281,7 +277,7 @@ __global__ __launch_bounds__(256, (D <= 128 ? ROW_LSE_WGS : 1)) void row_lse_ker
   using no = std::false_type;
 
   // prologue: the first stage gives the reference
-  wait_fills(0);
+  wait_fills();
   __syncthreads();
   f32x16 sa0, sa1, sb0, sb1;
   qk_tile(0, sa0, sa1);
@@ -309,7 +305,7 @@ __global__ __launch_bounds__(256, (D <= 128 ? ROW_LSE_WGS : 1)) void row_lse_ker
       step(buf, 2 * s, sa0, sa1, sb0, sb1, no{}, no{});
       if (SCORES) left--;
       step(buf, 2 * s + 1, sb0, sb1, sa0, sa1, yes{}, no{});
-      wait_fills(min(s + PF, S - 1) - (s + 1));
+      wait_fills();
       __syncthreads();
     };
     if constexpr (SCORES) {
