@@ -66,6 +66,11 @@ struct Swz {
   __device__ static __forceinline__ int fv(int row) { return (D >= 128) ? ((row & 3) << 2) : (((row >> 1) & 1) << 2); }
 };
 
+// Token-list instances whose list readers know two rows (AttnParams::remap_gs): 192-row groups in one workgroup of eight waves,
+// or at head_dim 64 in two of three.  The others would pay the choice of a row per entry for nothing.
+template <int D, int NWAVES, int MODE, int NPROD>
+constexpr bool reads_remapped = MODE == MODE_GATHER && (NPROD > 0 || (D == 64 && NWAVES == 3));
+
 // LDS of a workgroup: K and V buffers; the epilogue's transpose buffer of eight computing waves is larger
 template <int D, int NCOMP, int MODE>
 constexpr int attn_lds_bytes() {
@@ -124,7 +129,7 @@ __device__ __forceinline__ void attn_item(const AttnParams& p, char* smem, const
   // Token lists formed from another scale's (see AttnParams): the waves that read the list take the entries straight from the
   // two rows they come from, so that no launch writes the lists and the count is not waited for.  Step at the last scale with
   // 20 % of the keys and a local run, B2 H16 d128: 30 x 30 32.8 -> 29.7 us, 48 x 48 84.5 -> 81.4, 64 x 64 169.3 -> 164.5.
-  constexpr bool REMAP = MODE == MODE_GATHER && !SK && (NPROD > 0 || D == 64);
+  constexpr bool REMAP = !SK && reads_remapped<D, NWAVES, MODE, NPROD>;
   int n_src = 0x7fffffff;             // entries from `list`, the others from `local`:
   const int32_t* local = nullptr;     // low words of 64-bit entries
   // first four entries of a block list, read together with the count (not after it): one memory
@@ -1041,6 +1046,7 @@ static int launch_one(const AttnParams& p0, hipStream_t stream) {
   constexpr int SMEM = attn_lds_bytes<D, NWAVES - NPROD, MODE>();
   if (MODE == MODE_BLOCK && p.list == nullptr) p.group_rows = WGROWS;  // dense: any row grouping
   if (p.group_rows % WGROWS != 0) return LVAR_EINVAL;
+  if (p.remap_gs > 0 && !reads_remapped<D, NWAVES, MODE, NPROD>) return LVAR_EUNSUPPORTED;
   p.nqt = (p.Lq + WGROWS - 1) / WGROWS;
   p.total_wg = p.B * p.H * p.nqt;
   constexpr bool WIDE = MODE == MODE_BLOCK && NWAVES == 8;   // 256 query rows, or 128 and fetch waves

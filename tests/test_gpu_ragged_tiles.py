@@ -57,18 +57,45 @@ def test_ragged_last_tile(B, H, rows):
         qg, kg, vg = q.cuda(), k.cuda(), v.cuda()
         out = ops.csp_attn(qg, kg, vg, None, idx.cuda(), cnt.cuda(), o0.cuda(), 1)
         assert _close(out, oracle.csp_attn(q, k, v, None, idx, cnt, o0, 1))
-        # 256-row workgroups (many tiles) are covered by the full-size checks; here 128-row tiles with the same remainder
+        # 128-row tiles with the same remainder (256-row ones: test_ragged_last_tile_of_256_rows)
         Lq = 128 + min(rows, 127)
         o, _ = ops.dense_attn(qg[:, :, :Lq].contiguous(), kg, vg)
         assert _close(o, oracle.dense_attn(q[:, :, :Lq], k, v)[0])
 
 
-def test_ragged_last_tile_of_256_rows():
+# 256-row workgroups: one per compute unit of the launch's single round, seven 128-row tiles per head (1.75 per compute unit,
+# the same round shared by two) in the other form; the last of four tiles has 40 of its 256 rows, six of eight waves idle
+@pytest.mark.parametrize("Lk", [1, 64, 65, 128, 190, 257, 320])
+def test_ragged_last_tile_of_256_rows(Lk):
     from lvar_amd import sparse_attn_ops as ops
-    H, Lq, Lk = 80, 3 * 256 + 40, 200
-    (q, k, v), _ = _rand(1, H, Lq, Lk, 128, seed=7)
-    o, (M, L) = ops.dense_attn(q.cuda(), k.cuda(), v.cuda())
+    H, Lq = torch.cuda.get_device_properties(0).multi_processor_count // 4, 3 * 256 + 40
+    (q, k, v), g = _rand(1, H, Lq, Lk, 128, seed=7)
+    qg, kg, vg = q.cuda(), k.cuda(), v.cuda()
+    o, (M, L) = ops.dense_attn(qg, kg, vg)
     h = slice(H - 2, H)
-    o1, (M1, L1) = ops.dense_attn(*[t[:, h].contiguous().cuda() for t in (q, k, v)])      # few tiles: 128-row workgroups
+    part = [t[:, h].contiguous() for t in (qg, kg, vg)]
+    o1, (M1, L1) = ops.dense_attn(*part)      # few tiles: 128-row workgroups with fetch-only waves
     assert torch.equal(o1, o[:, h]) and torch.equal(M1, M[:, h]) and torch.equal(L1, L[:, h])
     assert _close(o1, oracle.dense_attn(q[:, h], k[:, h], v[:, h])[0])
+    mask = torch.rand(1, H, 4, -(-Lk // 64), generator=g) < 0.7          # lists of 256-row query blocks, some of them empty
+    num, idx = oracle.block_mask_to_lists(mask)
+    o, (M, L) = ops.block_sparse_attn(qg, kg, vg, num.cuda(), idx.cuda(), 256, 64)
+    o1, (M1, L1) = ops.block_sparse_attn(*part, num[:, h].contiguous().cuda(), idx[:, h].contiguous().cuda(), 256, 64)
+    assert torch.equal(o1, o[:, h]) and torch.equal(M1, M[:, h]) and torch.equal(L1, L[:, h])
+    assert _close(o1, oracle.block_sparse_attn(q[:, h], k[:, h], v[:, h], num[:, h], idx[:, h], 256, 64)[0])
+
+
+# token lists whose ragged groups run behind the whole ones: more groups than compute units, fewer than one per head in the
+# last round, 30 of 192 rows in a head's last group
+@pytest.mark.parametrize("d", [64, 128])
+def test_ragged_groups_behind_the_whole_ones(d):
+    from lvar_amd import sparse_attn_ops as ops
+    cus = torch.cuda.get_device_properties(0).multi_processor_count
+    H, Lq, Lk = cus // 2 + 19, 192 + 30, 300
+    assert cus < 2 * H and 2 * H - cus < H
+    (q, k, v), g = _rand(1, H, Lq, Lk, d, seed=d)
+    idx = torch.randint(0, Lk, (1, H, 2, Lk), generator=g, dtype=torch.int32)
+    cnt = torch.randint(0, 201, (1, H, 2), generator=g, dtype=torch.int32)
+    o0 = (torch.randn(1, H, Lq, d, generator=g) * 0.5).to(torch.bfloat16)
+    out = ops.csp_attn(q.cuda(), k.cuda(), v.cuda(), None, idx.cuda(), cnt.cuda(), o0.cuda(), 1)
+    assert _close(out, oracle.csp_attn(q, k, v, None, idx, cnt, o0, 1))
