@@ -43,14 +43,13 @@ LVAR_HD TileOrder tile_order(int slices, int nqt, bool ragged_last) {
 // XCD x go to ragged ones, in slice order.
 LVAR_HD bool tile_of(const TileOrder& t, unsigned id, int& slice, int& qt) {
   const int x = (int)(id % TILE_XCDS), i = (int)(id / TILE_XCDS);
-  const int w = x * t.whole_per_xcd + i;
-  if (i < t.whole_per_xcd && w < t.whole) {
-    slice = w / t.nqt;
-    qt = w - slice * t.nqt;
-    return true;
-  }
   const int first = x * t.whole_per_xcd < t.whole ? x * t.whole_per_xcd : t.whole;   // whole tiles of the XCDs before x
   const int mine = t.whole - first < t.whole_per_xcd ? t.whole - first : t.whole_per_xcd;
+  if (i < mine) {
+    slice = (first + i) / t.nqt;
+    qt = first + i - slice * t.nqt;
+    return true;
+  }
   slice = x * t.per_xcd - first + (i - mine);
   qt = t.nqt;
   return i < t.per_xcd && slice < t.ragged;
