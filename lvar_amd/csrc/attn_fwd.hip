@@ -112,7 +112,7 @@ __device__ __forceinline__ void attn_item(const AttnParams& p, char* smem, const
   // LDS map: K buffers at 0 and TILE, V buffers at 2*TILE and 3*TILE
 
   const int b = bh / p.H, h = bh - b * p.H;
-  const int tid = threadIdx.x, lane = tid & 63;
+  const int tid = __builtin_amdgcn_workitem_id_x(), lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int hh = lane >> 5, r = lane & 31;
   const int fwave = NPROD ? wave - NCOMP : wave;   // index among the filling waves (negative: this wave does not fill)
@@ -868,8 +868,12 @@ __global__ __launch_bounds__(NWAVES * 64, ((NWAVES <= 4 && D <= 128) ? (THIRD ? 
   // silently drops the stub when the body uses the LDS-DMA builtins.
 #if defined(__HIP_DEVICE_COMPILE__)
   extern __shared__ __attribute__((aligned(1024))) char smem[];
+  // The place is worked out in scalar registers (blockIdx would be a call, as threadIdx: library functions are compiled with the
+  // target's own features and so not inlined here, and their result counts as different per lane) and then handed on as if it
+  // differed per lane: known to be uniform, it leads the compiler to 30 .. 40 more vector registers, and spills.
   int bh, qt;
-  if (!tile_of(p.order, blockIdx.x, bh, qt)) return;
+  if (!tile_of(p.order, __builtin_amdgcn_workgroup_id_x(), bh, qt)) return;
+  asm volatile("" : "+v"(bh), "+v"(qt));
   attn_item<D, NWAVES, MODE, ACCUM, LSE_ONLY, false, NPROD, IDLE>(p, smem, 0, bh, qt, 0, 0, true, SkCtx{});
 #endif
 }

@@ -165,7 +165,7 @@ __global__ __launch_bounds__(NT, (KPT >= 1 && KPT <= 24) ? (NT == 512 ? 6 : 4) :
     kmax = (uint32_t)wgt[lane & 15];
     kmin = (uint32_t)weq[lane & 15];
     wide = score_width(kmin, kmax);
-    narrow = wide > 0.f ? wide : INFINITY;
+    narrow = wide > 0.f && ((lane & 15) + 1) * KPT * 64 <= n ? wide : INFINITY;   // (the last wave's may be that of a few columns)
     row_all([](uint32_t a, uint32_t b) { return max(a, b); }, kmax);
     row_all([](uint32_t a, uint32_t b) { return min(a, b); }, kmin);
     row_all([](float a, float b) { return fmaxf(a, b); }, wide);

@@ -51,7 +51,7 @@ LVAR_HD bool score_bins(uint32_t lo, uint32_t hi, float narrow, float wide, Scor
   union { float f; uint32_t u; } range;
   range.f = 2.5f * width;
   if (range.u <= 0x08000000u || range.u >= 0x7f800000u) return false;   // 2^-111; infinite
-  if (!(wide <= 12.f * narrow)) return false;   // (waves of normal scores differ by up to 5, of exp(12 |x|) by 13 and more)
+  if (!(wide <= 12.f * narrow)) return false;   // (full waves of normal scores differ by up to 5, of exp(12 |x|) by 13 and more)
   b.x0 = 0.5f * score_of_key(lo) + 0.5f * score_of_key(hi) - 0.5f * range.f;
   b.xs = (float)(SCORE_BINS - 1) / range.f;
   return true;
