@@ -4,7 +4,7 @@
 // dozen bins and the bin of the threshold holds several hundred keys of 10521: two more passes.  Bins of equal width hold a
 // few dozen keys at most, but between the smallest and the largest score they do so only while no score lies far from the
 // others: one that does leaves the others in a handful of bins, whose counts then serialise, and the pass is lost.  So the
-// bins span two and a half times the range that every group of neighbouring threads reaches: the smallest of the largest keys
+// bins span twice the range that every group of neighbouring threads reaches: the smallest of the largest keys
 // of a group's threads, over the groups the largest.  Keys beyond it count in the end bins.  A far score changes it only
 // where it comes with one in every thread of a group; of normal scores it is 1.5 .. 2 standard deviations each way.  Scores
 // spread over many orders of magnitude have no such range: it differs by as much between waves, and the digits are as good
@@ -49,7 +49,7 @@ LVAR_HD float score_width(uint32_t lo, uint32_t hi) {
 LVAR_HD bool score_bins(uint32_t lo, uint32_t hi, float narrow, float wide, ScoreBins& b) {
   const float width = score_width(lo, hi);
   union { float f; uint32_t u; } range;
-  range.f = 2.5f * width;
+  range.f = 2.f * width;
   if (range.u <= 0x08000000u || range.u >= 0x7f800000u) return false;   // 2^-111; infinite
   if (!(wide <= 12.f * narrow)) return false;   // (full waves of normal scores differ by up to 5, of exp(12 |x|) by 13 and more)
   b.x0 = 0.5f * score_of_key(lo) + 0.5f * score_of_key(hi) - 0.5f * range.f;
