@@ -33,16 +33,25 @@ __device__ __forceinline__ uint32_t wave_umax(uint32_t v) {
 __device__ __forceinline__ uint32_t wave_umin(uint32_t v) {
   return (uint32_t)__builtin_amdgcn_readlane(wave_scan((int)v, -1, [](int a, int b) { return (int)min((uint32_t)a, (uint32_t)b); }), 63);
 }
-// Smallest value of each aligned group of G lanes (2, 4 or 8), in all of them
+// Smallest value of each aligned group of G lanes (2, 4 or 8; ~0 does not count), over the groups of the wave the largest (0: none)
 template <int G>
-__device__ __forceinline__ uint32_t group_umin(uint32_t v) {
+__device__ __forceinline__ uint32_t wave_max_of_group_min(uint32_t v) {
   auto mv = [](uint32_t x, auto ctrl) { return (uint32_t)__builtin_amdgcn_update_dpp(0, (int)x, decltype(ctrl)::value, 0xf, 0xf, true); };
-  v = min(v, mv(v, std::integral_constant<int, 0xB1>{}));                        // quad_perm: neighbours
-  if constexpr (G >= 4) v = min(v, mv(v, std::integral_constant<int, 0x4E>{}));  // quad_perm: pairs
-  if constexpr (G >= 8) v = min(v, mv(v, std::integral_constant<int, 0x141>{})); // row_half_mirror: fours
-  return v;
+  auto close = [&](auto last) { if constexpr (decltype(last)::value) v = v == 0xffffffffu ? 0u : v; };
+  uint32_t o = mv(v, std::integral_constant<int, 0xB1>{});    // quad_perm: neighbours
+  v = min(v, o);
+  close(std::bool_constant<G == 2>{});
+  o = mv(v, std::integral_constant<int, 0x4E>{});             // quad_perm: pairs
+  v = G >= 4 ? min(v, o) : max(v, o);
+  close(std::bool_constant<G == 4>{});
+  o = mv(v, std::integral_constant<int, 0x141>{});            // row_half_mirror: fours
+  v = G >= 8 ? min(v, o) : max(v, o);
+  close(std::bool_constant<G == 8>{});
+  v = max(v, mv(v, std::integral_constant<int, 0x140>{}));    // row_mirror: eights
+  v = max(v, (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x142, 0xa, 0xf, false));   // row_bcast:15 into rows 1 and 3
+  v = max(v, (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x143, 0xc, 0xf, false));   // row_bcast:31 into rows 2 and 3
+  return (uint32_t)__builtin_amdgcn_readlane((int)v, 63);
 }
-
 // Reduction over each row of 16 lanes, in all of them
 template <class Op, class T>
 __device__ __forceinline__ void row_all(Op op, T& v) {
@@ -150,25 +159,24 @@ __global__ __launch_bounds__(NT, (KPT >= 1 && KPT <= 24) ? (NT == 512 ? 6 : 4) :
     // the bulk of the row, see score_bins.h (threads without a score stay out of it)
     constexpr int G = score_group(KPT);
     const bool any = kmin <= kmax;
-    const uint32_t gmax = group_umin<G>(any ? kmax : 0xffffffffu), gmin = ~group_umin<G>(any ? ~kmin : 0xffffffffu);
-    kmax = gmax == 0xffffffffu ? 0u : gmax;
-    kmin = gmin == 0u ? 0xffffffffu : gmin;
+    kmax = wave_max_of_group_min<G>(any ? kmax : 0xffffffffu);
+    kmin = ~wave_max_of_group_min<G>(any ? ~kmin : 0xffffffffu);
+  } else {
+    kmax = wave_umax(kmax);
+    kmin = wave_umin(kmin);
   }
-  kmax = wave_umax(kmax);
-  kmin = wave_umin(kmin);
   if (lane == 0) { wgt[wave] = (int)kmax; weq[wave] = (int)kmin; }
   if (tid == 0) ncand = 0;
   __syncthreads();
-  float narrow = 0.f, wide = 0.f;   // UNION: of the waves' bulks
+  float narrow = 0.f;   // UNION: width of the narrowest bulk of a wave
   if constexpr (UNION) {
     static_assert(NW == 16, "one wave per lane of a row of 16");
     kmax = (uint32_t)wgt[lane & 15];
     kmin = (uint32_t)weq[lane & 15];
-    wide = score_width(kmin, kmax);
-    narrow = wide > 0.f && ((lane & 15) + 1) * KPT * 64 <= n ? wide : INFINITY;   // (the last wave's may be that of a few columns)
+    const float width = score_width(kmin, kmax);
+    narrow = width > 0.f && ((lane & 15) + 1) * KPT * 64 <= n ? width : INFINITY;   // (the last wave's may be that of a few columns)
     row_all([](uint32_t a, uint32_t b) { return max(a, b); }, kmax);
     row_all([](uint32_t a, uint32_t b) { return min(a, b); }, kmin);
-    row_all([](float a, float b) { return fmaxf(a, b); }, wide);
     row_all([](float a, float b) { return fminf(a, b); }, narrow);
     kmax = __builtin_amdgcn_readfirstlane(kmax);
     kmin = __builtin_amdgcn_readfirstlane(kmin);
@@ -283,7 +291,7 @@ __global__ __launch_bounds__(NT, (KPT >= 1 && KPT <= 24) ? (NT == 512 ? 6 : 4) :
   bool found = false, first = true;
   if constexpr (UNION) {
     ScoreBins bins;
-    if (score_bins(kmin, kmax, narrow, wide, bins)) {
+    if (score_bins(kmin, kmax, narrow, bins)) {
 #pragma unroll
       for (int c = 0; c < KPT; c++) bin[c] = score_bin(bins, keys[c]);
 #pragma unroll

@@ -9,8 +9,8 @@
 // where it comes with one in every thread of a group; of normal scores it is 1.5 .. 2 standard deviations each way.  Scores
 // spread over many orders of magnitude have no such range: it differs by as much between waves, and the digits are as good
 // as bins can be there.  32 rows of 10521 scores, 1792 kept; digits only / bins from the smallest to the largest / these, us:
-// normal 16.0 / 12.2 / 12.1, one score 100 times the others 16.0 / 24.1 / 12.1, two at +-1e30 16.0 / 28.4 / 12.1, a hundredth
-// of them far 16.1 / 24.1 / 12.1, a Cauchy distribution 20.0 / 31.1 / 12.2, exp(12 |x|) 13.6 / 26.0 / 15.0.
+// normal 16.0 / 12.1 / 11.9, one score 100 times the others 16.0 / 24.1 / 12.0, two at +-1e30 16.0 / 28.3 / 11.9, a hundredth
+// of them far 16.1 / 24.1 / 11.9, a Cauchy distribution 20.0 / 31.1 / 12.3, exp(12 |x|) 13.6 / 26.0 / 14.8.
 // Arithmetic shared by the device code and by a host-side test.
 #pragma once
 #include <stdint.h>
@@ -44,14 +44,14 @@ LVAR_HD float score_width(uint32_t lo, uint32_t hi) {
   return KEY_NEG_INF < lo && lo < hi && hi < KEY_POS_INF ? score_of_key(hi) - score_of_key(lo) : 0.f;
 }
 
-// Bins for a bulk of [lo, hi] whose waves' widths are `narrow` (of those that have one) to `wide`, or false where it is
-// empty, not finite, spread over orders of magnitude, or so narrow that 1 / width is not finite.
-LVAR_HD bool score_bins(uint32_t lo, uint32_t hi, float narrow, float wide, ScoreBins& b) {
+// Bins for a bulk of [lo, hi] whose narrowest full wave has a bulk of width `narrow`, or false where it is empty, not finite,
+// spread over orders of magnitude, or so narrow that 1 / width is not finite.
+LVAR_HD bool score_bins(uint32_t lo, uint32_t hi, float narrow, ScoreBins& b) {
   const float width = score_width(lo, hi);
   union { float f; uint32_t u; } range;
   range.f = 2.f * width;
   if (range.u <= 0x08000000u || range.u >= 0x7f800000u) return false;   // 2^-111; infinite
-  if (!(wide <= 12.f * narrow)) return false;   // (full waves of normal scores differ by up to 5, of exp(12 |x|) by 13 and more)
+  if (!(width <= 24.f * narrow)) return false;   // (of normal scores up to 6 times, with a mean that rises by 20 deviations 12, of exp(12 |x|) 27 and more)
   b.x0 = 0.5f * score_of_key(lo) + 0.5f * score_of_key(hi) - 0.5f * range.f;
   b.xs = (float)(SCORE_BINS - 1) / range.f;
   return true;

@@ -56,16 +56,15 @@ static void bulk(const std::vector<uint32_t>& keys, int t0, int t1, uint32_t& lo
 
 static bool row_bins(const std::vector<uint32_t>& keys, ScoreBins& b) {
   uint32_t lo, hi;
-  float narrow = std::numeric_limits<float>::infinity(), wide = 0.f;
+  float narrow = std::numeric_limits<float>::infinity();
   const int n = (int)keys.size(), kpt = (n + THREADS - 1) / THREADS;
   for (int t = 0; t < THREADS; t += 64) {
     bulk(keys, t, t + 64, lo, hi);
     const float w = score_width(lo, hi);
     if (w > 0.f && (t / 64 + 1) * kpt * 64 <= n) narrow = std::min(narrow, w);
-    wide = std::max(wide, w);
   }
   bulk(keys, 0, THREADS, lo, hi);
-  return score_bins(lo, hi, narrow, wide, b);
+  return score_bins(lo, hi, narrow, b);
 }
 
 static std::vector<float> scores(const std::string& kind, int n, unsigned seed) {
@@ -113,7 +112,7 @@ int main() {
   const float ranges[][2] = {{-1.f, 1.f}, {0.f, 1e-3f}, {-1e30f, 2e30f}, {5.f, 5.001f}, {-1e-30f, 1e-30f}};
   for (auto& r : ranges) {
     ScoreBins b;
-    if (!score_bins(key_of(r[0]), key_of(r[1]), 1.f, 1.f, b)) { printf("no bins for %g .. %g\n", r[0], r[1]); return 1; }
+    if (!score_bins(key_of(r[0]), key_of(r[1]), 1e38f, b)) { printf("no bins for %g .. %g\n", r[0], r[1]); return 1; }
     int last = 0;
     for (uint32_t k : edge) {
       const int at = score_bin(b, k);
@@ -123,12 +122,12 @@ int main() {
     }
   }
   ScoreBins b;
-  if (score_bins(key_of(1.f), key_of(1.f), 1.f, 1.f, b) || score_bins(0xffffffffu, 0u, 1.f, 1.f, b) || score_bins(key_of(0.f), KEY_POS_INF, 1.f, 1.f, b) ||
-      score_bins(key_of(-3e38f), key_of(3e38f), 1.f, 1.f, b) || score_bins(key_of(1e-42f), key_of(2e-42f), 1.f, 1.f, b)) { printf("bins without a bulk\n"); return 1; }
+  if (score_bins(key_of(1.f), key_of(1.f), 1e38f, b) || score_bins(0xffffffffu, 0u, 1e38f, b) || score_bins(key_of(0.f), KEY_POS_INF, 1e38f, b) ||
+      score_bins(key_of(-3e38f), key_of(3e38f), 1e38f, b) || score_bins(key_of(1e-42f), key_of(2e-42f), 1e38f, b)) { printf("bins without a bulk\n"); return 1; }
   // candidates of the threshold
   // every remainder of the last wave: a row whose bulk is that of normal scores has bins
-  for (const char* kind : {"plain", "holes", "pooled"})
-    for (int n = 200; n <= 16384; n += n < 2000 ? 1 : 7) {
+  for (const char* kind : {"plain", "holes", "pooled", "trend"})
+    for (int n = kind[0] == 't' ? 1025 : 200; n <= 16384; n += n < 2000 ? 1 : 7) {
       const std::vector<float> x = scores(kind, n, n);
       std::vector<uint32_t> keys(n);
       for (int j = 0; j < n; j++) keys[j] = key_of(x[j]);
