@@ -358,7 +358,7 @@ def run_hbm_workload(args, dev, wl):
         win = torch.randint(Lk - Lq, Lk, (B, H, W), generator=g).to(dev)
         fn = lambda: ops.window_key_scores(q, k, win, 5, "avgpool")
         nbytes = B * H * (Lk * d * 2 + Lk * 4 + W * (d * 2 + 8))
-        kernel, unit_desc = "window_scores_kernel<128>", f"{B * H} (batch,head) x {Lk} keys, {W} window queries, avg pool 5"
+        kernel, unit_desc = "window_scores_kernel<128, 512>", f"{B * H} (batch,head) x {Lk} keys, {W} window queries, avg pool 5"
         if not args.no_cpu_baseline:
             torch.set_num_threads(os.cpu_count() or 1)
             qc, kc, wc = q.cpu(), k.cpu(), win.cpu()

@@ -128,7 +128,8 @@ __device__ __forceinline__ void attn_item(const AttnParams& p, char* smem, const
   int avail = 0;   // entries of the list row from `list` on (token lists)
   // Token lists formed from another scale's (see AttnParams): the waves that read the list take the entries straight from the
   // two rows they come from, so that no launch writes the lists and the count is not waited for.  Step at the last scale with
-  // 20 % of the keys and a local run, B2 H16 d128: 30 x 30 32.8 -> 29.7 us, 48 x 48 84.5 -> 81.4, 64 x 64 169.3 -> 164.5.
+  // 20 % of the keys and a local run, B2 H16 d128: 30 x 30 32.8 -> 29.7 us, 48 x 48 84.5 -> 81.4; the whole 64 x 64
+  // step 178.6 -> 176.2.
   constexpr bool REMAP = !SK && reads_remapped<D, NWAVES, MODE, NPROD>;
   int n_src = 0x7fffffff;             // entries from `list`, the others from `local`:
   const int32_t* local = nullptr;     // low words of 64-bit entries
@@ -1043,7 +1044,11 @@ static bool third_workgroup(int total_wg) { return total_wg > 2 * device_cus(); 
 // tile beside its MFMAs are fills.  Without / with four fetch waves, B2 H16 d128: 144 x 265 9.8 / 9.0 us, 576 x 1497 27.3 /
 // 24.4, 1024 x 2521 (256 workgroups) 46.5 / 44.3; B1 H4 4096 x 10521 153 / 134; d64 B8 H16 256 x 680 12.2 / 11.4; lists
 // alike (B1 H16 784 x 1924 at 25 % 20.6 / 18.4).  With a second workgroup on a compute unit there are no empty slots, and at
-// head_dim 256 a wave fills its SIMD.  Same bits.
+// head_dim 256 a wave fills its SIMD.  Same bits.  A workgroup with fetch waves has its compute unit to itself, so launches
+// on two streams that together need more than one per compute unit no longer share any: a pair of calls, without / with,
+// B1 d128 1024 x 2521: 2 x 128 workgroups 49.1 / 45.0 us, 2 x 160 (576 x 1497) 56.8 / 52.3, 2 x 192 67.1 / 68.2, 2 x 224 72.7 / 78.9,
+// 2 x 256 78.9 / 88.0 (one stream 50.2 / 46.0); d64 2 x 256 49.0 / 59.0 (31.8 / 30.0).  A launch cannot know what runs beside it,
+// and one stream is the usual case.
 static bool fetch_waves(int total_wg) { return total_wg <= device_cus(); }
 
 template <int D, int NWAVES, int MODE, bool ACCUM, bool LSE_ONLY, int NPROD = (MODE == MODE_GATHER && NWAVES == 8) ? 2 : 0>

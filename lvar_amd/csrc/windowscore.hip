@@ -15,8 +15,10 @@ constexpr int WS_T = 512;      // threads per workgroup
 // of round trips inside a workgroup is the time; 32 x 265 keys, 16 window queries 6.3 -> 4.7 us, 4 x 10521 7.1 -> 6.6).
 // 512 threads with four rows in flight each (62 registers, four workgroups per compute unit) against 256 with eight: twice
 // the window rows per round trip and half the rows per lane: 32 x 10521 keys, d128, 256 window queries 20.6 -> 18.3 us
-// (4.9 TB/s), 72 x 10521 36.1 -> 33.7 (5.9), 32 x 4121 12.8 -> 9.8.  Requesting key rows ahead of the window queries, or a
-// batch ahead of the dots, costs registers and with them resident workgroups: 21 .. 25 us.
+// (4.9 TB/s), 72 x 10521 36.1 -> 33.7 (5.9), 32 x 4121 12.8 -> 9.8.  The window rows are added up in twice as many partial
+// sums of half as many rows each, in fp32 (another order than with 256 threads: rms error of a score +0.2 % at most).
+// Requesting key rows ahead of the window queries, or a batch ahead of the dots, costs registers and with them resident
+// workgroups: 21 .. 25 us.
 template <int D, int KEYS>
 __global__ __launch_bounds__(WS_T) void window_scores_kernel(const WinScoreParams p) {
   constexpr int LPR = D / 8;          // lanes that share one key row (8 bf16 = 16 bytes each)
