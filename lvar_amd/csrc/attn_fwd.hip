@@ -232,7 +232,14 @@ __device__ __forceinline__ void attn_item(const AttnParams& p, char* smem, const
     // Written as inline assembly so that the compiler does not serialise later LDS reads of the
     // OTHER buffers behind these fills; completion is awaited with vmcnt(0) before the barrier.
     // issue_slot: the s-th of the SLOTS fill instructions this wave contributes to a tile; issue: all of them.
-    auto issue_slot = [&](const i32x4& rsrc, int srb, bool is_v, const int (&rows)[NR], uint32_t dst, int s) {
+    // `left`: std::true_type, or (in a scalar register) the number of tiles from the current one on, and nothing is fetched
+    // where that is less than three.  The skip is a branch inside the assembly: one that the compiler sees ends its basic
+    // block, and it then moves the softmax instructions of the steps before, whose results are only used later, behind it
+    // (every other tile ran its 16 QK MFMAs with no vector work beside them).  With two waves per SIMD the other wave covers
+    // most of that: 4096 x 10521 in lists of 25 % 183.9 -> 182.5 us, d128 2304 x 6425 in 64 x 64 blocks 106.3 -> 104.8; with one,
+    // d256 1600 x 4121 220.9 -> 217.3.
+    auto issue_slot = [&](const i32x4& rsrc, int srb, bool is_v, const int (&rows)[NR], uint32_t dst, int s, auto left) {
+      constexpr bool ALWAYS = std::is_same_v<decltype(left), std::true_type>;
       const int i = fwave + s * FW;
       if (!((NI % FW == 0) || i < NI)) return;
       const uint32_t m0v = dst + i * 1024;
@@ -248,6 +255,19 @@ __device__ __forceinline__ void attn_item(const AttnParams& p, char* smem, const
         const int trow0 = (fwave + (s % CONST_PER) * FW) * RPI + lrow;
         const int voff = trow0 * srb + ((lcs ^ (is_v ? Swz<D>::fv(trow0) : Swz<D>::fk(trow0))) << 4);
         const int soff = (row0 + (s / CONST_PER) * CONST_PER * FW * RPI) * srb;
+        if constexpr (!ALWAYS) {
+          asm volatile(
+              "s_cmp_lt_i32 %4, 3\n\t"
+              "s_cbranch_scc1 .Lno_fill%=\n\t"
+              "s_mov_b32 m0, %0\n\t"
+              "s_nop 0\n\t"
+              "buffer_load_dwordx4 %1, %2, %3 offen lds\n"
+              ".Lno_fill%=:"
+              :
+              : "s"(m0v), "v"(voff), "s"(rsrc), "s"(soff), "s"(left)
+              : "memory", "scc");
+          return;
+        }
         asm volatile(
             "s_mov_b32 m0, %0\n\t"
             "s_nop 0\n\t"
@@ -277,7 +297,7 @@ __device__ __forceinline__ void attn_item(const AttnParams& p, char* smem, const
     };
     auto issue = [&](const i32x4& rsrc, int srb, bool is_v, const int (&rows)[NR], uint32_t dst) {
 #pragma unroll
-      for (int s = 0; s < SLOTS; s++) issue_slot(rsrc, srb, is_v, rows, dst, s);
+      for (int s = 0; s < SLOTS; s++) issue_slot(rsrc, srb, is_v, rows, dst, s, std::true_type{});
     };
 
     // valid keys of tile t of a token list (only the last tile can be ragged)
@@ -497,14 +517,14 @@ __device__ __forceinline__ void attn_item(const AttnParams& p, char* smem, const
       constexpr int NQK_ = 2 * KS;
       constexpr int NFILL = NPROD ? 0 : (LSE_ONLY ? SLOTS : 2 * SLOTS);
       constexpr int FSTRIDE = (CONST_OFF && NFILL > 0 && NFILL <= NQK_) ? NQK_ / NFILL : 0;
-      const bool fill_k = t + 2 < T;
+      const int left = __builtin_amdgcn_readfirstlane(T - t);   // tiles from this one on; K(t+2) is only fetched where there is one
       auto fill_step = [&](auto jc) {
         constexpr int j = decltype(jc)::value;
         if constexpr (FSTRIDE > 0) {
           if constexpr (j % FSTRIDE == 0 && j / FSTRIDE < NFILL) {
             constexpr int f = j / FSTRIDE;
-            if constexpr (!LSE_ONLY && f < SLOTS) issue_slot(vrsrc, v_srb, true, rows_v, lds0 + (3 - PAR) * TILE, f);
-            else if (fill_k) issue_slot(krsrc, k_srb, false, rows_k, lds0 + PAR * TILE, LSE_ONLY ? f : f - SLOTS);
+            if constexpr (!LSE_ONLY && f < SLOTS) issue_slot(vrsrc, v_srb, true, rows_v, lds0 + (3 - PAR) * TILE, f, std::true_type{});
+            else issue_slot(krsrc, k_srb, false, rows_k, lds0 + PAR * TILE, LSE_ONLY ? f : f - SLOTS, left);
           }
         }
       };
@@ -513,7 +533,7 @@ __device__ __forceinline__ void attn_item(const AttnParams& p, char* smem, const
       } else {
         if constexpr (!NPROD && FSTRIDE == 0) {
           if (!LSE_ONLY) issue(vrsrc, v_srb, true, rows_v, lds0 + (3 - PAR) * TILE);
-          if (fill_k) issue(krsrc, k_srb, false, rows_k, lds0 + PAR * TILE);
+          if (left > 2) issue(krsrc, k_srb, false, rows_k, lds0 + PAR * TILE);
         }
         if (t + 3 < T) finish_rows(t + 3, raw, rows_n, nv3);
         if (t + 4 < T) prefetch_raw(t + 4, raw);
