@@ -87,6 +87,13 @@ struct SkCtx {
   int tile_units;   // units of the whole tile
 };
 
+// Wait until at most N of this wave's global reads and LDS fills are outstanding (they complete in order)
+template <int N>
+__device__ __forceinline__ void wait_fills() {
+  static_assert(N < 64, "six bits of the counter");
+  __builtin_amdgcn_s_waitcnt(0x0f70 | (N & 15) | ((N >> 4) << 14));
+}
+
 // One query tile w (or, in a balanced launch, the units [u0, u1) of its tile list; `whole` = all of them).
 template <int D, int NWAVES, int MODE, bool ACCUM, bool LSE_ONLY, bool SK, int NPROD, bool IDLE>
 __device__ __forceinline__ void attn_item(const AttnParams& p, char* smem, const int w, const int bh, const int qt,
@@ -300,6 +307,15 @@ __device__ __forceinline__ void attn_item(const AttnParams& p, char* smem, const
       for (int s = 0; s < SLOTS; s++) issue_slot(rsrc, srb, is_v, rows, dst, s, std::true_type{});
     };
 
+    // K(0), the oldest of the fills of the prologue, has landed: S(0) does not need V(0) and K(1), which are waited for
+    // after it.  (Every filling wave issues at least NI / FW fills per tile.)  B2 H16 d128: 144 x 265 9.12 -> 8.83 us, 576 x 1497
+    // 24.4 -> 24.2, sink + window lists at 48 x 48 57.0 -> 56.3; d64 B8 256 x 680 11.4 -> 11.3.
+    auto wait_first = [&]() {
+      constexpr int PER = NI / FW;
+      if (T > 1) wait_fills<LSE_ONLY ? PER : 2 * PER>();
+      else wait_fills<LSE_ONLY ? 0 : PER>();
+    };
+
     // valid keys of tile t of a token list (only the last tile can be ragged)
     auto nvalid_gather = [&](int t) { return max(0, min(64, count - (t << 6))); };
 
@@ -339,8 +355,9 @@ __device__ __forceinline__ void attn_item(const AttnParams& p, char* smem, const
         if (!LSE_ONLY) issue(vrsrc, v_srb, true, rows0, lds0 + 2 * TILE);
         if (T > 1) issue(krsrc, k_srb, false, rows_v, lds0 + TILE);
       }
-      __builtin_amdgcn_s_waitcnt(0x0f70);
+      wait_first();
       __syncthreads();
+      wait_fills<0>();
       __syncthreads();   // the computing waves have read K(0): its buffer may be refilled
       for (int t = 0; t + 1 < T; t++) {
         if (fills) {
@@ -350,7 +367,7 @@ __device__ __forceinline__ void attn_item(const AttnParams& p, char* smem, const
           if (t + 3 < T) finish_rows(t + 3, raw, rows_n, nv_unused);
           if (t + 4 < T) prefetch_raw(t + 4, raw);
         }
-        __builtin_amdgcn_s_waitcnt(0x0f70);
+        wait_fills<0>();
         __syncthreads();
 #pragma unroll
         for (int s = 0; s < NR; s++) { rows_v[s] = rows_k[s]; rows_k[s] = rows_n[s]; }
@@ -491,12 +508,13 @@ __device__ __forceinline__ void attn_item(const AttnParams& p, char* smem, const
         if (T > 1) issue(krsrc, k_srb, false, rows_v, lds0 + TILE);
       }
     }
-    __builtin_amdgcn_s_waitcnt(0x0f70);  // vmcnt(0): this wave's LDS fills have landed
+    if constexpr (NPROD) wait_fills<0>(); else wait_first();
     __syncthreads();
     f32x16 sa0, sa1, sb0, sb1;
     qk_tile(smem, sa0, sa1);
     // K(2) is fetched into the buffer of K(0) at the top of the first iteration: every wave must have read
-    // K(0) before any wave issues that fill
+    // K(0) before any wave issues that fill; and V(0) and K(1) have landed
+    wait_fills<0>();
     __syncthreads();
     if (nv0 < 64) mask_tile(sa0, sa1, nv0);
     rescale_check(max_tile(sa0, sa1));
@@ -641,7 +659,7 @@ __device__ __forceinline__ void attn_item(const AttnParams& p, char* smem, const
       }
       lsum += la + lb;
       const float mx = xhalf_max(fmaxf(ma, mb));
-      __builtin_amdgcn_s_waitcnt(0x0f70);
+      wait_fills<0>();
       __syncthreads();
       rescale_check(mx);
       nv0 = nv1; nv1 = nv2; nv2 = nv3;
@@ -717,7 +735,7 @@ __device__ __forceinline__ void attn_item(const AttnParams& p, char* smem, const
         put1(st + 128 * NCOMP, m_true);
       }
       __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");   // compiler ordering only
-      __builtin_amdgcn_s_waitcnt(0x0f70);                        // vmcnt(0): this wave's stores have been written through
+      wait_fills<0>();                                           // this wave's stores have been written through
       __syncthreads();
       volatile int* flag = (volatile int*)smem;   // the K/V buffers are idle from here on
       if (tid == 0) {
