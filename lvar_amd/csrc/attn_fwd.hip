@@ -2,7 +2,7 @@
 // (flex BlockMask layout) and token-list (column-sparse, gathered keys) variants.
 //
 // Work decomposition
-//   workgroup  = NWAVES waves, 32 query rows per wave, all waves share the K/V tiles in LDS
+//   workgroup  = NWAVES waves, 32 query rows per wave (small launches: per two waves, see PAIR), all share the K/V tiles in LDS
 //                (token lists with 192-row groups: 8 waves = 6 computing waves + 2 waves that only fetch, see NPROD)
 //   wave       = S^T[64 keys x 32 queries] = K_tile . Q^T with 32x32x16 bf16 MFMA (K rows are
 //                the A operand read from LDS, Q^T is the B operand held in registers), so a
@@ -41,6 +41,12 @@ struct ExpSlots {
   }
 };
 
+// The same for the 16 elements of a wave of a pair, over G slots
+template <int G>
+struct HalfSlots {
+  static constexpr int lo(int g) { return g <= 0 ? 0 : g >= G ? 16 : g * 16 / G; }
+};
+
 // f(integral_constant<int, i>) for i = LO .. HI-1, unrolled at compile time
 template <int LO, int HI, class F>
 __device__ __forceinline__ void static_for(F&& f) {
@@ -71,10 +77,12 @@ struct Swz {
 template <int D, int NWAVES, int MODE, int NPROD>
 constexpr bool reads_remapped = MODE == MODE_GATHER && (NPROD > 0 || (D == 64 && NWAVES == 3));
 
-// LDS of a workgroup: K and V buffers; the epilogue's transpose buffer of eight computing waves is larger
-template <int D, int NCOMP, int MODE>
+// LDS of a workgroup: K and V buffers; the epilogue's transpose buffer of eight computing waves is larger.  Pairs of waves: behind
+// the K and V buffers, two deep, every computing wave's half of P and one float per lane.
+template <int D, int NCOMP, int MODE, bool PAIR = false>
 constexpr int attn_lds_bytes() {
   const int bufs = 4 * 64 * D * 2, epi = NCOMP * 32 * (D * 2 + 16);
+  if (PAIR) return bufs + 2 * NCOMP * (2048 + 256);
   return (MODE == MODE_BLOCK && epi > bufs) ? epi : bufs;
 }
 
@@ -94,8 +102,21 @@ __device__ __forceinline__ void wait_fills() {
   __builtin_amdgcn_s_waitcnt(0x0f70 | (N & 15) | ((N >> 4) << 14));
 }
 
+// x, never fused with what is added to it: whether the compiler would depends on the instance, and all have the same bits
+__device__ __forceinline__ float rounded(float x) {
+  asm volatile("" : "+v"(x));
+  return x;
+}
+
 // One query tile w (or, in a balanced launch, the units [u0, u1) of its tile list; `whole` = all of them).
-template <int D, int NWAVES, int MODE, bool ACCUM, bool LSE_ONLY, bool SK, int NPROD, bool IDLE>
+//
+// PAIR: two waves share 32 query rows, for launches that leave compute units idle: there a wave is alone on its SIMD and its chain
+// of instructions per tile is the time of a tile (1800 .. 1900 cycles, 1066 of them MFMAs, however they are arranged).  Wave
+// `half` of a pair forms S^T of keys 32 * half .. +31 of every tile, their softmax and their half of P, and accumulates columns
+// half * D/2 .. of O over all 64 keys: half of the MFMAs and of the vector work each (1400 cycles).  P and the row maxima pass
+// between the two through LDS behind the barrier that a tile has anyway: O is one tile behind S, so nothing in an iteration waits
+// for anything else in it.  The order of every sum is the same as without: same bits.
+template <int D, int NWAVES, int MODE, bool ACCUM, bool LSE_ONLY, bool SK, int NPROD, bool IDLE, bool PAIR = false>
 __device__ __forceinline__ void attn_item(const AttnParams& p, char* smem, const int w, const int bh, const int qt,
                                           const int u0, const int u1, const bool whole, const SkCtx& sk) {
   // NPROD: the last waves only fetch -- they read the list, form the addresses and issue every K/V fill -- and the
@@ -104,8 +125,11 @@ __device__ __forceinline__ void attn_item(const AttnParams& p, char* smem, const
   // CU: four and four (see fetch_waves).  Everywhere else all waves do both.
   constexpr int NCOMP = NWAVES - NPROD;     // computing waves, 32 query rows each
   constexpr int FW = NPROD ? NPROD : NWAVES;  // waves that issue the fills
-  constexpr int WGROWS = NCOMP * 32;
+  constexpr int RB = PAIR ? NCOMP / 2 : NCOMP;   // 32-row blocks
+  constexpr int WGROWS = RB * 32;
   constexpr int KS = D / 16, MTD = D / 32;
+  constexpr int MTW = PAIR ? MTD / 2 : MTD;      // 32-column blocks of O that a wave accumulates
+  static_assert(!PAIR || (MODE == MODE_BLOCK && NPROD > 0 && !ACCUM && !LSE_ONLY && !SK), "pairs: dense and block lists with fetch waves");
   constexpr int ROWB = Swz<D>::ROWB, CPR = Swz<D>::CPR;
   constexpr int RPI = 1024 / ROWB;          // rows filled by one 64-lane x 16 B load
   constexpr int NI = 64 / RPI;              // loads per 64-row tile
@@ -115,13 +139,15 @@ __device__ __forceinline__ void attn_item(const AttnParams& p, char* smem, const
   constexpr bool CONST_OFF = MODE == MODE_BLOCK && ((FW * RPI) % 16 == 0 || 16 % (FW * RPI) == 0) && NI % FW == 0;
   constexpr int CONST_PER = (FW * RPI) >= 16 ? 1 : 16 / (FW * RPI);
   constexpr int OSTR = D * 2 + 16;  // epilogue transpose buffer row stride (bytes)
-  static_assert(NCOMP * 32 * OSTR <= attn_lds_bytes<D, NCOMP, MODE>(), "the epilogue buffer must fit");
+  static_assert(RB * 32 * OSTR <= attn_lds_bytes<D, NCOMP, MODE, PAIR>(), "the epilogue buffer must fit");
   // LDS map: K buffers at 0 and TILE, V buffers at 2*TILE and 3*TILE
 
   const int b = bh / p.H, h = bh - b * p.H;
   const int tid = __builtin_amdgcn_workitem_id_x(), lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int hh = lane >> 5, r = lane & 31;
+  const int half = (PAIR && wave >= RB) ? 1 : 0;   // which wave of a pair
+  const int rblk = PAIR ? wave - half * RB : wave; // the block of 32 rows that it works on (fetch waves: no matter)
   const int fwave = NPROD ? wave - NCOMP : wave;   // index among the filling waves (negative: this wave does not fill)
   const int q0 = qt * WGROWS;
   const int g = q0 / p.group_rows;
@@ -174,12 +200,13 @@ __device__ __forceinline__ void attn_item(const AttnParams& p, char* smem, const
   const int sub_shift = identity ? 0 : p.sub_shift;
 
   // accumulators and softmax state (one query column per lane pair l, l^32)
-  f32x16 oacc[MTD];
+  f32x16 oacc[MTW];
 #pragma unroll
-  for (int m = 0; m < MTD; m++)
+  for (int m = 0; m < MTW; m++)
 #pragma unroll
     for (int i = 0; i < 16; i++) oacc[m][i] = 0.f;
-  float m_ref = NEG_BIG, m_true = -INFINITY, lsum = 0.f;
+  float m_ref = NEG_BIG, m_true = -INFINITY;
+  float lsum[2] = {0.f, 0.f};   // row sums of keys 0 .. 31 and of keys 32 .. 63 of every tile (what the two waves of a pair hold)
   const float c = p.c;
 
   if (T > 0) do {
@@ -333,14 +360,14 @@ __device__ __forceinline__ void attn_item(const AttnParams& p, char* smem, const
     // meets the barriers, so the waves with rows have the matrix cores and the LDS reads to themselves, and a launch at
     // the power limit keeps its clock (dense B2 H16 d128, 1600 x 4121 in 256-row tiles, an eighth of them padding: 111.7 ->
     // 106.5 us).  Where no wave has that role otherwise (IDLE, see idle_waves_pay) it is an instance of its own.
-    const bool no_rows = !SK && (NPROD > 0 || IDLE) && q0 + wave * 32 >= p.Lq;
+    const bool no_rows = !SK && (NPROD > 0 || IDLE) && q0 + rblk * 32 >= p.Lq;
     if ((NPROD > 0 && wave >= NCOMP) || no_rows) {
       // ---- fetch waves: the fill schedule of the loop below and nothing else; one barrier per tile ----
       const bool fills = !NPROD || wave >= NCOMP;
-      int rows_v[NR], rows_k[NR], rows_n[NR], raw[NR], rows0[NR];
+      int rows_u[NR], rows_v[NR], rows_k[NR], rows_n[NR], raw[NR], rows0[NR];   // rows_u: tile t (pairs)
       int nv_unused;
 #pragma unroll
-      for (int s = 0; s < NR; s++) { rows_v[s] = 0; rows_k[s] = 0; rows_n[s] = 0; raw[s] = 0; }
+      for (int s = 0; s < NR; s++) { rows_u[s] = 0; rows_v[s] = 0; rows_k[s] = 0; rows_n[s] = 0; raw[s] = 0; }
       // the list entries of the first four tiles are requested together (one memory round trip, not one per tile)
       int raw0[NR], raw1[NR], raw2[NR];
       if (fills) {
@@ -362,7 +389,11 @@ __device__ __forceinline__ void attn_item(const AttnParams& p, char* smem, const
       for (int t = 0; t + 1 < T; t++) {
         if (fills) {
           const int par = t & 1;
-          if (!LSE_ONLY) issue(vrsrc, v_srb, true, rows_v, lds0 + (3 - par) * TILE);
+          if constexpr (PAIR) {
+            if (t > 0) issue(vrsrc, v_srb, true, rows_u, lds0 + (2 + par) * TILE);
+          } else if (!LSE_ONLY) {
+            issue(vrsrc, v_srb, true, rows_v, lds0 + (3 - par) * TILE);
+          }
           if (t + 2 < T) issue(krsrc, k_srb, false, rows_k, lds0 + par * TILE);
           if (t + 3 < T) finish_rows(t + 3, raw, rows_n, nv_unused);
           if (t + 4 < T) prefetch_raw(t + 4, raw);
@@ -370,7 +401,13 @@ __device__ __forceinline__ void attn_item(const AttnParams& p, char* smem, const
         wait_fills<0>();
         __syncthreads();
 #pragma unroll
-        for (int s = 0; s < NR; s++) { rows_v[s] = rows_k[s]; rows_k[s] = rows_n[s]; }
+        for (int s = 0; s < NR; s++) { rows_u[s] = rows_v[s]; rows_v[s] = rows_k[s]; rows_k[s] = rows_n[s]; }
+      }
+      if constexpr (PAIR) {   // V of the last tile
+        const int last = __builtin_amdgcn_readfirstlane(T - 1);
+        if (fills && last > 0) issue(vrsrc, v_srb, true, rows_u, lds0 + (2 + (last & 1)) * TILE);
+        wait_fills<0>();
+        __syncthreads();
       }
       __syncthreads();   // the one after the last tile
       if (SK) break;     // a balanced launch has more barriers to meet below
@@ -378,7 +415,7 @@ __device__ __forceinline__ void attn_item(const AttnParams& p, char* smem, const
     }
 
     // Q^T fragments stay in registers for the whole key loop
-    const int qrow = min(q0 + wave * 32 + r, p.Lq - 1);
+    const int qrow = min(q0 + rblk * 32 + r, p.Lq - 1);
     const bf16_t* qp = p.q + b * p.q_sb + h * p.q_sh + (int64_t)qrow * p.q_sr + hh * 8;
     bf16x8 qf[KS];
 #pragma unroll
@@ -431,7 +468,8 @@ __device__ __forceinline__ void attn_item(const AttnParams& p, char* smem, const
       if (__builtin_amdgcn_ballot_w64(mt > m_ref + RESCALE_TAU) != 0) {
         const float m_new = fmaxf(m_ref, mt);
         const float alpha = fast_exp2(m_ref - m_new);
-        lsum *= alpha;
+        lsum[0] = rounded(lsum[0] * alpha);
+        lsum[1] = rounded(lsum[1] * alpha);
         if (!LSE_ONLY) {
 #pragma unroll
           for (int m = 0; m < MTD; m++)
@@ -452,7 +490,8 @@ __device__ __forceinline__ void attn_item(const AttnParams& p, char* smem, const
         la += s0[i];
         lb += s1[i];
       }
-      lsum += la + lb;
+      lsum[0] += la;
+      lsum[1] += lb;
       pb[0] = pack8(s0[0], s0[1], s0[2], s0[3], s0[4], s0[5], s0[6], s0[7]);
       pb[1] = pack8(s0[8], s0[9], s0[10], s0[11], s0[12], s0[13], s0[14], s0[15]);
       pb[2] = pack8(s1[0], s1[1], s1[2], s1[3], s1[4], s1[5], s1[6], s1[7]);
@@ -510,6 +549,183 @@ __device__ __forceinline__ void attn_item(const AttnParams& p, char* smem, const
     }
     if constexpr (NPROD) wait_fills<0>(); else wait_first();
     __syncthreads();
+    if constexpr (PAIR) {
+      char* const pbuf = smem + 4 * TILE;                        // [parity][row block][quarter of the keys][lane] x 16 bytes
+      constexpr int PPAR = NCOMP * 2048;                         // bytes of one parity
+      float* const xbuf = (float*)(pbuf + 2 * PPAR);             // [parity][computing wave][lane]
+      const int mate = half ? wave - RB : wave + RB;
+      const int kb_l = kbase_l + half * 32 * ROWB;
+      int vb_l[MTW];
+#pragma unroll
+      for (int m = 0; m < MTW; m++) vb_l[m] = vbase_l ^ ((half * MTW + m) << 6);
+      char* const pmine = pbuf + (rblk * 4 + half * 2) * 1024 + lane * 16;
+      const char* const prow = pbuf + rblk * 4096 + lane * 16;
+      const int tiles = __builtin_amdgcn_readfirstlane(T);
+      f32x16 sa, sb;
+      float mown, alpha = 1.f;
+      bool pend = false;
+      auto kread = [&](const char* kbuf, int j) -> bf16x8 { return *(const bf16x8*)(kbuf + (kb_l ^ (j << 5))); };
+      auto vread = [&](const char* vbuf, int j) -> bf16x8 {
+        const char* a = vbuf + vb_l[j % MTW] + (j / MTW) * 16 * ROWB;
+        bf16x4 lo = lds_read_tr(a);
+        bf16x4 hi = lds_read_tr(a + 8 * ROWB);
+        return __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7);
+      };
+      auto mask_half = [&](f32x16& x, int nvalid) {
+        const int lim = nvalid - 32 * half - 4 * hh;
+#pragma unroll
+        for (int i = 0; i < 16; i++) x[i] = (8 * (i >> 2) + (i & 3) < lim) ? x[i] : -INFINITY;
+      };
+      auto max_half = [&](const f32x16& x) -> float {
+        float a = fmaxf(x[0], x[1]);
+#pragma unroll
+        for (int i = 2; i < 16; i += 2) a = fmaxf(fmaxf(a, x[i]), x[i + 1]);
+        return xhalf_max(a);
+      };
+      // the reference maximum of tile t, from the row maxima of both waves; O lacks P(t-1) V(t-1) yet, so its factor waits (pend)
+      auto settle = [&](float mx) {
+        const float mt = mx * c;
+        m_true = fmaxf(m_true, mt);
+        pend = __builtin_amdgcn_ballot_w64(mt > m_ref + RESCALE_TAU) != 0;
+        if (pend) {
+          const float m_new = fmaxf(m_ref, mt);
+          alpha = fast_exp2(m_ref - m_new);
+          lsum[0] = rounded(lsum[0] * alpha);
+          m_ref = m_new;
+        }
+      };
+      // Iteration t: the matrix cores run S(t+1) = K(t+1) Q^T (this wave's keys; hasqk) and O += P(t-1) V(t-1) (its columns; haspv)
+      // while the vector ALU turns S(t) into P(t); K(t+1) is in K buffer 1 - PAR, V(t-1) in V buffer 1 - PAR.
+      auto half_tile = [&](int t, auto par, auto masked, auto hasqk, auto haspv, f32x16& cs, f32x16& ns) {
+        constexpr int PAR = decltype(par)::value;
+        constexpr bool MASKED = decltype(masked)::value, QK = decltype(hasqk)::value, PV = decltype(haspv)::value;
+        constexpr int NQK = QK ? KS : 0, NPV = PV ? 4 * MTW : 0, NS = NQK + NPV, AHEAD = READ_AHEAD, PAHEAD = 3;
+        // the maximum is settled two MFMAs into the iteration: the other wave's arrives from LDS with the first fragments
+        constexpr int CHK = NS >= 8 ? 2 : 0;
+        using Sch = HalfSlots<(NS - CHK > 3 ? NS - CHK - 2 : 1)>;
+        if constexpr (QK) {
+          if (t + 3 < tiles) finish_rows(t + 3, raw, rows_n, nv3);
+          if (t + 4 < tiles) prefetch_raw(t + 4, raw);
+        }
+        const char* kbuf = smem + (1 - PAR) * TILE;
+        const char* vbuf = smem + (3 - PAR) * TILE;
+        const float mother = xbuf[(PAR * NCOMP + mate) * 64 + lane];
+        bf16x8 frag[NS > 0 ? NS : 1], pb[4];
+        auto operand = [&](auto ic) {
+          constexpr int i = decltype(ic)::value;
+          if constexpr (i < NQK) frag[i] = kread(kbuf, i); else frag[i] = vread(vbuf, i - NQK);
+        };
+        // quarter kb of P(t-1), PAHEAD steps ahead of its first use
+        auto p_operand = [&](auto ic) {
+          constexpr int i = decltype(ic)::value - NQK + PAHEAD;
+#pragma unroll
+          for (int kb = 0; kb < 4; kb++)
+            if (PV && (kb * MTW == i || (decltype(ic)::value == 0 && kb * MTW < i))) pb[kb] = *(const bf16x8*)(prow + (1 - PAR) * PPAR + kb * 1024);
+        };
+        uint32_t pw[8];
+        float ls = 0.f, negm = 0.f, ma = -INFINITY;
+        auto softmax_step = [&](auto gc) {
+          constexpr int g = decltype(gc)::value;
+          static_for<Sch::lo(g - 2), Sch::lo(g - 1)>([&](auto ec) {
+            constexpr int e = decltype(ec)::value;
+            ls += cs[e];
+            if constexpr (e & 1) pw[e >> 1] = pack_bf16(cs[e - 1], cs[e]);
+            if constexpr (e == 7 || e == 15) {
+              const u32x4 u = {pw[(e >> 1) - 3], pw[(e >> 1) - 2], pw[(e >> 1) - 1], pw[e >> 1]};
+              *(u32x4*)(pmine + PAR * PPAR + (e >> 3) * 1024) = u;
+            }
+          });
+          static_for<Sch::lo(g - 1), Sch::lo(g)>([&](auto ec) { constexpr int e = decltype(ec)::value; cs[e] = fast_exp2(cs[e]); });
+          static_for<Sch::lo(g), Sch::lo(g + 1)>([&](auto ec) { constexpr int e = decltype(ec)::value; cs[e] = fmaf(cs[e], c, negm); });
+        };
+        static_for<0, (AHEAD < NS ? AHEAD : NS)>(operand);
+        __builtin_amdgcn_sched_barrier(0);
+        if constexpr (CHK == 0) { settle(fmaxf(mown, mother)); negm = -m_ref; }
+        static_for<0, NS>([&](auto ic) {
+          constexpr int i = decltype(ic)::value;
+          if constexpr (CHK > 0 && i == CHK) { settle(fmaxf(mown, mother)); negm = -m_ref; }
+          if constexpr (i + AHEAD < NS) operand(std::integral_constant<int, i + AHEAD>{});
+          p_operand(ic);
+          if constexpr (i >= NQK) oacc[(i - NQK) % MTW] = mfma32(frag[i], pb[(i - NQK) / MTW], oacc[(i - NQK) % MTW]);
+          else if constexpr (i == 0) ns = mfma32(frag[0], qf[0], f32x16{0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0});
+          else ns = mfma32(frag[i], qf[i], ns);
+          if constexpr (i >= CHK) softmax_step(std::integral_constant<int, i - CHK>{});
+          // row maximum of S(t+1), next to the PV steps
+          if constexpr (QK && PV && i > NQK + 1) {
+            if constexpr (MASKED && i == NQK + 2) mask_half(ns, nv1);
+            constexpr int n = NPV - 2, k = i - NQK - 2;
+#pragma unroll
+            for (int e = k * 8 / n; e < (k + 1) * 8 / n; e++) ma = fmaxf(fmaxf(ma, ns[2 * e]), ns[2 * e + 1]);
+          }
+          __builtin_amdgcn_sched_barrier(0);
+        });
+        static_for<NS - CHK, 16 + 3>(softmax_step);   // what is left of the softmax
+        lsum[0] += ls;
+        if constexpr (PV) {
+          if (pend) {
+#pragma unroll
+            for (int m = 0; m < MTW; m++)
+#pragma unroll
+              for (int i = 0; i < 16; i++) oacc[m][i] *= alpha;
+          }
+        }
+        if constexpr (QK && PV) mown = xhalf_max(ma);
+        if constexpr (QK && !PV) {
+          if constexpr (MASKED) mask_half(ns, nv1);
+          mown = max_half(ns);
+        }
+        xbuf[((1 - PAR) * NCOMP + wave) * 64 + lane] = QK ? mown : lsum[0];   // behind the last tile the row sums change hands
+        __syncthreads();
+        nv1 = nv2; nv2 = nv3;
+#pragma unroll
+        for (int s = 0; s < NR; s++) { rows_v[s] = rows_k[s]; rows_k[s] = rows_n[s]; }
+      };
+#pragma unroll
+      for (int i = 0; i < 16; i++) sa[i] = 0.f;
+#pragma unroll
+      for (int ks = 0; ks < KS; ks++) sa = mfma32(kread(smem, ks), qf[ks], sa);
+      if (nv0 < 64) mask_half(sa, nv0);
+      mown = max_half(sa);
+      xbuf[wave * 64 + lane] = mown;
+      __syncthreads();   // all have read K(0), and V(0) and K(1) have landed
+      using P0 = std::integral_constant<int, 0>;
+      using P1 = std::integral_constant<int, 1>;
+      using Yes = std::true_type;
+      using No = std::false_type;
+      auto step = [&](int t, auto par, auto haspv, f32x16& cs, f32x16& ns) {
+        if (nv1 < 64) half_tile(t, par, Yes{}, Yes{}, haspv, cs, ns);
+        else half_tile(t, par, No{}, Yes{}, haspv, cs, ns);
+      };
+      auto last = [&](auto par, auto haspv, f32x16& cs, f32x16& ns) {
+        constexpr int PAR = decltype(par)::value;
+        half_tile(tiles - 1, par, No{}, No{}, haspv, cs, ns);
+        lsum[1] = xbuf[((1 - PAR) * NCOMP + mate) * 64 + lane];
+#pragma unroll
+        for (int kb = 0; kb < 4; kb++) {
+          const bf16x8 pq = *(const bf16x8*)(prow + PAR * PPAR + kb * 1024);
+#pragma unroll
+          for (int m = 0; m < MTW; m++) oacc[m] = mfma32(vread(smem + (2 + PAR) * TILE, kb * MTW + m), pq, oacc[m]);
+        }
+        __syncthreads();
+      };
+      if (tiles == 1) {
+        last(P0{}, No{}, sa, sb);
+        break;
+      }
+      step(0, P0{}, No{}, sa, sb);
+      int t = 1;
+      for (; t + 2 < tiles; t += 2) {
+        step(t, P1{}, Yes{}, sb, sa);
+        step(t + 1, P0{}, Yes{}, sa, sb);
+      }
+      if (t + 1 < tiles) {
+        step(t, P1{}, Yes{}, sb, sa);
+        last(P0{}, Yes{}, sa, sb);
+      } else {
+        last(P1{}, Yes{}, sb, sa);
+      }
+      break;
+    } else {
     f32x16 sa0, sa1, sb0, sb1;
     qk_tile(smem, sa0, sa1);
     // K(2) is fetched into the buffer of K(0) at the top of the first iteration: every wave must have read
@@ -594,13 +810,11 @@ __device__ __forceinline__ void attn_item(const AttnParams& p, char* smem, const
         constexpr int e = decltype(ec)::value;
         float r;
         if constexpr (e < 16) r = c0[e]; else r = c1[e - 16];
+        if constexpr (e < 16) la += r; else lb += r;
         if constexpr (e & 1) {
-          lb += r;
           float prev;
           if constexpr (e < 16) prev = c0[e - 1]; else prev = c1[e - 17];
           pw[e >> 1] = pack_bf16(prev, r);
-        } else {
-          la += r;
         }
       };
       using Sch = ExpSlots<2 * KS, (LSE_ONLY ? 0 : 4 * MTD) / 2, LSE_ONLY ? 32 : EXP_IN_QK>;
@@ -657,7 +871,8 @@ __device__ __forceinline__ void attn_item(const AttnParams& p, char* smem, const
 #pragma unroll
         for (int e = 0; e < 16; e++) ma = fmaxf(fmaxf(ma, n0[e]), n1[e]);
       }
-      lsum += la + lb;
+      lsum[0] += la;
+      lsum[1] += lb;
       const float mx = xhalf_max(fmaxf(ma, mb));
       wait_fills<0>();
       __syncthreads();
@@ -693,6 +908,7 @@ __device__ __forceinline__ void attn_item(const AttnParams& p, char* smem, const
       last(P1{}, sb0, sb1);
     } else {
       last(P0{}, sa0, sa1);
+    }
     }
   } while (false);
 
@@ -731,7 +947,7 @@ __device__ __forceinline__ void attn_item(const AttnParams& p, char* smem, const
           for (int a = 0; a < 8; a++) put2(slot + ((m * 8 + a) * NCOMP + wave) * 128 + lane * 2, oacc[m][2 * a], oacc[m][2 * a + 1]);
         float* st = slot + D * 32 * NCOMP + wave * 64 + lane;
         put1(st, m_ref);
-        put1(st + 64 * NCOMP, lsum);
+        put1(st + 64 * NCOMP, lsum[0] + lsum[1]);
         put1(st + 128 * NCOMP, m_true);
       }
       __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");   // compiler ordering only
@@ -765,12 +981,12 @@ __device__ __forceinline__ void attn_item(const AttnParams& p, char* smem, const
         for (int m = 0; m < MTD; m++)
 #pragma unroll
           for (int i = 0; i < 16; i++) oacc[m][i] = 0.f;
-        lsum = 0.f;
+        lsum[0] = lsum[1] = 0.f;
         for (int kp = 0; kp < sk.pieces; kp++) {
           const float* slot = p.sk_slots + (int64_t)(sk.slot0 + kp) * SLOT_FLOATS;
           const float* st = slot + D * 32 * NCOMP + wave * 64 + lane;
           const float alpha = fast_exp2(get1(st) - m_star);
-          lsum = fmaf(get1(st + 64 * NCOMP), alpha, lsum);
+          lsum[0] = fmaf(get1(st + 64 * NCOMP), alpha, lsum[0]);
 #pragma unroll
           for (int m = 0; m < MTD; m++)
 #pragma unroll
@@ -788,11 +1004,11 @@ __device__ __forceinline__ void attn_item(const AttnParams& p, char* smem, const
 
   // ---- epilogue ----
   if (NPROD && wave >= NCOMP) return;   // fetch waves own no query rows (only reached with an empty list)
-  const float ltot = xhalf_sum(lsum);
+  const float ltot = xhalf_sum(lsum[0] + lsum[1]);
   const bool empty = !(ltot > 0.f);
   const float inv = empty ? 0.f : 1.0f / ltot;
-  const int qrow_w = q0 + wave * 32 + r;
-  if (hh == 0 && qrow_w < p.Lq) {
+  const int qrow_w = q0 + rblk * 32 + r;
+  if (hh == 0 && half == 0 && qrow_w < p.Lq) {
     const int64_t off = ((int64_t)b * p.H + h) * p.Lq + qrow_w;
     if (p.M) p.M[off] = empty ? -INFINITY : m_true;
     if (p.L) p.L[off] = empty ? 1.0f : ltot * fast_exp2(m_ref - m_true);
@@ -869,9 +1085,9 @@ __device__ __forceinline__ void attn_item(const AttnParams& p, char* smem, const
       return;
     }
   }
-  char* ob = smem + wave * (32 * OSTR);
+  char* ob = smem + rblk * (32 * OSTR) + half * D;   // a pair: each wave its columns
 #pragma unroll
-  for (int m = 0; m < MTD; m++) {
+  for (int m = 0; m < MTW; m++) {
 #pragma unroll
     for (int a = 0; a < 4; a++) {
       const int dcol = m * 32 + 8 * a + 4 * hh;
@@ -886,22 +1102,22 @@ __device__ __forceinline__ void attn_item(const AttnParams& p, char* smem, const
   __builtin_amdgcn_s_waitcnt(0xc07f);  // lgkmcnt(0)
   __builtin_amdgcn_wave_barrier();
   bf16_t* op = p.o + b * p.o_sb + h * p.o_sh;
-  constexpr int OCPR = D / 8;
+  constexpr int OCPR = MTW * 4;
 #pragma unroll
   for (int i = 0; i < (32 * OCPR) / 64; i++) {
     const int cidx = lane + i * 64;
     const int orow = cidx / OCPR, ocol = cidx - orow * OCPR;
-    const int grow = q0 + wave * 32 + orow;
+    const int grow = q0 + rblk * 32 + orow;
     if (grow < p.Lq) {
       u32x4 val = *(const u32x4*)(ob + orow * OSTR + ocol * 16);
-      *(u32x4*)(op + (int64_t)grow * p.o_sr + ocol * 8) = val;
+      *(u32x4*)(op + (int64_t)grow * p.o_sr + half * (D / 2) + ocol * 8) = val;
     }
   }
 }
 #endif  // __HIP_DEVICE_COMPILE__
 
 // THIRD: registers of a wave limited so that three workgroups share a compute unit, see third_workgroup
-template <int D, int NWAVES, int MODE, bool ACCUM, bool LSE_ONLY, int NPROD, bool IDLE, bool THIRD = false>
+template <int D, int NWAVES, int MODE, bool ACCUM, bool LSE_ONLY, int NPROD, bool IDLE, bool THIRD = false, bool PAIR = false>
 __global__ __launch_bounds__(NWAVES * 64, ((NWAVES <= 4 && D <= 128) ? (THIRD ? 3 : 2) : 1)) void attn_fwd_kernel(const AttnParams p) {
   // The body is compiled for the device only: the host pass just needs the launch stub, and it
   // silently drops the stub when the body uses the LDS-DMA builtins.
@@ -917,7 +1133,7 @@ __global__ __launch_bounds__(NWAVES * 64, ((NWAVES <= 4 && D <= 128) ? (THIRD ? 
   int bh, qt;
   if (!tile_of(p.order, __builtin_amdgcn_workgroup_id_x(), bh, qt)) return;
   asm volatile("" : "+v"(bh), "+v"(qt));
-  attn_item<D, NWAVES, MODE, ACCUM, LSE_ONLY, false, NPROD, IDLE>(p, smem, 0, bh, qt, 0, 0, true, SkCtx{});
+  attn_item<D, NWAVES, MODE, ACCUM, LSE_ONLY, false, NPROD, IDLE, PAIR>(p, smem, 0, bh, qt, 0, 0, true, SkCtx{});
 #endif
 }
 
@@ -1080,7 +1296,8 @@ static bool third_workgroup(int total_wg) { return total_wg > 2 * device_cus(); 
 // Fetch-only waves beside four computing ones.  A launch of at most one 128-row workgroup per compute unit leaves half of
 // the wave slots empty, and its lone waves pay for every instruction in full: 16 of the 100-odd that a wave issues per
 // tile beside its MFMAs are fills.  Without / with four fetch waves, B2 H16 d128: 144 x 265 9.8 / 9.0 us, 576 x 1497 27.3 /
-// 24.4, 1024 x 2521 (256 workgroups) 46.5 / 44.3; B1 H4 4096 x 10521 153 / 134; d64 B8 H16 256 x 680 12.2 / 11.4; lists
+// 24.4, 1024 x 2521 (256 workgroups) 46.5 / 44.3; B1 H4 4096 x 10521 153 / 134; d64 B8 H16 256 x 680 12.2 / 11.4 (the smaller ones of
+// these are launches of pairs now); lists
 // alike (B1 H16 784 x 1924 at 25 % 20.6 / 18.4).  With a second workgroup on a compute unit there are no empty slots, and at
 // head_dim 256 a wave fills its SIMD.  Same bits.  A workgroup with fetch waves has its compute unit to itself, so launches
 // on two streams that together need more than one per compute unit no longer share any: a pair of calls, without / with,
@@ -1089,12 +1306,22 @@ static bool third_workgroup(int total_wg) { return total_wg > 2 * device_cus(); 
 // and one stream is the usual case.
 static bool fetch_waves(int total_wg) { return total_wg <= device_cus(); }
 
-template <int D, int NWAVES, int MODE, bool ACCUM, bool LSE_ONLY, int NPROD = (MODE == MODE_GATHER && NWAVES == 8) ? 2 : 0>
+// Pairs of waves (see attn_item) with four fetch waves, where 64-row workgroups of them have a compute unit each.  128-row
+// workgroups with four fetch waves / 64-row ones of pairs, B2 H16 d128: 36 x 85 5.82 / 5.53 us, 64 x 149 6.73 / 6.10, 144 x 265
+// 8.89 / 7.38, 256 x 521 12.1 / 9.86, 400 x 921 17.1 / 13.8, 256 x 1497 23.9 / 19.0; B1 H4 4096 x 10521 133 / 117; d64 B1 H16
+// 256 x 680 10.7 / 9.0; lists alike (B1 H8 576 x 1497 at 30 % 16.0 / 12.8, sink + window B1 H4 3025 x 9450 31.6 / 25.2); a single key tile
+// alike.  Not beyond: pairs that share their SIMDs take twice as long (96-row workgroups of three pairs, 576 x 1497 24.3 /
+// 25.8, 6000 x 10521 136 / 165; 128-row ones 24.4 / 29.6).  Two streams with such a launch each, B1 d128: 2 x 8 heads 576 x 1497
+// 23.7 / 23.1, 2 x 16 heads 25.3 / 24.7, 2 x 8 heads 1024 x 2521 72.7 / 55.5, but 2 x 16 heads, which fill the chip together as 128-row
+// workgroups, 51.2 / 64.9 (one stream 40.5 / 33.0).
+static bool pairs_of_waves(const AttnParams& p) { return (int64_t)p.B * p.H * ((p.Lq + 63) / 64) <= device_cus(); }
+
+template <int D, int NWAVES, int MODE, bool ACCUM, bool LSE_ONLY, int NPROD = (MODE == MODE_GATHER && NWAVES == 8) ? 2 : 0, bool PAIR = false>
 static int launch_one(const AttnParams& p0, hipStream_t stream) {
   AttnParams p = p0;
   if (p.kv_group < 1) p.kv_group = 1;
-  constexpr int WGROWS = (NWAVES - NPROD) * 32;
-  constexpr int SMEM = attn_lds_bytes<D, NWAVES - NPROD, MODE>();
+  constexpr int WGROWS = (NWAVES - NPROD) * (PAIR ? 16 : 32);
+  constexpr int SMEM = attn_lds_bytes<D, NWAVES - NPROD, MODE, PAIR>();
   if (MODE == MODE_BLOCK && p.list == nullptr) p.group_rows = WGROWS;  // dense: any row grouping
   if (p.group_rows % WGROWS != 0) return LVAR_EINVAL;
   if (p.remap_gs > 0 && !reads_remapped<D, NWAVES, MODE, NPROD>) return LVAR_EUNSUPPORTED;
@@ -1144,6 +1371,7 @@ static int launch_one(const AttnParams& p0, hipStream_t stream) {
   }
   if constexpr (MODE == MODE_BLOCK && !LSE_ONLY && NWAVES == 4 && D <= 128) {
     if (wide_tiles(p0, D)) return launch_one<D, 8, MODE_BLOCK, false, false>(p0, stream);
+    if (pairs_of_waves(p)) return launch_one<D, 8, MODE_BLOCK, false, false, 4, true>(p0, stream);
     if (fetch_waves(p.total_wg)) return launch_one<D, 8, MODE_BLOCK, false, false, 4>(p0, stream);
   }
   const int rest = p.Lq % WGROWS;
@@ -1168,7 +1396,7 @@ static int launch_one(const AttnParams& p0, hipStream_t stream) {
       return hipGetLastError() == hipSuccess ? LVAR_OK : LVAR_ELAUNCH;
     }
   }
-  auto kern = attn_fwd_kernel<D, NWAVES, MODE, ACCUM, LSE_ONLY, NPROD, false>;
+  auto kern = attn_fwd_kernel<D, NWAVES, MODE, ACCUM, LSE_ONLY, NPROD, false, false, PAIR>;
   static std::atomic<uint64_t> lds_ready{0};
   if (!ensure_lds_limit((const void*)kern, SMEM, lds_ready)) return LVAR_ELAUNCH;
   hipLaunchKernelGGL(kern, dim3(grid), dim3(NWAVES * 64), SMEM, stream, p);
