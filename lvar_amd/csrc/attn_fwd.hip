@@ -1116,6 +1116,20 @@ __device__ __forceinline__ void attn_item(const AttnParams& p, char* smem, const
 }
 #endif  // __HIP_DEVICE_COMPILE__
 
+// The tile with the place-th longest list of the n tiles that run in order, of lists that all slices share (see ranked_slice)
+template <int WGROWS>
+__device__ __forceinline__ int tile_by_length(const AttnParams& p, int place, int n) {
+  const int lane = __builtin_amdgcn_workitem_id_x() & 63;
+  // length and position in one number; never equal
+  const int key = lane < n ? (max(0, min(p.cnt[lane * WGROWS / p.group_rows], p.list_len)) << 6) + 63 - lane : -1;
+  int longer = 0;
+  for (int k = 0; k < n; k++) longer += __builtin_amdgcn_readlane(key, k) > key ? 1 : 0;
+  return __builtin_ctzll(__builtin_amdgcn_ballot_w64(lane < n && longer == place));
+}
+
+template <int D, int NWAVES, int MODE, bool LSE_ONLY>
+constexpr bool ranks_tiles = MODE == MODE_BLOCK && !LSE_ONLY && D == 128 && NWAVES == 4;
+
 // THIRD: registers of a wave limited so that three workgroups share a compute unit, see third_workgroup
 template <int D, int NWAVES, int MODE, bool ACCUM, bool LSE_ONLY, int NPROD, bool IDLE, bool THIRD = false, bool PAIR = false>
 __global__ __launch_bounds__(NWAVES * 64, ((NWAVES <= 4 && D <= 128) ? (THIRD ? 3 : 2) : 1)) void attn_fwd_kernel(const AttnParams p) {
@@ -1132,6 +1146,9 @@ __global__ __launch_bounds__(NWAVES * 64, ((NWAVES <= 4 && D <= 128) ? (THIRD ? 
   asm volatile("" : : "s"(p.q), "s"(p.q_sb), "s"(p.v_sb), "s"(p.o_sh), "s"(p.H), "s"(p.list_sb));
   int bh, qt;
   if (!tile_of(p.order, __builtin_amdgcn_workgroup_id_x(), bh, qt)) return;
+  if constexpr (ranks_tiles<D, NWAVES, MODE, LSE_ONLY>) {
+    if (p.round_places > 0 && qt < p.order.nqt && ranked_slice(p.order, bh, p.round_places)) qt = tile_by_length<NWAVES * 32>(p, qt, p.order.nqt);
+  }
   asm volatile("" : "+v"(bh), "+v"(qt));
   attn_item<D, NWAVES, MODE, ACCUM, LSE_ONLY, false, NPROD, IDLE, PAIR>(p, smem, 0, bh, qt, 0, 0, true, SkCtx{});
 #endif
@@ -1306,6 +1323,16 @@ static bool third_workgroup(int total_wg) { return total_wg > 2 * device_cus(); 
 // and one stream is the usual case.
 static bool fetch_waves(int total_wg) { return total_wg <= device_cus(); }
 
+// Lists that all slices share (one mask for every batch and head, as the sink + window layers have): their lengths are one row of
+// counts, which a wave can rank, one tile per lane.  That costs a workgroup a read that its list waits for, so only those of a
+// slice that reaches into a last, partial round do it.  Natural order / longest first, sink + window d128 128 x 128: B2 H16
+// 48 x 48 (576 workgroups on 512 places) 58.5 / 55.8 us, 55 x 55 94.0 / 93.2, B2 H12 56 x 56 106.2 / 104.7, B3 H20 48 x 48 95.1 /
+// 93.7; launches without such a round, or whose heads lie across two XCDs, alike.  head_dim 64 loses 1 % (a third workgroup per
+// compute unit covers the end), 64-row blocks gain nothing: no code for it there.
+static bool lists_by_length(const AttnParams& p) {
+  return p.list && p.B * p.H > 1 && p.cnt_sb == 0 && p.cnt_sh == 0 && p.order.nqt > 1 && p.order.nqt <= 64;
+}
+
 // Pairs of waves (see attn_item) with four fetch waves, where 64-row workgroups of them have a compute unit each.  128-row
 // workgroups with four fetch waves / 64-row ones of pairs, B2 H16 d128: 36 x 85 5.82 / 5.53 us, 64 x 149 6.73 / 6.10, 144 x 265
 // 8.89 / 7.38, 256 x 521 12.1 / 9.86, 400 x 921 17.1 / 13.8, 256 x 1497 23.9 / 19.0; B1 H4 4096 x 10521 133 / 117; d64 B1 H16
@@ -1379,6 +1406,7 @@ static int launch_one(const AttnParams& p0, hipStream_t stream) {
                                           : p.list != nullptr && ragged_lists_last(p.B * p.H, p.nqt, rest, device_cus());
   p.order = tile_order(p.B * p.H, p.nqt, ragged);
   const int grid = TILE_XCDS * p.order.per_xcd;
+  if constexpr (ranks_tiles<D, NWAVES, MODE, LSE_ONLY>) p.round_places = lists_by_length(p) ? device_cus() / TILE_XCDS * 2 : 0;
   if constexpr (D == 64 && NWAVES == 4 && MODE == MODE_BLOCK && !LSE_ONLY) {
     if (third_workgroup(p.total_wg)) {
       static_assert(SMEM <= 48 * 1024, "three workgroups share the LDS of a compute unit; no larger limit has to be asked for");

@@ -55,6 +55,14 @@ LVAR_HD bool tile_of(const TileOrder& t, unsigned id, int& slice, int& qt) {
   return i < t.per_xcd && slice < t.ragged;
 }
 
+// Whether the tiles of a slice run longest list first: slices that lie in one XCD and reach into a last round that is not full.
+// What starts late is then short.
+LVAR_HD bool ranked_slice(const TileOrder& t, int slice, int round_places) {
+  const int full = t.per_xcd / round_places * round_places;   // places before the last round
+  const int first = slice * t.nqt, last = first + t.nqt - 1, x = first / t.whole_per_xcd;
+  return full > 0 && full < t.per_xcd && x == last / t.whole_per_xcd && last - x * t.whole_per_xcd >= full;
+}
+
 // Whether the ragged last tiles of token lists with fetch-only waves (one workgroup per compute unit) run behind the whole
 // ones.  The waves without rows do not compute, so with at least half of them idle such a tile is the shorter workgroup, and
 // it pays where the launch can end on a round of nothing else, with every whole tile in the full rounds before it.  832 of
