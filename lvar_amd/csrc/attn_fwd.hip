@@ -1116,12 +1116,16 @@ __device__ __forceinline__ void attn_item(const AttnParams& p, char* smem, const
 }
 #endif  // __HIP_DEVICE_COMPILE__
 
-// The tile with the place-th longest list of the n tiles that run in order, of lists that all slices share (see ranked_slice)
+// The tile of slice bh with its place-th longest list, of the n tiles that run in order (see ranked_slice)
 template <int WGROWS>
-__device__ __forceinline__ int tile_by_length(const AttnParams& p, int place, int n) {
-  const int lane = __builtin_amdgcn_workitem_id_x() & 63;
-  // length and position in one number; never equal
-  const int key = lane < n ? (max(0, min(p.cnt[lane * WGROWS / p.group_rows], p.list_len)) << 6) + 63 - lane : -1;
+__device__ __forceinline__ int tile_by_length(const AttnParams& p, int bh, int place, int n) {
+  const int lane = __builtin_amdgcn_workitem_id_x() & 63, b = bh / p.H, h = bh - b * p.H;
+  const int len = lane < n ? max(0, min(p.cnt[b * p.cnt_sb + h * p.cnt_sh + lane * WGROWS / p.group_rows], p.list_len)) : 0;
+  // the list of the tile in natural order is asked for at the same time: with lists of equal length it is the one that is read next
+  const int head = p.list_len > 0 ? p.list[b * p.list_sb + h * p.list_sh + (int64_t)(place * WGROWS / p.group_rows) * p.list_sg] : 0;
+  asm volatile("" : : "v"(head));
+  if (__builtin_amdgcn_ballot_w64(lane < n && len != __builtin_amdgcn_readfirstlane(len)) == 0) return place;
+  const int key = lane < n ? (len << 6) + 63 - lane : -1;   // length and position in one number; never equal
   int longer = 0;
   for (int k = 0; k < n; k++) longer += __builtin_amdgcn_readlane(key, k) > key ? 1 : 0;
   return __builtin_ctzll(__builtin_amdgcn_ballot_w64(lane < n && longer == place));
@@ -1147,7 +1151,7 @@ __global__ __launch_bounds__(NWAVES * 64, ((NWAVES <= 4 && D <= 128) ? (THIRD ? 
   int bh, qt;
   if (!tile_of(p.order, __builtin_amdgcn_workgroup_id_x(), bh, qt)) return;
   if constexpr (ranks_tiles<D, NWAVES, MODE, LSE_ONLY>) {
-    if (p.round_places > 0 && qt < p.order.nqt && ranked_slice(p.order, bh, p.round_places)) qt = tile_by_length<NWAVES * 32>(p, qt, p.order.nqt);
+    if (p.round_places > 0 && qt < p.order.nqt && ranked_slice(p.order, bh, p.round_places)) qt = tile_by_length<NWAVES * 32>(p, bh, qt, p.order.nqt);
   }
   asm volatile("" : "+v"(bh), "+v"(qt));
   attn_item<D, NWAVES, MODE, ACCUM, LSE_ONLY, false, NPROD, IDLE, PAIR>(p, smem, 0, bh, qt, 0, 0, true, SkCtx{});
@@ -1323,15 +1327,8 @@ static bool third_workgroup(int total_wg) { return total_wg > 2 * device_cus(); 
 // and one stream is the usual case.
 static bool fetch_waves(int total_wg) { return total_wg <= device_cus(); }
 
-// Lists that all slices share (one mask for every batch and head, as the sink + window layers have): their lengths are one row of
-// counts, which a wave can rank, one tile per lane.  That costs a workgroup a read that its list waits for, so only those of a
-// slice that reaches into a last, partial round do it.  Natural order / longest first, sink + window d128 128 x 128: B2 H16
-// 48 x 48 (576 workgroups on 512 places) 58.5 / 55.8 us, 55 x 55 94.0 / 93.2, B2 H12 56 x 56 106.2 / 104.7, B3 H20 48 x 48 95.1 /
-// 93.7; launches without such a round, or whose heads lie across two XCDs, alike.  head_dim 64 loses 1 % (a third workgroup per
-// compute unit covers the end), 64-row blocks gain nothing: no code for it there.
-static bool lists_by_length(const AttnParams& p) {
-  return p.list && p.B * p.H > 1 && p.cnt_sb == 0 && p.cnt_sh == 0 && p.order.nqt > 1 && p.order.nqt <= 64;
-}
+// Lists whose lengths a wave can rank, one tile per lane.
+static bool lists_by_length(const AttnParams& p) { return p.list && p.order.nqt > 1 && p.order.nqt <= 64; }
 
 // Pairs of waves (see attn_item) with four fetch waves, where 64-row workgroups of them have a compute unit each.  128-row
 // workgroups with four fetch waves / 64-row ones of pairs, B2 H16 d128: 36 x 85 5.82 / 5.53 us, 64 x 149 6.73 / 6.10, 144 x 265
