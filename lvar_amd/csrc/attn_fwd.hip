@@ -1120,10 +1120,12 @@ __device__ __forceinline__ void attn_item(const AttnParams& p, char* smem, const
 template <int WGROWS>
 __device__ __forceinline__ int tile_by_length(const AttnParams& p, int bh, int place, int n) {
   const int lane = __builtin_amdgcn_workitem_id_x() & 63, b = bh / p.H, h = bh - b * p.H;
-  const int len = lane < n ? max(0, min(p.cnt[b * p.cnt_sb + h * p.cnt_sh + lane * WGROWS / p.group_rows], p.list_len)) : 0;
-  // the list of the tile in natural order is asked for at the same time: with lists of equal length it is the one that is read next
-  const int head = p.list_len > 0 ? p.list[b * p.list_sb + h * p.list_sh + (int64_t)(place * WGROWS / p.group_rows) * p.list_sg] : 0;
-  asm volatile("" : : "v"(head));
+  const int g = lane * WGROWS / p.group_rows;
+  const int raw = lane < n ? p.cnt[b * p.cnt_sb + h * p.cnt_sh + g] : 0;
+  // the heads of all lists are asked for at the same time: whichever is read next is then in the L2
+  const int head = lane < n && p.list_len > 0 ? p.list[b * p.list_sb + h * p.list_sh + (int64_t)g * p.list_sg] : 0;
+  asm volatile("" : : "v"(head), "v"(raw));
+  const int len = max(0, min(raw, p.list_len));
   if (__builtin_amdgcn_ballot_w64(lane < n && len != __builtin_amdgcn_readfirstlane(len)) == 0) return place;
   const int key = lane < n ? (len << 6) + 63 - lane : -1;   // length and position in one number; never equal
   int longer = 0;

@@ -58,9 +58,9 @@ LVAR_HD bool tile_of(const TileOrder& t, unsigned id, int& slice, int& qt) {
 // Whether the tiles of a slice run longest list first: slices that lie in one XCD and reach into a last round that is at most half
 // full, so that what starts late is short.  `round_places`: places of an XCD that run at once.  The others keep their order and pay
 // nothing; a ranked tile waits for the lengths of its slice's lists before its own list is read.  Natural order / longest first,
-// d128, 128-row tiles, two per compute unit: random lists B2 H16 48 x 48 (576 tiles on 512 places) at 25 % 81.7 / 76.4 us, at 10 %
-// 43.7 / 39.5, B1 H24 56 x 56 106.4 / 102.6; sink + window 48 x 48 58.6 / 56.0, B2 H12 56 x 56 106.2 / 104.7; best-scoring blocks,
-// nearly or exactly of one length, 48 x 48 25 % 74.0 / 74.2, 10 % 65.1 / 64.4, B1 H24 56 x 56 121.2 / 119.2, B2 H20 44 x 44 82.3 / 82.7.
+// d128, 128-row tiles, two per compute unit: random lists B2 H16 48 x 48 (576 tiles on 512 places) at 25 % 81.6 / 75.5 us, at 10 %
+// 43.9 / 39.3, B1 H24 56 x 56 106.9 / 102.0; sink + window 48 x 48 58.1 / 55.6, B2 H12 56 x 56 106.2 / 104.7; best-scoring blocks,
+// nearly or exactly of one length, 48 x 48 25 % 74.3 / 73.7, 10 % 64.8 / 63.8, B1 H24 56 x 56 120.4 / 117.9, B2 H20 44 x 44 81.5 / 82.0.
 // With the last round 46 / 64 full random lists lose 1.8 %.  head_dim 64 loses 1 % (a third workgroup per compute unit covers the
 // end), 64-row tiles gain nothing.
 LVAR_HD bool ranked_slice(const TileOrder& t, int slice, int round_places) {
