@@ -554,7 +554,7 @@ __device__ __forceinline__ void attn_item(const AttnParams& p, char* smem, const
       constexpr int PPAR = NCOMP * 2048;                         // bytes of one parity
       float* const xbuf = (float*)(pbuf + 2 * PPAR);             // [parity][computing wave][lane]
       const int mate = half ? wave - RB : wave + RB;
-      const int kb_l = kbase_l + half * 32 * ROWB;
+      int kb_l = kbase_l + half * 32 * ROWB;
       int vb_l[MTW];
 #pragma unroll
       for (int m = 0; m < MTW; m++) vb_l[m] = vbase_l ^ ((half * MTW + m) << 6);
@@ -599,7 +599,7 @@ __device__ __forceinline__ void attn_item(const AttnParams& p, char* smem, const
       auto half_tile = [&](int t, auto par, auto masked, auto hasqk, auto haspv, f32x16& cs, f32x16& ns) {
         constexpr int PAR = decltype(par)::value;
         constexpr bool MASKED = decltype(masked)::value, QK = decltype(hasqk)::value, PV = decltype(haspv)::value;
-        constexpr int NQK = QK ? KS : 0, NPV = PV ? 4 * MTW : 0, NS = NQK + NPV, AHEAD = READ_AHEAD, PAHEAD = 3;
+        constexpr int NQK = QK ? KS : 0, NPV = PV ? 4 * MTW : 0, NS = NQK + NPV, AHEAD = D == 256 ? 3 : READ_AHEAD, PAHEAD = D == 256 ? 2 : 3;
         // the maximum is settled two MFMAs into the iteration: the other wave's arrives from LDS with the first fragments
         constexpr int CHK = NS >= 8 ? 2 : 0;
         using Sch = HalfSlots<(NS - CHK > 3 ? NS - CHK - 2 : 1)>;
@@ -609,6 +609,9 @@ __device__ __forceinline__ void attn_item(const AttnParams& p, char* smem, const
         }
         const char* kbuf = smem + (1 - PAR) * TILE;
         const char* vbuf = smem + (3 - PAR) * TILE;
+        // head_dim 256: the 16 offsets of the K fragments are formed per tile and a fragment less is read ahead, or 50 registers are
+        // spilled (400 x 921 29.4 us, 21.7 without)
+        if constexpr (D == 256) asm volatile("" : "+v"(kb_l));
         const float mother = xbuf[(PAR * NCOMP + mate) * 64 + lane];
         bf16x8 frag[NS > 0 ? NS : 1], pb[4];
         auto operand = [&](auto ic) {
@@ -1336,7 +1339,8 @@ static bool lists_by_length(const AttnParams& p) { return p.list && p.order.nqt 
 // workgroups with four fetch waves / 64-row ones of pairs, B2 H16 d128: 36 x 85 5.82 / 5.53 us, 64 x 149 6.73 / 6.10, 144 x 265
 // 8.89 / 7.38, 256 x 521 12.1 / 9.86, 400 x 921 17.1 / 13.8, 256 x 1497 23.9 / 19.0; B1 H4 4096 x 10521 133 / 117; d64 B1 H16
 // 256 x 680 10.7 / 9.0; lists alike (B1 H8 576 x 1497 at 30 % 16.0 / 12.8, sink + window B1 H4 3025 x 9450 31.6 / 25.2); a single key tile
-// alike.  Not beyond: pairs that share their SIMDs take twice as long (96-row workgroups of three pairs, 576 x 1497 24.3 /
+// alike; head_dim 256, where the waves of 128-row workgroups fill their SIMDs and nothing only fetches: 16 x 21 7.12 / 5.54, 144 x 265
+// 15.1 / 10.9, 400 x 921 29.8 / 21.7, 512 x 1000 31.1 / 26.7, B1 H4 3000 x 9000 206 / 142.  Not beyond: pairs that share their SIMDs take twice as long (96-row workgroups of three pairs, 576 x 1497 24.3 /
 // 25.8, 6000 x 10521 136 / 165; 128-row ones 24.4 / 29.6).  Two streams with such a launch each, B1 d128: 2 x 8 heads 576 x 1497
 // 23.7 / 23.1, 2 x 16 heads 25.3 / 24.7, 2 x 8 heads 1024 x 2521 72.7 / 55.5, but 2 x 16 heads, which fill the chip together as 128-row
 // workgroups, 51.2 / 64.9 (one stream 40.5 / 33.0).
@@ -1395,9 +1399,11 @@ static int launch_one(const AttnParams& p0, hipStream_t stream) {
       return hipGetLastError() == hipSuccess ? LVAR_OK : LVAR_ELAUNCH;
     }
   }
+  if constexpr (MODE == MODE_BLOCK && !LSE_ONLY && NWAVES == 4) {
+    if (pairs_of_waves(p)) return launch_one<D, 8, MODE_BLOCK, false, false, 4, true>(p0, stream);
+  }
   if constexpr (MODE == MODE_BLOCK && !LSE_ONLY && NWAVES == 4 && D <= 128) {
     if (wide_tiles(p0, D)) return launch_one<D, 8, MODE_BLOCK, false, false>(p0, stream);
-    if (pairs_of_waves(p)) return launch_one<D, 8, MODE_BLOCK, false, false, 4, true>(p0, stream);
     if (fetch_waves(p.total_wg)) return launch_one<D, 8, MODE_BLOCK, false, false, 4>(p0, stream);
   }
   const int rest = p.Lq % WGROWS;

@@ -15,7 +15,7 @@ def _inputs(H, Lq, Lk, d, seed, growth):
 
 
 @pytest.mark.parametrize("growth", [0.0, 0.7])
-@pytest.mark.parametrize("d", [64, 128])
+@pytest.mark.parametrize("d", [64, 128, 256])
 @pytest.mark.parametrize("Lq,Lk", [(1, 1), (33, 64), (64, 65), (65, 128), (96, 129), (127, 200), (128, 257), (130, 640), (40, 1000)])
 def test_pairs_give_the_bits_of_larger_launches(Lq, Lk, d, growth):
     from lvar_amd import sparse_attn_ops as ops
@@ -34,13 +34,14 @@ def test_pairs_give_the_bits_of_larger_launches(Lq, Lk, d, growth):
         assert torch.equal(o1, ob[:, h]) and torch.equal(M1, Mb[:, h]) and torch.equal(L1, Lb[:, h])
 
 
+@pytest.mark.parametrize("d", [64, 128, 256])
 @pytest.mark.parametrize("growth", [0.0, 0.7])
-def test_pairs_against_float64(growth):
+def test_pairs_against_float64(growth, d):
     """bf16 inputs, P rounded to bf16: 2^-9 per probability and per output, so 1 % of the largest output is four times that."""
     from lvar_amd import sparse_attn_ops as ops
-    q, k, v = _inputs(3, 150, 500, 128, seed=1, growth=growth)
+    q, k, v = _inputs(3, 150, 500, d, seed=1, growth=growth)
     o, (M, L) = ops.dense_attn(q, k, v)
-    s = (q.double().cpu() @ k.double().cpu().transpose(-1, -2).contiguous()) / 128 ** 0.5
+    s = (q.double().cpu() @ k.double().cpu().transpose(-1, -2).contiguous()) / d ** 0.5
     ref = s.softmax(-1) @ v.double().cpu()
     assert (o.double().cpu() - ref).abs().max() < 1e-2 * ref.abs().max()
     lse = (M.double() + L.double().log2()).cpu().reshape(1, 3, 150)
