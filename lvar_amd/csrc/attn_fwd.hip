@@ -3,7 +3,8 @@
 //
 // Work decomposition
 //   workgroup  = NWAVES waves, 32 query rows per wave (small launches: per two waves, see PAIR), all share the K/V tiles in LDS
-//                (token lists with 192-row groups: 8 waves = 6 computing waves + 2 waves that only fetch, see NPROD)
+//                (token lists with 192-row groups: 8 waves = 6 computing waves + 2 waves that only fetch, see NPROD; fewer rows
+//                and four fetch waves where that leaves no compute unit idle, see half_groups)
 //   wave       = S^T[64 keys x 32 queries] = K_tile . Q^T with 32x32x16 bf16 MFMA (K rows are
 //                the A operand read from LDS, Q^T is the B operand held in registers), so a
 //                lane owns ONE query column: the softmax row max / sum are in-register
@@ -129,7 +130,7 @@ __device__ __forceinline__ void attn_item(const AttnParams& p, char* smem, const
   constexpr int WGROWS = RB * 32;
   constexpr int KS = D / 16, MTD = D / 32;
   constexpr int MTW = PAIR ? MTD / 2 : MTD;      // 32-column blocks of O that a wave accumulates
-  static_assert(!PAIR || (MODE == MODE_BLOCK && NPROD > 0 && !ACCUM && !LSE_ONLY && !SK), "pairs: dense and block lists with fetch waves");
+  static_assert(!PAIR || (NPROD > 0 && !LSE_ONLY && !SK), "pairs have fetch waves beside them");
   constexpr int ROWB = Swz<D>::ROWB, CPR = Swz<D>::CPR;
   constexpr int RPI = 1024 / ROWB;          // rows filled by one 64-lane x 16 B load
   constexpr int NI = 64 / RPI;              // loads per 64-row tile
@@ -603,7 +604,9 @@ __device__ __forceinline__ void attn_item(const AttnParams& p, char* smem, const
         // the maximum is settled two MFMAs into the iteration: the other wave's arrives from LDS with the first fragments
         constexpr int CHK = NS >= 8 ? 2 : 0;
         using Sch = HalfSlots<(NS - CHK > 3 ? NS - CHK - 2 : 1)>;
-        if constexpr (QK) {
+        if constexpr (MODE == MODE_GATHER) {
+          nv3 = nvalid_gather(t + 3);
+        } else if constexpr (QK) {
           if (t + 3 < tiles) finish_rows(t + 3, raw, rows_n, nv3);
           if (t + 4 < tiles) prefetch_raw(t + 4, raw);
         }
@@ -1035,7 +1038,7 @@ __device__ __forceinline__ void attn_item(const AttnParams& p, char* smem, const
       const bf16_t* abase = p.o_accum + b * p.oa_sb + h * p.oa_sh;
       bf16_t* op = p.o + b * p.o_sb + h * p.o_sh;
 #pragma unroll
-      for (int pass = 0; pass < 2; pass++) {
+      for (int pass = 0; pass < (PAIR ? 1 : 2); pass++) {   // (a wave of a pair holds its half alone)
 #pragma unroll
         for (int mm = 0; mm < MTD / 2; mm++) {
           const int m = pass * (MTD / 2) + mm;
@@ -1053,11 +1056,11 @@ __device__ __forceinline__ void attn_item(const AttnParams& p, char* smem, const
         for (int i = 0; i < ITER; i++) {
           const int cidx = lane + i * 64;
           const int orow = cidx / CPRH, oc = cidx - orow * CPRH;
-          const int grow = q0 + wave * 32 + orow;
+          const int grow = q0 + rblk * 32 + orow;
           if (grow < p.Lq) {
             const f32x4 xa = *(const f32x4*)(fb + orow * FSTR + oc * 32), xb = *(const f32x4*)(fb + orow * FSTR + oc * 32 + 16);
             float x[8] = {xa[0], xa[1], xa[2], xa[3], xb[0], xb[1], xb[2], xb[3]};
-            const int col = pass * HD + oc * 8;
+            const int col = (PAIR ? half : pass) * HD + oc * 8;
             if (p.up_src > 0) {
               const int y = grow / p.up_dst, xq = grow - y * p.up_dst;
               const float sc = (float)p.up_src / (float)p.up_dst;
@@ -1358,7 +1361,7 @@ static int launch_one(const AttnParams& p0, hipStream_t stream) {
   p.nqt = (p.Lq + WGROWS - 1) / WGROWS;
   p.total_wg = p.B * p.H * p.nqt;
   constexpr bool WIDE = MODE == MODE_BLOCK && NWAVES == 8;   // 256 query rows, or 128 and fetch waves
-  if constexpr (!LSE_ONLY && !(MODE == MODE_BLOCK && NPROD > 0)) {
+  if constexpr (!LSE_ONLY && NPROD != 4) {
     const bool dense = (MODE == MODE_BLOCK && p.list == nullptr);
     const int64_t per_tile = (MODE == MODE_BLOCK) ? (p.list ? p.list_len : (p.Lk + 63) / 64) : (p.list_len + 63) / 64;
     const int sub = (MODE == MODE_BLOCK && p.list) ? p.sub_shift : 0;
@@ -1436,6 +1439,14 @@ static int launch_one(const AttnParams& p0, hipStream_t stream) {
   return hipGetLastError() == hipSuccess ? LVAR_OK : LVAR_ELAUNCH;
 }
 
+// 192-row groups of token lists that leave compute units idle.  A group's six computing waves share four SIMDs, and the two SIMDs
+// with two of them set its time.  As 64-row workgroups of pairs (pairs_of_waves), or as 96-row ones of three computing and four
+// fetch waves, a computing wave has its SIMD to itself; either where every workgroup has a compute unit.  192 rows / 64 rows of
+// pairs, d128 last step with 20 % of the keys, the whole step: B1 H4 64 x 64 49.3 / 32.4 us, B1 H8 40 x 40 32.0 / 18.2, B2 H4 33 x 33 at
+// 5 % 22.5 / 12.5, d64 B1 H4 64 x 64 32.6 / 19.8.  192 / 96 rows: B1 H16 36 x 36 at 10 % 30.4 / 22.6, B1 H8 50 x 50 at 30 % 48.1 /
+// 35.4, d64 18.8 / 15.4 and 31.1 / 23.7.
+static bool half_groups(const AttnParams& p) { return (int64_t)p.B * p.H * ((p.Lq + 95) / 96) <= device_cus(); }
+
 // Token lists at head_dim 64: 192-row groups as two 3-wave workgroups (several share a compute unit, each fetches for
 // itself) instead of one of 8 waves, with the same bits, where the 8-wave workgroups leave their last round at most half
 // full.  832 / 2560 keys per list, 8-wave against 3-wave: 96 groups 18.9 / 43.2 against 16.3 / 37.7 us, 384 groups 36.2 /
@@ -1456,6 +1467,8 @@ static int launch_d(const AttnParams& p, int mode, bool accum, bool lse_only, in
   } else if (mode == MODE_GATHER) {
     // (head_dim 256: a wave needs more than 256 registers, so one wave per SIMD: 192-row groups run as two 3-wave workgroups)
     if constexpr (D > 128) { if (nwaves == 8) nwaves = 3; }
+    else if (nwaves == 8 && !p.sk_ws && pairs_of_waves(p)) return launch_one<D, 8, MODE_GATHER, true, false, 4, true>(p, s);
+    else if (nwaves == 8 && !p.sk_ws && half_groups(p)) return launch_one<D, 7, MODE_GATHER, true, false, 4>(p, s);
     else if (D == 64 && nwaves == 8 && !p.sk_ws && three_wave_groups(p)) return launch_one<D, 3, MODE_GATHER, true, false>(p, s);
     else if (nwaves == 8) return launch_one<D, 8, MODE_GATHER, true, false>(p, s);
     if (nwaves == 3) return launch_one<D, 3, MODE_GATHER, true, false>(p, s);

@@ -1,5 +1,6 @@
-"""Launches whose waves work in pairs (64-row workgroups that have a compute unit each) against larger launches of the same heads,
-which do not: the same bits, whatever the number of key tiles, ragged rows or keys and growth of the row maximum."""
+"""Launches whose waves work in pairs (64-row workgroups that have a compute unit each), and token lists in half groups, against
+larger launches of the same heads, which do neither: the same bits, whatever the number of key tiles, ragged rows or keys and
+growth of the row maximum."""
 import pytest
 import torch
 
@@ -32,6 +33,27 @@ def test_pairs_give_the_bits_of_larger_launches(Lq, Lk, d, growth):
         assert torch.equal(o1, o[:, h]) and torch.equal(M1, M[:, h]) and torch.equal(L1, L[:, h])
         o1, (M1, L1) = ops.block_sparse_attn(*part, num[:, h].contiguous(), idx[:, h].contiguous(), 128, 64)
         assert torch.equal(o1, ob[:, h]) and torch.equal(M1, Mb[:, h]) and torch.equal(L1, Lb[:, h])
+
+
+# rows: one part-filled pair, whole groups of 192, 64, 96 and 160 rows in the last one
+@pytest.mark.parametrize("growth", [0.0, 0.7])
+@pytest.mark.parametrize("d", [64, 128])
+@pytest.mark.parametrize("Lq,Lk,keys", [(20, 70, 33), (192, 400, 64), (256, 700, 129), (288, 500, 200), (400, 900, 450), (544, 300, 300)])
+def test_token_lists_give_the_bits_of_larger_launches(Lq, Lk, keys, d, growth):
+    from lvar_amd import sparse_attn_ops as ops
+    cus = torch.cuda.get_device_properties(0).multi_processor_count
+    H, G = cus + 3, -(-Lq // 192)                                                             # more groups than compute units
+    q, k, v = _inputs(H, Lq, Lk, d, seed=Lq + keys, growth=growth)
+    g = torch.Generator(device="cuda").manual_seed(keys)
+    idx = torch.rand(1, H, G, Lk, generator=g, device="cuda").argsort(-1).int()
+    cnt = torch.randint(0, keys + 1, (1, H, G), generator=g, device="cuda", dtype=torch.int32)  # empty and part-filled lists
+    cache = torch.randn(1, H, Lq, d, generator=g, device="cuda").to(torch.bfloat16)
+    o = ops.csp_attn(q, k, v, None, idx, cnt, cache, -1.0)
+    pair_heads, half_heads = cus // -(-Lq // 64), cus // -(-Lq // 96)                         # the most that either form takes
+    for h in (slice(0, 1), slice(H - pair_heads, H), slice(H - half_heads, H)):
+        q1, k1, v1, idx1, cnt1, cache1 = (t[:, h].contiguous() for t in (q, k, v, idx, cnt, cache))
+        o1 = ops.csp_attn(q1, k1, v1, None, idx1, cnt1, cache1, -1.0)
+        assert torch.equal(o1, o[:, h])
 
 
 @pytest.mark.parametrize("d", [64, 128, 256])
