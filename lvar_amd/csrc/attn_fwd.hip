@@ -1338,6 +1338,14 @@ static bool fetch_waves(int total_wg) { return total_wg <= device_cus(); }
 // Lists whose lengths a wave can rank, one tile per lane.
 static bool lists_by_length(const AttnParams& p) { return p.list && p.order.nqt > 1 && p.order.nqt <= 64; }
 
+// 96 rows per workgroup, three computing and four fetch waves, for dense launches that leave compute units idle as 128-row
+// workgroups: a chain of tiles takes as long, with a quarter less operand reads and power per compute unit.  128 / 96 rows, B2 H16
+// d128: 576 x 1497 24.2 / 23.8 us, 576 x 660 13.8 / 13.6, 520 x 100 6.88 / 6.63, 576 x 4000 54.4 / 54.1; d64 576 x 330 7.89 / 7.64.  With
+// more keys the K/V reads of the additional workgroups cost more than that: B1 H4 6000 x 10521 136 / 138.
+static bool third_less_rows(const AttnParams& p) {
+  return p.list == nullptr && p.Lk <= 4096 && (int64_t)p.B * p.H * ((p.Lq + 95) / 96) <= device_cus();
+}
+
 // Pairs of waves (see attn_item) with four fetch waves, where 64-row workgroups of them have a compute unit each.  128-row
 // workgroups with four fetch waves / 64-row ones of pairs, B2 H16 d128: 36 x 85 5.82 / 5.53 us, 64 x 149 6.73 / 6.10, 144 x 265
 // 8.89 / 7.38, 256 x 521 12.1 / 9.86, 400 x 921 17.1 / 13.8, 256 x 1497 23.9 / 19.0; B1 H4 4096 x 10521 133 / 117; d64 B1 H16
@@ -1407,6 +1415,7 @@ static int launch_one(const AttnParams& p0, hipStream_t stream) {
   }
   if constexpr (MODE == MODE_BLOCK && !LSE_ONLY && NWAVES == 4 && D <= 128) {
     if (wide_tiles(p0, D)) return launch_one<D, 8, MODE_BLOCK, false, false>(p0, stream);
+    if (third_less_rows(p)) return launch_one<D, 7, MODE_BLOCK, false, false, 4>(p0, stream);
     if (fetch_waves(p.total_wg)) return launch_one<D, 8, MODE_BLOCK, false, false, 4>(p0, stream);
   }
   const int rest = p.Lq % WGROWS;

@@ -56,6 +56,19 @@ def test_token_lists_give_the_bits_of_larger_launches(Lq, Lk, keys, d, growth):
         assert torch.equal(o1, o[:, h])
 
 
+# dense launches in 96-row workgroups: more 64-row ones than compute units, but not more 96-row ones
+@pytest.mark.parametrize("d", [64, 128])
+@pytest.mark.parametrize("Lq,Lk", [(65, 64), (96, 130), (97, 700), (190, 321)])
+def test_96_row_workgroups_give_the_bits_of_larger_launches(Lq, Lk, d):
+    from lvar_amd import sparse_attn_ops as ops
+    cus = torch.cuda.get_device_properties(0).multi_processor_count
+    q, k, v = _inputs(2 * cus + 3, Lq, Lk, d, seed=Lq, growth=0.7)
+    o, (M, L) = ops.dense_attn(q, k, v)
+    h = slice(5, 5 + cus // -(-Lq // 96))
+    o1, (M1, L1) = ops.dense_attn(*(t[:, h].contiguous() for t in (q, k, v)))
+    assert torch.equal(o1, o[:, h]) and torch.equal(M1, M[:, h]) and torch.equal(L1, L[:, h])
+
+
 @pytest.mark.parametrize("d", [64, 128, 256])
 @pytest.mark.parametrize("growth", [0.0, 0.7])
 def test_pairs_against_float64(growth, d):
