@@ -73,8 +73,8 @@ struct Swz {
   __device__ static __forceinline__ int fv(int row) { return (D >= 128) ? ((row & 3) << 2) : (((row >> 1) & 1) << 2); }
 };
 
-// Token-list instances whose list readers know two rows (AttnParams::remap_gs): 192-row groups in one workgroup of eight waves,
-// or at head_dim 64 in two of three.  The others would pay the choice of a row per entry for nothing.
+// Token-list instances whose list readers know two rows (AttnParams::remap_gs): 192-row groups in workgroups with fetch waves, or
+// at head_dim 64 in two of three waves.  The others would pay the choice of a row per entry for nothing.
 template <int D, int NWAVES, int MODE, int NPROD>
 constexpr bool reads_remapped = MODE == MODE_GATHER && (NPROD > 0 || (D == 64 && NWAVES == 3));
 
