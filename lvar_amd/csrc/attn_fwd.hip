@@ -117,7 +117,7 @@ __device__ __forceinline__ float rounded(float x) {
 // half * D/2 .. of O over all 64 keys: half of the MFMAs and of the vector work each (1400 cycles).  P and the row maxima pass
 // between the two through LDS behind the barrier that a tile has anyway: O is one tile behind S, so nothing in an iteration waits
 // for anything else in it.  The order of every sum is the same as without: same bits.
-template <int D, int NWAVES, int MODE, bool ACCUM, bool LSE_ONLY, bool SK, int NPROD, bool IDLE, bool PAIR = false>
+template <int D, int NWAVES, int MODE, bool ACCUM, bool LSE_ONLY, bool SK, int NPROD, bool IDLE, bool PAIR = false, bool THIRD = false>
 __device__ __forceinline__ void attn_item(const AttnParams& p, char* smem, const int w, const int bh, const int qt,
                                           const int u0, const int u1, const bool whole, const SkCtx& sk) {
   // NPROD: the last waves only fetch -- they read the list, form the addresses and issue every K/V fill -- and the
@@ -757,14 +757,23 @@ __device__ __forceinline__ void attn_item(const AttnParams& p, char* smem, const
       constexpr int NQK_ = 2 * KS;
       constexpr int NFILL = NPROD ? 0 : (LSE_ONLY ? SLOTS : 2 * SLOTS);
       constexpr int FSTRIDE = (CONST_OFF && NFILL > 0 && NFILL <= NQK_) ? NQK_ / NFILL : 0;
-      const int left = __builtin_amdgcn_readfirstlane(T - t);   // tiles from this one on; K(t+2) is only fetched where there is one
+      // K(t+2) is only fetched if there is one.  The skip is inside the fill (see issue_slot) where fills are spread over the steps, but
+      // not in the instance of three workgroups per compute unit: its third wave covers a branch, its registers are limited, and the
+      // assembly's operands had 21 of them spilled (B3 H24 1024 x 1100 36.2 us, 33.6 with the branch; 10 % of 128 x 128 blocks at
+      // 4096 x 10521 48.0, 43.9).  Fills in one burst up front (token lists) keep the branch, too, on T itself: on a copy of it in a
+      // scalar register the 64-row groups of head_dim 128 spilled 69 registers, now 21 (4096 x 10521, 832 keys 210 / 137 us; 96-row
+      // groups 154 / 117).
+      constexpr bool SKIP_IN_FILL = FSTRIDE > 0 && !THIRD;
+      const int left = SKIP_IN_FILL ? __builtin_amdgcn_readfirstlane(T - t) : 0;   // tiles from this one on
+      const bool fill_k = t + 2 < T;
       auto fill_step = [&](auto jc) {
         constexpr int j = decltype(jc)::value;
         if constexpr (FSTRIDE > 0) {
           if constexpr (j % FSTRIDE == 0 && j / FSTRIDE < NFILL) {
             constexpr int f = j / FSTRIDE;
             if constexpr (!LSE_ONLY && f < SLOTS) issue_slot(vrsrc, v_srb, true, rows_v, lds0 + (3 - PAR) * TILE, f, std::true_type{});
-            else issue_slot(krsrc, k_srb, false, rows_k, lds0 + PAR * TILE, LSE_ONLY ? f : f - SLOTS, left);
+            else if constexpr (SKIP_IN_FILL) issue_slot(krsrc, k_srb, false, rows_k, lds0 + PAR * TILE, LSE_ONLY ? f : f - SLOTS, left);
+            else if (fill_k) issue_slot(krsrc, k_srb, false, rows_k, lds0 + PAR * TILE, LSE_ONLY ? f : f - SLOTS, std::true_type{});
           }
         }
       };
@@ -773,7 +782,7 @@ __device__ __forceinline__ void attn_item(const AttnParams& p, char* smem, const
       } else {
         if constexpr (!NPROD && FSTRIDE == 0) {
           if (!LSE_ONLY) issue(vrsrc, v_srb, true, rows_v, lds0 + (3 - PAR) * TILE);
-          if (left > 2) issue(krsrc, k_srb, false, rows_k, lds0 + PAR * TILE);
+          if (fill_k) issue(krsrc, k_srb, false, rows_k, lds0 + PAR * TILE);
         }
         if (t + 3 < T) finish_rows(t + 3, raw, rows_n, nv3);
         if (t + 4 < T) prefetch_raw(t + 4, raw);
@@ -1162,7 +1171,7 @@ __global__ __launch_bounds__(NWAVES * 64, ((NWAVES <= 4 && D <= 128) ? (THIRD ? 
     if (p.round_places > 0 && qt < p.order.nqt && ranked_slice(p.order, bh, p.round_places)) qt = tile_by_length<NWAVES * 32>(p, bh, qt, p.order.nqt);
   }
   asm volatile("" : "+v"(bh), "+v"(qt));
-  attn_item<D, NWAVES, MODE, ACCUM, LSE_ONLY, false, NPROD, IDLE, PAIR>(p, smem, 0, bh, qt, 0, 0, true, SkCtx{});
+  attn_item<D, NWAVES, MODE, ACCUM, LSE_ONLY, false, NPROD, IDLE, PAIR, THIRD>(p, smem, 0, bh, qt, 0, 0, true, SkCtx{});
 #endif
 }
 
