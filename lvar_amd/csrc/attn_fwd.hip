@@ -807,6 +807,12 @@ __device__ __forceinline__ void attn_item(const AttnParams& p, char* smem, const
       bf16x8 frag[NQK > NPV ? NQK : NPV];
       uint32_t pw[16];
       const float negm = -m_ref;
+      // A half's sum joins the row sum as soon as it is complete: held to the end of the tile, the two cost a register more while the
+      // V fragments and P need theirs (64- and 96-row token-list groups at head_dim 128 spill 14 and 0 registers, not 21 and 19:
+      // 4096 x 10521, 832 keys 137 / 133 and 117 / 95 us; the statistics at head_dim 64 keep to 128, four waves per SIMD: 4096 x 10521
+      // 266 / 260).  Where registers are to spare the chain of additions is better split: the other instances of head_dim 64 lose 1 %
+      // of their lists' time with it, the statistics at head_dim 256 1.5 %.
+      constexpr bool SUM_EARLY = LSE_ONLY ? D < 256 : D > 64 || THIRD;
       float la = 0.f, lb = 0.f;
       // The softmax of S(t) runs as a three-stage pipeline over the MFMA steps so that no vector instruction
       // waits for the one before it: step g scales the elements of slot g, takes exp2 of slot g-1 and
@@ -826,6 +832,8 @@ __device__ __forceinline__ void attn_item(const AttnParams& p, char* smem, const
         float r;
         if constexpr (e < 16) r = c0[e]; else r = c1[e - 16];
         if constexpr (e < 16) la += r; else lb += r;
+        if constexpr (SUM_EARLY && e == 15) lsum[0] += la;
+        if constexpr (SUM_EARLY && e == 31) lsum[1] += lb;
         if constexpr (e & 1) {
           float prev;
           if constexpr (e < 16) prev = c0[e - 1]; else prev = c1[e - 17];
@@ -886,8 +894,10 @@ __device__ __forceinline__ void attn_item(const AttnParams& p, char* smem, const
 #pragma unroll
         for (int e = 0; e < 16; e++) ma = fmaxf(fmaxf(ma, n0[e]), n1[e]);
       }
-      lsum[0] += la;
-      lsum[1] += lb;
+      if constexpr (!SUM_EARLY) {
+        lsum[0] += la;
+        lsum[1] += lb;
+      }
       const float mx = xhalf_max(fmaxf(ma, mb));
       wait_fills<0>();
       __syncthreads();
