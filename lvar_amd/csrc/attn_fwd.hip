@@ -1178,7 +1178,8 @@ __global__ __launch_bounds__(NWAVES * 64, ((NWAVES <= 4 && D <= 128) ? (THIRD ? 
   int bh, qt;
   if (!tile_of(p.order, __builtin_amdgcn_workgroup_id_x(), bh, qt)) return;
   if constexpr (ranks_tiles<D, NWAVES, MODE, LSE_ONLY>) {
-    if (p.round_places > 0 && qt < p.order.nqt && ranked_slice(p.order, bh, p.round_places)) qt = tile_by_length<NWAVES * 32>(p, bh, qt, p.order.nqt);
+    const int x = __builtin_amdgcn_workgroup_id_x() % TILE_XCDS;
+    if (p.last_round > 0 && qt < p.order.nqt && ranked_slice(p.order, bh, x, p.last_round)) qt = tile_by_length<NWAVES * 32>(p, bh, qt, p.order.nqt);
   }
   asm volatile("" : "+v"(bh), "+v"(qt));
   attn_item<D, NWAVES, MODE, ACCUM, LSE_ONLY, false, NPROD, IDLE, PAIR, THIRD>(p, smem, 0, bh, qt, 0, 0, true, SkCtx{});
@@ -1442,7 +1443,7 @@ static int launch_one(const AttnParams& p0, hipStream_t stream) {
                                           : p.list != nullptr && ragged_lists_last(p.B * p.H, p.nqt, rest, device_cus());
   p.order = tile_order(p.B * p.H, p.nqt, ragged);
   const int grid = TILE_XCDS * p.order.per_xcd;
-  if constexpr (ranks_tiles<D, NWAVES, MODE, LSE_ONLY>) p.round_places = lists_by_length(p) ? device_cus() / TILE_XCDS * 2 : 0;
+  if constexpr (ranks_tiles<D, NWAVES, MODE, LSE_ONLY>) p.last_round = lists_by_length(p) ? short_last_round(p.order, device_cus() / TILE_XCDS * 2) : 0;
   if constexpr (D == 64 && NWAVES == 4 && MODE == MODE_BLOCK && !LSE_ONLY) {
     if (third_workgroup(p.total_wg)) {
       static_assert(SMEM <= 48 * 1024, "three workgroups share the LDS of a compute unit; no larger limit has to be asked for");

@@ -43,7 +43,7 @@ struct AttnParams {
   int remap_gs, remap_gk, remap_cnt, remap_len;
   int nqt, total_wg;
   TileOrder order;   // plain launch: which query tile a workgroup takes
-  int round_places;  // places of an XCD that run at once, where tiles are ranked by the lengths of their lists (0 = not ranked)
+  int last_round;    // where tiles are ranked by the lengths of their lists: place of an XCD at which the last round begins (0 = not ranked)
   // balanced launch: workspace handed in by the caller (null = plain launch).  The launch code fills in sk_wgs
   // (0 = plain launch after all), sk_counters (per-query-tile arrival counters, all zero between launches) and
   // sk_slots (2 * sk_wgs slots of partial results).

@@ -55,19 +55,28 @@ LVAR_HD bool tile_of(const TileOrder& t, unsigned id, int& slice, int& qt) {
   return i < t.per_xcd && slice < t.ragged;
 }
 
-// Whether the tiles of a slice run longest list first: slices that lie in one XCD and reach into a last round that is at most half
-// full, so that what starts late is short.  `round_places`: places of an XCD that run at once.  The others keep their order and pay
-// nothing; a ranked tile waits for the lengths of its slice's lists before its own list is read.  Natural order / longest first,
-// d128, 128-row tiles, two per compute unit: random lists B2 H16 48 x 48 (576 tiles on 512 places) at 25 % 81.6 / 75.5 us, at 10 %
-// 43.9 / 39.3, B1 H24 56 x 56 106.9 / 102.0; sink + window 48 x 48 58.1 / 55.6, B2 H12 56 x 56 106.2 / 104.7; best-scoring blocks,
-// nearly or exactly of one length, 48 x 48 25 % 74.3 / 73.7, 10 % 64.8 / 63.8, B1 H24 56 x 56 120.4 / 117.9, B2 H20 44 x 44 81.5 / 82.0.
+// The place of an XCD at which a last round of at most half of its places begins, or 0 where a launch ends otherwise.  `round_places`:
+// places of an XCD that run at once.
+LVAR_HD int short_last_round(const TileOrder& t, int round_places) {
+  if (round_places <= 0) return 0;
+  const int full = t.per_xcd / round_places * round_places;   // places before the last round
+  return full < t.per_xcd && 2 * (t.per_xcd - full) <= round_places ? full : 0;
+}
+
+// Whether the tiles of a slice, one of which runs on XCD x, run longest list first: slices that lie in that XCD and reach from the
+// rounds before into a short last one (its place from short_last_round), so that what starts late is short.  The others keep their
+// order: a ranked tile waits for the lengths of its slice's lists before its own list is read, and where a whole slice starts in the
+// last round that wait is all that would come of it (ranked / not, B3 H24 900 x 2000 at 30 % 38.6 / 37.6 us, B1 H300 256 x 4000 at 10 %
+// 34.2 / 33.0).  Natural order / longest first, d128, 128-row tiles, two per compute unit: random lists B2 H16 48 x 48 (576 tiles on
+// 512 places) at 25 % 80.7 / 74.6 us, at 10 % 43.1 / 39.0, B2 H20 44 x 44 78.7 / 78.4 and 45.1 / 41.5; sink + window 48 x 48 57.7 / 55.3,
+// B2 H12 56 x 56 82.9 / 81.7; best-scoring blocks, nearly of one length, 48 x 48 25 % 72.6 / 72.7, 10 % 64.2 / 63.3; lists of exactly
+// one length lose the wait, 0.3 us.  With ragged tiles behind the whole ones it is the draw: B1 H24 56 x 56 115.0 / 118.4 and 56.4 /
+// 56.3, lists of a few entries (48 heads 1600 x 4121, 5 % of the 128-key blocks, eight draws) -5 .. +8 %.
 // With the last round 46 / 64 full random lists lose 1.8 %.  head_dim 64 loses 1 % (a third workgroup per compute unit covers the
 // end), 64-row tiles gain nothing.
-LVAR_HD bool ranked_slice(const TileOrder& t, int slice, int round_places) {
-  const int full = t.per_xcd / round_places * round_places;   // places before the last round
-  const int first = slice * t.nqt, last = first + t.nqt - 1, x = first / t.whole_per_xcd;
-  return full > 0 && full < t.per_xcd && 2 * (t.per_xcd - full) <= round_places && x == last / t.whole_per_xcd &&
-         last - x * t.whole_per_xcd >= full;
+LVAR_HD bool ranked_slice(const TileOrder& t, int slice, int x, int last_round) {
+  const int first = slice * t.nqt - x * t.whole_per_xcd, last = first + t.nqt - 1;   // places on XCD x
+  return first >= 0 && first < last_round && last >= last_round && last < t.whole_per_xcd;
 }
 
 // Whether the ragged last tiles of token lists with fetch-only waves (one workgroup per compute unit) run behind the whole

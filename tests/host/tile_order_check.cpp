@@ -3,7 +3,8 @@
 //   * no XCD gets more tiles than an even split gives the fullest one,
 //   * on every XCD the ragged last tiles come behind the whole ones, and the whole ones are a contiguous range,
 //   * the rules that take ragged tiles out of the order, on both sides of each of their bounds,
-//   * the rule that takes the instance with idle waves, likewise.
+//   * the rule that takes the instance with idle waves, likewise,
+//   * the rule that orders tiles by the lengths of their lists, likewise; a slice's workgroups agree on it.
 // Prints "ok <cases>" or the first violation.
 #include <cstdio>
 #include <vector>
@@ -14,7 +15,8 @@ using namespace lvar;
 static const char* check(int slices, int nqt, bool ragged) {
   const TileOrder t = tile_order(slices, nqt, ragged);
   const int tiles = slices * nqt;
-  std::vector<int> taken(tiles, 0);
+  std::vector<int> taken(tiles, 0), ranked(slices, -1);
+  const int last_round = short_last_round(t, 64);
   for (int x = 0; x < TILE_XCDS; x++) {
     int here = 0, last = -1;
     bool behind = false;
@@ -24,6 +26,11 @@ static const char* check(int slices, int nqt, bool ragged) {
       if (s < 0 || s >= slices || q < 0 || q >= nqt) return "tile out of range";
       taken[s * nqt + q]++;
       here++;
+      if (q < t.nqt && last_round > 0) {
+        const int r = ranked_slice(t, s, x, last_round);
+        if (ranked[s] >= 0 && ranked[s] != r) return "workgroups of a slice that do not agree on its order";
+        ranked[s] = r;
+      }
       if (ragged && q == nqt - 1) { behind = true; continue; }
       if (behind) return "whole tile behind a ragged one";
       const int w = s * t.nqt + q;
@@ -73,6 +80,26 @@ int main() {
   for (auto& r : idle) {
     cases++;
     if (idle_waves_pay(r.waves, r.nqt, r.rest) != r.pay) { printf("idle waves of %d in %d tiles per head, rest %d\n", r.waves, r.nqt, r.rest); return 1; }
+  }
+  // longest list first (64 places of an XCD at once): slices that reach from the rounds before into a last one of at most half of them
+  struct { int slices, nqt; bool ragged; int slice, x, last_round; bool ranked; } len[] = {
+      {32, 18, false, 3, 0, 64, true}, {32, 18, false, 2, 0, 64, false},      // places 54 .. 71 and 36 .. 53 of 72
+      {32, 18, false, 31, 7, 64, true}, {32, 18, false, 30, 7, 64, false},
+      {72, 8, false, 8, 0, 64, false}, {72, 8, false, 7, 0, 64, false},       // 64 .. 71, wholly inside the last round; 56 .. 63, up to it
+      {40, 15, false, 4, 0, 64, true}, {40, 15, false, 3, 0, 64, false},      // 60 .. 74 of 75
+      {20, 27, false, 2, 0, 64, false},                                       // 54 .. 80 of 68: across two XCDs
+      {20, 27, false, 2, 1, 64, false}, {8, 64, false, 0, 0, 0, false},       // (seen from the other one; whole rounds)
+      {32, 24, false, 2, 0, 64, true}, {32, 25, false, 2, 0, 0, false},       // last round of 32 places, of 36
+      {32, 16, false, 0, 0, 0, false}, {24, 8, false, 2, 0, 0, false},        // no round before, whole rounds
+      {34, 17, true, 4, 0, 64, false}, {32, 19, true, 3, 0, 64, true}};       // ragged tiles behind: 64 .. 79 of 68 whole, 54 .. 71 of 72
+  for (auto& r : len) {
+    cases++;
+    const TileOrder t = tile_order(r.slices, r.nqt, r.ragged);
+    const int last_round = short_last_round(t, 64);
+    if (last_round != r.last_round || (last_round > 0 && ranked_slice(t, r.slice, r.x, last_round)) != r.ranked) {
+      printf("slice %d of %d with %d tiles: last round %d, ranked %d\n", r.slice, r.slices, r.nqt, last_round, last_round > 0 && ranked_slice(t, r.slice, r.x, last_round));
+      return 1;
+    }
   }
   printf("ok %ld\n", cases);
   return 0;
