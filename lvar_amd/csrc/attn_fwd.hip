@@ -26,6 +26,7 @@
 #include <type_traits>
 #include "common.h"
 #include "launch.h"
+#include "launch_forms.h"
 #include "sk_partition.h"
 
 namespace lvar {
@@ -1317,65 +1318,15 @@ __global__ __launch_bounds__(256) void plan_kernel(const AttnParams p, int* plan
   }
 }
 
-// 256 query rows per workgroup (eight waves on one pair of K/V buffers, one workgroup per compute
-// unit): half the L2->LDS fills per flop, 4 % faster than two 128-row workgroups side by side (B2 H16 d128: 4096 x 10521
-// 635 -> 608 us, 1600 x 4121 117 -> 113 us) unless the coarser tiles leave more of the last round idle.  In units of a
-// lone 128-row tile: a pair of 128-row workgroups takes 1.6 of it, a 256-row one 1.6 * 0.95; at head_dim 64 three small
-// workgroups share a compute unit and only launches of a single round gain.
-static bool wide_tiles(const AttnParams& p, int head_dim) {
-  if (p.list && p.group_rows % 256 != 0) return false;   // (lists of 256-row query blocks run the same way)
-  const int64_t bh = (int64_t)p.B * p.H, cus = device_cus();
-  if (cus <= 0) return false;
-  const int64_t n128 = bh * ((p.Lq + 127) / 128), n256 = bh * ((p.Lq + 255) / 256);
-  if (n128 <= cus) return false;
-  if (head_dim == 64) return n256 <= cus;
-  const int64_t full = n128 / (2 * cus), rest = n128 % (2 * cus);
-  const double narrow = 1.6 * full + (rest == 0 ? 0.0 : rest <= cus ? 1.0 : 1.6);
-  const double wide = 1.6 * 0.95 * ((n256 + cus - 1) / cus);
-  return wide < narrow;
-}
-
-// Three 128-row workgroups per compute unit at head_dim 64: 168 registers per wave instead of 180, two of them spilled.  Where
-// two per compute unit hold the launch the third slot stays empty and the spills cost 1 to 4 % (two against three: B8 H16
-// 256 x 680 12.4 / 12.9 us, B2 H16 2048 x 4121 in lists of 30 % 29.3 / 29.9 us); larger launches are up to 9 % faster (B2 H17
-// 2048 x 4121 115 / 105 us, B2 H16 2304 x 6425 177 / 164 us).  The 2-wave workgroups of 64-row query blocks are not (B2 H16
-// 4096 x 10521 in lists of 30 %: 149 / 162 us).
+// Three 128-row workgroups per compute unit at head_dim 64: 168 registers per wave instead of 174, two of them spilled.  Where
+// two per compute unit hold the launch the third slot stays empty and the spills cost 1 to 2 % (two against three, lists of 30 %:
+// B2 H12 1600 x 4121 30.8 / 31.4 us, B2 H16 2048 x 4121 35.0 / 35.3); larger launches are up to 10 % faster (B3 H24 1024 x 1100
+// 37.1 / 33.4 us, B2 H17 2048 x 4121 117 / 107, B2 H16 2304 x 6425 179 / 165, in lists of 25 % 49.4 / 45.6).  The 2-wave workgroups of
+// 64-row query blocks are not (B2 H16 4096 x 10521 in lists of 30 %: 149 / 162 us).
 static bool third_workgroup(int total_wg) { return total_wg > 2 * device_cus(); }
-
-// Fetch-only waves beside four computing ones.  A launch of at most one 128-row workgroup per compute unit leaves half of
-// the wave slots empty, and its lone waves pay for every instruction in full: 16 of the 100-odd that a wave issues per
-// tile beside its MFMAs are fills.  Without / with four fetch waves, B2 H16 d128: 144 x 265 9.8 / 9.0 us, 576 x 1497 27.3 /
-// 24.4, 1024 x 2521 (256 workgroups) 46.5 / 44.3; B1 H4 4096 x 10521 153 / 134; d64 B8 H16 256 x 680 12.2 / 11.4 (the smaller ones of
-// these are launches of pairs now); lists
-// alike (B1 H16 784 x 1924 at 25 % 20.6 / 18.4).  With a second workgroup on a compute unit there are no empty slots, and at
-// head_dim 256 a wave fills its SIMD.  Same bits.  A workgroup with fetch waves has its compute unit to itself, so launches
-// on two streams that together need more than one per compute unit no longer share any: a pair of calls, without / with,
-// B1 d128 1024 x 2521: 2 x 128 workgroups 49.1 / 45.0 us, 2 x 160 (576 x 1497) 56.8 / 52.3, 2 x 192 67.1 / 68.2, 2 x 224 72.7 / 78.9,
-// 2 x 256 78.9 / 88.0 (one stream 50.2 / 46.0); d64 2 x 256 49.0 / 59.0 (31.8 / 30.0).  A launch cannot know what runs beside it,
-// and one stream is the usual case.
-static bool fetch_waves(int total_wg) { return total_wg <= device_cus(); }
 
 // Lists whose lengths a wave can rank, one tile per lane.
 static bool lists_by_length(const AttnParams& p) { return p.list && p.order.nqt > 1 && p.order.nqt <= 64; }
-
-// 96 rows per workgroup, three computing and four fetch waves, for dense launches that leave compute units idle as 128-row
-// workgroups: a chain of tiles takes as long, with a quarter less operand reads and power per compute unit.  128 / 96 rows, B2 H16
-// d128: 576 x 1497 24.2 / 23.8 us, 576 x 660 13.8 / 13.6, 520 x 100 6.88 / 6.63, 576 x 4000 54.4 / 54.1; d64 576 x 330 7.89 / 7.64.  With
-// more keys the K/V reads of the additional workgroups cost more than that: B1 H4 6000 x 10521 136 / 138.
-static bool third_less_rows(const AttnParams& p) {
-  return p.list == nullptr && p.Lk <= 4096 && (int64_t)p.B * p.H * ((p.Lq + 95) / 96) <= device_cus();
-}
-
-// Pairs of waves (see attn_item) with four fetch waves, where 64-row workgroups of them have a compute unit each.  128-row
-// workgroups with four fetch waves / 64-row ones of pairs, B2 H16 d128: 36 x 85 5.82 / 5.53 us, 64 x 149 6.73 / 6.10, 144 x 265
-// 8.89 / 7.38, 256 x 521 12.1 / 9.86, 400 x 921 17.1 / 13.8, 256 x 1497 23.9 / 19.0; B1 H4 4096 x 10521 133 / 117; d64 B1 H16
-// 256 x 680 10.7 / 9.0; lists alike (B1 H8 576 x 1497 at 30 % 16.0 / 12.8, sink + window B1 H4 3025 x 9450 31.6 / 25.2); a single key tile
-// alike; head_dim 256, where the waves of 128-row workgroups fill their SIMDs and nothing only fetches: 16 x 21 7.12 / 5.54, 144 x 265
-// 15.1 / 10.9, 400 x 921 29.8 / 21.7, 512 x 1000 31.1 / 26.7, B1 H4 3000 x 9000 206 / 142.  Not beyond: pairs that share their SIMDs take twice as long (96-row workgroups of three pairs, 576 x 1497 24.3 /
-// 25.8, 6000 x 10521 136 / 165; 128-row ones 24.4 / 29.6).  Two streams with such a launch each, B1 d128: 2 x 8 heads 576 x 1497
-// 23.7 / 23.1, 2 x 16 heads 25.3 / 24.7, 2 x 8 heads 1024 x 2521 72.7 / 55.5, but 2 x 16 heads, which fill the chip together as 128-row
-// workgroups, 51.2 / 64.9 (one stream 40.5 / 33.0).
-static bool pairs_of_waves(const AttnParams& p) { return (int64_t)p.B * p.H * ((p.Lq + 63) / 64) <= device_cus(); }
 
 template <int D, int NWAVES, int MODE, bool ACCUM, bool LSE_ONLY, int NPROD = (MODE == MODE_GATHER && NWAVES == 8) ? 2 : 0, bool PAIR = false>
 static int launch_one(const AttnParams& p0, hipStream_t stream) {
@@ -1431,12 +1382,13 @@ static int launch_one(const AttnParams& p0, hipStream_t stream) {
     }
   }
   if constexpr (MODE == MODE_BLOCK && !LSE_ONLY && NWAVES == 4) {
-    if (pairs_of_waves(p)) return launch_one<D, 8, MODE_BLOCK, false, false, 4, true>(p0, stream);
-  }
-  if constexpr (MODE == MODE_BLOCK && !LSE_ONLY && NWAVES == 4 && D <= 128) {
-    if (wide_tiles(p0, D)) return launch_one<D, 8, MODE_BLOCK, false, false>(p0, stream);
-    if (third_less_rows(p)) return launch_one<D, 7, MODE_BLOCK, false, false, 4>(p0, stream);
-    if (fetch_waves(p.total_wg)) return launch_one<D, 8, MODE_BLOCK, false, false, 4>(p0, stream);
+    const BlockForm form = block_form((int64_t)p.B * p.H, p.Lq, p.Lk, D, p.list != nullptr, p.group_rows, device_cus());
+    if (form == BlockForm::PAIRS) return launch_one<D, 8, MODE_BLOCK, false, false, 4, true>(p0, stream);
+    if constexpr (D <= 128) {
+      if (form == BlockForm::WIDE) return launch_one<D, 8, MODE_BLOCK, false, false>(p0, stream);
+      if (form == BlockForm::ROWS_96) return launch_one<D, 7, MODE_BLOCK, false, false, 4>(p0, stream);
+      if (form == BlockForm::FETCH) return launch_one<D, 8, MODE_BLOCK, false, false, 4>(p0, stream);
+    }
   }
   const int rest = p.Lq % WGROWS;
   const bool ragged = MODE == MODE_GATHER ? NPROD > 0 && ragged_runs_last(p.B * p.H, p.nqt, rest, WGROWS, device_cus())
@@ -1468,25 +1420,6 @@ static int launch_one(const AttnParams& p0, hipStream_t stream) {
   return hipGetLastError() == hipSuccess ? LVAR_OK : LVAR_ELAUNCH;
 }
 
-// 192-row groups of token lists that leave compute units idle.  A group's six computing waves share four SIMDs, and the two SIMDs
-// with two of them set its time.  As 64-row workgroups of pairs (pairs_of_waves), or as 96-row ones of three computing and four
-// fetch waves, a computing wave has its SIMD to itself; either where every workgroup has a compute unit.  192 rows / 64 rows of
-// pairs, d128 last step with 20 % of the keys, the whole step: B1 H4 64 x 64 49.3 / 32.4 us, B1 H8 40 x 40 32.0 / 18.2, B2 H4 33 x 33 at
-// 5 % 22.5 / 12.5, d64 B1 H4 64 x 64 32.6 / 19.8.  192 / 96 rows: B1 H16 36 x 36 at 10 % 30.4 / 22.6, B1 H8 50 x 50 at 30 % 48.1 /
-// 35.4, d64 18.8 / 15.4 and 31.1 / 23.7.
-static bool half_groups(const AttnParams& p) { return (int64_t)p.B * p.H * ((p.Lq + 95) / 96) <= device_cus(); }
-
-// Token lists at head_dim 64: 192-row groups as two 3-wave workgroups (several share a compute unit, each fetches for
-// itself) instead of one of 8 waves, with the same bits, where the 8-wave workgroups leave their last round at most half
-// full.  832 / 2560 keys per list, 8-wave against 3-wave: 96 groups 18.9 / 43.2 against 16.3 / 37.7 us, 384 groups 36.2 /
-// 84.3 against 32.7 / 79.2 us; full rounds the other way (256 groups 20.7 / 44.9 against 23.2 / 52.1 us, 704 groups 53.3 /
-// 127 against 56.2 / 140 us).  From the fourth round on the choice is within a few percent and stays.  (At head_dim 128 the
-// 3-wave form wins only on nearly empty launches: 16 groups 25.1 against 23.2 us, 96 groups 27.1 against 27.9 us.)
-static bool three_wave_groups(const AttnParams& p) {
-  const int64_t n = (int64_t)p.B * p.H * ((p.Lq + 191) / 192), cus = device_cus();
-  return cus > 0 && p.group_rows % 192 == 0 && n < 3 * cus && n % cus != 0 && 2 * (n % cus) <= cus;
-}
-
 template <int D>
 static int launch_d(const AttnParams& p, int mode, bool accum, bool lse_only, int nwaves, hipStream_t s) {
   if (mode == MODE_BLOCK) {
@@ -1495,11 +1428,15 @@ static int launch_d(const AttnParams& p, int mode, bool accum, bool lse_only, in
     return lse_only ? launch_one<D, 4, MODE_BLOCK, false, true>(p, s) : launch_one<D, 4, MODE_BLOCK, false, false>(p, s);
   } else if (mode == MODE_GATHER) {
     // (head_dim 256: a wave needs more than 256 registers, so one wave per SIMD: 192-row groups run as two 3-wave workgroups)
-    if constexpr (D > 128) { if (nwaves == 8) nwaves = 3; }
-    else if (nwaves == 8 && !p.sk_ws && pairs_of_waves(p)) return launch_one<D, 8, MODE_GATHER, true, false, 4, true>(p, s);
-    else if (nwaves == 8 && !p.sk_ws && half_groups(p)) return launch_one<D, 7, MODE_GATHER, true, false, 4>(p, s);
-    else if (D == 64 && nwaves == 8 && !p.sk_ws && three_wave_groups(p)) return launch_one<D, 3, MODE_GATHER, true, false>(p, s);
-    else if (nwaves == 8) return launch_one<D, 8, MODE_GATHER, true, false>(p, s);
+    if constexpr (D > 128) {
+      if (nwaves == 8) nwaves = 3;
+    } else if (nwaves == 8) {
+      const TokenForm form = p.sk_ws ? TokenForm::PLAIN : token_form((int64_t)p.B * p.H, p.Lq, D, device_cus());
+      if (form == TokenForm::PAIRS) return launch_one<D, 8, MODE_GATHER, true, false, 4, true>(p, s);
+      if (form == TokenForm::HALF_GROUPS) return launch_one<D, 7, MODE_GATHER, true, false, 4>(p, s);
+      if constexpr (D == 64) if (form == TokenForm::THREE_WAVES) return launch_one<D, 3, MODE_GATHER, true, false>(p, s);
+      return launch_one<D, 8, MODE_GATHER, true, false>(p, s);
+    }
     if (nwaves == 3) return launch_one<D, 3, MODE_GATHER, true, false>(p, s);
     if (nwaves == 2) return launch_one<D, 2, MODE_GATHER, true, false>(p, s);
   }

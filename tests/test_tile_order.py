@@ -18,3 +18,15 @@ def test_every_tile_once_and_no_xcd_over_its_share(tmp_path):
                    check=True, timeout=300)
     out = subprocess.run([exe], capture_output=True, text=True, timeout=300)
     assert out.returncode == 0 and out.stdout.startswith("ok "), out.stdout + out.stderr
+
+
+def test_form_of_a_launch_on_both_sides_of_every_bound(tmp_path):
+    """lvar_amd/csrc/launch_forms.h: the rules that the launch code takes its form of workgroup from."""
+    cxx = shutil.which("g++")
+    if cxx is None:
+        pytest.skip("g++ not available")
+    exe = str(tmp_path / "launch_forms_check")
+    subprocess.run([cxx, "-O2", "-std=c++17", os.path.join(ROOT, "tests", "host", "launch_forms_check.cpp"), "-o", exe],
+                   check=True, timeout=300)
+    out = subprocess.run([exe], capture_output=True, text=True, timeout=300)
+    assert out.returncode == 0 and out.stdout.startswith("ok "), out.stdout + out.stderr
