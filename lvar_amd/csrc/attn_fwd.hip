@@ -599,9 +599,9 @@ __device__ __forceinline__ void attn_item(const AttnParams& p, char* smem, const
       // Iteration t: the matrix cores run S(t+1) = K(t+1) Q^T (this wave's keys; hasqk) and O += P(t-1) V(t-1) (its columns; haspv)
       // while the vector ALU turns S(t) into P(t); K(t+1) is in K buffer 1 - PAR, V(t-1) in V buffer 1 - PAR.
       auto half_tile = [&](int t, auto par, auto masked, auto hasqk, auto haspv, f32x16& cs, f32x16& ns) {
-        constexpr int PAR = decltype(par)::value;
+        const int PAR = par;
         constexpr bool MASKED = decltype(masked)::value, QK = decltype(hasqk)::value, PV = decltype(haspv)::value;
-        constexpr int NQK = QK ? KS : 0, NPV = PV ? 4 * MTW : 0, NS = NQK + NPV, AHEAD = D == 256 ? 3 : READ_AHEAD, PAHEAD = D == 256 ? 2 : 3;
+        constexpr int NQK = QK ? KS : 0, NPV = PV ? 4 * MTW : 0, NS = NQK + NPV, AHEAD = READ_AHEAD, PAHEAD = 3;
         // the maximum is settled two MFMAs into the iteration: the other wave's arrives from LDS with the first fragments
         constexpr int CHK = NS >= 8 ? 2 : 0;
         using Sch = HalfSlots<(NS - CHK > 3 ? NS - CHK - 2 : 1)>;
@@ -613,9 +613,6 @@ __device__ __forceinline__ void attn_item(const AttnParams& p, char* smem, const
         }
         const char* kbuf = smem + (1 - PAR) * TILE;
         const char* vbuf = smem + (3 - PAR) * TILE;
-        // head_dim 256: the 16 offsets of the K fragments are formed per tile and a fragment less is read ahead, or 50 registers are
-        // spilled (400 x 921 29.4 us, 21.7 without)
-        if constexpr (D == 256) asm volatile("" : "+v"(kb_l));
         const float mother = xbuf[(PAR * NCOMP + mate) * 64 + lane];
         bf16x8 frag[NS > 0 ? NS : 1], pb[4];
         auto operand = [&](auto ic) {
@@ -703,20 +700,21 @@ __device__ __forceinline__ void attn_item(const AttnParams& p, char* smem, const
         if (nv1 < 64) half_tile(t, par, Yes{}, Yes{}, haspv, cs, ns);
         else half_tile(t, par, No{}, Yes{}, haspv, cs, ns);
       };
-      auto last = [&](auto par, auto haspv, f32x16& cs, f32x16& ns) {
-        constexpr int PAR = decltype(par)::value;
+      // The last tile, of either parity: as two instances behind a branch O was held twice, for the path not taken, too, and at
+      // head_dim 256 an even number of tiles spilled 36 registers on its way out (2 tiles 11.0 -> 8.3 us, 24 31.9 -> 28.2).
+      auto last = [&](int par, auto haspv, f32x16& cs, f32x16& ns) {
         half_tile(tiles - 1, par, No{}, No{}, haspv, cs, ns);
-        lsum[1] = xbuf[((1 - PAR) * NCOMP + mate) * 64 + lane];
+        lsum[1] = xbuf[((1 - par) * NCOMP + mate) * 64 + lane];
 #pragma unroll
         for (int kb = 0; kb < 4; kb++) {
-          const bf16x8 pq = *(const bf16x8*)(prow + PAR * PPAR + kb * 1024);
+          const bf16x8 pq = *(const bf16x8*)(prow + par * PPAR + kb * 1024);
 #pragma unroll
-          for (int m = 0; m < MTW; m++) oacc[m] = mfma32(vread(smem + (2 + PAR) * TILE, kb * MTW + m), pq, oacc[m]);
+          for (int m = 0; m < MTW; m++) oacc[m] = mfma32(vread(smem + (2 + par) * TILE, kb * MTW + m), pq, oacc[m]);
         }
         __syncthreads();
       };
       if (tiles == 1) {
-        last(P0{}, No{}, sa, sb);
+        last(0, No{}, sa, sb);
         break;
       }
       step(0, P0{}, No{}, sa, sb);
@@ -725,12 +723,9 @@ __device__ __forceinline__ void attn_item(const AttnParams& p, char* smem, const
         step(t, P1{}, Yes{}, sb, sa);
         step(t + 1, P0{}, Yes{}, sa, sb);
       }
-      if (t + 1 < tiles) {
-        step(t, P1{}, Yes{}, sb, sa);
-        last(P0{}, Yes{}, sa, sb);
-      } else {
-        last(P1{}, Yes{}, sb, sa);
-      }
+      if (t + 1 < tiles) step(t, P1{}, Yes{}, sb, sa);
+      else sa = sb;
+      last((tiles - 1) & 1, Yes{}, sa, sb);
       break;
     } else {
     f32x16 sa0, sa1, sb0, sb1;

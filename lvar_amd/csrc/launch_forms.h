@@ -11,9 +11,8 @@ inline int64_t workgroups(int64_t slices, int Lq, int rows) { return slices * ((
 // workgroups with four fetch waves / 64-row ones of pairs, B2 H16 d128: 36 x 85 5.82 / 5.53 us, 64 x 149 6.73 / 6.10, 144 x 265
 // 8.78 / 7.42, 256 x 521 11.9 / 9.87, 400 x 921 16.8 / 13.8, 256 x 1497 23.7 / 18.7; B1 H4 4096 x 10521 134 / 120; d64 B1 H16
 // 256 x 680 10.7 / 9.0; lists alike (B1 H8 576 x 1497 at 30 % 14.2 / 11.3, sink + window B1 H4 3025 x 9450 31.6 / 25.2); a single key
-// tile alike; head_dim 256, where the waves of 128-row workgroups fill their SIMDs and nothing only fetches: 16 x 21 7.2 / 6.7,
-// 144 x 265 15.1 / 10.9, 400 x 921 29.7 / 22.0, 512 x 1000 31.3 / 27.5, B1 H4 3000 x 9000 206 / 149; two key tiles of nearly as many
-// workgroups as compute units lose a little there (B1 H48 300 x 90 10.9 / 11.1).  Not beyond: pairs that share their SIMDs take twice
+// tile alike; head_dim 256, where the waves of 128-row workgroups fill their SIMDs and nothing only fetches: 16 x 21 6.9 / 5.0,
+// 144 x 265 15.1 / 10.2, 400 x 921 30.5 / 21.5, 512 x 1000 32.1 / 24.1, B1 H4 3000 x 9000 213 / 137.  Not beyond: pairs that share their SIMDs take twice
 // as long (96-row workgroups of three pairs, 576 x 1497 24.3 / 25.8, 6000 x 10521 136 / 165; 128-row ones 24.4 / 29.6).  Two streams
 // with such a launch each, B1 d128: 2 x 8 heads 576 x 1497 23.7 / 23.1, 2 x 16 heads 25.3 / 24.7, 2 x 8 heads 1024 x 2521 72.7 / 55.5,
 // but 2 x 16 heads, which fill the chip together as 128-row workgroups, 51.2 / 64.9 (one stream 40.5 / 33.0).

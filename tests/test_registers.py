@@ -66,7 +66,6 @@ MAY_SPILL = {
     ("attn_fwd_kernel", 128, 2, 2, 1, 0, 0, 0, 0, 0): 14,    # token lists of 64-row groups
     ("attn_fwd_balanced_kernel", 128, 3, 2, 1): 6,
     ("attn_fwd_kernel", 256, 2, 2, 1, 0, 0, 0, 0, 0): 4,
-    ("attn_fwd_kernel", 256, 8, 1, 0, 0, 4, 0, 0, 1): 36,    # pairs of waves: behind the key loop
 }
 
 
