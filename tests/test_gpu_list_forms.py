@@ -291,7 +291,7 @@ def test_sparse_steps_do_not_depend_on_the_host_path(B, d, strided, monkeypatch)
         assert torch.equal(a, b)
 
 
-# lists formed while they are read: one, two and three workgroups per group (head_dim 64 with few groups takes 3-wave ones),
+# lists formed while they are read: few groups, so 64-row workgroups of pairs of waves (the other forms: the test after this one);
 # either row empty or ending inside a tile, more and fewer groups than the lists come from
 @pytest.mark.parametrize("d", [64, 128])
 @pytest.mark.parametrize("side,Gs,bm", [(5, 1, 192), (14, 3, 192), (20, 9, 192), (28, 2, 384)])
@@ -316,3 +316,43 @@ def test_attention_over_remapped_rows_is_the_attention_over_the_written_lists(d,
     assert lib.lvar_csp_attn_remap_fwd(ops._view(q), ops._view(k), ops._view(v), ops._view(cache), src_side, side, ops._view(o),
                                        src.data_ptr(), Ks, Ks, Gs, count, loc, L, L, bm, B, H, Lq, Lk, d, 1.0, 0.125, s) == 0
     assert torch.equal(o, want)
+
+
+# the same in every form of workgroup that reads two rows, by the number of heads: pairs of waves, half groups, 192-row groups of six
+# computing and two fetch waves, and at head_dim 64 two 3-wave workgroups per group; the first heads against the form of few groups
+@pytest.mark.parametrize("d", [64, 128])
+@pytest.mark.parametrize("form", ["pairs", "half groups", "192 rows", "three waves"])
+@pytest.mark.parametrize("count,L", [(0, 70), (64, 0), (65, 63), (330, 130)])
+@pytest.mark.parametrize("side", [14, 20])
+def test_remapped_rows_in_every_form_of_workgroup(side, count, L, form, d):
+    from lvar_amd import _lib, sparse_attn_ops as ops
+    cus = torch.cuda.get_device_properties(0).multi_processor_count
+    lib, Lq, Lk, src_side, bm, Gs = _lib.load(), side * side, 700, 3, 192, 2
+    groups = -(-Lq // bm)
+    H = {"pairs": cus // -(-Lq // 64), "half groups": cus // -(-Lq // 96), "192 rows": cus // groups, "three waves": (cus + cus // 8) // groups + 1}[form]
+    q, k, v = _inputs(1, H, H, Lq, Lk, d, False, seed=side)
+    cache = _inputs(1, H, H, src_side * src_side, Lk, d, False, seed=1)[0]
+    Ks = count + 3
+    g = torch.Generator(device="cuda").manual_seed(count)
+    src = torch.randint(-2, Lk + 2, (1, H, Gs, Ks), generator=g, device="cuda", dtype=torch.int32)
+    local = torch.randint(0, Lk, (groups, L), generator=g, device="cuda")
+    loc = local.data_ptr() if L else None
+    s = torch.cuda.current_stream().cuda_stream
+
+    def attention(h, remapped):
+        qh, kh, vh, ch, sh = (t[:, :h].contiguous() for t in (q, k, v, cache, src))
+        o = torch.full_like(qh, 7.0)
+        if remapped:
+            assert lib.lvar_csp_attn_remap_fwd(ops._view(qh), ops._view(kh), ops._view(vh), ops._view(ch), src_side, side, ops._view(o),
+                                               sh.data_ptr(), Ks, Ks, Gs, count, loc, L, L, bm, 1, h, Lq, Lk, d, 1.0, 0.125, s) == 0
+            return o
+        lists = torch.empty((1, h, groups, count + L), dtype=torch.int32, device="cuda")
+        counts = torch.empty((1, h, groups), dtype=torch.int32, device="cuda")
+        assert lib.lvar_remap_concat_lists(sh.data_ptr(), Ks, Ks, loc, L, L, lists.data_ptr(), count + L, counts.data_ptr(), h, Gs, groups, count, Lk, 0, s) == 0
+        assert lib.lvar_csp_attn_upsample_fwd(ops._view(qh), ops._view(kh), ops._view(vh), ops._view(ch), src_side, side, ops._view(o), None, None,
+                                              lists.data_ptr(), counts.data_ptr(), groups, count + L, bm, 1, h, Lq, Lk, d, 1.0, 0.125, s) == 0
+        return o
+
+    o = attention(H, True)
+    assert torch.equal(o, attention(H, False))
+    assert torch.equal(o[:, :3], attention(3, True))

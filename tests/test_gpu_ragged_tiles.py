@@ -22,7 +22,7 @@ def _close(o, ref):
 @pytest.mark.parametrize("Lq,Lk", [(1, 1), (32, 64), (33, 65), (128, 128), (129, 192), (160, 193), (250, 257), (300, 330)])
 def test_few_query_tiles(Lq, Lk, d):
     from lvar_amd import sparse_attn_ops as ops
-    H = 270                                                     # more query tiles than compute units: no fetch-only waves
+    H = 270                                                     # more query tiles than compute units: no fetch-only waves; `part`: pairs of waves
     (q, k, v), g = _rand(1, H, Lq, Lk, d, seed=Lq + d)
     qg, kg, vg = q.cuda(), k.cuda(), v.cuda()
     h = slice(H - 3, H)
@@ -41,6 +41,30 @@ def test_few_query_tiles(Lq, Lk, d):
         assert torch.equal(o, ob[:, h]) and torch.equal(M, Mb[:, h]) and torch.equal(L, Lb[:, h])
         o_ref, _, _ = oracle.block_sparse_attn(q[:, h], k[:, h], v[:, h], num[:, h], idx[:, h], 128, bk)
         assert _close(o, o_ref)
+
+
+# 128-row workgroups of four computing and four fetch waves, where 64-row ones (dense: and 96-row ones) are more than the compute
+# units: every count of key tiles around the depth of the pipeline, waves without rows and empty lists, against a larger launch
+@pytest.mark.parametrize("d", [64, 128])
+@pytest.mark.parametrize("Lk", [1, 64, 65, 128, 190, 257, 320])
+@pytest.mark.parametrize("tiles,Lq,dense", [(1, 97, True), (1, 128, True), (2, 193, True), (2, 250, True), (1, 65, False), (1, 96, False), (2, 129, False), (2, 225, False)])
+def test_four_computing_and_four_fetch_waves(tiles, Lq, dense, Lk, d):
+    from lvar_amd import sparse_attn_ops as ops
+    cus = torch.cuda.get_device_properties(0).multi_processor_count
+    H = cus // tiles
+    g = torch.Generator(device="cuda").manual_seed(Lq + Lk + d)
+    q, k, v = ((torch.randn(1, 2 * cus // tiles + 3, L, d, generator=g, device="cuda") * 0.5).to(torch.bfloat16) for L in (Lq, Lk, Lk))
+    part = [t[:, 1:H + 1].contiguous() for t in (q, k, v)]
+    if dense:
+        o, (M, L) = ops.dense_attn(q, k, v)
+        o1, (M1, L1) = ops.dense_attn(*part)
+    else:
+        num, idx = ops.mask_to_lists(torch.rand(1, q.shape[1], tiles, -(-Lk // 64), generator=g, device="cuda") < 0.6)
+        o, (M, L) = ops.block_sparse_attn(q, k, v, num, idx, 128, 64)
+        o1, (M1, L1) = ops.block_sparse_attn(*part, num[:, 1:H + 1].contiguous(), idx[:, 1:H + 1].contiguous(), 128, 64)
+    assert torch.equal(o1, o[:, 1:H + 1]) and torch.equal(M1, M[:, 1:H + 1]) and torch.equal(L1, L[:, 1:H + 1])
+    if dense:
+        assert _close(o1[:, :2], oracle.dense_attn(*(t[:, :2].cpu() for t in part))[0])
 
 
 # rows of the last query group / tile: one, a wave less one row, a wave, all but a wave; heads that do not divide by eight
@@ -74,7 +98,7 @@ def test_ragged_last_tile_of_256_rows(Lk):
     o, (M, L) = ops.dense_attn(qg, kg, vg)
     h = slice(H - 2, H)
     part = [t[:, h].contiguous() for t in (qg, kg, vg)]
-    o1, (M1, L1) = ops.dense_attn(*part)      # few tiles: 128-row workgroups with fetch-only waves
+    o1, (M1, L1) = ops.dense_attn(*part)      # few tiles: 64-row workgroups of pairs of waves
     assert torch.equal(o1, o[:, h]) and torch.equal(M1, M[:, h]) and torch.equal(L1, L[:, h])
     assert _close(o1, oracle.dense_attn(q[:, h], k[:, h], v[:, h])[0])
     mask = torch.rand(1, H, 4, -(-Lk // 64), generator=g) < 0.7          # lists of 256-row query blocks, some of them empty

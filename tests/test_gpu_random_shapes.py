@@ -166,9 +166,8 @@ def _csp_abi(q, k, v, idx, cnt, o0, group_rows, o_scale):
 
 @pytest.mark.parametrize("d", [64, 128, 256])
 def test_token_lists_every_workgroup_shape(d):
-    """Query groups of 192 rows run as 8-wave workgroups (six computing waves + two fetch waves; at head_dim 256 as
-    two 3-wave workgroups), other multiples
-    of 96 / 64 rows as 3- / 2-wave workgroups that fetch for themselves.  Each variant against the oracle at its
+    """Query groups of 192 rows run, so few, as three workgroups of pairs of waves (at head_dim 256 as two 3-wave workgroups),
+    other multiples of 96 / 64 rows as 3- / 2-wave workgroups that fetch for themselves.  Each variant against the oracle at its
     own group size, and, with every 192-row list repeated for its 96- / 64-row parts, bit for bit against each
     other: the arithmetic of a query row does not depend on the workgroup shape."""
     from lvar_amd import _lib
