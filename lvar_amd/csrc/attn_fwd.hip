@@ -4,7 +4,7 @@
 // Work decomposition
 //   workgroup  = NWAVES waves, 32 query rows per wave (small launches: per two waves, see PAIR), all share the K/V tiles in LDS
 //                (token lists with 192-row groups: 8 waves = 6 computing waves + 2 waves that only fetch, see NPROD; fewer rows
-//                and four fetch waves where that leaves no compute unit idle, see half_groups)
+//                and four fetch waves in small launches; launch_forms.h says which launch takes which form)
 //   wave       = S^T[64 keys x 32 queries] = K_tile . Q^T with 32x32x16 bf16 MFMA (K rows are
 //                the A operand read from LDS, Q^T is the B operand held in registers), so a
 //                lane owns ONE query column: the softmax row max / sum are in-register
@@ -807,8 +807,8 @@ __device__ __forceinline__ void attn_item(const AttnParams& p, char* smem, const
       // V fragments and P need theirs (64- and 96-row token-list groups at head_dim 128 spill 14 and 0 registers, not 21 and 19:
       // 4096 x 10521, 832 keys 137 / 133 and 117 / 95 us; the statistics at head_dim 64 keep to 128, four waves per SIMD: 4096 x 10521
       // 266 / 260).  Where registers are to spare the chain of additions is better split: the other instances of head_dim 64 lose 1 %
-      // of their lists' time with it, the statistics at head_dim 256 1.5 %.
-      constexpr bool SUM_EARLY = LSE_ONLY ? D < 256 : D > 64 || THIRD;
+      // of their lists' time with it, the statistics at head_dim 128 (up to 2 %, 130 x 147 5.37 / 5.50) and 256 1.5 %.
+      constexpr bool SUM_EARLY = LSE_ONLY ? D == 64 : D > 64 || THIRD;
       float la = 0.f, lb = 0.f;
       // The softmax of S(t) runs as a three-stage pipeline over the MFMA steps so that no vector instruction
       // waits for the one before it: step g scales the elements of slot g, takes exp2 of slot g-1 and
